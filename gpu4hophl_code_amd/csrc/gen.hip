@@ -114,6 +114,9 @@ struct Ctrl {
   // the running batch attempt (k_set_batch): the kernels take these instead
   // of their arguments' s0 / B / tag, so one captured batch replays for any
   uint32_t bs0, bB, btag;
+  uint32_t lm_on;                // the landmark test runs in this batch
+  unsigned long long lm_tested;  // candidates the landmark test looked at
+  unsigned long long lm_caught;  // of these, pruned by it
 };
 
 // A piece of a large frontier group: its cnt labels (at pool offset off)
@@ -191,6 +194,10 @@ struct GenArgs {
   uint32_t *gtile;
   unsigned long long gtile_cap;  // u32 words
   Ctrl *ctrl;
+  // landmark rows (k_lm_build), 16 << lm_lw bytes per vertex; nullptr: none
+  const uint4 *lm;
+  uint32_t lm_lw;     // log2 of a row's 16-byte chunks, one lane each
+  uint32_t lm_parts;  // chunks per hop (landmarks / 8)
 };
 
 __device__ inline Item *frontier(const GenArgs &a, uint32_t which) { return which ? a.F1 : a.F0; }
@@ -201,12 +208,14 @@ __device__ inline void with_batch(GenArgs &a) {
   a.s0 = __builtin_amdgcn_readfirstlane(a.ctrl->bs0);
   a.B = __builtin_amdgcn_readfirstlane(a.ctrl->bB);
   a.tag = __builtin_amdgcn_readfirstlane(a.ctrl->btag);
+  if (!__builtin_amdgcn_readfirstlane(a.ctrl->lm_on)) a.lm = nullptr;
 }
 
-__global__ void k_set_batch(Ctrl *c, uint32_t s0, uint32_t B, uint32_t tag) {
+__global__ void k_set_batch(Ctrl *c, uint32_t s0, uint32_t B, uint32_t tag, uint32_t lm_on) {
   c->bs0 = s0;
   c->bB = B;
   c->btag = tag;
+  c->lm_on = lm_on;
 }
 
 // Dense slot of (hub slot b, vertex y): the slots of a window of 2^slot_lw
@@ -680,9 +689,122 @@ __device__ inline bool rows_chosen(const GenArgs &a) {
                                 (uint64_t)cands * a.row_density >= (uint64_t)a.B * a.n));
 }
 
+// -------------------------------------------------------------- landmarks
+// The first hubs of the sequence (16 by default) are landmarks.  Row v holds,
+// for hop x = 1..K-1 and landmark i, the smallest distance of landmark i's
+// labels in L(v) of hop <= x (0xFFFF: none), 16 bits each, hop-major, 8
+// landmarks to a 16-byte chunk.  Rows are built once, when the batch that
+// holds the last landmark has finished; later hubs s rank below every
+// landmark, so a landmark's labels in L(s) and L(y) no longer change, and
+//   min over x, i of row(y)[x][i] + row(s)[h - x][i] <= d
+// is a witness for candidate (s, y, d) of round h: the prune would reject it.
+// Top-ranked hubs lie on most short walks, so this test rejects most of the
+// candidates a prune rejects (83 % on R-MAT scale 16, K = 5) from one
+// 128-byte line each, eight candidates per wave step, where the search takes a
+// wave and about four lines per candidate.  A candidate it does not catch
+// takes the search, so the labels are the same.  R-MAT scale 18, K = 5:
+// labels the prune reads 62.7 -> 40.8 billion, row items 133 -> 100 ms, list
+// items 19 -> 13 ms, the build 319 -> 284 ms (8 landmarks 286 ms, 24 289,
+// 32 287, 64 296: more lines per candidate than they save searches).
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+
+// smallest of the eight saturated 16-bit sums
+__device__ inline uint32_t lm_min_sum(uint4 x, uint4 y) {
+  auto sum = [](uint32_t p, uint32_t q) {
+    return __builtin_elementwise_add_sat(__builtin_bit_cast(us2, p), __builtin_bit_cast(us2, q));
+  };
+  const us2 m = __builtin_elementwise_min(
+      __builtin_elementwise_min(sum(x.x, y.x), sum(x.y, y.y)),
+      __builtin_elementwise_min(sum(x.z, y.z), sum(x.w, y.w)));
+  return min((uint32_t)m.x, (uint32_t)m.y);
+}
+
+// This lane's chunk of a row y in round h, and the chunk of a row s it adds
+// to (hop x with hop h - x); `use` is false for hops the round cannot pair.
+struct LmLane {
+  uint32_t mine, other;
+  bool use;
+};
+__device__ inline LmLane lm_lane(const GenArgs &a) {
+  const uint32_t c = (uint32_t)lane_id() & ((1u << a.lm_lw) - 1u);
+  const uint32_t x = c / a.lm_parts + 1, part = c % a.lm_parts;
+  LmLane l;
+  l.use = x < a.h;
+  l.mine = l.use ? c : 0u;
+  l.other = l.use ? (a.h - x - 1) * a.lm_parts + part : 0u;
+  return l;
+}
+
+// Lane i holds candidate (s, y, d), d = 0 for none (a sum is at least 2);
+// returns whether a landmark rejects it.  U: loads in flight per lane.
+template <int U>
+__device__ inline bool lm_caught(const GenArgs &a, uint32_t s, uint32_t y, uint32_t d) {
+  const uint32_t lane = (uint32_t)lane_id(), lw = a.lm_lw, per_lw = 6 - lw;
+  const uint32_t grp = lane >> lw;
+  const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
+  const LmLane l = lm_lane(a);
+  bool caught = false;
+  for (uint32_t s0 = 0; s0 < (1u << lw); s0 += U) {
+    uint4 ry[U], rs[U];
+    uint32_t dd[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int src = (int)(((s0 + u) << per_lw) + grp);
+      const uint32_t yy = __shfl(y, src, kWave), ss = __shfl(s, src, kWave);
+      dd[u] = l.use ? (uint32_t)__shfl(d, src, kWave) : 0u;
+      ry[u] = a.lm[((uint64_t)yy << lw) + l.mine];
+      rs[u] = a.lm[((uint64_t)ss << lw) + l.other];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t m = __ballot(lm_min_sum(ry[u], rs[u]) <= dd[u]);
+      if ((lane >> per_lw) == s0 + u)
+        caught = ((m >> ((lane & ((1u << per_lw) - 1u)) << lw)) & gmask) != 0;
+    }
+  }
+  return caught;
+}
+__device__ inline bool lm_caught(const GenArgs &a, uint32_t s, uint32_t y, uint32_t d) {
+  return a.lm_lw >= 3 ? lm_caught<8>(a, s, y, d) : lm_caught<2>(a, s, y, d);
+}
+
+// One wave per vertex; LDS: a row of 32-bit minima per wave.
+__global__ void __launch_bounds__(256) k_lm_build(GenArgs a, uint32_t *rows, uint32_t nlm) {
+  extern __shared__ uint32_t lm_lds[];
+  const uint32_t lane = (uint32_t)lane_id(), wib = threadIdx.x / kWave;
+  const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + wib;
+  const uint32_t nwaves = gridDim.x * (blockDim.x / kWave);
+  const uint32_t words = 4u << a.lm_lw;  // two values each
+  const uint32_t per_hop = 8 * a.lm_parts;
+  uint32_t *row = lm_lds + wib * 2 * words;
+  for (uint64_t v = wave; v < a.n; v += nwaves) {
+    for (uint32_t i = lane; i < 2 * words; i += kWave) row[i] = 0xFFFFu;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const unsigned long long st = a.seg_start[v];
+    const uint32_t len = a.seg_len[v];
+    for (uint32_t j = lane; j < len; j += kWave) {
+      uint32_t hub, hop, dist;
+      pool_label(a, st + j, hub, hop, dist);
+      uint32_t i = hub;
+      if (a.hubs) {  // the landmark's place among the group's first hubs
+        i = 0;
+        while (i < nlm && a.hubs[i] < hub) ++i;
+        if (i < nlm && a.hubs[i] != hub) i = nlm;
+      }
+      if (i >= nlm || hop == 0) continue;
+      for (uint32_t x = hop; x < a.K; ++x) atomicMin(&row[(x - 1) * per_hop + i], dist);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    for (uint32_t i = lane; i < words; i += kWave)
+      rows[v * words + i] = row[2 * i] | (row[2 * i + 1] << 16);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  }
+}
+
 // Per-hub candidate counts of a round that takes list items: a workgroup
-// takes 2048 consecutive entries of the flat list, counts their hubs in an
-// LDS hash and adds each hub's count with one global atomic.
+// takes 2048 consecutive entries of the flat list, drops those a landmark
+// rejects (they become empty entries), counts the others' hubs in an LDS hash
+// and adds each hub's count with one global atomic.
 constexpr uint32_t kGroupThreads = 256;
 constexpr uint32_t kGroupPer = 8;                                 // entries per thread
 constexpr uint32_t kGroupChunk = kGroupThreads * kGroupPer;       // 2048
@@ -714,10 +836,19 @@ __global__ void __launch_bounds__(kGroupThreads) k_count(GenArgs a) {
       hcnt[i] = 0;
     }
     __syncthreads();
-#pragma unroll
+    // (not unrolled: the landmark test keeps 16 row loads in flight)
     for (uint32_t r = 0; r < kGroupPer; ++r) {
       const uint64_t i = c0 + r * kGroupThreads + tid;
-      const unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
+      unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
+      if (a.lm && a.h > 1) {
+        const bool some = e != kEmptyEntry;
+        const uint32_t b = (uint32_t)(e >> 32), y = (uint32_t)e;
+        const uint32_t d = some ? slot_dist(a, a.cand_d[slot_at(a, b, y)]) : 0u;
+        if (lm_caught(a, some ? hub_of(a, b) : 0u, some ? y : 0u, d)) {
+          a.cflat[i] = kEmptyEntry;
+          e = kEmptyEntry;
+        }
+      }
       if (e != kEmptyEntry) atomicAdd(&hcnt[group_slot(hkey, (uint32_t)(e >> 32))], 1u);
     }
     __syncthreads();
@@ -782,6 +913,10 @@ __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
     a.ctrl->total_chunks = (dead || rows) ? 0u : run;
     a.ctrl->work_ctr = 0;
     a.ctrl->cand_total += a.ctrl->cand_round;
+    if (!dead && !rows && a.lm && a.h > 1) {
+      a.ctrl->lm_tested += a.ctrl->cand_round;
+      a.ctrl->lm_caught += a.ctrl->cand_round - runc;
+    }
     a.ctrl->item_total += min(a.ctrl->fcnt[a.cur], a.fcap);
   }
 }
@@ -1213,10 +1348,11 @@ constexpr uint32_t kClaimSpread = 2 * (kPruneThreads / kWave);
 // loads their vertices, then their slot distances and list extents, in one
 // round trip per level (lane i: claimed candidate i); the first 64 labels of
 // the next claimed candidate's list are loaded before the current one's probes.
-// Instantiated once for an LDS tile and once for an arena tile.
-template <class V, class LT, class KP>
+// cand(i, y, dy) gives candidate i.  Instantiated once for an LDS tile and
+// once for an arena tile.
+template <class V, class LT, class KP, class Cand>
 __device__ __attribute__((always_inline)) inline void prune_candidates(
-    const GenArgs &a, uint32_t b, uint32_t c_beg, uint32_t c_end, const uint32_t *cands, KP rec,
+    const GenArgs &a, uint32_t b, uint32_t c_beg, uint32_t c_end, Cand cand, KP rec,
     uint32_t cap, uint32_t &sh_next, uint32_t &sh_acc_n, Item *sh_acc,
     unsigned long long &wave_reads) {
   const uint32_t sh = rec_shift<V>(a.K + 1);
@@ -1241,8 +1377,7 @@ __device__ __attribute__((always_inline)) inline void prune_candidates(
     ListView vw{0, 0, 0, 0};
     unsigned long long st = 0;
     if (lane < cn) {
-      y = cands[c + lane];
-      dy = slot_dist(a, a.cand_d[slot_at(a, b, y)]);
+      cand(c + lane, y, dy);
       st = a.seg_start[y];
       const uint32_t len = a.seg_len[y];
       uint32_t sorted = 0, pre = 1;
@@ -1357,7 +1492,11 @@ k_prune(GenArgs a) {
     // could overflow the staging slots (c_end - c_beg <= tile <= kAccSlots)
     if (sh_acc_n + (c_end - c_beg) > kAccSlots)
       publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
-    const uint32_t *cands = a.cgroup + a.hub_off[b];
+    const uint32_t *run = a.cgroup + a.hub_off[b];
+    auto cands = [&](uint32_t i, uint32_t &y, uint32_t &dy) {
+      y = run[i];
+      dy = slot_dist(a, a.cand_d[slot_at(a, b, y)]);
+    };
     const ListView sv = tile_view(a, s);
     const uint32_t cap = tile_cap_for(sv.len);
     const uint32_t icap = sv.len > a.idx_tiles
@@ -1430,8 +1569,13 @@ k_prune_rows(GenArgs a) {
   __shared__ Item sh_acc[kAccSlots];
   __shared__ uint32_t sh_rank[kAccSlots];
   __shared__ uint32_t sh_touch[kAccSlots];
-  __shared__ uint32_t sh_cand[kPruneThreads];
+  // candidates of a 1024-vertex step, as offset | distance << 10 with 16-bit
+  // distances, else the offset alone: found (0), past the landmarks (1)
+  __shared__ uint32_t sh_cand[2][kPruneThreads];
+  __shared__ uint32_t sh_cnt1;
   if (!a.ctrl->row_mode) return;
+  constexpr bool kPacked = sizeof(V) == 2;
+  static_assert(kPruneThreads == 1024, "offsets of 10 bits");
   const int lane = lane_id();
   const uint32_t K1 = a.K + 1;
   const uint32_t lds_bytes = a.lds_slots << (rec_shift<V>(K1) + 2);
@@ -1443,6 +1587,10 @@ k_prune_rows(GenArgs a) {
   const uint32_t nblk = (uint32_t)(((uint64_t)a.n + a.row_block - 1) / a.row_block);
   const uint32_t home = blockIdx.x % kXcds;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const bool lm = kPacked && a.lm && a.h > 1;
+  unsigned long long lm_tested = 0, lm_caught = 0;
+  LmLane ll{0, 0, false};
+  if (lm) ll = lm_lane(a);
   if (threadIdx.x == 0) {
     sh_q = 0;
     sh_acc_n = 0;
@@ -1489,6 +1637,8 @@ k_prune_rows(GenArgs a) {
       __syncthreads();
       continue;
     }
+    uint4 lm_s = make_uint4(kInf32, kInf32, kInf32, kInf32);
+    if (lm && ll.use) lm_s = a.lm[((uint64_t)s << a.lm_lw) + ll.other];
     bool built = false;
     // the run's blocks k, k + 8, ..., 1024 vertices at a time
     const uint32_t kSubs = a.row_block / kPruneThreads;
@@ -1500,7 +1650,10 @@ k_prune_rows(GenArgs a) {
       if (y0 >= y_end) continue;
       row_slots += min(kPruneThreads, y_end - y0);
       // this hub's candidates among [y0, y0 + 1024), compacted into sh_cand
-      if (threadIdx.x == 0) sh_cnt = 0;
+      if (threadIdx.x == 0) {
+        sh_cnt = 0;
+        sh_cnt1 = 0;
+      }
       __syncthreads();
       const uint32_t y = y0 + threadIdx.x;
       const uint32_t v = y < y_end ? a.cand_d[slot_at(a, b, y)] : kInf32;
@@ -1509,10 +1662,44 @@ k_prune_rows(GenArgs a) {
       uint32_t base = 0;
       if (lane == 0 && m) base = atomicAdd(&sh_cnt, (uint32_t)__popcll(m));
       base = __shfl(base, 0, kWave);
-      if (cand) sh_cand[base + (uint32_t)__popcll(m & lt_mask)] = y;
+      if (cand)
+        sh_cand[0][base + (uint32_t)__popcll(m & lt_mask)] =
+            kPacked ? threadIdx.x | (slot_dist(a, v) << 10) : threadIdx.x;
       __syncthreads();
-      const uint32_t cnt = sh_cnt;
+      uint32_t cnt = sh_cnt;
       if (cnt == 0) continue;
+      const uint32_t *found = sh_cand[0];
+      if (lm) {
+        // 64 >> lm_lw candidates per wave step, a row chunk per lane
+        const uint32_t lw = a.lm_lw, per = kWave >> lw, grp = (uint32_t)lane >> lw;
+        const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
+        for (uint32_t i0 = threadIdx.x / kWave * per; i0 < cnt;
+             i0 += kPruneThreads / kWave * per) {
+          const uint32_t i = i0 + grp;
+          const uint32_t e = i < cnt ? sh_cand[0][i] : 0u;
+          const uint4 r = a.lm[((uint64_t)(y0 + (e & 1023u)) << lw) + ll.mine];
+          const uint64_t hit = __ballot(lm_min_sum(r, lm_s) <= (e >> 10));
+          const bool keep = i < cnt && ((uint32_t)lane & ((1u << lw) - 1u)) == 0 &&
+                            ((hit >> lane) & gmask) == 0;
+          const uint64_t km = __ballot(keep);
+          if (!km) continue;
+          uint32_t at = 0;
+          if (lane == 0) at = atomicAdd(&sh_cnt1, (uint32_t)__popcll(km));
+          at = __shfl(at, 0, kWave);
+          if (keep) sh_cand[1][at + (uint32_t)__popcll(km & lt_mask)] = e;
+        }
+        __syncthreads();
+        lm_tested += cnt;
+        lm_caught += cnt - sh_cnt1;
+        cnt = sh_cnt1;
+        if (cnt == 0) continue;
+        found = sh_cand[1];
+      }
+      auto cands = [&](uint32_t i, uint32_t &yc, uint32_t &dy) {
+        const uint32_t e = found[i];
+        yc = y0 + (e & 1023u);
+        dy = kPacked ? e >> 10 : slot_dist(a, a.cand_d[slot_at(a, b, yc)]);
+      };
       if (!built) {
         if (in_lds) {
           if (tile_b != b) {
@@ -1541,16 +1728,16 @@ k_prune_rows(GenArgs a) {
         if (threadIdx.x == 0) sh_next = 0;
         __syncthreads();
         if (icap)
-          prune_candidates<V, LT>(a, b, c0, c1, sh_cand,
+          prune_candidates<V, LT>(a, b, c0, c1, cands,
                                   IdxTile{(lds_ptr<const uint32_t>)lds,
                                           (uint32_t)(uintptr_t)(lds_ptr<const uint32_t>)(lds + icap),
                                           K1 * (uint32_t)sizeof(V)},
                                   icap, sh_next, sh_acc_n, sh_acc, wave_reads);
         else if (in_lds)
-          prune_candidates<V, LT>(a, b, c0, c1, sh_cand, (lds_ptr<const uint32_t>)lds, lcap,
+          prune_candidates<V, LT>(a, b, c0, c1, cands, (lds_ptr<const uint32_t>)lds, lcap,
                                   sh_next, sh_acc_n, sh_acc, wave_reads);
         else
-          prune_candidates<V, LT>(a, b, c0, c1, sh_cand, (glb_ptr<const uint32_t>)gkeys, cap,
+          prune_candidates<V, LT>(a, b, c0, c1, cands, (glb_ptr<const uint32_t>)gkeys, cap,
                                   sh_next, sh_acc_n, sh_acc, wave_reads);
         __syncthreads();
       }
@@ -1560,6 +1747,10 @@ k_prune_rows(GenArgs a) {
   if (lane == 0 && wave_reads) atomicAdd(&a.ctrl->label_reads, wave_reads);
   if (threadIdx.x == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
   if (threadIdx.x == 0 && row_slots) atomicAdd(&a.ctrl->row_slots, row_slots);
+  if (threadIdx.x == 0 && lm_tested) {
+    atomicAdd(&a.ctrl->lm_tested, lm_tested);
+    atomicAdd(&a.ctrl->lm_caught, lm_caught);
+  }
 }
 
 // -------------------------------------------------------- reserve / append
@@ -1924,7 +2115,7 @@ enum ScratchId : int {
   kScSegStart, kScSegLen, kScSegCap, kScAddCnt, kScTouched, kScFgrp, kScHubSlot,
   kScSortedLen, kScHcnt, kScSortTmp, kScSortTmp32, kScCflat, kScCgroup, kScHubCcnt, kScHubOff,
   kScHubCur, kScChunkOff, kScF0, kScF1, kScGtile, kScCtrl, kScHeavy, kScExpKeys, kScExpSorted,
-  kScExpTmp, kScFrank, kScCount
+  kScExpTmp, kScFrank, kScLm, kScCount
 };
 static_assert(kScCount <= hsdl_graph::kScratch, "scratch slots");
 
@@ -1938,6 +2129,8 @@ struct Gen {
   DevBuf cflat, cgroup, hub_ccnt, hub_off, hub_cur, chunk_off, F0, F1, gtile, ctrl, heavy;
   DevBuf exp_keys, exp_sorted, exp_tmp;  // export: 32-bit keys, sorted keys, sort space
   DevBuf frank;                          // ranks of the next frontier's items
+  DevBuf lm;                             // landmark rows (k_lm_build)
+  bool lm_on = false;
   uint64_t budget = 0;  // device bytes the build may hold
   uint64_t fixed = 0;   // per-vertex state and the dense slots
   int grid = 0;
@@ -1964,11 +2157,23 @@ struct Gen {
            frank.bytes +
            gtile.bytes + sort_tmp.bytes + sort_tmp32.bytes;
   }
+  // Whether the build may hold `want` bytes beside the landmark rows; the
+  // rows only save time, so they go when the build needs their room.
+  bool fits(uint64_t want) {
+    if (want > budget) return false;
+    if (lm.p && want + lm.bytes > budget) {
+      (void)hipStreamSynchronize(st);
+      lm.release();
+      a.lm = nullptr;
+      lm_on = false;
+    }
+    return true;
+  }
   DevBuf *by_id(int id) {
     DevBuf *t[kScCount] = {&seg_start, &seg_len, &seg_cap, &add_cnt, &touched, &fgrp,
                            &hub_slot, &sorted_len, &hcnt, &sort_tmp, &sort_tmp32, &cflat, &cgroup,
                            &hub_ccnt, &hub_off, &hub_cur, &chunk_off, &F0, &F1, &gtile, &ctrl,
-                           &heavy, &exp_keys, &exp_sorted, &exp_tmp, &frank};
+                           &heavy, &exp_keys, &exp_sorted, &exp_tmp, &frank, &lm};
     return t[id];
   }
   // Buffer `id` of at least n bytes: the graph's kept one when it is large
@@ -2027,7 +2232,7 @@ static int grow_pool(Gen &g, uint64_t used, uint64_t min_cap) {
   while (ncap < min_cap) ncap *= 2;
   const bool p32 = g.a.pool32 != nullptr;  // then there is no 8-byte pool
   const uint64_t per_label = p32 ? 4 : 8;
-  if (g.held() - g.pool.bytes - g.pool32.bytes + ncap * per_label > g.budget)
+  if (!g.fits(g.held() - g.pool.bytes - g.pool32.bytes + ncap * per_label))
     return fail(HSDL_ENOMEM, "label pool exceeds the HBM budget");
   DevBuf np, np32;
   int rc = p32 ? np32.alloc(ncap * 4) : np.alloc(ncap * 8);
@@ -2051,7 +2256,7 @@ static int grow_pool(Gen &g, uint64_t used, uint64_t min_cap) {
 
 static int grow_gtile(Gen &g) {
   const uint64_t nw = g.a.gtile_cap * 2;
-  if (g.held() - g.gtile.bytes + nw * 4 > g.budget)
+  if (!g.fits(g.held() - g.gtile.bytes + nw * 4))
     return fail(HSDL_ENOMEM, "tile arena exceeds the HBM budget");
   g.gtile.release();
   int rc = g.take(kScGtile, nw * 4);
@@ -2066,7 +2271,7 @@ static int alloc_lists(Gen &g, uint32_t ccap, uint32_t fcap) {
   if (ccap != g.a.ccap) {
     g.cflat.release();
     g.cgroup.release();
-    if (g.held() + (uint64_t)ccap * 12 > g.budget)
+    if (!g.fits(g.held() + (uint64_t)ccap * 12))
       return fail(HSDL_ENOMEM, "candidate lists exceed the HBM budget");
     if ((rc = g.take(kScCflat, (uint64_t)ccap * 8)) || (rc = g.take(kScCgroup, (uint64_t)ccap * 4)))
       return rc;
@@ -2078,7 +2283,7 @@ static int alloc_lists(Gen &g, uint32_t ccap, uint32_t fcap) {
     g.F0.release();
     g.F1.release();
     g.frank.release();
-    if (g.held() + (uint64_t)fcap * (2 * sizeof(Item) + 4) > g.budget)
+    if (!g.fits(g.held() + (uint64_t)fcap * (2 * sizeof(Item) + 4)))
       return fail(HSDL_ENOMEM, "frontier lists exceed the HBM budget");
     if ((rc = g.take(kScF0, (uint64_t)fcap * sizeof(Item))) ||
         (rc = g.take(kScF1, (uint64_t)fcap * sizeof(Item))) ||
@@ -2143,7 +2348,7 @@ static bool same_buffers(const GenArgs &x, const GenArgs &y) {
   return x.pool == y.pool && x.pool_cap == y.pool_cap && x.pool32 == y.pool32 &&
          x.gtile == y.gtile && x.gtile_cap == y.gtile_cap && x.cflat == y.cflat &&
          x.cgroup == y.cgroup && x.ccap == y.ccap && x.F0 == y.F0 && x.F1 == y.F1 &&
-         x.frank == y.frank && x.fcap == y.fcap;
+         x.frank == y.frank && x.fcap == y.fcap && x.lm == y.lm;
 }
 
 // Captures the batch sequence (with or without the row-item prune) into a
@@ -2182,7 +2387,8 @@ static int enqueue_batch(Gen &g, uint32_t s0, uint32_t B, uint32_t K, uint32_t n
   // k_batch_begin writes the B hubs into the first frontier unchecked
   if (B == 0 || B > g.a.fcap || B > g.bmax || s0 + (uint64_t)B > nhubs)
     return fail(HSDL_EINVAL, "hub batch does not fit the frontier list or the hub sequence");
-  hipLaunchKernelGGL(k_set_batch, dim3(1), dim3(1), 0, g.st, g.a.ctrl, s0, B, g.a.tag);
+  hipLaunchKernelGGL(k_set_batch, dim3(1), dim3(1), 0, g.st, g.a.ctrl, s0, B, g.a.tag,
+                     g.lm_on ? 1u : 0u);
   const bool rows = B > 1 || g.a.row_policy == 2;
   // one graph launch per batch instead of 1 + 11 K launches (the plain form
   // is bound by the host's launch rate); not with per-launch timing events
@@ -2210,7 +2416,7 @@ static int sort_zones(Gen &g, uint32_t maxlen, uint32_t resort_div) {
     per = std::min(per, slice_cap);
     const bool p32 = g.a.pool32 != nullptr, p64 = g.a.pool != nullptr;
     const uint64_t bytes = waves * per * ((p64 ? 8ull : 0ull) + (p32 ? 4ull : 0ull));
-    if (g.held() - g.sort_tmp.bytes - g.sort_tmp32.bytes + bytes > g.budget) {
+    if (!g.fits(g.held() - g.sort_tmp.bytes - g.sort_tmp32.bytes + bytes)) {
       // no room for bigger slices: the longer lists stay unsorted
       if (!g.sort_per_wave) return HSDL_OK;
     } else {
@@ -2545,6 +2751,20 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     c0v.pool_top = (unsigned long long)n * c0;
     HSDL_HIP(hipMemcpyAsync(g.ctrl.p, &c0v, sizeof(Ctrl), hipMemcpyHostToDevice, g.st));
   }
+  // landmark rows: 16-bit distances, at least two hops and two batches, not
+  // in the plain form (whose rounds are launch latency).  Tuning knob
+  // HSDL_LANDMARKS: their count, in eights, 0 for none.
+  uint32_t nlm = 0;
+  if (g.small_vals && K >= 2 && !plain) {
+    a.lm_parts = env_u32("HSDL_LANDMARKS", 16, 0, 64) / 8;
+    a.lm_lw = 0;
+    while ((1u << a.lm_lw) < (K - 1) * a.lm_parts) ++a.lm_lw;
+    nlm = std::min(8 * a.lm_parts, nhubs);
+    const uint64_t bytes = (uint64_t)n * (16ull << a.lm_lw);
+    if (nlm && a.lm_lw <= 6 && a.lm_lw >= 1 && g.held() + bytes <= g.budget &&
+        g.take(kScLm, bytes) == HSDL_OK)
+      a.lm = g.lm.as<uint4>();
+  }
   hipLaunchKernelGGL(k_init_labels, dim3(1024), dim3(256), 0, g.st, a, c0);
   // The slots hold the values of the last build on this graph.  When it used
   // the same slot encoding, this build continues its tag count-down (those
@@ -2683,7 +2903,17 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     }
     const double work = (double)(c.cand_total - c_ok.cand_total) +
                         (double)(c.edge_total - c_ok.edge_total) / 8.0;
+    // a landmark test that rejects less than an eighth of what it looks at
+    // (graphs without hubs that many walks meet) ends
+    const uint64_t tested = c.lm_tested - c_ok.lm_tested;
+    if (g.lm_on && tested >= 4096 && (c.lm_caught - c_ok.lm_caught) * 8 < tested) g.lm_on = false;
     c_ok = c;
+    if (g.a.lm && s0 < nlm && s0 + B >= nlm && s0 + B < nhubs) {
+      hipLaunchKernelGGL(k_lm_build, dim3(g.grid), dim3(256), (size_t)128 << g.a.lm_lw, g.st, g.a,
+                         g.lm.as<uint32_t>(), nlm);
+      HSDL_HIP(hipGetLastError());
+      g.lm_on = true;
+    }
     // (no prune follows the last batch: its lists stay as they are)
     if (zones && B > 1 && s0 + B < nhubs && (rc = sort_zones(g, c.maxlen, resort_div)))
       return rc;

@@ -1,0 +1,51 @@
+"""Kernel variants that a size, a type or an option selects, at the edges of
+their ranges, against the oracle.  Integer work: every comparison is exact."""
+import numpy as np
+import pytest
+
+import gpu4hophl_code_amd as H
+import oracle_lib as O
+from test_gpu_parity import csr_of, same_labels
+
+pytestmark = pytest.mark.gpu
+
+
+def ragged(n, seed, wmax, ef=8):
+    """The n top-ranked vertices of an R-MAT graph, renamed by degree."""
+    g = H.Graph.rmat(max(1, (n - 1).bit_length()), ef, seed, 1, wmax)
+    off, col, w = g.csr()
+    row = np.repeat(np.arange(len(off) - 1, dtype=np.uint32), np.diff(off.astype(np.int64)))
+    keep = (row < col) & (col < n)
+    g = H.Graph.from_edges(n, row[keep], col[keep], w[keep])
+    g.reorder_by_degree()
+    return g
+
+
+@pytest.mark.parametrize("landmarks", ["0", "8", "24", "64"])
+@pytest.mark.parametrize("rows", ["0", "2"])
+def test_landmark_test_keeps_the_labels(monkeypatch, landmarks, rows):
+    """Candidates are tested against the first hubs' rows before the prune
+    searches (rows of 2 to 64 chunks by K and the landmark count, by lists
+    and by rows): the labels are the oracle's, for whole builds, batches that
+    end inside and past the landmarks, groups (landmarks are the group's own
+    hubs) and 8-byte labels."""
+    monkeypatch.setenv("HSDL_LANDMARKS", landmarks)
+    monkeypatch.setenv("HSDL_PRUNE_ROWS", rows)
+    for n, K, wmax in ((1500, 4, 100), (1031, 2, 3), (700, 9, 2), (2049, 5, 13000), (90, 3, 9)):
+        g = ragged(n, n, wmax)
+        c = csr_of(g)
+        want = O.kround(c, K).arrays()
+        for batch in (0, 7, 65):
+            print(f"[landmarks] n={n} K={K} hubs={landmarks} rows={rows} batch={batch}", flush=True)
+            same_labels(H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=batch), want)
+        hubs = np.arange(1, n, 3, dtype=np.uint32)
+        gid = np.ones(n, np.uint32)
+        gid[hubs] = 0
+        got = H.hop_constrained_two_hop_labels_generation(g, K, hubs=hubs, hub_batch=40)
+        ref = O.kround_gid(c, K, gid).arrays()
+        keep = np.isin(ref[1], hubs)
+        for x, y in zip(got.labels()[1:], ref[1:]):
+            assert np.array_equal(x, np.asarray(y)[keep])
+    monkeypatch.setenv("HSDL_STREAM32", "0")
+    g = ragged(1500, 4, 100)
+    same_labels(H.hop_constrained_two_hop_labels_generation(g, 4), O.kround(csr_of(g), 4).arrays())
