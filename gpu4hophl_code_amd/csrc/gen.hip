@@ -142,6 +142,7 @@ struct GenArgs {
   uint32_t row_block;    // vertices per y-block (a multiple of 1024)
   uint32_t claim_max;    // candidates a prune wave claims at once, at most
   uint32_t idx_tiles;    // LDS tiles of more labels than this are indexed (kInf32: none)
+  uint32_t direct_tiles; // LDS tiles addressed by hub id, where they fit
   uint32_t heavy_pairs;  // frontier groups with more pairs go to heavy pieces
   uint32_t piece_pairs;  // pairs per heavy piece (whole edges)
   uint32_t lds_slots;  // LDS tile capacity (slots)
@@ -1215,6 +1216,95 @@ __device__ void build_idx_tile(const GenArgs &a, uint32_t s, const ListView &vie
   __syncthreads();
 }
 
+// Direct LDS tiles, for hub ranges small enough to address by hub id (the
+// batch's last hub bounds every hub in the lists, the self labels aside, and
+// hop zones keep those out of the views).  Values are kept for hops 1..h - 1
+// of the streamed label, and an empty one for any higher hop: hub w's label
+// of hop ha reads value min(ha, h) - 1 of its h values, 16 bits each.
+//   values: w * h + min(ha, h) - 1         while limit * h * 2 bytes fit
+//   rows:   row index (16 bits) of hub w, then that row's h values
+// A probe has no chain: in a hash tile at load factor 1/8 a wave still took
+// about three turns, those of its longest lane, of 14 instructions each.
+// Early hubs, whose ids are small, hold most of a build's candidates (R-MAT
+// scale 18: 80 % of the time in hubs below 4,096).
+struct DirTile {
+  uint32_t vals;     // LDS byte address of value -1 of hub 0
+  uint32_t stride;   // bytes per hub
+  uint32_t h;
+};
+struct DirIdxTile {
+  uint32_t idx;      // LDS byte address of hub 0's row index
+  uint32_t vals;     // LDS byte address of value -1 of row 0 (empty)
+  uint32_t stride;   // bytes per row
+  uint32_t h;
+};
+template <class V, class LT>
+__device__ inline bool probe_label(const GenArgs &a, LT l, uint32_t dy, DirTile t, uint32_t,
+                                   uint32_t) {
+  uint32_t hub, ha, da;
+  unpack(a, l, hub, ha, da);
+  const uint32_t at = mul_u24(hub, t.stride) + t.vals + 2u * min(ha, t.h);
+  return da + *(lds_ptr<const uint16_t>)(uintptr_t)at <= dy;
+}
+template <class V, class LT>
+__device__ inline bool probe_label(const GenArgs &a, LT l, uint32_t dy, DirIdxTile t, uint32_t,
+                                   uint32_t) {
+  uint32_t hub, ha, da;
+  unpack(a, l, hub, ha, da);
+  const uint32_t row = *(lds_ptr<const uint16_t>)(uintptr_t)(t.idx + 2u * hub);
+  const uint32_t at = mul_u24(row, t.stride) + t.vals + 2u * min(ha, t.h);
+  return da + *(lds_ptr<const uint16_t>)(uintptr_t)at <= dy;
+}
+// fills `bytes` (a multiple of 16) of LDS with the byte pattern w
+__device__ inline void fill_lds(uint32_t *p, uint32_t bytes, uint32_t w) {
+  uint4 *q = reinterpret_cast<uint4 *>(p);
+  for (uint32_t i = threadIdx.x; i < bytes / 16; i += blockDim.x) q[i] = make_uint4(w, w, w, w);
+}
+__device__ inline uint32_t dir_bytes(uint32_t x) { return (x + 15u) & ~15u; }
+__device__ inline void build_dir_tile(const GenArgs &a, uint32_t s, const ListView &view,
+                                      uint32_t *lds, uint32_t limit) {
+  fill_lds(lds, dir_bytes(limit * a.h * 2), kInf32);
+  __syncthreads();
+  uint16_t *vals = reinterpret_cast<uint16_t *>(lds);
+  const unsigned long long st = a.seg_start[s];
+  for (uint32_t i = threadIdx.x; i < view.len; i += blockDim.x) {
+    uint32_t hub, hb, db;
+    pool_label(a, st + view.at(i), hub, hb, db);
+    for (uint32_t ha = 1; ha + hb <= a.h && ha < a.h; ++ha)
+      atomic_min_v(&vals[hub * a.h + ha - 1], db);
+  }
+  __syncthreads();
+}
+// Row 1 + i belongs to the hub whose first claimer is label i of the view.
+__device__ inline void build_diridx_tile(const GenArgs &a, uint32_t s, const ListView &view,
+                                         uint32_t *lds, uint32_t limit) {
+  const uint32_t ib = dir_bytes(limit * 2);
+  fill_lds(lds, ib, 0u);
+  fill_lds(lds + ib / 4, dir_bytes((view.len + 1) * a.h * 2), kInf32);
+  __syncthreads();
+  uint16_t *rows = reinterpret_cast<uint16_t *>(lds + ib / 4);
+  const unsigned long long st = a.seg_start[s];
+  for (uint32_t i = threadIdx.x; i < view.len; i += blockDim.x) {
+    uint32_t hub, hb, db;
+    pool_label(a, st + view.at(i), hub, hb, db);
+    uint32_t *w = lds + hub / 2;
+    const uint32_t sh = (hub & 1u) * 16u;
+    for (uint32_t old = *w; ((old >> sh) & 0xFFFFu) == 0;) {
+      const uint32_t got = atomicCAS(w, old, old | ((i + 1) << sh));
+      if (got == old) break;
+      old = got;
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < view.len; i += blockDim.x) {
+    uint32_t hub, hb, db;
+    pool_label(a, st + view.at(i), hub, hb, db);
+    uint16_t *vals = rows + (uint32_t)reinterpret_cast<uint16_t *>(lds)[hub] * a.h;
+    for (uint32_t ha = 1; ha + hb <= a.h && ha < a.h; ++ha) atomic_min_v(&vals[ha - 1], db);
+  }
+  __syncthreads();
+}
+
 // Label `lane` of a list view, clamped to it (a lane past the end reloads
 // the last label); an empty view reads the list's position 0, its self label.
 template <class LT>
@@ -1342,19 +1432,18 @@ __device__ inline void publish_accepted(const GenArgs &a, Item *Fn, Item *sh_acc
 // item's end, where the slowest wave decides when the workgroup moves on).
 constexpr uint32_t kClaimSpread = 2 * (kPruneThreads / kWave);
 
-// The waves of a prune workgroup take the item's candidates [c_beg, c_end) of
-// hub slot b (L(y) lengths vary widely, so dynamically) and stage the
-// accepted ones in LDS.  A wave claims up to a.claim_max candidates at once and
+// The waves of a prune workgroup take the candidates [c_beg, c_end) of hub
+// slot b (L(y) lengths vary widely, so dynamically) and hand the accepted
+// ones to accept(i, y, d).  A wave claims up to a.claim_max candidates at once and
 // loads their vertices, then their slot distances and list extents, in one
 // round trip per level (lane i: claimed candidate i); the first 64 labels of
 // the next claimed candidate's list are loaded before the current one's probes.
 // cand(i, y, dy) gives candidate i.  Instantiated once for an LDS tile and
 // once for an arena tile.
-template <class V, class LT, class KP, class Cand>
+template <class V, class LT, class KP, class Cand, class Acc>
 __device__ __attribute__((always_inline)) inline void prune_candidates(
-    const GenArgs &a, uint32_t b, uint32_t c_beg, uint32_t c_end, Cand cand, KP rec,
-    uint32_t cap, uint32_t &sh_next, uint32_t &sh_acc_n, Item *sh_acc,
-    unsigned long long &wave_reads) {
+    const GenArgs &a, uint32_t b, uint32_t c_beg, uint32_t c_end, Cand cand, Acc accept, KP rec,
+    uint32_t cap, uint32_t &sh_next, unsigned long long &wave_reads) {
   const uint32_t sh = rec_shift<V>(a.K + 1);
   const uint32_t lane = (uint32_t)lane_id();
   for (;;) {
@@ -1411,17 +1500,85 @@ __device__ __attribute__((always_inline)) inline void prune_candidates(
       uint32_t reads = 0;
       const bool pruned = witness_search<V>(a, Lc, vc, f0, di, rec, cap, sh, reads);
       wave_reads += reads;
-      if (lane == 0) {
-        if (!pruned) {
-          const uint32_t p = atomicAdd(&sh_acc_n, 1u);
-          sh_acc[p] = Item{b, yi, di};
-        }
-      }
+      if (lane == 0 && !pruned) accept(c + i, yi, di);
       Lc = Ln;
       vc = vn;
       f0 = g0;
     }
   }
+}
+
+// The tile of a hub whose view holds `len` labels: in LDS addressed by hub
+// id (values, or a row index), else hashed (indexed, or records), else a
+// record tile in the workgroup's slice (gwords) of the arena.
+enum : uint32_t { kTileDir, kTileDirIdx, kTileIdx, kTileRec, kTileArena, kTileNoRoom };
+struct TilePlan {
+  uint32_t kind, cap;
+};
+// Direct tiles hold 16-bit values, and only 32-bit labels take them: graphs
+// with wider labels spread their lists over many hubs (the 1024 x 1024 grid's
+// prune ran 1.5 % slower with the two variants in its kernel).
+template <class V, class LT>
+constexpr bool kDirect = sizeof(V) == 2 && sizeof(LT) == 4;
+template <class V, class LT>
+__device__ inline TilePlan tile_plan(const GenArgs &a, uint32_t len, uint64_t gwords) {
+  const uint32_t K1 = a.K + 1;
+  const uint32_t lds_bytes = a.lds_slots << (rec_shift<V>(K1) + 2);
+  if (kDirect<V, LT> && a.direct_tiles && a.hcnt && a.h > 1) {
+    const uint64_t limit = (uint64_t)hub_of(a, a.B - 1) + 1;
+    if (((limit * a.h * 2 + 15) & ~15ull) <= lds_bytes)
+      return TilePlan{kTileDir, (uint32_t)limit};
+    if (((limit * 2 + 15) & ~15ull) + (((uint64_t)(len + 1) * a.h * 2 + 15) & ~15ull) <= lds_bytes)
+      return TilePlan{kTileDirIdx, (uint32_t)limit};
+  }
+  if (len > a.idx_tiles) {
+    const uint32_t icap = idx_tile_cap(len, K1 * (uint32_t)sizeof(V), lds_bytes);
+    if (icap) return TilePlan{kTileIdx, icap};
+  }
+  const uint32_t cap = tile_cap_for(len);
+  if (cap <= a.lds_slots) return TilePlan{kTileRec, lds_tile_cap(len, a.lds_slots)};
+  return TilePlan{rec_tile_words<V>(cap, K1) > gwords ? kTileNoRoom : kTileArena, cap};
+}
+template <class V>
+__device__ inline void tile_build(const GenArgs &a, uint32_t s, const ListView &sv, TilePlan p,
+                                  uint32_t *lds, uint32_t *gkeys, uint32_t &sh_rows) {
+  if (p.kind == kTileDir) {
+    build_dir_tile(a, s, sv, lds, p.cap);
+  } else if (p.kind == kTileDirIdx) {
+    build_diridx_tile(a, s, sv, lds, p.cap);
+  } else if (p.kind == kTileIdx) {
+    build_idx_tile<V>(a, s, sv, lds, p.cap, sh_rows);
+  } else if (p.kind == kTileRec) {
+    build_tile<V>(a, s, sv, lds, p.cap);
+  } else {
+    build_tile<V>(a, s, sv, gkeys, p.cap);
+    // the tile was written through L2 (atomics); drop stale L1 lines of
+    // this workgroup's arena slice before plain loads read it
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+}
+template <class V, class LT, class Cand, class Acc>
+__device__ __attribute__((always_inline)) inline void tile_prune(
+    const GenArgs &a, uint32_t b, uint32_t c_beg, uint32_t c_end, Cand cand, Acc accept,
+    TilePlan p, uint32_t *lds, uint32_t *gkeys, uint32_t &sh_next,
+    unsigned long long &wave_reads) {
+  auto run = [&](auto tile) __attribute__((always_inline)) {
+    prune_candidates<V, LT>(a, b, c_beg, c_end, cand, accept, tile, p.cap, sh_next, wave_reads);
+  };
+  auto at = [&](uint32_t bytes) {
+    return (uint32_t)(uintptr_t)(lds_ptr<const uint32_t>)lds + bytes;
+  };
+  const uint32_t K1 = a.K + 1;
+  if (kDirect<V, LT> && p.kind == kTileDir)
+    run(DirTile{at(0) - 2u, a.h * 2u, a.h});
+  else if (kDirect<V, LT> && p.kind == kTileDirIdx)
+    run(DirIdxTile{at(0), at(dir_bytes(p.cap * 2)) - 2u, a.h * 2u, a.h});
+  else if (p.kind == kTileIdx)
+    run(IdxTile{(lds_ptr<const uint32_t>)lds, at(4 * p.cap), K1 * (uint32_t)sizeof(V)});
+  else if (p.kind == kTileRec)
+    run((lds_ptr<const uint32_t>)lds);
+  else
+    run((glb_ptr<const uint32_t>)gkeys);
 }
 
 // LT: label type of the stream (uint32_t: the pool's 32-bit copy).
@@ -1436,8 +1593,6 @@ k_prune(GenArgs a) {
   __shared__ uint32_t sh_rank[kAccSlots];
   __shared__ uint32_t sh_touch[kAccSlots];
   const int lane = lane_id();
-  const uint32_t K1 = a.K + 1;
-  const uint32_t lds_bytes = a.lds_slots << (rec_shift<V>(K1) + 2);
   Item *Fn = frontier(a, a.cur ^ 1);
   uint32_t tile_b = kInf32;  // hub slot whose tile is in LDS
   unsigned long long wave_reads = 0, tile_reads = 0;
@@ -1498,47 +1653,23 @@ k_prune(GenArgs a) {
       dy = slot_dist(a, a.cand_d[slot_at(a, b, y)]);
     };
     const ListView sv = tile_view(a, s);
-    const uint32_t cap = tile_cap_for(sv.len);
-    const uint32_t icap = sv.len > a.idx_tiles
-                              ? idx_tile_cap(sv.len, K1 * (uint32_t)sizeof(V), lds_bytes)
-                              : 0u;
-    if (icap) {
-      if (tile_b != b) {
-        build_idx_tile<V>(a, s, sv, lds, icap, sh_rows);
-        tile_b = b;
-        tile_reads += sv.len;
-      }
-      const IdxTile it{(lds_ptr<const uint32_t>)lds,
-                       (uint32_t)(uintptr_t)(lds_ptr<const uint32_t>)(lds + icap),
-                       K1 * (uint32_t)sizeof(V)};
-      prune_candidates<V, LT>(a, b, c_beg, c_end, cands, it, icap, sh_next, sh_acc_n, sh_acc,
-                              wave_reads);
-    } else if (cap <= a.lds_slots) {
-      const uint32_t lcap = lds_tile_cap(sv.len, a.lds_slots);
-      if (tile_b != b) {
-        build_tile<V>(a, s, sv, lds, lcap);
-        tile_b = b;
-        tile_reads += sv.len;
-      }
-      prune_candidates<V, LT>(a, b, c_beg, c_end, cands, (lds_ptr<const uint32_t>)lds, lcap,
-                              sh_next, sh_acc_n, sh_acc, wave_reads);
-    } else {
-      if (rec_tile_words<V>(cap, K1) > gwords) {
-        // arena too small: the host rolls the batch back, grows the arena
-        // and runs the batch again
-        if (threadIdx.x == 0) atomicOr(&a.ctrl->overflow, kOvfArena);
-        __syncthreads();
-        continue;
-      }
-      build_tile<V>(a, s, sv, gkeys, cap);
-      // the tile was written through L2 (atomics); drop stale L1 lines of
-      // this workgroup's arena slice before plain loads read it
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      tile_b = kInf32;
-      tile_reads += sv.len;
-      prune_candidates<V, LT>(a, b, c_beg, c_end, cands, (glb_ptr<const uint32_t>)gkeys, cap,
-                              sh_next, sh_acc_n, sh_acc, wave_reads);
+    const TilePlan plan = tile_plan<V, LT>(a, sv.len, gwords);
+    if (plan.kind == kTileNoRoom) {
+      // arena too small: the host rolls the batch back, grows the arena
+      // and runs the batch again
+      if (threadIdx.x == 0) atomicOr(&a.ctrl->overflow, kOvfArena);
+      __syncthreads();
+      continue;
     }
+    if (tile_b != b) {
+      tile_build<V>(a, s, sv, plan, lds, gkeys, sh_rows);
+      tile_b = plan.kind == kTileArena ? kInf32 : b;
+      tile_reads += sv.len;
+    }
+    auto accept = [&](uint32_t, uint32_t y, uint32_t d) {
+      sh_acc[atomicAdd(&sh_acc_n, 1u)] = Item{b, y, d};
+    };
+    tile_prune<V, LT>(a, b, c_beg, c_end, cands, accept, plan, lds, gkeys, sh_next, wave_reads);
     __syncthreads();
   }
   publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
@@ -1559,26 +1690,34 @@ k_prune(GenArgs a) {
 // are dealt to XCDs round-robin by id; a workgroup whose queue runs dry takes
 // items from the other queues in turn.  The decisions do not depend on the order: a round's
 // prune reads only labels of earlier rounds and batches.
+//
+// An item's vertices are taken kRowSteps * 1024 at a time: every thread loads
+// its kRowSteps slots at once, the candidates gather in an LDS list (in as
+// few pieces as the list takes), the landmark test thins each piece, and the
+// search runs over up to kRowList survivors.  What binds is the chain of
+// memory round trips and barriers per step, not bytes or instructions: taken
+// 1024 vertices at a time, R-MAT scale 18 had 10 million steps of 4.5 us.
+constexpr uint32_t kRowSteps = 8;
+// two lists of this beside 64 KB of tile: two workgroups in a CU's 160 KB
+constexpr uint32_t kRowList = 1984;
+static_assert(kRowList >= kPruneThreads && kRowList <= 2 * kPruneThreads, "a step fits; publish");
+
 template <class V, class LT>
 __global__ void __launch_bounds__(kPruneThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_prune_rows(GenArgs a) {
   with_batch(a);
   extern __shared__ uint32_t lds[];
-  __shared__ uint32_t sh_b, sh_k, sh_kn, sh_q, sh_next, sh_cnt, sh_rows;
-  __shared__ uint32_t sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base;
-  __shared__ Item sh_acc[kAccSlots];
-  __shared__ uint32_t sh_rank[kAccSlots];
-  __shared__ uint32_t sh_touch[kAccSlots];
-  // candidates of a 1024-vertex step, as offset | distance << 10 with 16-bit
-  // distances, else the offset alone: found (0), past the landmarks (1)
-  __shared__ uint32_t sh_cand[2][kPruneThreads];
-  __shared__ uint32_t sh_cnt1;
+  __shared__ uint32_t sh_b, sh_k, sh_kn, sh_q, sh_next, sh_rows;
+  __shared__ uint32_t sh_nf, sh_ns, sh_acc, sh_touch, sh_acc_base, sh_touch_base;
+  __shared__ uint32_t sh_step[kRowSteps];  // candidates of each step
+  __shared__ uint32_t sh_y0[kRowSteps];    // first vertex of each step
+  // candidates found, and those past the landmarks: offset in the steps
+  // (13 bits), with 16-bit distances the distance << 13, accepted: bit 31
+  __shared__ uint32_t sh_found[kRowList], sh_surv[kRowList];
   if (!a.ctrl->row_mode) return;
   constexpr bool kPacked = sizeof(V) == 2;
-  static_assert(kPruneThreads == 1024, "offsets of 10 bits");
-  const int lane = lane_id();
-  const uint32_t K1 = a.K + 1;
-  const uint32_t lds_bytes = a.lds_slots << (rec_shift<V>(K1) + 2);
+  static_assert(kPruneThreads == 1024 && kRowSteps == 8, "offsets of 13 bits");
+  const uint32_t lane = (uint32_t)lane_id(), tid = threadIdx.x, wv = tid / kWave;
   Item *Fn = frontier(a, a.cur ^ 1);
   uint32_t tile_b = kInf32;  // hub slot whose tile is in LDS
   unsigned long long wave_reads = 0, tile_reads = 0, row_slots = 0;
@@ -1591,14 +1730,10 @@ k_prune_rows(GenArgs a) {
   unsigned long long lm_tested = 0, lm_caught = 0;
   LmLane ll{0, 0, false};
   if (lm) ll = lm_lane(a);
-  if (threadIdx.x == 0) {
-    sh_q = 0;
-    sh_acc_n = 0;
-    sh_touch_n = 0;
-  }
+  if (tid == 0) sh_q = 0;
   __syncthreads();
   for (;;) {
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
       sh_b = kInf32;
       while (sh_q < kXcds) {
         // queue x: its blocks k = x + 8i, in runs of row_run blocks; item j
@@ -1624,130 +1759,178 @@ k_prune_rows(GenArgs a) {
     const uint32_t k = sh_k;
     const uint32_t s = hub_of(a, b);
     const ListView sv = tile_view(a, s);
-    const uint32_t cap = tile_cap_for(sv.len);
-    const uint32_t icap = sv.len > a.idx_tiles
-                              ? idx_tile_cap(sv.len, K1 * (uint32_t)sizeof(V), lds_bytes)
-                              : 0u;
-    const bool in_lds = icap || cap <= a.lds_slots;
-    const uint32_t lcap = icap ? icap : in_lds ? lds_tile_cap(sv.len, a.lds_slots) : cap;
-    if (!in_lds && rec_tile_words<V>(cap, K1) > gwords) {
+    const TilePlan plan = tile_plan<V, LT>(a, sv.len, gwords);
+    if (plan.kind == kTileNoRoom) {
       // arena too small: the host rolls the batch back, grows the arena and
       // runs the batch again
-      if (threadIdx.x == 0) atomicOr(&a.ctrl->overflow, kOvfArena);
+      if (tid == 0) atomicOr(&a.ctrl->overflow, kOvfArena);
       __syncthreads();
       continue;
     }
     uint4 lm_s = make_uint4(kInf32, kInf32, kInf32, kInf32);
     if (lm && ll.use) lm_s = a.lm[((uint64_t)s << a.lm_lw) + ll.other];
     bool built = false;
-    // the run's blocks k, k + 8, ..., 1024 vertices at a time
+    auto vertex = [&](uint32_t e) { return sh_y0[(e >> 10) & 7u] + (e & 1023u); };
+    auto dist_of = [&](uint32_t e, uint32_t y) {
+      return kPacked ? (e >> 13) & 0xFFFFu : slot_dist(a, a.cand_d[slot_at(a, b, y)]);
+    };
+    // the run's blocks k, k + 8, ..., kRowSteps * 1024 vertices at a time
     const uint32_t kSubs = a.row_block / kPruneThreads;
-    const uint32_t kn = sh_kn;
-    for (uint32_t i = 0; i < kn * kSubs; ++i) {
-      const uint32_t kb = k + kXcds * (i / kSubs);
-      const uint32_t y0 = kb * a.row_block + (i % kSubs) * kPruneThreads;
-      const uint32_t y_end = min(a.n, (kb + 1) * a.row_block);
-      if (y0 >= y_end) continue;
-      row_slots += min(kPruneThreads, y_end - y0);
-      // this hub's candidates among [y0, y0 + 1024), compacted into sh_cand
-      if (threadIdx.x == 0) {
-        sh_cnt = 0;
-        sh_cnt1 = 0;
+    const uint32_t steps = sh_kn * kSubs;
+    for (uint32_t g0 = 0; g0 < steps; g0 += kRowSteps) {
+      uint32_t v[kRowSteps];
+      auto load_slots = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < kRowSteps; ++u) {
+          const uint32_t i = g0 + u;
+          const uint32_t kb = k + kXcds * (i / kSubs);
+          const uint32_t y0 = kb * a.row_block + (i % kSubs) * kPruneThreads;
+          const uint32_t y_end = i < steps ? min(a.n, (kb + 1) * a.row_block) : 0u;
+          if (tid == u) sh_y0[u] = y0;
+          v[u] = y0 + tid < y_end ? a.cand_d[slot_at(a, b, y0 + tid)] : kInf32;
+          row_slots += y0 < y_end ? min(kPruneThreads, y_end - y0) : 0u;
+        }
+      };
+      load_slots();
+      if (tid < kRowSteps) sh_step[tid] = 0;
+      __syncthreads();
+#pragma unroll
+      for (uint32_t u = 0; u < kRowSteps; ++u) {
+        const uint64_t m = __ballot(slot_current(a, v[u]));
+        if (m && lane == 0) atomicAdd(&sh_step[u], (uint32_t)__popcll(m));
       }
       __syncthreads();
-      const uint32_t y = y0 + threadIdx.x;
-      const uint32_t v = y < y_end ? a.cand_d[slot_at(a, b, y)] : kInf32;
-      const bool cand = y < y_end && slot_current(a, v);
-      const unsigned long long m = __ballot(cand);
-      uint32_t base = 0;
-      if (lane == 0 && m) base = atomicAdd(&sh_cnt, (uint32_t)__popcll(m));
-      base = __shfl(base, 0, kWave);
-      if (cand)
-        sh_cand[0][base + (uint32_t)__popcll(m & lt_mask)] =
-            kPacked ? threadIdx.x | (slot_dist(a, v) << 10) : threadIdx.x;
-      __syncthreads();
-      uint32_t cnt = sh_cnt;
-      if (cnt == 0) continue;
-      const uint32_t *found = sh_cand[0];
-      if (lm) {
-        // 64 >> lm_lw candidates per wave step, a row chunk per lane
-        const uint32_t lw = a.lm_lw, per = kWave >> lw, grp = (uint32_t)lane >> lw;
-        const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
-        for (uint32_t i0 = threadIdx.x / kWave * per; i0 < cnt;
-             i0 += kPruneThreads / kWave * per) {
-          const uint32_t i = i0 + grp;
-          const uint32_t e = i < cnt ? sh_cand[0][i] : 0u;
-          const uint4 r = a.lm[((uint64_t)(y0 + (e & 1023u)) << lw) + ll.mine];
-          const uint64_t hit = __ballot(lm_min_sum(r, lm_s) <= (e >> 10));
-          const bool keep = i < cnt && ((uint32_t)lane & ((1u << lw) - 1u)) == 0 &&
-                            ((hit >> lane) & gmask) == 0;
-          const uint64_t km = __ballot(keep);
-          if (!km) continue;
-          uint32_t at = 0;
-          if (lane == 0) at = atomicAdd(&sh_cnt1, (uint32_t)__popcll(km));
-          at = __shfl(at, 0, kWave);
-          if (keep) sh_cand[1][at + (uint32_t)__popcll(km & lt_mask)] = e;
+      for (uint32_t u0 = 0, u1 = 0; u0 < kRowSteps; u0 = u1) {
+        // steps [u0, u1): as many as the list takes
+        uint32_t sum = 0;
+        while (u1 < kRowSteps && sum + sh_step[u1] <= kRowList) sum += sh_step[u1++];
+        if (sum == 0) break;  // nothing left
+        // a later piece loads its slots again (from L2) rather than keep them
+        // in registers over the search
+        if (u0) load_slots();
+        if (tid == 0) {
+          sh_nf = 0;
+          sh_ns = 0;
+          sh_next = 0;
+          sh_acc = 0;
+          sh_touch = 0;
         }
         __syncthreads();
-        lm_tested += cnt;
-        lm_caught += cnt - sh_cnt1;
-        cnt = sh_cnt1;
-        if (cnt == 0) continue;
-        found = sh_cand[1];
-      }
-      auto cands = [&](uint32_t i, uint32_t &yc, uint32_t &dy) {
-        const uint32_t e = found[i];
-        yc = y0 + (e & 1023u);
-        dy = kPacked ? e >> 10 : slot_dist(a, a.cand_d[slot_at(a, b, yc)]);
-      };
-      if (!built) {
-        if (in_lds) {
-          if (tile_b != b) {
-            if (icap)
-              build_idx_tile<V>(a, s, sv, lds, icap, sh_rows);
-            else
-              build_tile<V>(a, s, sv, lds, lcap);
-            tile_b = b;
+#pragma unroll
+        for (uint32_t u = 0; u < kRowSteps; ++u) {
+          if (u < u0 || u >= u1) continue;
+          const bool cand = slot_current(a, v[u]);
+          const uint64_t m = __ballot(cand);
+          if (!m) continue;
+          uint32_t base = 0;
+          if (lane == 0) base = atomicAdd(&sh_nf, (uint32_t)__popcll(m));
+          base = __shfl(base, 0, kWave);
+          if (cand)
+            sh_found[base + (uint32_t)__popcll(m & lt_mask)] =
+                u << 10 | tid | (kPacked ? slot_dist(a, v[u]) << 13 : 0u);
+        }
+        __syncthreads();
+        uint32_t *list = sh_found;
+        uint32_t cnt = sum;
+        if (lm) {
+          // 64 >> lm_lw candidates per wave step, a row chunk per lane
+          const uint32_t lw = a.lm_lw, per = kWave >> lw, grp = lane >> lw;
+          const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
+          for (uint32_t i0 = wv * per; i0 < sum; i0 += kPruneThreads / kWave * per) {
+            const uint32_t i = i0 + grp;
+            const uint32_t e = i < sum ? sh_found[i] : 0u;
+            const uint4 r = a.lm[((uint64_t)vertex(e) << lw) + ll.mine];
+            const uint64_t hit = __ballot(lm_min_sum(r, lm_s) <= (e >> 13));
+            const bool keep = i < sum && (lane & ((1u << lw) - 1u)) == 0 &&
+                              ((hit >> lane) & gmask) == 0;
+            const uint64_t km = __ballot(keep);
+            if (!km) continue;
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&sh_ns, (uint32_t)__popcll(km));
+            at = __shfl(at, 0, kWave);
+            if (keep) sh_surv[at + (uint32_t)__popcll(km & lt_mask)] = e;
+          }
+          __syncthreads();
+          list = sh_surv;
+          cnt = sh_ns;
+          lm_tested += sum;
+          lm_caught += sum - cnt;
+        }
+        if (cnt) {
+          if (!built && tile_b != b) {
+            tile_build<V>(a, s, sv, plan, lds, gkeys, sh_rows);
+            tile_b = plan.kind == kTileArena ? kInf32 : b;
             tile_reads += sv.len;
           }
-        } else {
-          build_tile<V>(a, s, sv, gkeys, cap);
-          // written through L2 (atomics): drop stale L1 lines of the slice
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-          tile_b = kInf32;
-          tile_reads += sv.len;
+          built = true;
+          tile_prune<V, LT>(
+              a, b, 0, cnt,
+              [&](uint32_t i, uint32_t &y, uint32_t &dy) {
+                const uint32_t e = list[i];
+                y = vertex(e);
+                dy = dist_of(e, y);
+              },
+              [&](uint32_t i, uint32_t, uint32_t) { list[i] |= 1u << 31; }, plan, lds, gkeys,
+              sh_next, wave_reads);
         }
-        built = true;
-      }
-      for (uint32_t c0 = 0; c0 < cnt; c0 += a.tile) {
-        const uint32_t c1 = min(cnt, c0 + a.tile);
-        // staged labels are published once this chunk's could overflow them
-        if (sh_acc_n + (c1 - c0) > kAccSlots)
-          publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n,
-                           sh_touch_base);
-        if (threadIdx.x == 0) sh_next = 0;
         __syncthreads();
-        if (icap)
-          prune_candidates<V, LT>(a, b, c0, c1, cands,
-                                  IdxTile{(lds_ptr<const uint32_t>)lds,
-                                          (uint32_t)(uintptr_t)(lds_ptr<const uint32_t>)(lds + icap),
-                                          K1 * (uint32_t)sizeof(V)},
-                                  icap, sh_next, sh_acc_n, sh_acc, wave_reads);
-        else if (in_lds)
-          prune_candidates<V, LT>(a, b, c0, c1, cands, (lds_ptr<const uint32_t>)lds, lcap,
-                                  sh_next, sh_acc_n, sh_acc, wave_reads);
-        else
-          prune_candidates<V, LT>(a, b, c0, c1, cands, (glb_ptr<const uint32_t>)gkeys, cap,
-                                  sh_next, sh_acc_n, sh_acc, wave_reads);
+        // the accepted labels: per-vertex add counts (the count before a label
+        // is its rank among the vertex's new labels, the append's slot past its
+        // list), one reservation each on the frontier and the touched list
+        uint32_t ry[2], rr[2], rd[2], at[2], tat[2];
+        bool acc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const uint32_t i = u * kPruneThreads + tid;
+          const uint32_t e = i < cnt ? list[i] : 0u;
+          acc[u] = e >> 31;
+          ry[u] = rr[u] = rd[u] = at[u] = tat[u] = 0;
+          if (acc[u]) {
+            ry[u] = vertex(e);
+            rd[u] = dist_of(e, ry[u]);
+            rr[u] = atomicAdd(&a.add_cnt[ry[u]], 1u);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const uint64_t m = __ballot(acc[u]), mt = __ballot(acc[u] && rr[u] == 0);
+          if (!m) continue;
+          if (lane == 0) {
+            at[u] = atomicAdd(&sh_acc, (uint32_t)__popcll(m));
+            tat[u] = mt ? atomicAdd(&sh_touch, (uint32_t)__popcll(mt)) : 0u;
+          }
+          at[u] = __shfl(at[u], 0, kWave) + (uint32_t)__popcll(m & lt_mask);
+          tat[u] = __shfl(tat[u], 0, kWave) + (uint32_t)__popcll(mt & lt_mask);
+        }
+        __syncthreads();
+        const uint32_t nacc = sh_acc;
+        if (nacc) {
+          if (tid == 0) {
+            sh_acc_base = atomicAdd(&a.ctrl->fcnt[a.cur ^ 1], nacc);
+            if (sh_acc_base + nacc > a.fcap) atomicOr(&a.ctrl->overflow, kOvfFront);
+            if (sh_touch) sh_touch_base = atomicAdd(&a.ctrl->touched_cnt, sh_touch);
+          }
+          __syncthreads();
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            if (!acc[u]) continue;
+            const uint32_t p = sh_acc_base + at[u];
+            if (p < a.fcap) {
+              Fn[p] = Item{b, ry[u], rd[u]};
+              a.frank[p] = rr[u];
+            }
+            if (rr[u] == 0) a.touched[sh_touch_base + tat[u]] = ry[u];
+          }
+        }
         __syncthreads();
       }
+      __syncthreads();
     }
   }
-  publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
   if (lane == 0 && wave_reads) atomicAdd(&a.ctrl->label_reads, wave_reads);
-  if (threadIdx.x == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
-  if (threadIdx.x == 0 && row_slots) atomicAdd(&a.ctrl->row_slots, row_slots);
-  if (threadIdx.x == 0 && lm_tested) {
+  if (tid == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
+  if (tid == 0 && row_slots) atomicAdd(&a.ctrl->row_slots, row_slots);
+  if (tid == 0 && lm_tested) {
     atomicAdd(&a.ctrl->lm_tested, lm_tested);
     atomicAdd(&a.ctrl->lm_caught, lm_caught);
   }
@@ -2691,6 +2874,8 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     const uint32_t mode = (uint64_t)n <= (1ull << (32 - kIdxBits))
                               ? env_u32("HSDL_PRUNE_INDEXED", 1, 0, 2) : 0u;
     a.idx_tiles = mode == 0 ? kInf32 : mode == 2 ? 0u : kRecSmall;
+    // (either setting of the knob also keeps hash tiles only)
+    a.direct_tiles = getenv("HSDL_PRUNE_INDEXED") ? 0u : 1u;
   }
   a.piece_pairs = env_u32("HSDL_PIECE_PAIRS", 8192, 1, 1u << 16);
   a.lds_slots = lds_slots;

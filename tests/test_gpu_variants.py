@@ -49,3 +49,22 @@ def test_landmark_test_keeps_the_labels(monkeypatch, landmarks, rows):
     monkeypatch.setenv("HSDL_STREAM32", "0")
     g = ragged(1500, 4, 100)
     same_labels(H.hop_constrained_two_hop_labels_generation(g, 4), O.kround(csr_of(g), 4).arrays())
+
+
+@pytest.mark.parametrize("rows,density", [("0", "32"), ("1", "32"), ("2", "32"), ("2", "1")])
+def test_prune_tiles_by_hub_id(monkeypatch, rows, density):
+    """Tiles addressed by hub id (values while the hub range is small, then
+    row indexes, then hashes: 21,001 vertices pass through all three in a
+    build, at a different hub in each round) and row items whose candidates
+    fill the list several times (dense rounds) or leave steps empty: the
+    oracle's labels, with K at both ends of a 3-bit hop field."""
+    monkeypatch.setenv("HSDL_PRUNE_ROWS", rows)
+    monkeypatch.setenv("HSDL_ROW_DENSITY", density)
+    for n, K, wmax, batch, lm in ((21001, 3, 50, 0, "16"), (21001, 3, 50, 1000, "0"),
+                                  (1025, 7, 4, 0, "0"), (4100, 4, 100, 3, "16"),
+                                  (9000, 3, 20000, 4096, "0")):
+        monkeypatch.setenv("HSDL_LANDMARKS", lm)
+        print(f"[tiles] n={n} K={K} batch={batch} rows={rows} landmarks={lm}", flush=True)
+        g = ragged(n, n + K, wmax)
+        same_labels(H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=batch),
+                    O.kround(csr_of(g), K).arrays())
