@@ -115,8 +115,8 @@ struct Ctrl {
   // of their arguments' s0 / B / tag, so one captured batch replays for any
   uint32_t bs0, bB, btag;
   uint32_t lm_on;                // the landmark test runs in this batch
-  unsigned long long lm_tested;  // candidates the landmark test looked at
-  unsigned long long lm_caught;  // of these, pruned by it
+  unsigned long long lm_tested;  // (label, edge) pairs the landmark test looked at
+  unsigned long long lm_caught;  // of these, rejected
 };
 
 // A piece of a large frontier group: its cnt labels (at pool offset off)
@@ -195,9 +195,9 @@ struct GenArgs {
   uint32_t *gtile;
   unsigned long long gtile_cap;  // u32 words
   Ctrl *ctrl;
-  // landmark rows (k_lm_build), 16 << lm_lw bytes per vertex; nullptr: none
+  // landmark chunks (k_lm_build): chunk c of vertex v at lm[c * n + v];
+  // nullptr: none
   const uint4 *lm;
-  uint32_t lm_lw;     // log2 of a row's 16-byte chunks, one lane each
   uint32_t lm_parts;  // chunks per hop (landmarks / 8)
 };
 
@@ -407,6 +407,79 @@ __device__ inline unsigned long long first_above(const uint2 *adj, unsigned long
 // (whole edges) for k_expand_heavy, so no wave is left alone with a large
 // group while the rest of the GPU idles.
 
+// The first hubs of the sequence (8 by default) are landmarks.  For hop x =
+// 1..K-1 and landmark i, a vertex v keeps the smallest distance of landmark
+// i's labels in L(v) of hop <= x (0xFFFF: none), 16 bits each, eight landmarks
+// of one hop to a 16-byte chunk.  The chunks are built once, when the batch
+// that holds the last landmark has finished; later hubs s rank below every
+// landmark, so a landmark's labels in L(s) and L(y) no longer change, and
+//   min over x, i of lm(y)[x][i] + lm(s)[h - x][i] <= d
+// is a witness for a candidate (s, y, d) of round h: the prune would reject
+// it, and every candidate of (s, y) at a larger distance.  Such a pair opens no
+// slot.  (A later round's candidate that a slot would have dropped for it
+// meets the same witness.)  Top-ranked hubs lie on most short walks, so the
+// test rejects most pairs: R-MAT scale 18, K = 5: candidates 636 -> 270
+// million, labels the prune reads 62.7 -> 40 billion, the prune 152 -> 66 ms;
+// a rejected pair costs two cached 16-byte loads per hop in place of a random
+// memory sector of the slots, which binds the expansion.  Builds with 8 / 16 /
+// 24 / 32 landmarks: 236.5 / 245 / 251 / 266 ms (267 with the candidates
+// tested after the expansion, 323 without a test).
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+
+// smallest of the eight saturated 16-bit sums
+__device__ inline uint32_t lm_min_sum(uint4 x, uint4 y) {
+  auto sum = [](uint32_t p, uint32_t q) {
+    return __builtin_elementwise_add_sat(__builtin_bit_cast(us2, p), __builtin_bit_cast(us2, q));
+  };
+  const us2 m = __builtin_elementwise_min(
+      __builtin_elementwise_min(sum(x.x, y.x), sum(x.y, y.y)),
+      __builtin_elementwise_min(sum(x.z, y.z), sum(x.w, y.w)));
+  return min((uint32_t)m.x, (uint32_t)m.y);
+}
+
+// Whether a landmark rejects candidate (s, y, d) of round h > 1.
+__device__ inline bool lm_rejects(const GenArgs &a, uint32_t s, uint32_t y, uint32_t d) {
+  uint32_t m = kInf32;
+  for (uint32_t x = 1; x < a.h; ++x)
+    for (uint32_t p = 0; p < a.lm_parts; ++p)
+      m = min(m, lm_min_sum(a.lm[(uint64_t)((x - 1) * a.lm_parts + p) * a.n + y],
+                            a.lm[(uint64_t)((a.h - x - 1) * a.lm_parts + p) * a.n + s]));
+  return m <= d;
+}
+
+// One wave per vertex; LDS: 32-bit minima per wave.
+__global__ void __launch_bounds__(256) k_lm_build(GenArgs a, uint32_t *lm, uint32_t nlm) {
+  extern __shared__ uint32_t lm_lds[];
+  const uint32_t lane = (uint32_t)lane_id(), wib = threadIdx.x / kWave;
+  const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + wib;
+  const uint32_t nwaves = gridDim.x * (blockDim.x / kWave);
+  const uint32_t per_hop = 8 * a.lm_parts, vals = (a.K - 1) * per_hop;
+  uint32_t *row = lm_lds + wib * vals;
+  for (uint64_t v = wave; v < a.n; v += nwaves) {
+    for (uint32_t i = lane; i < vals; i += kWave) row[i] = 0xFFFFu;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const unsigned long long st = a.seg_start[v];
+    const uint32_t len = a.seg_len[v];
+    for (uint32_t j = lane; j < len; j += kWave) {
+      uint32_t hub, hop, dist;
+      pool_label(a, st + j, hub, hop, dist);
+      uint32_t i = hub;
+      if (a.hubs) {  // the landmark's place among the group's first hubs
+        i = 0;
+        while (i < nlm && a.hubs[i] < hub) ++i;
+        if (i < nlm && a.hubs[i] != hub) i = nlm;
+      }
+      if (i >= nlm || hop == 0) continue;
+      for (uint32_t x = hop; x < a.K; ++x) atomicMin(&row[(x - 1) * per_hop + i], dist);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    // word w of chunk c: values 8 c + 2 w and the next
+    for (uint32_t i = lane; i < vals / 2; i += kWave)
+      lm[((uint64_t)(i / 4) * a.n + v) * 4 + i % 4] = row[2 * i] | (row[2 * i + 1] << 16);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  }
+}
+
 // Flat-list space is reserved per wave in blocks of kListBlock entries (one
 // atomic on the list counter per block instead of one per step); unused
 // tails are filled with empty entries that the counting and grouping skip.
@@ -416,6 +489,7 @@ constexpr unsigned long long kEmptyEntry = ~0ull;
 struct ListRes {
   uint32_t base = 0, used = kListBlock;  // starts exhausted
   uint32_t cands = 0;                    // candidates opened, not yet added to cand_round
+  uint32_t caught = 0;                   // pairs a landmark rejected (per lane)
 };
 
 // Writes empty entries over [base+used, base+kListBlock) (whole wave).
@@ -424,10 +498,20 @@ __device__ inline void list_pad(const GenArgs &a, const ListRes &r) {
     if (r.base + i < a.ccap) a.cflat[r.base + i] = kEmptyEntry;
 }
 
-// End of a kernel: pad the open block and add the wave's candidate count.
-__device__ inline void list_close(const GenArgs &a, const ListRes &r) {
+// End of a kernel: pad the open block and add the wave's counts (edges: pairs
+// this lane relaxed).
+__device__ inline void list_close(const GenArgs &a, const ListRes &r, uint64_t edges) {
   list_pad(a, r);
-  if (lane_id() == 0 && r.cands) atomicAdd(&a.ctrl->cand_round, r.cands);
+  edges = wave_sum_u64(edges);
+  const uint64_t caught = a.lm && a.h > 1 ? wave_sum_u64(r.caught) : 0;
+  if (lane_id() != 0) return;
+  if (r.cands) atomicAdd(&a.ctrl->cand_round, r.cands);
+  if (!edges) return;
+  atomicAdd(&a.ctrl->edge_total, (unsigned long long)edges);
+  if (a.lm && a.h > 1) {
+    atomicAdd(&a.ctrl->lm_tested, (unsigned long long)edges);
+    if (caught) atomicAdd(&a.ctrl->lm_caught, (unsigned long long)caught);
+  }
 }
 
 // A frontier label at pool offset `at`: its hub slot, hub and distance.
@@ -465,6 +549,8 @@ __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uin
     y = ed.x;
     if (y > kh) {  // rank pruning: hub kh labels only vertices ranked below it
       relaxed = true;
+      const bool rejected = a.lm && a.h > 1 && lm_rejects(a, kh, y, kd + ed.y);
+      res.caught += rejected;
       const uint32_t nv = slot_fresh(a, kd + ed.y);
       uint32_t *slot = &a.cand_d[slot_at(a, kb, y)];
       // A slot only falls while the expansion runs (atomicMin; clears happen
@@ -472,7 +558,7 @@ __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uin
       // the atomic would neither change the slot nor open it: most
       // relaxations end with this read, which costs less than a returning
       // atomic.
-      if (nv < *slot) {
+      if (!rejected && nv < *slot) {
         const uint32_t old = atomicMin(slot, nv);
         first = nv < old && slot_opens(a, old);
       }
@@ -618,9 +704,7 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
       }
     }
   }
-  list_close(a, res);
-  edges_seen = wave_sum_u64(edges_seen);
-  if (lane == 0 && edges_seen) atomicAdd(&a.ctrl->edge_total, (unsigned long long)edges_seen);
+  list_close(a, res, edges_seen);
 }
 
 // Heavy pieces: a workgroup takes one piece at a time and spreads its pairs
@@ -663,9 +747,7 @@ __global__ void __launch_bounds__(256) k_expand_heavy(GenArgs a) {
       edges_seen += relax_edge(a, p < pairs && ok, b, hub, d, ed, lt_mask, res);
     }
   }
-  list_close(a, res);
-  edges_seen = wave_sum_u64(edges_seen);
-  if (lane == 0 && edges_seen) atomicAdd(&a.ctrl->edge_total, (unsigned long long)edges_seen);
+  list_close(a, res, edges_seen);
 }
 
 // ------------------------------------------------------------ chunk scan
@@ -690,122 +772,9 @@ __device__ inline bool rows_chosen(const GenArgs &a) {
                                 (uint64_t)cands * a.row_density >= (uint64_t)a.B * a.n));
 }
 
-// -------------------------------------------------------------- landmarks
-// The first hubs of the sequence (16 by default) are landmarks.  Row v holds,
-// for hop x = 1..K-1 and landmark i, the smallest distance of landmark i's
-// labels in L(v) of hop <= x (0xFFFF: none), 16 bits each, hop-major, 8
-// landmarks to a 16-byte chunk.  Rows are built once, when the batch that
-// holds the last landmark has finished; later hubs s rank below every
-// landmark, so a landmark's labels in L(s) and L(y) no longer change, and
-//   min over x, i of row(y)[x][i] + row(s)[h - x][i] <= d
-// is a witness for candidate (s, y, d) of round h: the prune would reject it.
-// Top-ranked hubs lie on most short walks, so this test rejects most of the
-// candidates a prune rejects (83 % on R-MAT scale 16, K = 5) from one
-// 128-byte line each, eight candidates per wave step, where the search takes a
-// wave and about four lines per candidate.  A candidate it does not catch
-// takes the search, so the labels are the same.  R-MAT scale 18, K = 5:
-// labels the prune reads 62.7 -> 40.8 billion, row items 133 -> 100 ms, list
-// items 19 -> 13 ms, the build 319 -> 284 ms (8 landmarks 286 ms, 24 289,
-// 32 287, 64 296: more lines per candidate than they save searches).
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-
-// smallest of the eight saturated 16-bit sums
-__device__ inline uint32_t lm_min_sum(uint4 x, uint4 y) {
-  auto sum = [](uint32_t p, uint32_t q) {
-    return __builtin_elementwise_add_sat(__builtin_bit_cast(us2, p), __builtin_bit_cast(us2, q));
-  };
-  const us2 m = __builtin_elementwise_min(
-      __builtin_elementwise_min(sum(x.x, y.x), sum(x.y, y.y)),
-      __builtin_elementwise_min(sum(x.z, y.z), sum(x.w, y.w)));
-  return min((uint32_t)m.x, (uint32_t)m.y);
-}
-
-// This lane's chunk of a row y in round h, and the chunk of a row s it adds
-// to (hop x with hop h - x); `use` is false for hops the round cannot pair.
-struct LmLane {
-  uint32_t mine, other;
-  bool use;
-};
-__device__ inline LmLane lm_lane(const GenArgs &a) {
-  const uint32_t c = (uint32_t)lane_id() & ((1u << a.lm_lw) - 1u);
-  const uint32_t x = c / a.lm_parts + 1, part = c % a.lm_parts;
-  LmLane l;
-  l.use = x < a.h;
-  l.mine = l.use ? c : 0u;
-  l.other = l.use ? (a.h - x - 1) * a.lm_parts + part : 0u;
-  return l;
-}
-
-// Lane i holds candidate (s, y, d), d = 0 for none (a sum is at least 2);
-// returns whether a landmark rejects it.  U: loads in flight per lane.
-template <int U>
-__device__ inline bool lm_caught(const GenArgs &a, uint32_t s, uint32_t y, uint32_t d) {
-  const uint32_t lane = (uint32_t)lane_id(), lw = a.lm_lw, per_lw = 6 - lw;
-  const uint32_t grp = lane >> lw;
-  const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
-  const LmLane l = lm_lane(a);
-  bool caught = false;
-  for (uint32_t s0 = 0; s0 < (1u << lw); s0 += U) {
-    uint4 ry[U], rs[U];
-    uint32_t dd[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int src = (int)(((s0 + u) << per_lw) + grp);
-      const uint32_t yy = __shfl(y, src, kWave), ss = __shfl(s, src, kWave);
-      dd[u] = l.use ? (uint32_t)__shfl(d, src, kWave) : 0u;
-      ry[u] = a.lm[((uint64_t)yy << lw) + l.mine];
-      rs[u] = a.lm[((uint64_t)ss << lw) + l.other];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t m = __ballot(lm_min_sum(ry[u], rs[u]) <= dd[u]);
-      if ((lane >> per_lw) == s0 + u)
-        caught = ((m >> ((lane & ((1u << per_lw) - 1u)) << lw)) & gmask) != 0;
-    }
-  }
-  return caught;
-}
-__device__ inline bool lm_caught(const GenArgs &a, uint32_t s, uint32_t y, uint32_t d) {
-  return a.lm_lw >= 3 ? lm_caught<8>(a, s, y, d) : lm_caught<2>(a, s, y, d);
-}
-
-// One wave per vertex; LDS: a row of 32-bit minima per wave.
-__global__ void __launch_bounds__(256) k_lm_build(GenArgs a, uint32_t *rows, uint32_t nlm) {
-  extern __shared__ uint32_t lm_lds[];
-  const uint32_t lane = (uint32_t)lane_id(), wib = threadIdx.x / kWave;
-  const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + wib;
-  const uint32_t nwaves = gridDim.x * (blockDim.x / kWave);
-  const uint32_t words = 4u << a.lm_lw;  // two values each
-  const uint32_t per_hop = 8 * a.lm_parts;
-  uint32_t *row = lm_lds + wib * 2 * words;
-  for (uint64_t v = wave; v < a.n; v += nwaves) {
-    for (uint32_t i = lane; i < 2 * words; i += kWave) row[i] = 0xFFFFu;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    const unsigned long long st = a.seg_start[v];
-    const uint32_t len = a.seg_len[v];
-    for (uint32_t j = lane; j < len; j += kWave) {
-      uint32_t hub, hop, dist;
-      pool_label(a, st + j, hub, hop, dist);
-      uint32_t i = hub;
-      if (a.hubs) {  // the landmark's place among the group's first hubs
-        i = 0;
-        while (i < nlm && a.hubs[i] < hub) ++i;
-        if (i < nlm && a.hubs[i] != hub) i = nlm;
-      }
-      if (i >= nlm || hop == 0) continue;
-      for (uint32_t x = hop; x < a.K; ++x) atomicMin(&row[(x - 1) * per_hop + i], dist);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-    for (uint32_t i = lane; i < words; i += kWave)
-      rows[v * words + i] = row[2 * i] | (row[2 * i + 1] << 16);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-  }
-}
-
 // Per-hub candidate counts of a round that takes list items: a workgroup
-// takes 2048 consecutive entries of the flat list, drops those a landmark
-// rejects (they become empty entries), counts the others' hubs in an LDS hash
-// and adds each hub's count with one global atomic.
+// takes 2048 consecutive entries of the flat list, counts their hubs in an
+// LDS hash and adds each hub's count with one global atomic.
 constexpr uint32_t kGroupThreads = 256;
 constexpr uint32_t kGroupPer = 8;                                 // entries per thread
 constexpr uint32_t kGroupChunk = kGroupThreads * kGroupPer;       // 2048
@@ -837,19 +806,10 @@ __global__ void __launch_bounds__(kGroupThreads) k_count(GenArgs a) {
       hcnt[i] = 0;
     }
     __syncthreads();
-    // (not unrolled: the landmark test keeps 16 row loads in flight)
+#pragma unroll
     for (uint32_t r = 0; r < kGroupPer; ++r) {
       const uint64_t i = c0 + r * kGroupThreads + tid;
-      unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
-      if (a.lm && a.h > 1) {
-        const bool some = e != kEmptyEntry;
-        const uint32_t b = (uint32_t)(e >> 32), y = (uint32_t)e;
-        const uint32_t d = some ? slot_dist(a, a.cand_d[slot_at(a, b, y)]) : 0u;
-        if (lm_caught(a, some ? hub_of(a, b) : 0u, some ? y : 0u, d)) {
-          a.cflat[i] = kEmptyEntry;
-          e = kEmptyEntry;
-        }
-      }
+      const unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
       if (e != kEmptyEntry) atomicAdd(&hcnt[group_slot(hkey, (uint32_t)(e >> 32))], 1u);
     }
     __syncthreads();
@@ -914,10 +874,6 @@ __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
     a.ctrl->total_chunks = (dead || rows) ? 0u : run;
     a.ctrl->work_ctr = 0;
     a.ctrl->cand_total += a.ctrl->cand_round;
-    if (!dead && !rows && a.lm && a.h > 1) {
-      a.ctrl->lm_tested += a.ctrl->cand_round;
-      a.ctrl->lm_caught += a.ctrl->cand_round - runc;
-    }
     a.ctrl->item_total += min(a.ctrl->fcnt[a.cur], a.fcap);
   }
 }
@@ -1693,13 +1649,13 @@ k_prune(GenArgs a) {
 //
 // An item's vertices are taken kRowSteps * 1024 at a time: every thread loads
 // its kRowSteps slots at once, the candidates gather in an LDS list (in as
-// few pieces as the list takes), the landmark test thins each piece, and the
-// search runs over up to kRowList survivors.  What binds is the chain of
+// few pieces as the list takes), and the search runs over up to kRowList of
+// them.  What binds is the chain of
 // memory round trips and barriers per step, not bytes or instructions: taken
 // 1024 vertices at a time, R-MAT scale 18 had 10 million steps of 4.5 us.
 constexpr uint32_t kRowSteps = 8;
-// two lists of this beside 64 KB of tile: two workgroups in a CU's 160 KB
-constexpr uint32_t kRowList = 1984;
+// 8 KB beside 64 KB of tile: two workgroups in a CU's 160 KB
+constexpr uint32_t kRowList = 2048;
 static_assert(kRowList >= kPruneThreads && kRowList <= 2 * kPruneThreads, "a step fits; publish");
 
 template <class V, class LT>
@@ -1708,16 +1664,16 @@ k_prune_rows(GenArgs a) {
   with_batch(a);
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t sh_b, sh_k, sh_kn, sh_q, sh_next, sh_rows;
-  __shared__ uint32_t sh_nf, sh_ns, sh_acc, sh_touch, sh_acc_base, sh_touch_base;
+  __shared__ uint32_t sh_nf, sh_acc, sh_touch, sh_acc_base, sh_touch_base;
   __shared__ uint32_t sh_step[kRowSteps];  // candidates of each step
   __shared__ uint32_t sh_y0[kRowSteps];    // first vertex of each step
-  // candidates found, and those past the landmarks: offset in the steps
-  // (13 bits), with 16-bit distances the distance << 13, accepted: bit 31
-  __shared__ uint32_t sh_found[kRowList], sh_surv[kRowList];
+  // candidates: offset in the steps (13 bits), with 16-bit distances the
+  // distance << 13, accepted: bit 31
+  __shared__ uint32_t list[kRowList];
   if (!a.ctrl->row_mode) return;
   constexpr bool kPacked = sizeof(V) == 2;
   static_assert(kPruneThreads == 1024 && kRowSteps == 8, "offsets of 13 bits");
-  const uint32_t lane = (uint32_t)lane_id(), tid = threadIdx.x, wv = tid / kWave;
+  const uint32_t lane = (uint32_t)lane_id(), tid = threadIdx.x;
   Item *Fn = frontier(a, a.cur ^ 1);
   uint32_t tile_b = kInf32;  // hub slot whose tile is in LDS
   unsigned long long wave_reads = 0, tile_reads = 0, row_slots = 0;
@@ -1726,10 +1682,6 @@ k_prune_rows(GenArgs a) {
   const uint32_t nblk = (uint32_t)(((uint64_t)a.n + a.row_block - 1) / a.row_block);
   const uint32_t home = blockIdx.x % kXcds;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
-  const bool lm = kPacked && a.lm && a.h > 1;
-  unsigned long long lm_tested = 0, lm_caught = 0;
-  LmLane ll{0, 0, false};
-  if (lm) ll = lm_lane(a);
   if (tid == 0) sh_q = 0;
   __syncthreads();
   for (;;) {
@@ -1767,8 +1719,6 @@ k_prune_rows(GenArgs a) {
       __syncthreads();
       continue;
     }
-    uint4 lm_s = make_uint4(kInf32, kInf32, kInf32, kInf32);
-    if (lm && ll.use) lm_s = a.lm[((uint64_t)s << a.lm_lw) + ll.other];
     bool built = false;
     auto vertex = [&](uint32_t e) { return sh_y0[(e >> 10) & 7u] + (e & 1023u); };
     auto dist_of = [&](uint32_t e, uint32_t y) {
@@ -1810,7 +1760,6 @@ k_prune_rows(GenArgs a) {
         if (u0) load_slots();
         if (tid == 0) {
           sh_nf = 0;
-          sh_ns = 0;
           sh_next = 0;
           sh_acc = 0;
           sh_touch = 0;
@@ -1826,53 +1775,26 @@ k_prune_rows(GenArgs a) {
           if (lane == 0) base = atomicAdd(&sh_nf, (uint32_t)__popcll(m));
           base = __shfl(base, 0, kWave);
           if (cand)
-            sh_found[base + (uint32_t)__popcll(m & lt_mask)] =
+            list[base + (uint32_t)__popcll(m & lt_mask)] =
                 u << 10 | tid | (kPacked ? slot_dist(a, v[u]) << 13 : 0u);
         }
         __syncthreads();
-        uint32_t *list = sh_found;
-        uint32_t cnt = sum;
-        if (lm) {
-          // 64 >> lm_lw candidates per wave step, a row chunk per lane
-          const uint32_t lw = a.lm_lw, per = kWave >> lw, grp = lane >> lw;
-          const uint64_t gmask = lw == 6 ? ~0ull : (1ull << (1u << lw)) - 1ull;
-          for (uint32_t i0 = wv * per; i0 < sum; i0 += kPruneThreads / kWave * per) {
-            const uint32_t i = i0 + grp;
-            const uint32_t e = i < sum ? sh_found[i] : 0u;
-            const uint4 r = a.lm[((uint64_t)vertex(e) << lw) + ll.mine];
-            const uint64_t hit = __ballot(lm_min_sum(r, lm_s) <= (e >> 13));
-            const bool keep = i < sum && (lane & ((1u << lw) - 1u)) == 0 &&
-                              ((hit >> lane) & gmask) == 0;
-            const uint64_t km = __ballot(keep);
-            if (!km) continue;
-            uint32_t at = 0;
-            if (lane == 0) at = atomicAdd(&sh_ns, (uint32_t)__popcll(km));
-            at = __shfl(at, 0, kWave);
-            if (keep) sh_surv[at + (uint32_t)__popcll(km & lt_mask)] = e;
-          }
-          __syncthreads();
-          list = sh_surv;
-          cnt = sh_ns;
-          lm_tested += sum;
-          lm_caught += sum - cnt;
+        const uint32_t cnt = sum;
+        if (!built && tile_b != b) {
+          tile_build<V>(a, s, sv, plan, lds, gkeys, sh_rows);
+          tile_b = plan.kind == kTileArena ? kInf32 : b;
+          tile_reads += sv.len;
         }
-        if (cnt) {
-          if (!built && tile_b != b) {
-            tile_build<V>(a, s, sv, plan, lds, gkeys, sh_rows);
-            tile_b = plan.kind == kTileArena ? kInf32 : b;
-            tile_reads += sv.len;
-          }
-          built = true;
-          tile_prune<V, LT>(
-              a, b, 0, cnt,
-              [&](uint32_t i, uint32_t &y, uint32_t &dy) {
-                const uint32_t e = list[i];
-                y = vertex(e);
-                dy = dist_of(e, y);
-              },
-              [&](uint32_t i, uint32_t, uint32_t) { list[i] |= 1u << 31; }, plan, lds, gkeys,
-              sh_next, wave_reads);
-        }
+        built = true;
+        tile_prune<V, LT>(
+            a, b, 0, cnt,
+            [&](uint32_t i, uint32_t &y, uint32_t &dy) {
+              const uint32_t e = list[i];
+              y = vertex(e);
+              dy = dist_of(e, y);
+            },
+            [&](uint32_t i, uint32_t, uint32_t) { list[i] |= 1u << 31; }, plan, lds, gkeys,
+            sh_next, wave_reads);
         __syncthreads();
         // the accepted labels: per-vertex add counts (the count before a label
         // is its rank among the vertex's new labels, the append's slot past its
@@ -1930,10 +1852,6 @@ k_prune_rows(GenArgs a) {
   if (lane == 0 && wave_reads) atomicAdd(&a.ctrl->label_reads, wave_reads);
   if (tid == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
   if (tid == 0 && row_slots) atomicAdd(&a.ctrl->row_slots, row_slots);
-  if (tid == 0 && lm_tested) {
-    atomicAdd(&a.ctrl->lm_tested, lm_tested);
-    atomicAdd(&a.ctrl->lm_caught, lm_caught);
-  }
 }
 
 // -------------------------------------------------------- reserve / append
@@ -2312,7 +2230,7 @@ struct Gen {
   DevBuf cflat, cgroup, hub_ccnt, hub_off, hub_cur, chunk_off, F0, F1, gtile, ctrl, heavy;
   DevBuf exp_keys, exp_sorted, exp_tmp;  // export: 32-bit keys, sorted keys, sort space
   DevBuf frank;                          // ranks of the next frontier's items
-  DevBuf lm;                             // landmark rows (k_lm_build)
+  DevBuf lm;                             // landmark chunks (k_lm_build)
   bool lm_on = false;
   uint64_t budget = 0;  // device bytes the build may hold
   uint64_t fixed = 0;   // per-vertex state and the dense slots
@@ -2340,7 +2258,7 @@ struct Gen {
            frank.bytes +
            gtile.bytes + sort_tmp.bytes + sort_tmp32.bytes;
   }
-  // Whether the build may hold `want` bytes beside the landmark rows; the
+  // Whether the build may hold `want` bytes beside the landmark chunks; the
   // rows only save time, so they go when the build needs their room.
   bool fits(uint64_t want) {
     if (want > budget) return false;
@@ -2936,18 +2854,15 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     c0v.pool_top = (unsigned long long)n * c0;
     HSDL_HIP(hipMemcpyAsync(g.ctrl.p, &c0v, sizeof(Ctrl), hipMemcpyHostToDevice, g.st));
   }
-  // landmark rows: 16-bit distances, at least two hops and two batches, not
-  // in the plain form (whose rounds are launch latency).  Tuning knob
+  // landmarks: 16-bit distances, at least two hops and two batches, not in
+  // the plain form (whose rounds are launch latency).  Tuning knob
   // HSDL_LANDMARKS: their count, in eights, 0 for none.
   uint32_t nlm = 0;
   if (g.small_vals && K >= 2 && !plain) {
-    a.lm_parts = env_u32("HSDL_LANDMARKS", 16, 0, 64) / 8;
-    a.lm_lw = 0;
-    while ((1u << a.lm_lw) < (K - 1) * a.lm_parts) ++a.lm_lw;
+    a.lm_parts = env_u32("HSDL_LANDMARKS", 8, 0, 64) / 8;
     nlm = std::min(8 * a.lm_parts, nhubs);
-    const uint64_t bytes = (uint64_t)n * (16ull << a.lm_lw);
-    if (nlm && a.lm_lw <= 6 && a.lm_lw >= 1 && g.held() + bytes <= g.budget &&
-        g.take(kScLm, bytes) == HSDL_OK)
+    const uint64_t bytes = (uint64_t)n * 16 * (K - 1) * a.lm_parts;
+    if (nlm && g.held() + bytes <= g.budget && g.take(kScLm, bytes) == HSDL_OK)
       a.lm = g.lm.as<uint4>();
   }
   hipLaunchKernelGGL(k_init_labels, dim3(1024), dim3(256), 0, g.st, a, c0);
@@ -3094,7 +3009,8 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     if (g.lm_on && tested >= 4096 && (c.lm_caught - c_ok.lm_caught) * 8 < tested) g.lm_on = false;
     c_ok = c;
     if (g.a.lm && s0 < nlm && s0 + B >= nlm && s0 + B < nhubs) {
-      hipLaunchKernelGGL(k_lm_build, dim3(g.grid), dim3(256), (size_t)128 << g.a.lm_lw, g.st, g.a,
+      hipLaunchKernelGGL(k_lm_build, dim3(g.grid), dim3(256),
+                         (size_t)4 * (K - 1) * 8 * g.a.lm_parts * 4, g.st, g.a,
                          g.lm.as<uint32_t>(), nlm);
       HSDL_HIP(hipGetLastError());
       g.lm_on = true;
