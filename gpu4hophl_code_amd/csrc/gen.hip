@@ -143,6 +143,7 @@ struct GenArgs {
   uint32_t claim_max;    // candidates a prune wave claims at once, at most
   uint32_t idx_tiles;    // LDS tiles of more labels than this are indexed (kInf32: none)
   uint32_t direct_tiles; // LDS tiles addressed by hub id, where they fit
+  uint32_t group_min;    // least frontier groups per chunk of the light expansion
   uint32_t heavy_pairs;  // frontier groups with more pairs go to heavy pieces
   uint32_t piece_pairs;  // pairs per heavy piece (whole edges)
   uint32_t lds_slots;  // LDS tile capacity (slots)
@@ -533,6 +534,33 @@ __device__ inline void frontier_label(const GenArgs &a, unsigned long long at, u
   }
 }
 
+// Appends (kb, y) to the flat list for the lanes with `first` (all lanes of
+// the wave).
+__device__ inline void list_open(const GenArgs &a, bool first, uint32_t kb, uint32_t y,
+                                 unsigned long long lt_mask, ListRes &res) {
+  const int lane = lane_id();
+  const unsigned long long firsts = __ballot(first);
+  if (firsts) {
+    const uint32_t cnt = (uint32_t)__popcll(firsts);
+    if (res.used + cnt > kListBlock) {
+      list_pad(a, res);
+      uint32_t nb = 0;
+      if (lane == 0) nb = atomicAdd(&a.ctrl->ccnt, kListBlock);
+      res.base = __shfl(nb, 0, kWave);
+      res.used = 0;
+    }
+    if (first) {
+      const uint32_t pos = res.base + res.used + (uint32_t)__popcll(firsts & lt_mask);
+      if (pos < a.ccap)
+        a.cflat[pos] = ((unsigned long long)kb << 32) | y;
+      else
+        atomicOr(&a.ctrl->overflow, kOvfCand);
+    }
+    res.used += cnt;
+    res.cands += cnt;
+  }
+}
+
 // Relaxes edge ed = (vertex, weight) for hub slot kb (hub kh) at distance
 // kd, when valid and the edge's vertex ranks below the hub: atomicMin on the
 // tagged slot; first touches that undercut earlier rounds go to the flat list
@@ -542,7 +570,6 @@ __device__ inline void frontier_label(const GenArgs &a, unsigned long long at, u
 __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uint32_t kh,
                                   uint32_t kd, uint2 ed, unsigned long long lt_mask,
                                   ListRes &res) {
-  const int lane = lane_id();
   bool first = false, relaxed = false;
   uint32_t y = 0;
   if (valid) {
@@ -564,26 +591,7 @@ __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uin
       }
     }
   }
-  const unsigned long long firsts = __ballot(first);
-  if (firsts) {
-    const uint32_t cnt = (uint32_t)__popcll(firsts);
-    if (res.used + cnt > kListBlock) {
-      list_pad(a, res);
-      uint32_t nb = 0;
-      if (lane == 0) nb = atomicAdd(&a.ctrl->ccnt, kListBlock);
-      res.base = __shfl(nb, 0, kWave);
-      res.used = 0;
-    }
-    if (first) {
-      const uint32_t pos = res.base + res.used + (uint32_t)__popcll(firsts & lt_mask);
-      if (pos < a.ccap)
-        a.cflat[pos] = ((unsigned long long)kb << 32) | y;
-      else
-        atomicOr(&a.ctrl->overflow, kOvfCand);
-    }
-    res.used += cnt;
-    res.cands += cnt;
-  }
+  list_open(a, first, kb, y, lt_mask, res);
   return relaxed;
 }
 
@@ -606,8 +614,18 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   ListRes res;
   const uint32_t wave_id = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
+  // groups per chunk: 64 once that leaves every wave a chunk; smaller rounds
+  // spread over the waves, since a chunk's steps are a chain of memory round
+  // trips (64 groups of up to heavy_pairs pairs took a wave 60 us, which was
+  // the whole round on graphs of a few thousand vertices and on grids)
+  // -- but no chunk below about 64 edges, or the waves' claims on the flat list
+  // cost more than the chains (builds at 1,024 / 4,096 vertices and the
+  // 1024 x 1024 grid: one group and up 2.55 / 5.1 / 426 ms, 32 edges 2.57 /
+  // 4.84 / 367, 64 2.60 / 4.79 / 343, 128 2.77 / 5.0 / 344, 256 2.83 / 5.4 /
+  // 363, always 64 groups 2.93 / 6.15 / 363)
+  const uint32_t gw = min((uint32_t)kWave, max(a.group_min, (gcnt + nwaves - 1) / nwaves));
   for (bool first = true;; first = false) {
-    // chunks of 64 groups: a wave's first chunk is its own id and later ones
+    // chunks of gw groups: a wave's first chunk is its own id and later ones
     // come from a counter (waves with nothing to do never touch it; dealing
     // the chunks to XCDs in contiguous ranges instead cost every wave its
     // claims even in small rounds: the 1024x1024 grid's expansion took
@@ -617,13 +635,13 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
       if (lane == 0) chunk = nwaves + atomicAdd(&a.ctrl->expand_ctr, 1u);
       chunk = __shfl(chunk, 0, kWave);
     }
-    const uint64_t base = (uint64_t)chunk * kWave;
+    const uint64_t base = (uint64_t)chunk * gw;
     if (base >= gcnt) break;
     const uint64_t i = base + lane;
     uint32_t gc = 0, pairs = 0;
     unsigned long long goff = 0, beg = 0, deg = 0;
     bool kept = false;  // a large group this wave expands itself (heavy list full)
-    if (i < gcnt) {
+    if ((uint32_t)lane < gw && i < gcnt) {
       const FGroup gr = G[i];
       gc = gr.cnt;
       goff = gr.off;
@@ -707,19 +725,29 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   list_close(a, res, edges_seen);
 }
 
-// Heavy pieces: a workgroup takes one piece at a time and spreads its pairs
-// over its 256 lanes, edge-major like k_expand.
+// Heavy pieces: a workgroup takes one piece at a time.  A lane keeps one
+// label of the group (its hub, distance, slot base and the hub's landmark
+// chunks) in registers over all the edges its wave walks, so a pair costs an
+// edge load and the vertex's chunks, which the lanes on one edge share, and the
+// slot read of a pair no landmark rejects; walking the pairs edge-major took
+// a label load, a division and the hub's chunks per pair (R-MAT scale 18:
+// 62 -> 42 ms over its build, 4 edge steps at a time; 2: 45 ms).  Groups of at most 32 labels put several edges side by side.
+constexpr uint32_t kLmHeld = 4;  // chunks of its hub a lane holds
+constexpr int kHeavySteps = 4;   // edge steps with their loads in flight together
 __global__ void __launch_bounds__(256) k_expand_heavy(GenArgs a) {
   with_batch(a);
   __shared__ uint32_t sh_h;
   if (a.ctrl->overflow) return;
-  const int lane = lane_id();
-  const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const uint32_t wv = threadIdx.x / kWave;
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const uint32_t wv = threadIdx.x / kWave, nwv = 256 / kWave;
   const uint32_t cnt = min(a.ctrl->heavy_cnt, a.heavy_cap);
   if (blockIdx.x >= cnt) return;  // uniform: most launches find no pieces
   ListRes res;
   uint64_t edges_seen = 0;
+  const bool lm = a.lm && a.h > 1;
+  const uint32_t chunks = lm ? (a.h - 1) * a.lm_parts : 0u;
+  const bool held = chunks <= kLmHeld;
   for (bool first = true;; first = false) {
     // a workgroup's first piece is its own id and later ones come from a
     // counter
@@ -730,21 +758,89 @@ __global__ void __launch_bounds__(256) k_expand_heavy(GenArgs a) {
     __syncthreads();
     if (h >= cnt) break;
     const HeavyItem it = a.heavy[h];
-    // pairs <= max(piece_pairs, cnt) < 2^32; whole waves iterate together so
-    // the ballots see every lane
-    const uint32_t kc = max(1u, it.cnt);
-    const uint32_t pairs = it.cnt * it.ecnt;
-    for (uint32_t pb = wv * kWave; pb < pairs; pb += 256) {
-      const uint32_t p = pb + (uint32_t)lane;
-      const uint32_t q = p / kc;
+    // 2^lg lanes per edge, one label each
+    const uint32_t lg = it.cnt > 32 ? 6u : it.cnt > 1 ? 32u - (uint32_t)__builtin_clz(it.cnt - 1) : 0u;
+    const uint32_t per = kWave >> lg;  // edges per wave step
+    for (uint32_t l0 = 0; l0 < it.cnt; l0 += kWave) {
+      const uint32_t r = l0 + (lane & ((1u << lg) - 1u));
       uint32_t b = 0, hub = 0, d = 0;
       bool ok = false;
-      uint2 ed = make_uint2(0u, 0u);
-      if (p < pairs) {
-        ed = a.adj[it.beg + q];
-        frontier_label(a, it.off + (p - q * kc), b, hub, d, ok);
+      frontier_label(a, it.off + min(r, it.cnt - 1), b, hub, d, ok);
+      ok = ok && r < it.cnt;
+      const uint64_t sbase = ok ? slot_at(a, b, 0) : 0;
+      uint4 ls[kLmHeld];  // chunk c's partner in the hub: hop h - x, same landmarks
+      if (held) {
+#pragma unroll
+        for (uint32_t c = 0; c < kLmHeld; ++c) {
+          const uint32_t part = c % max(1u, a.lm_parts), x = c / max(1u, a.lm_parts) + 1;
+          if (c < chunks)
+            ls[c] = a.lm[(uint64_t)((a.h - x - 1) * a.lm_parts + part) * a.n + (ok ? hub : 0u)];
+        }
       }
-      edges_seen += relax_edge(a, p < pairs && ok, b, hub, d, ed, lt_mask, res);
+      for (uint32_t e0 = wv * per; e0 < it.ecnt; e0 += nwv * per * kHeavySteps) {
+        uint2 ed[kHeavySteps];
+        bool go[kHeavySteps];
+        uint32_t nv[kHeavySteps];
+#pragma unroll
+        for (int u = 0; u < kHeavySteps; ++u) {
+          const uint32_t e = e0 + u * nwv * per + (lane >> lg);
+          ed[u] = a.adj[it.beg + min(e, it.ecnt - 1)];
+          go[u] = ok && e < it.ecnt;
+        }
+#pragma unroll
+        for (int u = 0; u < kHeavySteps; ++u) {
+          go[u] = go[u] && ed[u].x > hub;  // rank pruning
+          edges_seen += go[u];
+          nv[u] = d + ed[u].y;
+        }
+        if (held) {
+          uint32_t m[kHeavySteps];
+#pragma unroll
+          for (int u = 0; u < kHeavySteps; ++u) m[u] = kInf32;
+#pragma unroll
+          for (uint32_t c = 0; c < kLmHeld; ++c) {
+            if (c >= chunks) break;
+            uint4 ly[kHeavySteps];
+#pragma unroll
+            for (int u = 0; u < kHeavySteps; ++u) ly[u] = a.lm[(uint64_t)c * a.n + ed[u].x];
+#pragma unroll
+            for (int u = 0; u < kHeavySteps; ++u) m[u] = min(m[u], lm_min_sum(ly[u], ls[c]));
+          }
+#pragma unroll
+          for (int u = 0; u < kHeavySteps; ++u) {
+            const bool rejected = go[u] && m[u] <= nv[u];
+            res.caught += rejected;
+            go[u] = go[u] && !rejected;
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < kHeavySteps; ++u) {
+            if (go[u] && lm_rejects(a, hub, ed[u].x, nv[u])) {
+              ++res.caught;
+              go[u] = false;
+            }
+          }
+        }
+        // the slots: a read first, an atomic only where it would lower the
+        // slot (relax_edge)
+        uint32_t old[kHeavySteps];
+#pragma unroll
+        for (int u = 0; u < kHeavySteps; ++u) {
+          nv[u] = slot_fresh(a, nv[u]);
+          old[u] = 0;
+          if (go[u]) old[u] = a.cand_d[sbase + ((uint64_t)ed[u].x << a.slot_lw)];
+        }
+#pragma unroll
+        for (int u = 0; u < kHeavySteps; ++u) {
+          bool opened = false;
+          if (nv[u] < old[u]) {  // old is 0 where no slot was read
+            const uint32_t was =
+                atomicMin(&a.cand_d[sbase + ((uint64_t)ed[u].x << a.slot_lw)], nv[u]);
+            opened = nv[u] < was && slot_opens(a, was);
+          }
+          list_open(a, opened, b, ed[u].x, lt_mask, res);
+        }
+      }
     }
   }
   list_close(a, res, edges_seen);
@@ -2775,13 +2871,14 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   // tuning knob HSDL_ROW_BLOCK: vertices per y-block, rounded to 1024
   a.row_block = ((env_u32("HSDL_ROW_BLOCK", 2048, 1024, 1u << 20) + 1023) / 1024) * 1024;
   // tuning knobs HSDL_HEAVY_PAIRS, HSDL_PIECE_PAIRS: (label, edge) pairs of a
-  // frontier group above which it is cut into heavy pieces, and per piece
-  // (a wave's light groups then hold at most 64 * heavy_pairs pairs).  Swept
-  // on R-MAT scale 18 / 20, K=5, expansion seconds: 256 / 2048 0.093 / 0.91,
-  // 256 / 8192 0.083 / 0.62, 512 / 16384 0.089 / 0.60, 1024 / 16384 0.099 /
-  // 0.66, 128 / 1024 0.13 / 1.44 (every 64 groups of a wave wait for its
-  // largest, so big light groups idle lanes; small pieces cost a claim each)
-  a.heavy_pairs = env_u32("HSDL_HEAVY_PAIRS", 256, 1, 1u << 16);
+  // frontier group above which it is cut into heavy pieces, and per piece.
+  // Builds of R-MAT scale 18 and at 40,001 and 4,096 vertices: 128 / 8192
+  // 232 / 48.3 / 5.3 ms, 256 / 8192 227.5 / 47.2 / 5.2, 512 / 8192 225.5 / 46.5 /
+  // 5.1, 1024 / 16384 227 / 46.0 / 5.9; 256 / 16384 226.5 / 47.2 / 5.1, 256 /
+  // 32768 227 / 47.4 / 5.1
+  a.group_min = (uint32_t)std::min<uint64_t>(
+      64, std::max<uint64_t>(1, 64ull * n / std::max<uint64_t>(1, hg->off[n])));
+  a.heavy_pairs = env_u32("HSDL_HEAVY_PAIRS", 512, 1, 1u << 16);
   // tuning knob HSDL_CLAIM_MAX: candidates a prune wave claims at once
   // (R-MAT scale 20 builds: 2 4.33 s, 4 4.27 s, 8 4.25 s, 16 4.24 s; scale
   // 18 the same within 1 %)
@@ -2795,7 +2892,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     // (either setting of the knob also keeps hash tiles only)
     a.direct_tiles = getenv("HSDL_PRUNE_INDEXED") ? 0u : 1u;
   }
-  a.piece_pairs = env_u32("HSDL_PIECE_PAIRS", 8192, 1, 1u << 16);
+  a.piece_pairs = env_u32("HSDL_PIECE_PAIRS", 16384, 1, 1u << 16);
   a.lds_slots = lds_slots;
   DevBuf hubs_buf, in_group;
   if (group) {

@@ -68,3 +68,24 @@ def test_prune_tiles_by_hub_id(monkeypatch, rows, density):
         g = ragged(n, n + K, wmax)
         same_labels(H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=batch),
                     O.kround(csr_of(g), K).arrays())
+
+
+@pytest.mark.parametrize("heavy,piece", [("1", "64"), ("1", "65536"), ("40", "300"), ("65536", "1")])
+def test_expansion_shapes(monkeypatch, heavy, piece):
+    """Frontier groups as pieces of a workgroup (every group, in pieces of an
+    edge and of all edges; groups of one label to a few hundred, so 1 to 64
+    lanes share an edge) and by waves (chunks of one group and more), with the
+    hub's landmark chunks held in registers (few hops) and read per pair (many,
+    or several chunks per hop): the oracle's labels."""
+    monkeypatch.setenv("HSDL_HEAVY_PAIRS", heavy)
+    monkeypatch.setenv("HSDL_PIECE_PAIRS", piece)
+    for n, K, wmax, lm in ((2500, 4, 100, "8"), (700, 7, 3, "8"), (1500, 4, 20, "24"),
+                           (300, 3, 30000, "8"), (65, 2, 5, "8")):
+        monkeypatch.setenv("HSDL_LANDMARKS", lm)
+        print(f"[expansion] n={n} K={K} landmarks={lm} heavy={heavy} piece={piece}", flush=True)
+        g = ragged(n, n + K, wmax, 16)
+        for batch in (0, 33):
+            same_labels(H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=batch),
+                        O.kround(csr_of(g), K).arrays())
+    g = H.Graph.grid(37, 41, 5, 1, 300)
+    same_labels(H.hop_constrained_two_hop_labels_generation(g, 6), O.kround(csr_of(g), 6).arrays())
