@@ -219,11 +219,13 @@ struct hsdl_index {
   hsdl::DevBuf par;  // u32[total]: parent vertex of each label (has_parents)
   bool has_parents = false;
   bool cleaned = false;
+  bool hubs_below = false;  // some label's hub may rank below its vertex (imported sets)
   hsdl_stats stats{};
   uint32_t dist_max = hsdl::kMaxDist;  // bound on every label's dist
   // Query copy of `lab`: hub << (hop_bits + dist_bits) | hop << dist_bits |
-  // dist in 32 bits (same per-vertex order), made by the first query call that
-  // may allocate when the fields fit; released whenever `lab` changes.
+  // dist in 32 bits, every list in hop order, then K prefix counts per vertex,
+  // made by the first query call that may allocate when the fields fit;
+  // released whenever `lab` changes.
   // q32: 0 not made yet, 1 made, 2 does not fit or switched off.
   mutable hsdl::DevBuf lab32;
   mutable std::atomic<uint32_t> q32{0};  // set with release after the fields below

@@ -155,11 +155,14 @@ static int index_from_labels_body(uint32_t n, uint8_t K, const uint64_t *off, co
     dist_max = std::max(dist_max, (uint32_t)dist[i]);
   }
   // per-vertex (hub, hop, dist) order; one label per (hub, hop)
+  bool below = false;
   for (uint32_t v = 0; v < n; ++v) {
     std::sort(lab.begin() + off[v], lab.begin() + off[v + 1]);
     for (uint64_t i = off[v] + 1; i < off[v + 1]; ++i)
       if ((lab[i] >> kDistBits) == (lab[i - 1] >> kDistBits))
         return fail(HSDL_EINVAL, "two labels with the same (hub, hop) at one vertex");
+    // (sorted by hub: the last one is the largest)
+    if (off[v + 1] > off[v] && label_hub(lab[off[v + 1] - 1]) > v) below = true;
     for (uint64_t i = off[v]; i < off[v + 1]; ++i)
       if (label_hop(lab[i]) == 0 && (label_hub(lab[i]) != v || label_dist(lab[i]) != 0))
         return fail(HSDL_EINVAL, "a hop-0 label must be the vertex's self label (v,0,0)");
@@ -173,6 +176,7 @@ static int index_from_labels_body(uint32_t n, uint8_t K, const uint64_t *off, co
   idx->K = K;
   idx->total = total;
   idx->dist_max = dist_max;
+  idx->hubs_below = below;
   if ((rc = idx->off.alloc(sizeof(uint64_t) * (n + 1ull))) ||
       (rc = idx->lab.alloc(sizeof(uint64_t) * std::max<uint64_t>(total, 1)))) {
     delete idx;

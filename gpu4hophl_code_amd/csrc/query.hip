@@ -8,30 +8,43 @@
 // The reference's GPU query (Query_mdnd/src/gpu_query.cu:5-177) launches three
 // kernels per query; here one launch answers a whole batch.
 //
-// One workgroup of four wavefronts per query, in a persistent loop over the
-// batch (workgroup g takes queries g, g+G, g+2G, ...).  Two paths:
-//  * merge path (|L(s)| + |L(t)| <= 4094): both lists are staged in LDS as
-//    packed labels, then the 256 lanes split the merged hub order evenly
-//    (merge path: each lane binary-searches its start on the diagonal and
-//    walks ceil(total/256) merged positions).  The shorter list A is the
-//    probing side: an element of A, met at B position j (= first B label
-//    with hub >= its hub, since A goes first on equal hubs), walks B's run of
-//    that hub (<= K+1 labels, hops ascending) while h1 + h2 <= k.
-//  * long path (longer pairs): the hubs of the longer list B are staged in
-//    LDS -- all of them up to 8188, else every stride-th one (a skip index);
-//    lanes take A 256 labels at a time, binary-search each hub in LDS (plus
-//    at most log2(stride) global probes) and walk B's run in global memory.
-// Memory latency is hidden by software pipelining across the workgroup's
-// queries: while query i is joined out of LDS, the labels of query i+1
-// (16 per lane in registers), the label offsets of query i+2 and the
-// (s,t,k) of query i+3 are in flight.  The prefetches are vector loads by
-// lane 0 of each wave (broadcast with readfirstlane), so they never hold up
-// the LDS waits of the join.  A min-reduction over the four waves gives the
-// answer.
+// A wavefront per query, with its own slice of LDS and no barriers, in one of
+// two forms.  A wave takes up to 64 consecutive queries of the batch at a time,
+// as many as leave every resident wave some: their requests are one coalesced
+// load and their answers one store, which counts where the server's requests
+// lie in host memory.
+//
+// k_query32 reads the index's 32-bit query copy, which keeps every list by hop
+// with prefix counts.  With a and b the endpoints (a's list the shorter one)
+// and c = k / 2, a pair falls in one of
+//   h1 in 1..c,     h2 in 1..k-1:    a's labels of hop 1..c are hashed by hub,
+//                                    b's labels of hop 1..k-1 probe them;
+//   h1 in c+1..k-1, h2 in 1..k-1-c:  b's labels of hop 1..k-1-c are hashed,
+//                                    a's labels of hop c+1..k-1 probe them;
+//   h1 = 0 or h2 = 0:                a label of hub a in L(b), or of hub b in
+//                                    L(a), with the other's self label.
+// Most labels have hops 2 and 3, so a query with k < K reads a part of its
+// lists and hashes a smaller one.  Labels of hop k matter only for hub a or b,
+// which ranks above the list's vertex: only the lower-ranked endpoint's list is
+// read that far, unless the index holds hubs ranked below their vertex
+// (imported label sets may).  A part of more labels than half the table is
+// hashed and probed in pieces.  What binds is instructions (a probe about 15
+// for 64 labels, a turn of its chain 10): 2^22 queries of an R-MAT 262,144
+// index at K = 5 (672 labels per list, k uniform in 1..5) take 5.98 ms, 701 M
+// q/s; a workgroup of four waves per query, with both whole lists in registers
+// and LDS, took 19.2 ms.  512 or 2,048 table slots per wave: 13.4 and 10.2 ms
+// (chunked parts; fewer waves resident).
+//
+// k_query64 reads the index's 8-byte labels, in (hub, hop, dist) order, where
+// there is no copy (fields wider than 32 bits, no memory, none made yet).  The
+// longer list is staged in LDS in pieces of 512 labels, and the shorter one's
+// labels whose hubs lie in the piece's range search it.  The same
+// 2^22 queries without the copy: 23.7 -> 10.9 ms; 100,003 queries on a 384 x 401
+// grid's index (63 labels per list, K = 8) from host arrays: 0.51 -> 0.18 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <climits>
+#include <cstdio>
 #include <mutex>
 #include <vector>
 
@@ -39,311 +52,290 @@
 
 namespace hsdl {
 
-constexpr uint32_t kQThreads = 256;                 // four wavefronts per query
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kQThreads = 256;  // four queries
 constexpr uint32_t kQWaves = kQThreads / kWave;
-constexpr uint32_t kStageWords = 4096;              // 32 KB of LDS per workgroup
-constexpr uint32_t kMergeCap = kStageWords - 2;     // last 16 B hold the wave minima
-constexpr uint32_t kLongHubs = 2 * kMergeCap;       // hubs of B staged on the long path
-constexpr uint32_t kLoadPerLane = kStageWords / kQThreads;  // 16 labels in flight per lane
 
-template <class Getter>
-__device__ inline uint32_t lower_bound_by(Getter get, uint32_t len, uint32_t w) {
-  uint32_t lo = 0, hi = len;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (get(mid) < w) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-__device__ inline uint32_t lane_u32(uint32_t v, int l) { return __builtin_amdgcn_readlane(v, l); }
-__device__ inline uint64_t lane_u64(uint64_t v, int l) {
-  return ((uint64_t)lane_u32((uint32_t)(v >> 32), l) << 32) | lane_u32((uint32_t)v, l);
-}
-
-// Prefetch loads.  Lanes 0-2 load (s, t, k) of a query and lanes 0-3 its two
-// label ranges; the per-lane addresses keep them vector loads (a scalar load
-// would share the wait counter of the LDS traffic and stall the join).
-__device__ inline uint32_t load_params(uint32_t lane, uint64_t x, const uint32_t *qs,
-                                       const uint32_t *qt, const int8_t *qk) {
-  uint32_t v = 0;
-  if (lane < 2) v = (lane == 0 ? qs : qt)[x];
-  else if (lane == 2) v = (uint32_t)(int32_t)qk[x];
-  return v;
-}
-__device__ inline uint64_t load_ranges(uint32_t lane, const unsigned long long *off, uint32_t s,
-                                       uint32_t t) {
-  uint64_t v = 0;
-  if (lane < 4) v = off[((lane & 2) ? t : s) + (lane & 1)];
-  return v;
-}
-
-// Label formats the kernel reads: the index's 8-byte labels, or its 32-bit
-// query copy (hub << (hop_bits + dist_bits) | hop << dist_bits | dist, same
-// per-vertex order), which halves the bytes, the registers of the label
-// prefetch and the LDS of the staging.
-struct Lab64 {
-  using T = unsigned long long;
-  __device__ uint32_t hub(T l) const { return label_hub(l); }
-  __device__ uint32_t hop(T l) const { return label_hop(l); }
-  __device__ uint32_t dist(T l) const { return label_dist(l); }
-};
+// The query copy's labels: hub << (hop_bits + dist_bits) | hop << dist_bits |
+// dist.  No label of hop >= 1 is 0.
 struct Lab32 {
-  using T = uint32_t;
   uint32_t db, hsh, hmask, dmask;  // dist bits, hop + dist bits, field masks
-  __device__ uint32_t hub(T l) const { return l >> hsh; }
-  __device__ uint32_t hop(T l) const { return (l >> db) & hmask; }
-  __device__ uint32_t dist(T l) const { return l & dmask; }
+  __device__ uint32_t hub(uint32_t l) const { return l >> hsh; }
+  __device__ uint32_t hop(uint32_t l) const { return (l >> db) & hmask; }
+  __device__ uint32_t dist(uint32_t l) const { return l & dmask; }
 };
 
-// A query after its (s,t,k) and label offsets are known; uniform over the
-// workgroup.  fixed >= 0 is an answer that needs no join.
-template <class T>
-struct QJob {
-  const T *A, *B;
-  uint32_t ls, lt, kk;
-  int32_t fixed;
+// Queries a wave takes at a time.
+struct QChunk {
+  uint32_t per;
+  __device__ QChunk(uint64_t nq, uint64_t waves)
+      : per((uint32_t)min<uint64_t>(kWave, (nq + waves - 1) / waves)) {}
 };
 
-__device__ inline bool needs_join(uint32_t n, uint32_t s, uint32_t t, int k) {
-  return k > 0 && s < n && t < n && s != t;
-}
-
-template <class T>
-__device__ inline QJob<T> make_job(uint32_t n, const T *lab, uint32_t s, uint32_t t, int k,
-                                   uint64_t sb, uint64_t se, uint64_t tb, uint64_t te) {
-  QJob<T> j;
-  j.A = j.B = lab;
-  j.ls = j.lt = 0;
-  j.kk = 0;
-  if (!needs_join(n, s, t, k)) {
-    j.fixed = (k >= 0 && s == t && s < n) ? 0 : INT32_MAX;
-    return j;
-  }
-  uint32_t ls = (uint32_t)(se - sb), lt = (uint32_t)(te - tb);
-  const T *A = lab + sb, *B = lab + tb;
-  if (ls > lt) {  // A = shorter list, B = longer list
-    const T *X = A; A = B; B = X;
-    const uint32_t tl = ls; ls = lt; lt = tl;
-  }
-  j.A = A; j.B = B; j.ls = ls; j.lt = lt; j.kk = (uint32_t)k;
-  j.fixed = ls == 0 ? INT32_MAX : -1;  // an empty list shares no hub
-  return j;
-}
-
-template <class T>
-__device__ inline bool merge_job(const QJob<T> &j, uint32_t merge_cap) {
-  return j.fixed < 0 && j.ls + j.lt <= merge_cap;
-}
-
-// LDS of a workgroup: kStageWords labels, then (32-bit labels) the four
-// wave minima, which the 8-byte form keeps in its last 16 bytes instead.
-template <class F>
-struct QStage {
-  static constexpr uint32_t kLabels = kStageWords + (sizeof(typename F::T) == 8 ? 0u : 4u);
-  static constexpr uint32_t kMinAt = sizeof(typename F::T) == 8 ? kMergeCap : kStageWords;
-  // hubs of B on the long path (u32 words)
-  static constexpr uint32_t kHubs = sizeof(typename F::T) == 8 ? kLongHubs : kStageWords;
-};
-
-template <class F>
-__global__ void __launch_bounds__(kQThreads) k_query(F fmt, uint32_t n,
-                                                     const unsigned long long *off,
-                                                     const typename F::T *lab, uint64_t nq,
-                                                     const uint32_t *qs, const uint32_t *qt,
-                                                     const int8_t *qk, int32_t *out,
-                                                     uint32_t merge_cap, uint32_t lds_hubs) {
-  using LT = typename F::T;
-  __shared__ LT stage[QStage<F>::kLabels];
-  uint32_t *wave_min = reinterpret_cast<uint32_t *>(stage + QStage<F>::kMinAt);
-  const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-  const uint64_t G = gridDim.x;
-  uint64_t q = blockIdx.x;
-  if (q >= nq) return;  // uniform over the workgroup
-
-  // ---- prologue: job of q (synchronous), ranges of q+G, (s,t,k) of q+2G
-  uint32_t pv = load_params(lane, q, qs, qt, qk);
-  uint32_t s = lane_u32(pv, 0), t = lane_u32(pv, 1);
-  int k = (int)lane_u32(pv, 2);
-  uint64_t rv = needs_join(n, s, t, k) ? load_ranges(lane, off, s, t) : 0;
-  QJob<LT> cur = make_job(n, lab, s, t, k, lane_u64(rv, 0), lane_u64(rv, 1), lane_u64(rv, 2),
-                         lane_u64(rv, 3));
-  pv = q + G < nq ? load_params(lane, q + G, qs, qt, qk) : 0;
-  uint32_t s1 = lane_u32(pv, 0), t1 = lane_u32(pv, 1);
-  int k1 = q + G < nq ? (int)lane_u32(pv, 2) : -1;
-  if (needs_join(n, s1, t1, k1)) rv = load_ranges(lane, off, s1, t1);
-  if (q + 2 * G < nq) pv = load_params(lane, q + 2 * G, qs, qt, qk);
-  // labels of q
-  LT v[kLoadPerLane];
-  if (merge_job(cur, merge_cap)) {
-    const uint32_t total = cur.ls + cur.lt;
-#pragma unroll
-    for (uint32_t u = 0; u < kLoadPerLane; ++u) {
-      const uint32_t i = u * kQThreads + tid;
-      const uint32_t ic = i < total ? i : total - 1;  // lanes past the end reload the last label
-      v[u] = ic < cur.ls ? cur.A[ic] : cur.B[ic - cur.ls];
-    }
-  }
-
-  for (; q < nq; q += G) {
-    // In flight now: labels of q (v), ranges of q+G (rv, lanes 0-3) and
-    // (s,t,k) of q+2G (pv, lanes 0-2).
-    const bool is_merge = merge_job(cur, merge_cap);
-    const uint32_t total = cur.ls + cur.lt;
-    const uint32_t ls = cur.ls;
-    // hash of A's hub groups: u16 indexes into the staged A, two per word,
-    // 2^tbits >= 2|A| slots (<= 4096 since |A| <= 2047), right after A
-    const uint32_t tbits = ls ? max(6u, 32u - (uint32_t)__builtin_clz(2 * ls - 1)) : 6u;
-    const uint32_t tmask = (1u << tbits) - 1u;
-    uint32_t *T = reinterpret_cast<uint32_t *>(stage + ls);
-    LT vc[kLoadPerLane];  // this query's labels; v takes the next one's
-    if (is_merge) {
-#pragma unroll
-      for (uint32_t u = 0; u < kLoadPerLane; ++u) {
-        vc[u] = v[u];
-        const uint32_t i = u * kQThreads + tid;
-        if (i < ls) stage[i] = vc[u];
+// hcnt[v * K + x], x < K: labels of v of hop <= x.  below: the index holds
+// hubs ranked below their vertex.  slots: table slots per wave, a power of two.
+__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
+          const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt, uint32_t below,
+          uint64_t nq, const uint32_t *__restrict__ qs, const uint32_t *__restrict__ qt,
+          const int8_t *__restrict__ qk, int32_t *out, uint32_t slots) {
+  extern __shared__ uint4 qlds[];  // 16-byte stores clear the tables
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  lds_ptr<uint32_t> T = (lds_ptr<uint32_t>)(reinterpret_cast<uint32_t *>(qlds) + wib * slots);
+  const uint64_t waves = (uint64_t)gridDim.x * kQWaves;
+  const QChunk ch(nq, waves);
+  for (uint64_t q0 = ((uint64_t)blockIdx.x * kQWaves + wib) * ch.per; q0 < nq;
+       q0 += waves * ch.per) {
+    // lane i: request q0 + i, then its answer
+    const uint32_t cnt = (uint32_t)min<uint64_t>(ch.per, nq - q0);
+    const bool mine = lane < cnt;
+    const uint32_t vs = mine ? qs[q0 + lane] : 0u, vt = mine ? qt[q0 + lane] : 0u;
+    const int vk = mine ? qk[q0 + lane] : 0;
+    int32_t ans = vk >= 0 && vs == vt && vs < n ? 0 : INT32_MAX;
+    // the others need a join
+    for (unsigned long long todo = __ballot(vk > 0 && vs < n && vt < n && vs != vt); todo;
+         todo &= todo - 1) {
+      const int qi = __ffsll((long long)todo) - 1;
+      const uint32_t s = __builtin_amdgcn_readlane(vs, qi), t = __builtin_amdgcn_readlane(vt, qi);
+      const int k = __builtin_amdgcn_readlane(vk, qi);
+      uint32_t a = s, b = t;
+      unsigned long long abeg = off[s], bbeg = off[t];
+      uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
+      if (alen > blen) {
+        const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
+        const uint32_t l = alen; alen = blen; blen = l;
+        a = t;
+        b = s;
       }
-      for (uint32_t j = tid; j < (1u << (tbits - 1)); j += kQThreads) T[j] = kInf32;
-    }
-    __syncthreads();
-    // ---- prefetch: labels of q+G, ranges of q+2G, (s,t,k) of q+3G
-    const bool has1 = q + G < nq;
-    const QJob<LT> nxt = make_job(n, lab, s1, t1, k1, lane_u64(rv, 0), lane_u64(rv, 1),
-                                 lane_u64(rv, 2), lane_u64(rv, 3));
-    const bool has2 = q + 2 * G < nq;
-    const uint32_t s2 = lane_u32(pv, 0), t2 = lane_u32(pv, 1);
-    const int k2 = has2 ? (int)lane_u32(pv, 2) : -1;
-    if (has1 && merge_job(nxt, merge_cap)) {
-      const uint32_t ntot = nxt.ls + nxt.lt;
-#pragma unroll
-      for (uint32_t u = 0; u < kLoadPerLane; ++u) {
-        const uint32_t i = u * kQThreads + tid;
-        const uint32_t ic = i < ntot ? i : ntot - 1;
-        v[u] = ic < nxt.ls ? nxt.A[ic] : nxt.B[ic - nxt.ls];
-      }
-    }
-    if (needs_join(n, s2, t2, k2)) rv = load_ranges(lane, off, s2, t2);
-    if (q + 3 * G < nq) pv = load_params(lane, q + 3 * G, qs, qt, qk);
+      const uint32_t *A = lab + abeg, *B = lab + bbeg;
+      const uint32_t kk = (uint32_t)k, c = kk >> 1;
+      // labels of v of hop <= x
+      auto upto = [&](uint32_t v, uint32_t len, uint32_t x) {
+        return x < K ? hcnt[(uint64_t)v * K + x] : len;
+      };
+      const uint32_t a0 = upto(a, alen, 0), b0 = upto(b, blen, 0);  // self labels
+      const uint32_t ac = upto(a, alen, c), bc = upto(b, blen, kk - 1 - c);
+      const uint32_t a1 = upto(a, alen, kk - 1), b1 = upto(b, blen, kk - 1);
+      const uint32_t ak = upto(a, alen, kk), bk = upto(b, blen, kk);
+      uint32_t best = kInf32;       // pairs of hops >= 1
+      uint32_t at_a = kInf32, at_b = kInf32;  // labels of hub a in L(b), of b in L(a)
 
-    // ---- join of q
-    uint32_t best = kInf32;
-    const uint32_t kk = cur.kk;
-    if (is_merge) {
-      const LT *SA = stage;
-      // insert the group heads of A (hubs are unique among heads)
-      for (uint32_t i = tid; i < ls; i += kQThreads) {
-        const uint32_t w = fmt.hub(SA[i]);
-        if (i > 0 && fmt.hub(SA[i - 1]) == w) continue;
-        uint32_t slot = (w * 0x9E3779B1u) >> (32 - tbits);
-        for (;;) {
-          uint32_t *wp = &T[slot >> 1];
-          const uint32_t sh = (slot & 1u) << 4;
-          uint32_t word = *wp;
-          bool done = false;
-          while (((word >> sh) & 0xFFFFu) == 0xFFFFu) {
-            const uint32_t got = atomicCAS(wp, word, (word & ~(0xFFFFu << sh)) | (i << sh));
-            if (got == word) { done = true; break; }
-            word = got;
-          }
-          if (done) break;
-          slot = (slot + 1) & tmask;
+      // Labels [beg, end) of L, four steps' loads at a time; use(l) sees every
+      // label (a lane past the end a copy of the last one).
+      auto walk = [&](const uint32_t *L, uint32_t beg, uint32_t end, auto &&use) {
+        for (uint32_t j = beg; j < end; j += 4 * kWave) {
+          uint32_t l[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) l[u] = L[min(j + u * kWave + lane, end - 1)];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            if (j + u * kWave < end) use(l[u]);
         }
-      }
-      __syncthreads();
-      // each lane probes its labels of B (held in registers) and walks A's
-      // run of that hub (<= K+1 labels, hops ascending) while h1 + h2 <= k
-#pragma unroll
-      for (uint32_t u = 0; u < kLoadPerLane; ++u) {
-        const uint32_t i = u * kQThreads + tid;
-        if (i < ls || i >= total) continue;
-        const LT b = vc[u];
-        const uint32_t w = fmt.hub(b), h2 = fmt.hop(b), d2 = fmt.dist(b);
-        if (h2 > kk) continue;
-        uint32_t slot = (w * 0x9E3779B1u) >> (32 - tbits);
-        for (;;) {
-          const uint32_t e = (T[slot >> 1] >> ((slot & 1u) << 4)) & 0xFFFFu;
-          if (e == 0xFFFFu) break;
-          if (fmt.hub(SA[e]) == w) {
-            for (uint32_t p = e; p < ls; ++p) {
-              const LT a = SA[p];
-              if (fmt.hub(a) != w || fmt.hop(a) + h2 > kk) break;
-              const uint32_t dsum = fmt.dist(a) + d2;
-              best = dsum < best ? dsum : best;
+      };
+      auto endpoint = [&](uint32_t l, uint32_t other, uint32_t &at) {
+        if (fmt.hub(l) == other) at = min(at, fmt.dist(l));
+      };
+      // hashes X[xb, xe), probes with Y[yb, ye)
+      auto join = [&](const uint32_t *X, uint32_t xb, uint32_t xe, const uint32_t *Y, uint32_t yb,
+                      uint32_t ye) {
+        while (xb < xe && yb < ye) {
+          // at most half the table; a quarter where it has room
+          const uint32_t part = min(xe - xb, slots / 2);
+          const uint32_t cap =
+              min(slots, 1u << (32 - __builtin_clz(max(64u, 4u * part) - 1)));
+          for (uint32_t i = lane; i < cap * 4 / 16; i += kWave)
+            ((lds_ptr<u32x4>)T)[i] = u32x4{0, 0, 0, 0};
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          for (uint32_t j = xb; j < xb + part; j += kWave) {
+            const uint32_t l = X[min(j + lane, xb + part - 1)];
+            if (j + lane < xb + part) {
+              uint32_t slot = hash_slot(fmt.hub(l), cap);
+              while (atomicCAS((uint32_t *)&T[slot], 0u, l) != 0u) slot = (slot + 1) & (cap - 1);
             }
-            break;
           }
-          slot = (slot + 1) & tmask;
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          walk(Y, yb, ye, [&](uint32_t l) {
+            const uint32_t w = fmt.hub(l), h = fmt.hop(l), d = fmt.dist(l);
+            uint32_t slot = hash_slot(w, cap);
+            uint32_t x = T[slot];
+            while (x != 0) {
+              if (fmt.hub(x) == w && fmt.hop(x) + h <= kk) best = min(best, d + fmt.dist(x));
+              slot = (slot + 1) & (cap - 1);
+              x = T[slot];
+            }
+          });
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          xb += part;
         }
+      };
+      if (below || b > a) walk(B, b0, bk, [&](uint32_t l) { endpoint(l, a, at_a); });
+      if (below || a > b) walk(A, a0, ak, [&](uint32_t l) { endpoint(l, b, at_b); });
+      join(A, a0, ac, B, b0, b1);
+      join(B, b0, bc, A, ac, a1);
+      if (a0) best = min(best, at_a);
+      if (b0) best = min(best, at_b);
+      best = wave_min_u32(best);
+      if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
+    }
+    if (mine) out[q0 + lane] = ans;
+  }
+}
+
+// 8-byte labels: pieces of the longer list B in LDS, searched by the shorter
+// list A's labels.  Both are hub-sorted, so a chunk of A whose hubs lie below
+// the piece is never read again; a run of B cut by a piece's end is found in
+// both pieces.
+constexpr uint32_t kQPiece = 512;  // labels, 4 KB per wave
+__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_query64(uint32_t n, const unsigned long long *__restrict__ off,
+          const unsigned long long *__restrict__ lab, uint64_t nq,
+          const uint32_t *__restrict__ qs, const uint32_t *__restrict__ qt,
+          const int8_t *__restrict__ qk, int32_t *out) {
+  __shared__ unsigned long long stage[kQWaves][kQPiece];
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  lds_ptr<unsigned long long> P = (lds_ptr<unsigned long long>)stage[wib];
+  const uint64_t waves = (uint64_t)gridDim.x * kQWaves;
+  const QChunk ch(nq, waves);
+  for (uint64_t q0 = ((uint64_t)blockIdx.x * kQWaves + wib) * ch.per; q0 < nq;
+       q0 += waves * ch.per) {
+    // lane i: request q0 + i, then its answer
+    const uint32_t cnt = (uint32_t)min<uint64_t>(ch.per, nq - q0);
+    const bool mine = lane < cnt;
+    const uint32_t vs = mine ? qs[q0 + lane] : 0u, vt = mine ? qt[q0 + lane] : 0u;
+    const int vk = mine ? qk[q0 + lane] : 0;
+    int32_t ans = vk >= 0 && vs == vt && vs < n ? 0 : INT32_MAX;
+    // the others need a join
+    for (unsigned long long todo = __ballot(vk > 0 && vs < n && vt < n && vs != vt); todo;
+         todo &= todo - 1) {
+      const int qi = __ffsll((long long)todo) - 1;
+      const uint32_t s = __builtin_amdgcn_readlane(vs, qi), t = __builtin_amdgcn_readlane(vt, qi);
+      const int k = __builtin_amdgcn_readlane(vk, qi);
+      const uint32_t kk = (uint32_t)k;
+      unsigned long long abeg = off[s], bbeg = off[t];
+      uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
+      if (alen > blen) {
+        const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
+        const uint32_t l = alen; alen = blen; blen = l;
       }
-    } else if (cur.fixed < 0) {
-      // long path: LDS skip index of B's hubs (stride 1 up to lds_hubs)
-      const LT *A = cur.A, *B = cur.B;
-      const uint32_t ls = cur.ls, lt = cur.lt;
-      uint32_t *hubs = reinterpret_cast<uint32_t *>(stage);
-      const uint32_t stride = (lt + lds_hubs - 1) / lds_hubs;
-      const uint32_t nsm = (lt + stride - 1) / stride;
-      for (uint32_t i = tid; i < nsm; i += kQThreads) hubs[i] = fmt.hub(B[(uint64_t)i * stride]);
-      __syncthreads();
-      for (uint32_t j = tid; j < ls; j += kQThreads) {
-        const LT a = A[j];
-        const uint32_t w = fmt.hub(a), h1 = fmt.hop(a), d1 = fmt.dist(a);
-        if (h1 > kk) continue;
-        // first sample >= w, then the first position >= w inside its block
-        const uint32_t si = lower_bound_by([&](uint32_t x) { return hubs[x]; }, nsm, w);
-        const uint32_t lo = si == 0 ? 0 : (si - 1) * stride + 1;
-        const uint32_t hi = si < nsm ? si * stride : lt;
-        uint32_t p = lo + lower_bound_by([&](uint32_t x) { return fmt.hub(B[lo + x]); }, hi - lo, w);
-        for (; p < lt; ++p) {
-          const LT b = B[p];
-          if (fmt.hub(b) != w || h1 + fmt.hop(b) > kk) break;  // hops ascend within a hub
-          const uint32_t dsum = d1 + fmt.dist(b);
-          best = dsum < best ? dsum : best;
+      const unsigned long long *A = lab + abeg, *B = lab + bbeg;
+      uint32_t best = kInf32;
+      uint32_t j0 = 0;  // chunks of A below this one are done
+      for (uint32_t p0 = 0; p0 < blen && j0 < alen; p0 += kQPiece) {
+        const uint32_t m = min(kQPiece, blen - p0);
+        for (uint32_t i = lane; i < m; i += 4 * kWave) {
+          unsigned long long l[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) l[u] = B[p0 + min(i + u * kWave, m - 1)];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            if (i + u * kWave < m) P[i + u * kWave] = l[u];
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint32_t lo_hub = label_hub(P[0]), hi_hub = label_hub(P[m - 1]);
+        for (uint32_t j = j0; j < alen; j += kWave) {
+          const unsigned long long a = A[min(j + lane, alen - 1)];
+          const uint32_t w = label_hub(a), h1 = label_hop(a);
+          if (__builtin_amdgcn_readlane(w, 0) > hi_hub) break;
+          if (__builtin_amdgcn_readlane(w, kWave - 1) < lo_hub) {
+            j0 = j + kWave;
+            continue;
+          }
+          if (w < lo_hub || w > hi_hub || h1 > kk) continue;
+          // first label of the piece with hub >= w (there is one)
+          uint32_t lo = 0, hi = m - 1;
+          while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
+          }
+          for (uint32_t x = lo; x < m; ++x) {  // <= K + 1 labels, hops ascending
+            const unsigned long long l = P[x];
+            if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
+            best = min(best, label_dist(a) + label_dist(l));
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
+      best = wave_min_u32(best);
+      if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
     }
-    best = wave_min_u32(best);
-    if (lane == 0) wave_min[wv] = best;
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t m = wave_min[0];
-      for (uint32_t x = 1; x < kQWaves; ++x) m = wave_min[x] < m ? wave_min[x] : m;
-      out[q] = cur.fixed >= 0 ? cur.fixed : (m == kInf32 ? INT32_MAX : (int32_t)m);
-    }
-    // advance the pipeline
-    cur = nxt;
-    s1 = s2; t1 = t2; k1 = k2;
+    if (mine) out[q0 + lane] = ans;
   }
 }
 
 // Workgroups resident at once on a device (the persistent grid), cached per
-// kernel form.
-template <class F>
-static uint32_t query_grid(int dev) {
+// kernel and LDS size.
+static uint32_t query_grid(int dev, bool copy, size_t lds) {
+  struct Cache {
+    int dev = -1;
+    size_t lds = 0;
+    uint32_t grid = 0;
+  };
   static std::mutex mu;
-  static int cached_dev = -1;
-  static uint32_t cached = 0;
+  static Cache cache[2];
   std::lock_guard<std::mutex> g(mu);
-  if (dev == cached_dev && cached) return cached;
+  Cache &c = cache[copy];
+  if (dev == c.dev && lds == c.lds) return c.grid;
   int cus = 0, per_cu = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_query<F>, kQThreads, 0) !=
-          hipSuccess ||
-      per_cu <= 0)
-    per_cu = 4;
-  cached = (uint32_t)(cus * per_cu);
-  cached_dev = dev;
-  return cached;
+  const hipError_t e =
+      copy ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_query32, kQThreads, lds)
+           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_query64, kQThreads, lds);
+  if (e != hipSuccess || per_cu <= 0) per_cu = 4;
+  c = Cache{dev, lds, (uint32_t)(cus * per_cu)};
+  return c.grid;
 }
 
-__global__ void __launch_bounds__(256) k_pack_query32(const unsigned long long *lab, uint64_t total,
-                                                      uint32_t *out, uint32_t hsh, uint32_t db) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < total;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const unsigned long long l = lab[i];
-    out[i] = (label_hub(l) << hsh) | (label_hop(l) << db) | label_dist(l);
+// The query copy: every list's labels as 32-bit words in hop order (any order
+// within a hop) and the prefix counts.  A wave per vertex counts its labels'
+// hops, then scatters them.
+__global__ void __launch_bounds__(256) k_pack_query32(uint32_t n, uint32_t K,
+                                                      const unsigned long long *off,
+                                                      const unsigned long long *lab, uint32_t *out,
+                                                      uint32_t *hcnt, uint32_t hsh, uint32_t db) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
+  for (uint32_t v = wave; v < n; v += nwaves) {
+    const unsigned long long b = off[v];
+    const uint32_t len = (uint32_t)(off[v + 1] - b);
+    uint32_t pos[kMaxK + 1];
+#pragma unroll
+    for (uint32_t x = 0; x <= kMaxK; ++x) pos[x] = 0;
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const unsigned long long l = lab[b + min(j0 + lane, len - 1)];
+      const uint32_t hop = j0 + lane < len ? label_hop(l) : kInf32;
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x)
+        if (x <= K) pos[x] += (uint32_t)__popcll(__ballot(hop == x));
+    }
+    uint32_t run = 0;
+#pragma unroll
+    for (uint32_t x = 0; x <= kMaxK; ++x) {
+      const uint32_t c = pos[x];
+      pos[x] = run;
+      run += c;
+      if (x < K && lane == 0) hcnt[(uint64_t)v * K + x] = run;
+    }
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const unsigned long long l = lab[b + min(j0 + lane, len - 1)];
+      const uint32_t hop = j0 + lane < len ? label_hop(l) : kInf32;
+      uint32_t dst = 0;
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x) {
+        if (x > K) continue;
+        const unsigned long long m = __ballot(hop == x);
+        if (hop == x) dst = pos[x] + (uint32_t)__popcll(m & lt_mask);
+        pos[x] += (uint32_t)__popcll(m);
+      }
+      if (hop != kInf32)
+        out[b + dst] = (label_hub(l) << hsh) | (hop << db) | label_dist(l);
+    }
   }
 }
 
@@ -368,15 +360,16 @@ static int ensure_query32(const hsdl_index *idx, hipStream_t st) {
     return HSDL_OK;
   }
   // the copy is an optimisation: without room for it, queries read the
-  // 8-byte labels
-  if (idx->lab32.alloc(std::max<uint64_t>(idx->total, 1) * 4) != HSDL_OK) {
+  // 8-byte labels.  The prefix counts lie after the labels.
+  if (idx->lab32.alloc((idx->total + (uint64_t)idx->n * idx->K) * 4) != HSDL_OK) {
     idx->q32.store(2, std::memory_order_release);
     return HSDL_OK;
   }
-  const uint32_t grid = (uint32_t)std::min<uint64_t>(4096, (idx->total + 255) / 256 + 1);
-  hipLaunchKernelGGL(k_pack_query32, dim3(grid), dim3(256), 0, st,
-                     idx->lab.as<unsigned long long>(), idx->total, idx->lab32.as<uint32_t>(),
-                     pb + db, db);
+  const uint32_t grid = (uint32_t)std::min<uint64_t>(4096, idx->n / kQWaves + 1ull);
+  hipLaunchKernelGGL(k_pack_query32, dim3(grid), dim3(256), 0, st, idx->n, (uint32_t)idx->K,
+                     idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
+                     idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total, pb + db,
+                     db);
   HSDL_HIP(hipGetLastError());
   // queries on other streams may read the copy as soon as it is marked made
   HSDL_HIP(hipStreamSynchronize(st));
@@ -392,13 +385,18 @@ int prepare_query(const hsdl_index *idx) {
   return ensure_query32(idx, nullptr);
 }
 
+// Table slots per wave: a list part is a few hundred labels, hashed at a load
+// of a quarter where the table has room; 1,024 slots are 16 KB per workgroup
+// and keep a CU's 32 waves resident, and indexes of longer lists take twice
+// that for 20 waves.  Tuning knob HSDL_QUERY_SLOTS (a power of two from 64).
+static uint32_t query_slots(const hsdl_index *idx) {
+  const uint64_t mean = idx->n ? idx->total / idx->n : 0;
+  return pow2_at_most(env_u32("HSDL_QUERY_SLOTS", mean <= 1024 ? 1024 : 2048, 64, 4096));
+}
+
 int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const uint32_t *d_t,
                  const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc) {
   if (nq == 0) return HSDL_OK;
-  // tuning knobs: labels staged for the merge path (<= 4094; 0 sends every
-  // query down the long path) and LDS skip-index capacity of the long path
-  const uint32_t merge_cap = env_u32("HSDL_QUERY_MERGE_CAP", kMergeCap, 0, kMergeCap);
-  const uint32_t lds_hubs = env_u32("HSDL_QUERY_LDS_HUBS", kLongHubs, 1, kLongHubs);
   const bool want32 = env_u32("HSDL_QUERY32", 1, 0, 1) != 0;
   if (want32 && may_alloc && !idx->q32.load(std::memory_order_acquire)) {
     // a stream under graph capture takes no allocation or synchronisation
@@ -409,20 +407,23 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
       if (rc) return rc;
     }
   }
-  if (want32 && idx->q32.load(std::memory_order_acquire) == 1) {
+  const bool copy = want32 && idx->q32.load(std::memory_order_acquire) == 1;
+  const uint32_t slots = copy ? query_slots(idx) : 0;
+  const size_t lds = (size_t)slots * 4 * kQWaves;
+  const uint32_t grid = (uint32_t)std::min<uint64_t>((nq + kQWaves - 1) / kQWaves,
+                                                     query_grid(idx->device, copy, lds));
+  if (copy) {
     const uint32_t db = idx->q32_dist_bits, pb = idx->q32_hop_bits;
-    const Lab32 fmt{db, pb + db, (1u << pb) - 1u, (1u << db) - 1u};
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(nq, query_grid<Lab32>(idx->device));
-    hipLaunchKernelGGL(k_query<Lab32>, dim3(grid), dim3(kQThreads), 0, st, fmt, idx->n,
-                       idx->off.as<unsigned long long>(), idx->lab32.as<uint32_t>(), (uint64_t)nq,
-                       d_s, d_t, d_k, d_out, merge_cap,
-                       std::min(lds_hubs, QStage<Lab32>::kHubs));
+    hipLaunchKernelGGL(k_query32, dim3(grid), dim3(kQThreads), lds, st,
+                       Lab32{db, pb + db, (1u << pb) - 1u, (1u << db) - 1u}, idx->n,
+                       (uint32_t)idx->K, idx->off.as<unsigned long long>(),
+                       idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total,
+                       idx->hubs_below ? 1u : 0u,
+                       (uint64_t)nq, d_s, d_t, d_k, d_out, slots);
   } else {
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(nq, query_grid<Lab64>(idx->device));
-    hipLaunchKernelGGL(k_query<Lab64>, dim3(grid), dim3(kQThreads), 0, st, Lab64{}, idx->n,
+    hipLaunchKernelGGL(k_query64, dim3(grid), dim3(kQThreads), 0, st, idx->n,
                        idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                       (uint64_t)nq, d_s, d_t, d_k, d_out, merge_cap,
-                       std::min(lds_hubs, QStage<Lab64>::kHubs));
+                       (uint64_t)nq, d_s, d_t, d_k, d_out);
   }
   HSDL_HIP(hipGetLastError());
   return HSDL_OK;

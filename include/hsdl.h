@@ -239,9 +239,9 @@ int hsdl_index_stats(const hsdl_index *idx, hsdl_stats *st);
  * (CPU_HopHL/include/HBPLL/hop_constrained_two_hop_labels.h:144-222) and
  * gpu_query (Query_mdnd/src/gpu_query.cu:84-177).  k < 0 -> INT32_MAX;
  * s == t -> 0; k == 0 -> INT32_MAX.  The first call on an index makes a
- * 32-bit copy of its labels (4 B per label, kept with the index) when hub,
- * hop and distance fit one word; hsdl_query_device does the same (waiting
- * for the copy once), except on a stream under graph capture. */
+ * 32-bit copy of its labels (4 B per label and 4 K B per vertex, kept with the
+ * index) when hub, hop and distance fit one word; hsdl_query_device does the
+ * same (waiting for the copy once), except on a stream under graph capture. */
 int hsdl_query(const hsdl_index *idx, size_t n, const uint32_t *s, const uint32_t *t,
                const int8_t *k, int32_t *out);
 

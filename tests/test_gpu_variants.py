@@ -89,3 +89,48 @@ def test_expansion_shapes(monkeypatch, heavy, piece):
                         O.kround(csr_of(g), K).arrays())
     g = H.Graph.grid(37, 41, 5, 1, 300)
     same_labels(H.hop_constrained_two_hop_labels_generation(g, 6), O.kround(csr_of(g), 6).arrays())
+
+
+@pytest.mark.parametrize("q32,slots", [("1", "1024"), ("1", "64"), ("0", "1024")])
+def test_query_forms(monkeypatch, q32, slots):
+    """Queries from the hop-ordered 32-bit copy (parts that fit the table, and
+    with 64 slots parts hashed in many pieces) and from the 8-byte labels (lists
+    of one piece of 512 labels and of several): every k from 0 past K, on a
+    graph of long lists, short lists at K = 15, a group's index (vertices
+    without their self label) and an imported set with hubs ranked below their
+    vertex: the oracle's answers."""
+    monkeypatch.setenv("HSDL_QUERY32", q32)
+    monkeypatch.setenv("HSDL_QUERY_SLOTS", slots)
+    rng = np.random.default_rng(17)
+
+    def check(name, idx, want, n, K):
+        print(f"[query] {name} q32={q32} slots={slots}", flush=True)
+        s, t = rng.integers(0, n, (2, 6000)).astype(np.uint32)
+        t[:50] = s[:50]
+        k = rng.integers(-1, K + 3, 6000).astype(np.int8)
+        assert np.array_equal(idx.query(s, t, k), O.query(want, s, t, k))
+
+    def imported(off, hub, hop, dist, K):
+        o = O.labels_from_arrays(len(off) - 1, off, hub, hop, dist)
+        return H.Index.from_labels(len(off) - 1, K, off, hub, hop, dist), o
+
+    for n, K, wmax, ef in ((6000, 4, 1000, 16), (400, 15, 2, 4), (33, 3, 5, 2)):
+        g = ragged(n, n, wmax, ef)
+        want = O.kround(csr_of(g), K)
+        check(f"n={n}", H.hop_constrained_two_hop_labels_generation(g, K), want, n, K)
+    hubs = np.arange(0, 6000, 2, dtype=np.uint32)
+    g = ragged(6000, 6000, 1000, 16)
+    idx = H.hop_constrained_two_hop_labels_generation(g, 4, hubs=hubs)
+    check("group", idx, O.labels_from_arrays(6000, *idx.labels()), 6000, 4)
+    # vertex v also holds, for some of its labels (u, h, d), the mirrored label at u
+    off, hub, hop, dist = idx.labels()
+    v = np.repeat(np.arange(6000), np.diff(off.astype(np.int64)))
+    pick = (rng.random(len(v)) < 0.2) & (hop > 0)
+    rows = np.concatenate([np.stack([v, hub, hop, dist], 1),
+                           np.stack([hub[pick], v[pick], hop[pick], dist[pick]], 1)]).astype(np.int64)
+    rows = rows[np.lexsort((rows[:, 2], rows[:, 1], rows[:, 0]))]
+    off = np.zeros(6001, np.uint64)
+    off[1:] = np.cumsum(np.bincount(rows[:, 0], minlength=6000))
+    idx, want = imported(off, rows[:, 1].astype(np.uint32), rows[:, 2].astype(np.uint8),
+                         rows[:, 3].astype(np.int32), 4)
+    check("hubs below", idx, want, 6000, 4)
