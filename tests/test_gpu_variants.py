@@ -134,3 +134,22 @@ def test_query_forms(monkeypatch, q32, slots):
     idx, want = imported(off, rows[:, 1].astype(np.uint32), rows[:, 2].astype(np.uint8),
                          rows[:, 3].astype(np.int32), 4)
     check("hubs below", idx, want, 6000, 4)
+
+
+def test_paths_over_pieces():
+    """Paths where a list spans several staged pieces of 512 labels, runs of a
+    hub cut by a piece's end, ties (weights 1..2), and lists far shorter than
+    the other side's: the oracle's edges."""
+    rng = np.random.default_rng(3)
+    for n, K, wmax, ef in ((6000, 4, 2, 16), (4000, 5, 1000, 16), (300, 9, 2, 4)):
+        g = ragged(n, n, wmax, ef)
+        print(f"[paths] n={n} K={K}", flush=True)
+        idx = H.hop_constrained_two_hop_labels_generation(g, K, parents=True)
+        want = O.kround(csr_of(g), K)
+        s, t = rng.integers(0, n, (2, 4000)).astype(np.uint32)
+        s[:1000] = np.arange(1000) % 40
+        k = rng.integers(0, K + 2, 4000).astype(np.int8)
+        edges, counts = idx.paths(s, t, k, cap=K + 1)
+        wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), K + 1)
+        assert np.array_equal(counts.astype(np.int32), wcounts)
+        assert np.array_equal(edges.astype(np.int32), wedges)
