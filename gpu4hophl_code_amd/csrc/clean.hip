@@ -942,6 +942,10 @@ extern "C" int hsdl_clean(hsdl_index *idx) {
 }
 
 static int release_scratch_body(int32_t device) {
+  int was = -1;
+  (void)hipGetDevice(&was);
+  hsdl::release_stages(device);
+  if (was >= 0) (void)hipSetDevice(was);
   std::lock_guard<std::mutex> lk(hsdl::g_clean_scratch_mu);
   int cur = -1;
   (void)hipGetDevice(&cur);

@@ -261,4 +261,40 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
 // Makes the index's 32-bit query copy now, when it fits (synchronous).
 int prepare_query(const hsdl_index *idx);
 
+// Staging of a host-array call: one or two slots, each a stream, pinned host
+// memory that kernels read and write in place, and device memory (when asked
+// for), of the bytes the call needs up to kStageBytes.  Calls take one from a
+// per-device pool of at most kStagesKept and give it back; a call that finds
+// none makes its own, so calls on several threads never share one.
+// hsdl_release_scratch frees the pool.
+constexpr size_t kStageBytes = 4u << 20;  // per slot that is kept
+constexpr int kStagesKept = 4;
+struct Stage {
+  int dev = 0;
+  hipStream_t st[2] = {nullptr, nullptr};
+  uint8_t *h[2] = {nullptr, nullptr};
+  size_t hbytes[2] = {0, 0};
+  DevBuf d[2];
+  ~Stage();
+};
+class StageLease {
+ public:
+  // `slots` slots of at least `bytes` each on the current device `dev`; device:
+  // with device memory of the same size
+  int take(int dev, size_t bytes, int slots, bool device);
+  Stage *operator->() const { return s_; }
+  ~StageLease();
+
+ private:
+  Stage *s_ = nullptr;
+};
+void release_stages(int dev);  // -1: every device
+
+// Whether every entry of a and b lies below n (no early exit: it vectorizes).
+inline bool all_below(const uint32_t *a, const uint32_t *b, size_t cnt, uint32_t n) {
+  uint32_t bad = 0;
+  for (size_t i = 0; i < cnt; ++i) bad |= (uint32_t)(a[i] >= n) | (uint32_t)(b[i] >= n);
+  return bad == 0;
+}
+
 }  // namespace hsdl

@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "device.hpp"
@@ -293,30 +294,54 @@ static int extract_paths_body(const hsdl_index *idx, size_t n, const uint32_t *s
   if (n == 0) return HSDL_OK;
   if (!s || !t || !k || !counts || (cap && !edges)) return fail(HSDL_EINVAL, "null path arrays");
   if (!idx->has_parents) return fail(HSDL_EINVAL, "index has no parents (build with opts.parents = 1)");
-  for (size_t i = 0; i < n; ++i)
-    if (s[i] >= idx->n || t[i] >= idx->n) return fail(HSDL_EINVAL, "query vertex out of range");
-  int rc = use_device(idx->device, nullptr);
+  if (!all_below(s, t, n, idx->n)) return fail(HSDL_EINVAL, "query vertex out of range");
+  int dev = 0;
+  int rc = use_device(idx->device, &dev);
   if (rc) return rc;
-  const size_t ebytes = std::max<size_t>((size_t)2 * cap * n * 4, 4);
-  DevBuf ds, dt, dk, de, dc;
-  if ((rc = ds.alloc(n * 4)) || (rc = dt.alloc(n * 4)) || (rc = dk.alloc(n)) ||
-      (rc = de.alloc(ebytes)) || (rc = dc.alloc(n * 4)))
-    return rc;
-  HSDL_HIP(hipMemcpy(ds.p, s, n * 4, hipMemcpyHostToDevice));
-  HSDL_HIP(hipMemcpy(dt.p, t, n * 4, hipMemcpyHostToDevice));
-  HSDL_HIP(hipMemcpy(dk.p, k, n, hipMemcpyHostToDevice));
+  // a slot: requests (9 B a query) read in place, then counts and edges, written
+  // in device memory and copied back together
+  const size_t per = 13 + (size_t)8 * cap;
+  // (a query whose edges exceed a kept slot gets slots of its own)
+  const size_t most = std::max<size_t>(1, (kStageBytes - 64) / per);
+  const size_t part = std::min(n, most >= 4 ? most & ~(size_t)3 : most);
+  StageLease stage;
+  if ((rc = stage.take(dev, part * per + 64, n > part ? 2 : 1, true))) return rc;
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, idx->device);
-  const size_t blocks = std::min<size_t>((n + 3) / 4, (size_t)cus * 16);
-  hipLaunchKernelGGL(k_paths, dim3((uint32_t)blocks), dim3(256), 0, nullptr, n,
-                     idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                     idx->par.as<uint32_t>(), ds.as<uint32_t>(), dt.as<uint32_t>(),
-                     dk.as<int8_t>(), cap, de.as<uint32_t>(), dc.as<uint32_t>());
-  HSDL_HIP(hipGetLastError());
-  HSDL_HIP(hipDeviceSynchronize());
-  if (cap) HSDL_HIP(hipMemcpy(edges, de.p, (size_t)2 * cap * n * 4, hipMemcpyDeviceToHost));
-  HSDL_HIP(hipMemcpy(counts, dc.p, n * 4, hipMemcpyDeviceToHost));
-  return HSDL_OK;
+  size_t sent = 0, first[2] = {0, 0}, cnt[2] = {0, 0};
+  for (int x = 0;; x ^= 1) {
+    uint8_t *h = stage->h[x], *d = stage->d[x].as<uint8_t>();
+    uint32_t *hs = reinterpret_cast<uint32_t *>(h), *ht = hs + part;
+    int8_t *hk = reinterpret_cast<int8_t *>(ht + part);
+    const size_t at = (part * 9 + 15) & ~(size_t)15;  // counts, then edges
+    if (cnt[x]) {
+      HSDL_HIP(hipStreamSynchronize(stage->st[x]));
+      std::memcpy(counts + first[x], h + at, cnt[x] * 4);
+      if (cap)
+        std::memcpy(edges + (size_t)2 * cap * first[x], h + at + cnt[x] * 4,
+                    (size_t)8 * cap * cnt[x]);
+      cnt[x] = 0;
+    }
+    if (sent < n) {
+      const size_t m = std::min(part, n - sent);
+      std::memcpy(hs, s + sent, m * 4);
+      std::memcpy(ht, t + sent, m * 4);
+      std::memcpy(hk, k + sent, m);
+      const size_t blocks = std::min<size_t>((m + 3) / 4, (size_t)cus * 16);
+      hipLaunchKernelGGL(k_paths, dim3((uint32_t)blocks), dim3(256), 0, stage->st[x], m,
+                         idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
+                         idx->par.as<uint32_t>(), hs, ht, hk, cap,
+                         reinterpret_cast<uint32_t *>(d + m * 4), reinterpret_cast<uint32_t *>(d));
+      HSDL_HIP(hipGetLastError());
+      HSDL_HIP(hipMemcpyAsync(h + at, d, m * 4 + (size_t)8 * cap * m, hipMemcpyDeviceToHost,
+                              stage->st[x]));
+      first[x] = sent;
+      cnt[x] = m;
+      sent += m;
+    } else if (!cnt[x ^ 1]) {
+      return HSDL_OK;
+    }
+  }
 }
 
 int hsdl_extract_paths(const hsdl_index *idx, size_t n, const uint32_t *s, const uint32_t *t,

@@ -45,6 +45,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -429,6 +430,93 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
   return HSDL_OK;
 }
 
+// ------------------------------------------------------------- staging
+static std::mutex g_stage_mu;
+// (never destroyed: no device call may run while the process ends)
+static std::vector<Stage *> &stage_pool() {
+  static std::vector<Stage *> *pool = new std::vector<Stage *>();
+  return *pool;
+}
+
+Stage::~Stage() {
+  for (int i = 0; i < 2; ++i) {
+    if (st[i]) (void)hipStreamDestroy(st[i]);
+    if (h[i]) (void)hipHostFree(h[i]);
+  }
+}
+
+int StageLease::take(int dev, size_t bytes, int slots, bool device) {
+  {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    std::vector<Stage *> &pool = stage_pool();
+    for (size_t i = 0; i < pool.size(); ++i)
+      if (pool[i]->dev == dev) {
+        s_ = pool[i];
+        pool.erase(pool.begin() + i);
+        break;
+      }
+  }
+  if (!s_) {
+    s_ = new Stage();
+    s_->dev = dev;
+  }
+  size_t want = 64u << 10;
+  while (want < bytes) want *= 2;
+  for (int i = 0; i < slots; ++i) {
+    if (!s_->st[i]) HSDL_HIP(hipStreamCreateWithFlags(&s_->st[i], hipStreamNonBlocking));
+    if (s_->hbytes[i] < bytes) {
+      if (s_->h[i]) (void)hipHostFree(s_->h[i]);
+      s_->h[i] = nullptr;
+      s_->hbytes[i] = 0;
+      HSDL_HIP(hipHostMalloc((void **)&s_->h[i], want, hipHostMallocMapped | hipHostMallocCoherent));
+      s_->hbytes[i] = want;
+    }
+    if (device && s_->d[i].bytes < bytes) {
+      const int rc = s_->d[i].alloc(want);
+      if (rc) return rc;
+    }
+  }
+  return HSDL_OK;
+}
+
+StageLease::~StageLease() {
+  if (!s_) return;
+  bool keep = true;
+  for (int i = 0; i < 2; ++i) {
+    // (a call that failed half-way may have work in flight)
+    if (s_->st[i]) (void)hipStreamSynchronize(s_->st[i]);
+    keep = keep && s_->hbytes[i] <= kStageBytes && s_->d[i].bytes <= kStageBytes;
+  }
+  if (keep) {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    std::vector<Stage *> &pool = stage_pool();
+    int kept = 0;
+    for (Stage *x : pool) kept += x->dev == s_->dev;
+    if (kept < kStagesKept) {
+      pool.push_back(s_);
+      return;
+    }
+  }
+  delete s_;
+}
+
+void release_stages(int dev) {
+  std::vector<Stage *> gone;
+  {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    std::vector<Stage *> &pool = stage_pool();
+    for (size_t i = pool.size(); i-- > 0;)
+      if (dev < 0 || pool[i]->dev == dev) {
+        gone.push_back(pool[i]);
+        pool.erase(pool.begin() + i);
+      }
+  }
+  for (Stage *x : gone) {
+    (void)hipSetDevice(x->dev);
+    delete x;
+  }
+}
+
 }  // namespace hsdl
 
 using namespace hsdl;
@@ -447,22 +535,41 @@ static int query_body(const hsdl_index *idx, size_t n, const uint32_t *s, const 
   if (!idx) return fail(HSDL_EINVAL, "null index");
   if (n == 0) return HSDL_OK;
   if (!s || !t || !k || !out) return fail(HSDL_EINVAL, "null query arrays");
-  for (size_t i = 0; i < n; ++i)
-    if (s[i] >= idx->n || t[i] >= idx->n) return fail(HSDL_EINVAL, "query vertex out of range");
-  int rc = use_device(idx->device, nullptr);
+  if (!all_below(s, t, n, idx->n)) return fail(HSDL_EINVAL, "query vertex out of range");
+  int dev = 0;
+  int rc = use_device(idx->device, &dev);
   if (rc) return rc;
-  DevBuf ds, dt, dk, dout;
-  if ((rc = ds.alloc(n * 4)) || (rc = dt.alloc(n * 4)) || (rc = dk.alloc(n)) ||
-      (rc = dout.alloc(n * 4)))
-    return rc;
-  HSDL_HIP(hipMemcpy(ds.p, s, n * 4, hipMemcpyHostToDevice));
-  HSDL_HIP(hipMemcpy(dt.p, t, n * 4, hipMemcpyHostToDevice));
-  HSDL_HIP(hipMemcpy(dk.p, k, n, hipMemcpyHostToDevice));
-  if ((rc = launch_query(idx, n, ds.as<uint32_t>(), dt.as<uint32_t>(), dk.as<int8_t>(),
-                         dout.as<int32_t>(), nullptr)))
-    return rc;
-  HSDL_HIP(hipMemcpy(out, dout.p, n * 4, hipMemcpyDeviceToHost));
-  return HSDL_OK;
+  // the kernel reads the requests from pinned memory and writes the answers
+  // there; a slot's copies overlap the other slot's queries
+  constexpr size_t kPart = (size_t)1 << 18;
+  static_assert(kPart * 13 <= kStageBytes, "a part fits a slot");
+  StageLease stage;
+  if ((rc = stage.take(dev, std::min(n, kPart) * 13, n > kPart ? 2 : 1, false))) return rc;
+  const size_t part = std::min(n, kPart);
+  size_t sent = 0, first[2] = {0, 0}, cnt[2] = {0, 0};
+  for (int x = 0;; x ^= 1) {
+    uint8_t *h = stage->h[x];
+    uint32_t *hs = reinterpret_cast<uint32_t *>(h), *ht = hs + part;
+    int32_t *ho = reinterpret_cast<int32_t *>(ht + part);
+    int8_t *hk = reinterpret_cast<int8_t *>(ho + part);
+    if (cnt[x]) {
+      HSDL_HIP(hipStreamSynchronize(stage->st[x]));
+      std::memcpy(out + first[x], ho, cnt[x] * 4);
+      cnt[x] = 0;
+    }
+    if (sent < n) {
+      const size_t m = std::min(part, n - sent);
+      std::memcpy(hs, s + sent, m * 4);
+      std::memcpy(ht, t + sent, m * 4);
+      std::memcpy(hk, k + sent, m);
+      if ((rc = launch_query(idx, m, hs, ht, hk, ho, stage->st[x]))) return rc;
+      first[x] = sent;
+      cnt[x] = m;
+      sent += m;
+    } else if (!cnt[x ^ 1]) {
+      return HSDL_OK;
+    }
+  }
 }
 
 int hsdl_query(const hsdl_index *idx, size_t n, const uint32_t *s, const uint32_t *t,
@@ -521,8 +628,7 @@ static int query_noalloc_body(const hsdl_index *idx, size_t n, const uint32_t *s
                              "queries per call");
   if (n == 0) return HSDL_OK;
   if (!s || !t || !k || !out) return fail(HSDL_EINVAL, "null query arrays");
-  for (size_t i = 0; i < n; ++i)
-    if (s[i] >= idx->n || t[i] >= idx->n) return fail(HSDL_EINVAL, "query vertex out of range");
+  if (!all_below(s, t, n, idx->n)) return fail(HSDL_EINVAL, "query vertex out of range");
   int dev = 0;
   int rc = use_device(idx->device, &dev);
   if (rc) return rc;

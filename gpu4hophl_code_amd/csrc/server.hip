@@ -35,7 +35,8 @@ struct Slot {
   uint8_t *h_req = nullptr;
   int32_t *h_out = nullptr;
   DevBuf d_req, d_out;
-  std::vector<uint64_t> ids, arrival;
+  uint64_t first = 0;  // id of the first request (a batch holds consecutive ones)
+  std::vector<uint64_t> arrival;
   size_t count = 0;
   bool busy = false;
   uint64_t t_close = 0, t_h2d = 0, t_kernel = 0, t_d2h = 0, t_launched = 0;
@@ -97,6 +98,18 @@ struct hsdl_server {
 
 namespace hsdl {
 
+// The ring entries [pos, pos + n) as at most two contiguous runs: f(index in
+// the ring, offset in the range, length).
+template <class F>
+static void ring_runs(uint64_t pos, size_t n, uint64_t cap, F &&f) {
+  for (size_t done = 0; done < n;) {
+    const uint64_t p = (pos + done) % cap;
+    const size_t m = (size_t)std::min<uint64_t>(n - done, cap - p);
+    f((size_t)p, done, m);
+    done += m;
+  }
+}
+
 // Mapped staging: the kernel reads the packed requests from and writes the
 // answers to pinned fine-grained host memory, so a batch costs one launch and
 // one event record.  Copy staging moves them through device buffers.
@@ -149,9 +162,13 @@ static void worker_loop(hsdl_server *srv) {
                            {sl.count, sl.count ? sl.arrival[0] : 0, sl.t_close, sl.t_h2d,
                             sl.t_kernel, sl.t_d2h, sl.t_launched, t}});
       const uint64_t rt = srv->r_tail.load(std::memory_order_relaxed);
-      for (size_t i = 0; i < sl.count; ++i)
-        srv->ring[(rt + i) % cap] =
-            Result{sl.ids[i], sl.h_out[i], t > sl.arrival[i] ? t - sl.arrival[i] : 0};
+      ring_runs(rt, sl.count, cap, [&](size_t p, size_t at, size_t m) {
+        Result *r = srv->ring.data() + p;
+        for (size_t i = 0; i < m; ++i) {
+          const uint64_t arr = sl.arrival[at + i];
+          r[i] = Result{sl.first + at + i, sl.h_out[at + i], t > arr ? t - arr : 0};
+        }
+      });
       srv->r_tail.store(rt + sl.count, std::memory_order_release);
       srv->completed += sl.count;
       sl.busy = false;
@@ -183,14 +200,13 @@ static void worker_loop(hsdl_server *srv) {
         uint32_t *hs = (uint32_t *)sl.h_req;
         uint32_t *ht = (uint32_t *)(sl.h_req + 4 * n);
         int8_t *hk = (int8_t *)(sl.h_req + 8 * n);
-        for (size_t i = 0; i < n; ++i) {
-          const uint64_t p = (srv->q_head + i) % cap;
-          hs[i] = srv->q_s[p];
-          ht[i] = srv->q_t[p];
-          hk[i] = srv->q_k[p];
-          sl.ids[i] = srv->q_head + i;
-          sl.arrival[i] = srv->q_arr[p];
-        }
+        ring_runs(srv->q_head, n, cap, [&](size_t p, size_t at, size_t m) {
+          std::memcpy(hs + at, srv->q_s.data() + p, m * 4);
+          std::memcpy(ht + at, srv->q_t.data() + p, m * 4);
+          std::memcpy(hk + at, srv->q_k.data() + p, m);
+          std::memcpy(sl.arrival.data() + at, srv->q_arr.data() + p, m * 8);
+        });
+        sl.first = srv->q_head;
         srv->q_head += n;
         g.unlock();
         srv->cv.notify_all();
@@ -273,7 +289,6 @@ static int server_create_body(const hsdl_index *idx, const hsdl_server_opts *opt
       hsdl_server_destroy(srv);
       return rc;
     }
-    sl.ids.resize(o.max_batch);
     sl.arrival.resize(o.max_batch);
     // warm the slot: the first copy and launch on a fresh stream pay one-time
     // costs that would otherwise land on the first requests' latency
@@ -311,8 +326,7 @@ static int enqueue_requests(hsdl_server *srv, size_t n, const uint32_t *s, const
                             bool partial, size_t *taken) {
   if (!srv) return fail(HSDL_EINVAL, "null server");
   if (n && (!s || !t || !k)) return fail(HSDL_EINVAL, "null request arrays");
-  for (size_t i = 0; i < n; ++i)
-    if (s[i] >= srv->idx->n || t[i] >= srv->idx->n) return fail(HSDL_EINVAL, "vertex out of range");
+  if (!all_below(s, t, n, srv->idx->n)) return fail(HSDL_EINVAL, "vertex out of range");
   const uint64_t cap = srv->o.queue_capacity;
   const uint64_t now = now_ns();
   std::lock_guard<std::mutex> g(srv->mu);
@@ -322,13 +336,15 @@ static int enqueue_requests(hsdl_server *srv, size_t n, const uint32_t *s, const
   if (!partial && n > room) return fail(HSDL_EBUSY, "request queue full");
   const size_t m = (size_t)std::min<uint64_t>(n, room);
   if (first_id) *first_id = srv->q_tail;
-  for (size_t i = 0; i < m; ++i) {
-    const uint64_t p = (srv->q_tail + i) % cap;
-    srv->q_s[p] = s[i];
-    srv->q_t[p] = t[i];
-    srv->q_k[p] = k[i];
-    srv->q_arr[p] = arrival_ns ? arrival_ns[i] : now;
-  }
+  ring_runs(srv->q_tail, m, cap, [&](size_t p, size_t at, size_t len) {
+    std::memcpy(srv->q_s.data() + p, s + at, len * 4);
+    std::memcpy(srv->q_t.data() + p, t + at, len * 4);
+    std::memcpy(srv->q_k.data() + p, k + at, len);
+    if (arrival_ns)
+      std::memcpy(srv->q_arr.data() + p, arrival_ns + at, len * 8);
+    else
+      std::fill_n(srv->q_arr.data() + p, len, now);
+  });
   srv->q_tail += m;
   if (taken) *taken = m;
   return HSDL_OK;
@@ -352,12 +368,14 @@ int hsdl_server_poll(hsdl_server *srv, size_t cap, uint64_t *ids, int32_t *answe
   const uint64_t h = srv->r_head.load(std::memory_order_relaxed);
   const uint64_t t = srv->r_tail.load(std::memory_order_acquire);
   const size_t n = (size_t)std::min<uint64_t>(cap, t - h);
-  for (size_t i = 0; i < n; ++i) {
-    const Result &r = srv->ring[(h + i) % rcap];
-    if (ids) ids[i] = r.id;
-    if (answers) answers[i] = r.ans;
-    if (latency_ns) latency_ns[i] = r.lat;
-  }
+  ring_runs(h, n, rcap, [&](size_t p, size_t at, size_t m) {
+    const Result *r = srv->ring.data() + p;
+    for (size_t i = 0; i < m; ++i) {
+      if (ids) ids[at + i] = r[i].id;
+      if (answers) answers[at + i] = r[i].ans;
+      if (latency_ns) latency_ns[at + i] = r[i].lat;
+    }
+  });
   srv->r_head.store(h + n, std::memory_order_release);
   *n_out = n;
   return srv->error ? fail(srv->error, "a batch launch failed") : HSDL_OK;
@@ -460,15 +478,16 @@ static int server_replay_body(hsdl_server *srv, size_t n, const uint32_t *s, con
       std::lock_guard<std::mutex> g(srv->rmu);
       const uint64_t h = srv->r_head.load(std::memory_order_relaxed);
       const uint64_t t = srv->r_tail.load(std::memory_order_acquire);
-      for (uint64_t p = h; p < t; ++p) {
-        const Result &r = srv->ring[p % rcap];
-        const uint64_t i = r.id - base_id;
-        if (i < n) {
-          if (answers) answers[i] = r.ans;
-          if (latency_ns) latency_ns[i] = r.lat;
-          ++got;
+      ring_runs(h, (size_t)(t - h), rcap, [&](size_t p, size_t, size_t m) {
+        for (const Result *r = srv->ring.data() + p, *e = r + m; r < e; ++r) {
+          const uint64_t i = r->id - base_id;
+          if (i < n) {
+            if (answers) answers[i] = r->ans;
+            if (latency_ns) latency_ns[i] = r->lat;
+            ++got;
+          }
         }
-      }
+      });
       fresh = (size_t)(t - h);
       srv->r_head.store(t, std::memory_order_release);
     }

@@ -153,3 +153,44 @@ def test_paths_over_pieces():
         wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), K + 1)
         assert np.array_equal(counts.astype(np.int32), wcounts)
         assert np.array_equal(edges.astype(np.int32), wedges)
+
+
+def test_host_calls_in_parts():
+    """Host-array queries and paths that end at, before and past a staging
+    slot's part and span several, paths whose cap exceeds a slot, and calls from
+    six threads at once on one index (more than the pool keeps), with the pool
+    released in between: the oracle's answers."""
+    from concurrent.futures import ThreadPoolExecutor
+    g = ragged(500, 3, 9)
+    want = O.kround(csr_of(g), 4)
+    idx = H.hop_constrained_two_hop_labels_generation(g, 4, parents=True)
+    s, t = (x.ravel().astype(np.uint32) for x in np.meshgrid(np.arange(500), np.arange(500)))
+    k = (np.arange(250000) % 6).astype(np.int8)
+    ans = O.query(want, s, t, k)
+    edges, counts = O.paths(want, s, t, k.astype(np.int32), 5)
+
+    def query(n, at):
+        i = (np.arange(n) + at) % 250000
+        return np.array_equal(idx.query(s[i], t[i], k[i]), ans[i])
+
+    def paths(n, at):
+        i = (np.arange(n) + at) % 250000
+        e, c = idx.paths(s[i], t[i], k[i], cap=5)
+        return np.array_equal(c, counts[i]) and np.array_equal(e, edges[i])
+
+    part = 1 << 18
+    for n in (1, part - 1, part, part + 1, 3 * part + 5):
+        print(f"[parts] queries {n}", flush=True)
+        assert query(n, n)
+    part = ((4 << 20) - 64) // 53 & ~3
+    for n in (part, part + 1, 3 * part - 1):
+        print(f"[parts] paths {n}", flush=True)
+        assert paths(n, n)
+    e, c = idx.paths(s[:3], t[:3], k[:3], cap=600000)
+    assert np.array_equal(c, counts[:3]) and np.array_equal(e[:, :5], edges[:3]) and not e[:, 5:].any()
+    for _ in range(2):
+        with ThreadPoolExecutor(6) as pool:
+            jobs = [pool.submit(query, 300001, 7 * i) for i in range(6)]
+            jobs += [pool.submit(paths, 90001, 11 * i) for i in range(6)]
+            assert all(j.result() for j in jobs)
+        H.release_scratch()
