@@ -9,20 +9,12 @@
 // oracle's tests require both readings to give the same output.
 //
 // Two passes, exact in every case:
-//  1. k_clean_tile: the predicate with `kept` replaced by every earlier label
+//  1. k_clean_pairs: the predicate with `kept` replaced by every earlier label
 //     of v.  That set contains the sequential kept set, so its minima are
 //     never larger: when it removes nothing from L(v), the sequential walk
-//     keeps every label of v as well.  Pass 1 has no order dependence.  One
-//     workgroup (16 wavefronts) takes a vertex v: it builds a hash tile of
-//     L(v) (hub -> per-hop prefix minimum distance; in LDS, or in the
-//     workgroup's slice of a global arena for long lists), then the waves take
-//     16-label windows of L(v) in turn, find the windows' group heads (hub u),
-//     load-balance the heads' lists L(u) over the lanes by a register prefix
-//     sum, and every element (w,h1,d1) of L(u) with w < u that could still
-//     remove a group label (h1 + 1 <= the group's largest hop and d1 <= its
-//     largest dist) looks w up once in the tile: a group label (u,h,d) falls
-//     when d1 + tile[w][h - h1] <= d.  Pairs through u itself (earlier labels
-//     of the same group) are checked directly.
+//     keeps every label of v as well.  Pass 1 has no order dependence: it
+//     tests the pairs of L(v)'s labels densely against a distance bound and
+//     looks L(u) up for the few that pass it; long lists take k_clean_tile.
 //  2. k_clean_seq: vertices where pass 1 would remove something are walked
 //     group by group in order with keep bits in LDS, exactly as the
 //     reference does.
@@ -85,6 +77,361 @@ __device__ inline uint32_t lb_hub(const unsigned long long *lab, uint32_t lo, ui
 }
 
 // ---------------------------------------------------------------- pass 1
+// A label i = (u,h,d) of v falls when an earlier label j = (w,h2,d2) of v has a
+// partner (w,h1,d1) in L(u) with h1 <= h - h2 and d1 <= d - d2.  The pairs
+// (i, j) of one list are tested densely against a bound that few pass, and
+// only those look L(u) up:
+//   w < u:  d2 <= d - m(u, h - h2), where m(u, x) is the least distance of
+//           L(u)'s labels of hop <= x and hub < u (k_clean_min): whatever the
+//           partner is, it is no nearer;
+//   w = u:  an earlier label of i's own hub group, at no larger distance.
+// Streaming every head's list L(u) through a hash tile of L(v) (k_clean_tile,
+// below) reads 174 labels per label of v on R-MAT scale 16 (K = 5); the pairs
+// of the same labels are 73 per label before the bound, at three VALU
+// instructions per 64 of them, and 7.5 after it.  The bound is that sharp in
+// this direction because L(u) is the list of the higher-ranked vertex.
+//
+// Pairs are walked by hop: the slice's labels are copied in hop order (hub
+// order within a hop, k_clean_sort), lanes hold 64 consecutive labels i of it,
+// and for each hop x below theirs a wave walks the labels j of hop x, which
+// are uniform (scalar loads, 16 or 32 to a load): per j one comparison with
+// the lane's packed (hub) limit, one with its distance bound, and a shift into
+// a 32-bit mask.  The walk of a hop ends at the largest hub among the lanes.
+// The mask's pairs go to a queue in LDS, and every 64 of them search L(u) in
+// the index, a pair per lane.
+struct Pair32 {
+  using T = uint32_t;
+  uint32_t hop_bits, dist_bits;
+  __device__ T pack(unsigned long long l) const {
+    return (label_hub(l) << (hop_bits + dist_bits)) | (label_hop(l) << dist_bits) | label_dist(l);
+  }
+  __device__ uint32_t hub(T l) const { return l >> (hop_bits + dist_bits); }
+  __device__ uint32_t hop(T l) const { return __builtin_amdgcn_ubfe(l, dist_bits, hop_bits); }
+  __device__ uint32_t dist(T l) const { return l & ((1u << dist_bits) - 1u); }
+  __device__ T below(uint32_t u) const { return u << (hop_bits + dist_bits); }  // labels of hubs < u
+};
+struct Pair64 {
+  using T = unsigned long long;
+  __device__ T pack(unsigned long long l) const { return l; }
+  __device__ uint32_t hub(T l) const { return label_hub(l); }
+  __device__ uint32_t hop(T l) const { return label_hop(l); }
+  __device__ uint32_t dist(T l) const { return label_dist(l); }
+  __device__ T below(uint32_t u) const { return (unsigned long long)u << 32; }
+};
+
+// m[u * K + x - 1], x = 1..K: least distance of L(u)'s labels of hop <= x and
+// hub < u (m may be null); maxima[0], [1]: the longest list and the largest
+// distance.  A wave per vertex.
+__global__ void __launch_bounds__(256) k_clean_min(uint32_t n, uint32_t K,
+                                                   const unsigned long long *off,
+                                                   const unsigned long long *lab, uint32_t *m,
+                                                   uint32_t *maxima) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
+  uint32_t ml = 0, md = 0;
+  for (uint32_t u = wave; u < n; u += nwaves) {
+    const unsigned long long b = off[u];
+    const uint32_t len = (uint32_t)(off[u + 1] - b);
+    ml = max(ml, len);
+    uint32_t best[kMaxK + 1];
+#pragma unroll
+    for (uint32_t x = 0; x <= kMaxK; ++x) best[x] = kInf32;
+    for (uint32_t j = lane; j < len; j += kWave) {
+      const unsigned long long l = lab[b + j];
+      const uint32_t h = label_hop(l), d = label_dist(l);
+      md = max(md, d);
+      if (!m || label_hub(l) >= u) continue;
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x)
+        if (x <= K && x >= h) best[x] = min(best[x], d);
+    }
+    if (!m) continue;
+    uint32_t mine = kInf32;
+#pragma unroll
+    for (uint32_t x = 1; x <= kMaxK; ++x) {
+      if (x > K) continue;
+      const uint32_t r = wave_min_u32(best[x]);
+      if (lane == x - 1) mine = r;
+    }
+    if (lane < K) m[(uint64_t)u * K + lane] = mine;
+  }
+  md = wave_max_u32(md);
+  // (one atomic per wave that could raise the maxima)
+  if (lane == 0) {
+    if (ml > __hip_atomic_load(&maxima[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&maxima[0], ml);
+    if (md > __hip_atomic_load(&maxima[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&maxima[1], md);
+  }
+}
+
+// The labels of vertices [v0, v1) in hop order (index order within a hop), from
+// out[0], and hcnt[(v - v0) * K + x], x < K: labels of v of hop <= x.  A wave
+// per vertex counts its labels' hops, then scatters them.
+template <class F>
+__global__ void __launch_bounds__(256) k_clean_sort(F f, uint32_t v0, uint32_t v1, uint32_t K,
+                                                    const unsigned long long *off,
+                                                    const unsigned long long *lab,
+                                                    typename F::T *out, uint32_t *hcnt) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
+  const unsigned long long base = off[v0];
+  for (uint32_t v = v0 + wave; v < v1; v += nwaves) {
+    const unsigned long long b = off[v];
+    const uint32_t len = (uint32_t)(off[v + 1] - b);
+    uint32_t pos[kMaxK + 1];
+#pragma unroll
+    for (uint32_t x = 0; x <= kMaxK; ++x) pos[x] = 0;
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const uint32_t hop = j0 + lane < len ? label_hop(lab[b + j0 + lane]) : kInf32;
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x)
+        if (x <= K) pos[x] += (uint32_t)__popcll(__ballot(hop == x));
+    }
+    uint32_t run = 0;
+#pragma unroll
+    for (uint32_t x = 0; x <= kMaxK; ++x) {
+      const uint32_t c = pos[x];
+      pos[x] = run;
+      run += c;
+      if (x < K && lane == 0) hcnt[(uint64_t)(v - v0) * K + x] = run;
+    }
+    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
+      const unsigned long long l = lab[b + min(j0 + lane, len - 1)];
+      const uint32_t hop = j0 + lane < len ? label_hop(l) : kInf32;
+      uint32_t dst = 0;
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x) {
+        if (x > K) continue;
+        const unsigned long long mk = __ballot(hop == x);
+        if (hop == x) dst = pos[x] + (uint32_t)__popcll(mk & lt_mask);
+        pos[x] += (uint32_t)__popcll(mk);
+      }
+      if (hop != kInf32) out[b - base + dst] = f.pack(l);
+    }
+  }
+}
+
+// Whether L(u) = lab[lo, lo + len) holds a label of hub w, hop <= x and
+// distance <= d (per lane).
+__device__ inline bool has_partner(const unsigned long long *__restrict__ lab,
+                                   unsigned long long lo, uint32_t len, uint32_t w, uint32_t x,
+                                   uint32_t d) {
+  const unsigned long long *L = lab + lo;
+  uint32_t p = 0, left = len;
+  while (left) {
+    const uint32_t half = left >> 1;
+    if (label_hub(L[p + half]) < w) {
+      p += half + 1;
+      left -= half + 1;
+    } else {
+      left = half;
+    }
+  }
+  for (; p < len; ++p) {  // one label per hop, hops ascending
+    const unsigned long long l = L[p];
+    if (label_hub(l) != w || label_hop(l) > x) return false;
+    if (label_dist(l) <= d) return true;
+  }
+  return false;
+}
+
+// Whether some pair of v's labels removes one of the 64 labels from position i0
+// of the hop-ordered list L (whole wave).  hc: v's prefix counts; q: the wave's
+// queue of 128 entries (position of j << 6 | lane of i).
+template <class F>
+__device__ bool chunk_removes(const F &f, uint32_t v, uint32_t K,
+                              const unsigned long long *__restrict__ off,
+                              const unsigned long long *__restrict__ lab,
+                              const typename F::T *__restrict__ L,
+                              const uint32_t *__restrict__ hc, const uint32_t *__restrict__ m,
+                              uint32_t len, uint32_t i0, lds_ptr<uint32_t> q, uint64_t &streamed) {
+  using T = typename F::T;
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const T li = L[min(i0 + lane, len - 1)];
+  const uint32_t u = f.hub(li), h = f.hop(li), d = f.dist(li);
+  const bool act = i0 + lane < len && u != v && h > 0;
+  const unsigned long long lo = off[u];
+  const uint32_t ulen = (uint32_t)(off[u + 1] - lo);
+  const uint32_t hmax = __builtin_amdgcn_readfirstlane(wave_max_u32(act ? h : 0u));
+  uint32_t qn = 0;
+  bool hit = false;
+  auto look_up = [&](uint32_t cnt) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t e = q[lane];
+    const int il = (int)(e & 63u);
+    const T lj = L[lane < cnt ? e >> 6 : 0u];
+    const T pi = __shfl(li, il, kWave);
+    const unsigned long long plo = __shfl(lo, il, kWave);
+    const uint32_t plen = __shfl(ulen, il, kWave);
+    if (lane < cnt && has_partner(lab, plo, plen, f.hub(lj), f.hop(pi) - f.hop(lj),
+                                  f.dist(pi) - f.dist(lj)))
+      hit = true;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  for (uint32_t x = 0; x < hmax; ++x) {
+    const uint32_t zb = x ? hc[x - 1] : 0u, ze = hc[x];
+    if (zb == ze) continue;
+    const uint32_t mu = act && h > x ? m[(uint64_t)u * K + (h - x - 1)] : kInf32;
+    const bool ok = mu <= d;
+    if (!__ballot(ok)) continue;
+    const uint32_t lim = ok ? d - mu : 0u;
+    const T ulim = ok ? f.below(u) : (T)0;  // no label lies below 0
+    const T umax = f.below(__builtin_amdgcn_readfirstlane(wave_max_u32(ok ? u : 0u)));
+    for (uint32_t j = zb; j < ze; j += 32) {
+      const T *Z = L + j;
+      if (Z[0] >= umax) break;
+      streamed += 32;
+      uint32_t mask = 0;
+#pragma unroll
+      for (uint32_t t = 0; t < 32; ++t) {
+        const T lj = Z[t];  // past the list's end: padding, masked below
+        mask = (mask << 1) | (uint32_t)(lj < ulim && f.dist(lj) <= lim);
+      }
+      if (ze - j < 32) mask &= ~0u << (32 - (ze - j));
+      for (;;) {
+        const unsigned long long any = __ballot(mask != 0);
+        if (!any) break;
+        const uint32_t t = (uint32_t)__builtin_clz(mask | 1u);
+        if (mask) {
+          q[qn + (uint32_t)__popcll(any & lt_mask)] = (j + t) << 6 | lane;
+          mask &= ~(0x80000000u >> t);
+        }
+        qn += (uint32_t)__popcll(any);
+        if (qn >= kWave) {
+          look_up(kWave);
+          qn -= kWave;
+          const uint32_t rest = q[kWave + lane];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          if (lane < qn) q[lane] = rest;
+          if (__ballot(hit)) return true;
+        }
+      }
+    }
+  }
+  if (qn) look_up(qn);
+  return __ballot(hit) != 0;
+}
+
+// Whether two labels of one hub group of v's list [vb, vb + len) remove the
+// later one, among the 64 from position i0 (index order; whole wave).
+__device__ inline bool group_removes(uint32_t v, const unsigned long long *__restrict__ off,
+                                     const unsigned long long *__restrict__ lab,
+                                     unsigned long long vb, uint32_t len, uint32_t i0) {
+  const uint32_t i = i0 + (uint32_t)lane_id();
+  bool hit = false;
+  if (i < len) {
+    const unsigned long long l = lab[vb + i];
+    const uint32_t u = label_hub(l), h = label_hop(l), d = label_dist(l);
+    for (uint32_t p = i; u != v && p > 0; --p) {
+      const unsigned long long e = lab[vb + p - 1];
+      if (label_hub(e) != u) break;
+      if (label_dist(e) <= d) {
+        const unsigned long long lo = off[u];
+        if (has_partner(lab, lo, (uint32_t)(off[u + 1] - lo), u, h - label_hop(e),
+                        d - label_dist(e)))
+          hit = true;
+      }
+    }
+  }
+  return __ballot(hit) != 0;
+}
+
+// ctr[0]: redo count, ctr[1]: long lists of the slice, ctr[2]: next vertex of
+// the slice (kLong: next entry of `longs`), ctr[4..5]: labels read (u64).
+// kLong = false: a wave per vertex, lists of more than kCleanLong labels are
+// left in `longs`.  kLong = true: a workgroup per list of `longs`, its waves
+// taking the chunks in turn.
+constexpr uint32_t kCleanLong = 2048;
+constexpr uint32_t kCleanClaim = 4;  // vertices a wave claims at once
+template <class F, bool kLong>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
+k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long long *__restrict__ off,
+              const unsigned long long *__restrict__ lab, const typename F::T *__restrict__ srt,
+              const uint32_t *__restrict__ hcnt, const uint32_t *__restrict__ m, uint32_t *redo,
+              uint32_t *longs, uint32_t *ctr) {
+  __shared__ uint32_t queue[256 / kWave][2 * kWave];
+  __shared__ uint32_t sh_l, sh_c, sh_hit;
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  lds_ptr<uint32_t> q = (lds_ptr<uint32_t>)queue[wib];
+  const unsigned long long base = off[v0];
+  uint64_t streamed = 0;
+  if constexpr (!kLong) {
+    for (;;) {
+      uint32_t c = 0;
+      if (lane == 0) c = atomicAdd(&ctr[2], kCleanClaim);
+      c = __builtin_amdgcn_readfirstlane(c);
+      if (c >= v1 - v0) break;
+      for (uint32_t v = v0 + c; v < min(v1, v0 + c + kCleanClaim); ++v) {
+        const unsigned long long vb = off[v];
+        const uint32_t len = (uint32_t)(off[v + 1] - vb);
+        if (len > kCleanLong) {
+          if (lane == 0) longs[atomicAdd(&ctr[1], 1u)] = v;
+          continue;
+        }
+        bool gone = false;
+        for (uint32_t i0 = 0; i0 < len && !gone; i0 += kWave)
+          gone = group_removes(v, off, lab, vb, len, i0) ||
+                 chunk_removes(f, v, K, off, lab, srt + (vb - base), hcnt + (uint64_t)(v - v0) * K,
+                               m, len, i0, q, streamed);
+        if (gone && lane == 0) redo[atomicAdd(&ctr[0], 1u)] = v;
+      }
+    }
+  } else {
+    const uint32_t cnt = ctr[1];
+    for (;;) {
+      if (threadIdx.x == 0) {
+        sh_l = atomicAdd(&ctr[2], 1u);
+        sh_c = 0;
+        sh_hit = 0;
+      }
+      __syncthreads();
+      const uint32_t li = __builtin_amdgcn_readfirstlane(sh_l);
+      if (li >= cnt) break;
+      const uint32_t v = longs[li];
+      const unsigned long long vb = off[v];
+      const uint32_t len = (uint32_t)(off[v + 1] - vb);
+      for (;;) {
+        uint32_t c = 0;
+        if (lane == 0) c = atomicAdd(&sh_c, 1u);
+        c = __builtin_amdgcn_readfirstlane(c);
+        const uint32_t seen = __hip_atomic_load(&sh_hit, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+        if ((uint64_t)c * kWave >= len || __builtin_amdgcn_readfirstlane(seen)) break;
+        if (group_removes(v, off, lab, vb, len, c * kWave) ||
+            chunk_removes(f, v, K, off, lab, srt + (vb - base), hcnt + (uint64_t)(v - v0) * K, m,
+                          len, c * kWave, q, streamed))
+          if (lane == 0)
+            __hip_atomic_store(&sh_hit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      __syncthreads();
+      if (threadIdx.x == 0 && sh_hit) redo[atomicAdd(&ctr[0], 1u)] = v;
+      __syncthreads();
+    }
+  }
+  if (lane == 0 && streamed)
+    atomicAdd(reinterpret_cast<unsigned long long *>(ctr) + 2, (unsigned long long)streamed);
+}
+
+// ------------------------------------------------- pass 1, long lists
+// Long lists (a mean above kPairMean labels): k_clean_tile, a workgroup of
+// sixteen waves per vertex.  It builds a hash tile of L(v) (hub -> per-hop
+// prefix minimum distance; in LDS, or in the workgroup's slice of a global arena
+// for long lists), then the waves take windows of L(v) in turn, find the windows'
+// group heads (hub u), stream the heads' lists L(u), and every element (w,h1,d1)
+// with w < u looks w up once in the tile: a group label (u,h,d) falls when d1 +
+// tile[w][h - h1] <= d.  Pairs through u itself (earlier labels of the same
+// group) are checked directly.  The pair form looks up about a dozen labels per
+// label there, at random in lists that no cache holds: R-MAT 262,144 at K = 5
+// (672 labels per list) takes 164 ms that way (1.1 TB past L2) against 64 ms with
+// tiles, 40,001 vertices (531) 7.4 against 6.3 ms, a group of 65,536 (190) 2.5
+// against 3.8 ms, and the 1024 x 1024 grid (66; 8-byte lists) 10.0 against 24.5 ms.
+constexpr uint64_t kPairMean = 256;
 // The heads' lists L(u) are streamed from the index's 8-byte labels, or from
 // a 32-bit copy of them (hub | hop | dist fields) when the fields fit one
 // word: the first pass reads far more list labels than anything else and
@@ -102,8 +449,7 @@ struct Stream64 {
   }
 };
 // The 32-bit copy keeps each list stably sorted by hop (hub order within a
-// hop), with hcnt[u * K + x] = elements of L(u) of hop <= x (x < K), when
-// hcnt is set: an element pairs with the tile through hop h1 + 1 or more
+// hop), with hcnt[u * K + x] = elements of L(u) of hop <= x (x < K): an element pairs with the tile through hop h1 + 1 or more
 // when w != v, so a group whose deepest label has hop maxh can use only
 // L(u)'s elements of hop <= maxh - 1 -- a prefix of the sorted list, which
 // the stream stops at (the self label, hop 0, is its first element).  Only a
@@ -117,7 +463,7 @@ struct Stream32 {
   uint32_t K;
   __device__ const T *list(unsigned long long b) const { return lab + b; }
   __device__ uint32_t upto(uint32_t u, uint32_t maxhop, uint32_t len) const {
-    return hcnt && maxhop < K ? hcnt[(uint64_t)u * K + maxhop] : len;
+    return maxhop < K ? hcnt[(uint64_t)u * K + maxhop] : len;
   }
   __device__ void dec(T l, uint32_t &w, uint32_t &h, uint32_t &d) const {
     w = l >> (hop_bits + dist_bits);
@@ -125,73 +471,6 @@ struct Stream32 {
     d = l & ((1u << dist_bits) - 1u);
   }
 };
-
-__device__ inline uint32_t pack32(unsigned long long l, uint32_t hop_bits, uint32_t dist_bits) {
-  return (label_hub(l) << (hop_bits + dist_bits)) | (label_hop(l) << dist_bits) | label_dist(l);
-}
-
-__global__ void k_pack32(uint64_t total, const unsigned long long *lab, uint32_t *out,
-                         uint32_t hop_bits, uint32_t dist_bits) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < total;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    out[i] = pack32(lab[i], hop_bits, dist_bits);
-}
-
-// The 32-bit copy with every list stably sorted by hop, and the per-hop
-// prefix counts (Stream32): a wave per vertex counts its labels' hops, then
-// scatters them in list order into their hop's run (positions by ballot).
-__global__ void __launch_bounds__(256) k_pack32_hop(uint32_t n, uint32_t K,
-                                                    const unsigned long long *off,
-                                                    const unsigned long long *lab, uint32_t *out,
-                                                    uint32_t *hcnt, uint32_t hop_bits,
-                                                    uint32_t dist_bits) {
-  const uint32_t lane = (uint32_t)lane_id();
-  const unsigned long long lt_mask = (1ull << lane) - 1ull;
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
-  const uint32_t K1 = K + 1;
-  for (uint32_t v = wave; v < n; v += nwaves) {
-    const unsigned long long b = off[v];
-    const uint32_t len = (uint32_t)(off[v + 1] - b);
-    uint32_t cnt[kMaxK + 1];
-#pragma unroll
-    for (uint32_t x = 0; x <= kMaxK; ++x) cnt[x] = 0;
-    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
-      const uint32_t j = j0 + lane;
-      const uint32_t hop = j < len ? label_hop(lab[b + j]) : kInf32;
-#pragma unroll
-      for (uint32_t x = 0; x <= kMaxK; ++x)
-        if (x < K1) cnt[x] += (uint32_t)__popcll(__ballot(hop == x));
-    }
-    uint32_t pos[kMaxK + 1];
-    uint32_t run = 0;
-#pragma unroll
-    for (uint32_t x = 0; x <= kMaxK; ++x) {
-      pos[x] = run;
-      run += x < K1 ? cnt[x] : 0u;
-      // hcnt[v * K + x]: labels of hop <= x, for x = 0..K-1
-      if (x < K && lane == 0) hcnt[(uint64_t)v * K + x] = run;
-    }
-    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
-      const uint32_t j = j0 + lane;
-      unsigned long long l = 0;
-      uint32_t hop = kInf32;
-      if (j < len) {
-        l = lab[b + j];
-        hop = label_hop(l);
-      }
-      uint32_t dst = 0;
-#pragma unroll
-      for (uint32_t x = 0; x <= kMaxK; ++x) {
-        if (x >= K1) continue;
-        const unsigned long long m = __ballot(hop == x);
-        if (hop == x) dst = pos[x] + (uint32_t)__popcll(m & lt_mask);
-        pos[x] += (uint32_t)__popcll(m);
-      }
-      if (j < len) out[b + dst] = pack32(l, hop_bits, dist_bits);
-    }
-  }
-}
 
 // True when the all-earlier predicate removes a label of a group whose head
 // lies in L(v)[p0, p0 + win).  The wave walks the window's heads in order
@@ -441,8 +720,8 @@ template <class V, class S>
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_clean_tile(uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
              const unsigned long long *__restrict__ lab, S str,
-             uint8_t *keep, uint32_t *new_len, uint32_t *redo, uint32_t *ctr, uint32_t lds_slots,
-             uint32_t *gtile, uint64_t gwords, uint32_t win, uint32_t indexed) {
+             uint32_t *redo, uint32_t *ctr, uint32_t lds_slots, uint32_t *gtile,
+             uint64_t gwords, uint32_t win, uint32_t indexed) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t sh_v, sh_win, sh_heads, sh_removed, sh_row;
   // LDS bytes for a tile (the launch gives lds_slots slots of key + values)
@@ -501,38 +780,17 @@ k_clean_tile(uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
                                sh_removed, sh_row, streamed);
       }
     }
-    if (sh_removed) {
-      if (tid == 0) redo[atomicAdd(&ctr[0], 1u)] = v;
-    } else {
-      for (uint32_t i = tid; i < len; i += kTileThreads) keep[vb + i] = 1;
-      if (tid == 0) new_len[v] = len;
-    }
+    if (sh_removed && tid == 0) redo[atomicAdd(&ctr[0], 1u)] = v;
     __syncthreads();  // shared state and the tile are reused for the next vertex
   }
   if (lane == 0 && streamed)
     atomicAdd(reinterpret_cast<unsigned long long *>(ctr) + 2, (unsigned long long)streamed);
 }
 
-// Largest list length and largest label distance of an index (out[0], out[1]).
-__global__ void __launch_bounds__(256) k_index_maxima(uint32_t n, const unsigned long long *off,
-                                                      const unsigned long long *lab,
-                                                      uint32_t *out) {
-  uint32_t ml = 0, md = 0;
-  const uint32_t nth = gridDim.x * blockDim.x;
-  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += nth) {
-    const unsigned long long b = off[v], e = off[v + 1];
-    ml = max(ml, (uint32_t)(e - b));
-  }
-  const unsigned long long total = off[n];
-  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < total;
-       i += nth)
-    md = max(md, label_dist(lab[i]));
-  ml = wave_max_u32(ml);
-  md = wave_max_u32(md);
-  if (lane_id() == 0) {
-    atomicMax(&out[0], ml);
-    atomicMax(&out[1], md);
-  }
+// Pass 2's start: every label kept, every length the old one.
+__global__ void k_clean_keep_all(uint32_t n, const unsigned long long *off, uint32_t *new_len) {
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+    new_len[v] = (uint32_t)(off[v + 1] - off[v]);
 }
 
 // ---------------------------------------------------------------- pass 2
@@ -709,13 +967,14 @@ __global__ void __launch_bounds__(256) k_compact(uint32_t n, const unsigned long
   }
 }
 
-// The clean's working buffers (keep flags, counts, the 32-bit copy and its
-// hop counts, the tile arena) and the index arrays a clean replaces are kept
+// The clean's working buffers (the hop-ordered copy and its counts, the least
+// distances, keep flags, lengths) and the index arrays a clean replaces are kept
 // per device for the next clean, sized for the largest so far: freeing and
 // allocating gigabytes inside every clean now and then cost a tenth of a
 // second there.  hsdl_release_scratch frees them.
 enum CleanScratchId : int {
-  kCsKeep, kCsNewLen, kCsRedo, kCsGtile, kCsLab32, kCsHcnt, kCsOff, kCsLab, kCsCount
+  kCsKeep, kCsNewLen, kCsRedo, kCsSrt, kCsHcnt, kCsMins, kCsLongs, kCsCtr, kCsGtile, kCsOff,
+  kCsLab, kCsCount
 };
 constexpr int kCsDevices = 64;
 struct CleanScratch {
@@ -769,163 +1028,220 @@ int clean_index(hsdl_index *idx) {
     hipStream_t s;
     ~G() { (void)hipStreamDestroy(s); }
   } guard{st};
-  DevBuf keep, new_len, noff, nlab, redo, ctr, gtile, lab32, hcnt;
+  DevBuf keep, new_len, noff, nlab, redo, ctr, srt, hcnt, mins, longs, gtile;
   const int dev = idx->device;
   // every buffer taken from the kept ones goes back when the clean ends
   struct Give {
     int dev;
-    DevBuf *b[6];
-    int id[6];
+    DevBuf *b[9];
+    int id[9];
     ~Give() {
-      for (int i = 0; i < 6; ++i) give_scratch(dev, id[i], *b[i]);
+      for (int i = 0; i < 9; ++i) give_scratch(dev, id[i], *b[i]);
     }
-  } give{dev, {&keep, &new_len, &redo, &gtile, &lab32, &hcnt},
-         {kCsKeep, kCsNewLen, kCsRedo, kCsGtile, kCsLab32, kCsHcnt}};
-  if ((rc = take_scratch(dev, kCsKeep, keep, std::max<uint64_t>(idx->total, 1))) ||
-      (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull)) ||
-      (rc = take_scratch(dev, kCsOff, noff, (n + 1ull) * 8)) ||
-      (rc = take_scratch(dev, kCsRedo, redo, n * 4ull + 4)) || (rc = ctr.alloc(32)))
+  } give{dev, {&keep, &new_len, &redo, &srt, &hcnt, &mins, &longs, &ctr, &gtile},
+         {kCsKeep, kCsNewLen, kCsRedo, kCsSrt, kCsHcnt, kCsMins, kCsLongs, kCsCtr, kCsGtile}};
+  if ((rc = take_scratch(dev, kCsRedo, redo, n * 4ull + 4)) ||
+      (rc = take_scratch(dev, kCsHcnt, hcnt, (uint64_t)n * idx->K * 4)) ||
+      (rc = take_scratch(dev, kCsCtr, ctr, 64)))
     return rc;
-  HSDL_HIP(hipMemsetAsync(ctr.p, 0, 32, st));
+  uint32_t *cnt = ctr.as<uint32_t>();  // see k_clean_pairs; [3]: pass 2's error bits; [8], [9]: maxima
+  HSDL_HIP(hipMemsetAsync(cnt, 0, 64, st));
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, idx->device);
   const int grid = std::max(1, cus * 8);
-  uint32_t *cnt = ctr.as<uint32_t>();
-  // list-length and distance maxima size the global tile arena and pick the
-  // tile's value width
-  DevBuf maxima;
-  if ((rc = maxima.alloc(8))) return rc;
-  HSDL_HIP(hipMemsetAsync(maxima.p, 0, 8, st));
-  hipLaunchKernelGGL(k_index_maxima, dim3(cus * 4), dim3(256), 0, st, n,
-                     idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                     maxima.as<uint32_t>());
+  const unsigned long long *off = idx->off.as<unsigned long long>();
+  const unsigned long long *lab = idx->lab.as<unsigned long long>();
+  // label pairs, or tiles for long lists (tuning knob HSDL_CLEAN_PAIRS: 0
+  // never pairs, 2 always; HSDL_CLEAN_HOP_SORT=0: tiles over the index's own
+  // order, no hop-ordered copy)
+  const bool hop_sort = env_u32("HSDL_CLEAN_HOP_SORT", 1, 0, 1);
+  const uint32_t form = hop_sort ? env_u32("HSDL_CLEAN_PAIRS", 1, 0, 2) : 0u;
+  const bool pairs = form == 2 || (form == 1 && idx->total <= kPairMean * n);
+  if (pairs && ((rc = take_scratch(dev, kCsLongs, longs, n * 4ull + 4)) ||
+                (rc = take_scratch(dev, kCsMins, mins, (uint64_t)n * idx->K * 4))))
+    return rc;
+  hipLaunchKernelGGL(k_clean_min, dim3(grid), dim3(256), 0, st, n, (uint32_t)idx->K, off, lab,
+                     pairs ? mins.as<uint32_t>() : nullptr, cnt + 8);
   HSDL_HIP(hipGetLastError());
   uint32_t mx[2] = {0, 0};
-  HSDL_HIP(hipMemcpyAsync(mx, maxima.p, 8, hipMemcpyDeviceToHost, st));
+  HSDL_HIP(hipMemcpyAsync(mx, cnt + 8, 8, hipMemcpyDeviceToHost, st));
   HSDL_HIP(hipStreamSynchronize(st));
-  const uint32_t K1 = (uint32_t)idx->K + 1;
-  const bool small_vals = mx[1] < 0xFFFFu;
-  // indexed LDS tiles need hub << kIdxBits to fit a word (tuning knob
-  // HSDL_CLEAN_INDEXED=0: per-slot values only)
-  const uint32_t indexed =
-      (uint64_t)n <= (1ull << (32 - kIdxBits)) ? env_u32("HSDL_CLEAN_INDEXED", 1, 0, 1) : 0u;
-  const uint32_t slot_bytes = 4 + K1 * (small_vals ? 2 : 4);
-  // tuning knob HSDL_CLEAN_LDS_SLOTS caps the LDS tile (small values send
-  // every vertex to the global arena)
-  uint32_t lds_slots = (kTileLdsBytes - 16) / slot_bytes;
-  lds_slots = env_u32("HSDL_CLEAN_LDS_SLOTS", lds_slots, 1, lds_slots);
-  const size_t lds_bytes = (size_t)lds_slots * slot_bytes + 16;
-  const int tgrid = std::max(1, cus * 2);
-  // tuning knob HSDL_CLEAN_WINDOW: labels of L(v) per wave work unit
-  const uint32_t win = env_u32("HSDL_CLEAN_WINDOW", kTileWindow, 1, kMaxWindow);
-  const uint32_t gcap = tile_cap_for(mx[0]);
-  const uint64_t gwords = small_vals ? tile_words<uint16_t>(gcap, K1) : tile_words<uint32_t>(gcap, K1);
-  if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
-  // 32-bit copy of the labels for the heads' list streams, when hub, hop and
-  // distance fields fit one word (tuning knob HSDL_STREAM32=0 keeps the
-  // 8-byte stream; so does a failed allocation of the copy)
+  // 32-bit copies of the labels when hub, hop and distance fit one word
+  // (tuning knob HSDL_STREAM32=0: 8-byte ones)
   uint32_t hub_bits = 1, hop_bits = 1, dist_bits = 1;
   while ((1ull << hub_bits) <= (uint64_t)(n ? n - 1 : 0)) ++hub_bits;
   while ((1ull << hop_bits) <= (uint64_t)idx->K) ++hop_bits;
   while ((1ull << dist_bits) <= (uint64_t)mx[1]) ++dist_bits;
-  bool use32 = env_u32("HSDL_STREAM32", 1, 0, 1) && idx->total > 0 &&
-               hub_bits + hop_bits + dist_bits <= 32;
-  // tuning knob HSDL_CLEAN_HOP_SORT=0 keeps the 32-bit copy in the index's
-  // (hub, hop, dist) order and streams whole lists
-  const bool hop_sort = use32 && env_u32("HSDL_CLEAN_HOP_SORT", 1, 0, 1);
-  if (use32) {
-    if (take_scratch(dev, kCsLab32, lab32, idx->total * 4) == HSDL_OK) {
-      if (hop_sort) {
-        if ((rc = take_scratch(dev, kCsHcnt, hcnt, (uint64_t)n * idx->K * 4))) return rc;
-        hipLaunchKernelGGL(k_pack32_hop, dim3(cus * 8), dim3(256), 0, st, n, (uint32_t)idx->K,
-                           idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                           lab32.as<uint32_t>(), hcnt.as<uint32_t>(), hop_bits, dist_bits);
-      } else {
-        hipLaunchKernelGGL(k_pack32, dim3(cus * 8), dim3(256), 0, st, (uint64_t)idx->total,
-                           idx->lab.as<unsigned long long>(), lab32.as<uint32_t>(), hop_bits,
-                           dist_bits);
+  const bool use32 =
+      env_u32("HSDL_STREAM32", 1, 0, 1) && hub_bits + hop_bits + dist_bits <= 32;
+  uint64_t width = use32 ? 4 : 8;
+  const uint64_t t_kern = now_ns();
+  if (pairs) {
+    // The hop-ordered copy holds a slice of the vertices: all of them up to
+    // kSliceBytes (tuning knob HSDL_CLEAN_SLICE: labels), fewer when there is no
+    // room for it, at least the longest list.
+    constexpr uint64_t kSliceBytes = 2ull << 30;
+    uint64_t cap = std::min<uint64_t>(idx->total, kSliceBytes / width);
+    cap = std::max<uint64_t>({std::min<uint64_t>(cap, env_u32("HSDL_CLEAN_SLICE", 0xFFFFFFFFu, 1,
+                                                             0xFFFFFFFFu)),
+                              mx[0], 1});
+    constexpr uint64_t kPad = 64;  // labels read past a list's end (masked)
+    while ((rc = take_scratch(dev, kCsSrt, srt, (cap + kPad) * width))) {
+      if (rc != HSDL_ENOMEM || cap <= mx[0]) return rc;
+      cap = std::max<uint64_t>(cap / 2, mx[0]);
+    }
+    std::vector<uint64_t> hoff;
+    if (idx->total > cap) {
+      hoff.resize(n + 1ull);
+      HSDL_HIP(hipMemcpy(hoff.data(), off, (n + 1ull) * 8, hipMemcpyDeviceToHost));
+    }
+    auto pass1 = [&](auto f) -> int {
+      using F = decltype(f);
+      using T = typename F::T;
+      for (uint32_t v0 = 0; v0 < n;) {
+        uint32_t v1 = n;
+        if (!hoff.empty()) {
+          const uint64_t end = hoff[v0] + cap;
+          v1 = (uint32_t)(std::upper_bound(hoff.begin() + v0, hoff.end(), end) - hoff.begin()) - 1;
+        }
+        hipLaunchKernelGGL(k_clean_sort<F>, dim3(grid), dim3(256), 0, st, f, v0, v1,
+                           (uint32_t)idx->K, off, lab, srt.as<T>(), hcnt.as<uint32_t>());
+        HSDL_HIP(hipGetLastError());
+        HSDL_HIP(hipMemsetAsync(cnt + 1, 0, 8, st));
+        hipLaunchKernelGGL((k_clean_pairs<F, false>), dim3(grid), dim3(256), 0, st, f, v0, v1,
+                           (uint32_t)idx->K, off, lab, srt.as<T>(), hcnt.as<uint32_t>(),
+                           mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(), cnt);
+        HSDL_HIP(hipGetLastError());
+        if (mx[0] > kCleanLong) {
+          HSDL_HIP(hipMemsetAsync(cnt + 2, 0, 4, st));
+          hipLaunchKernelGGL((k_clean_pairs<F, true>), dim3(grid), dim3(256), 0, st, f, v0, v1,
+                             (uint32_t)idx->K, off, lab, srt.as<T>(), hcnt.as<uint32_t>(),
+                             mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(), cnt);
+          HSDL_HIP(hipGetLastError());
+        }
+        v0 = v1;
       }
+      return HSDL_OK;
+    };
+    if (idx->total && (rc = use32 ? pass1(Pair32{hop_bits, dist_bits}) : pass1(Pair64{})))
+      return rc;
+  } else {
+    const uint32_t K1 = (uint32_t)idx->K + 1;
+    const bool small_vals = mx[1] < 0xFFFFu;
+    // indexed LDS tiles need hub << kIdxBits to fit a word (tuning knob
+    // HSDL_CLEAN_INDEXED=0: per-slot values only)
+    const uint32_t indexed =
+        (uint64_t)n <= (1ull << (32 - kIdxBits)) ? env_u32("HSDL_CLEAN_INDEXED", 1, 0, 1) : 0u;
+    const uint32_t slot_bytes = 4 + K1 * (small_vals ? 2 : 4);
+    // tuning knob HSDL_CLEAN_LDS_SLOTS caps the LDS tile (small values send
+    // every vertex to the global arena)
+    uint32_t lds_slots = (kTileLdsBytes - 16) / slot_bytes;
+    lds_slots = env_u32("HSDL_CLEAN_LDS_SLOTS", lds_slots, 1, lds_slots);
+    const size_t lds_bytes = (size_t)lds_slots * slot_bytes + 16;
+    const int tgrid = std::max(1, cus * 2);
+    // tuning knob HSDL_CLEAN_WINDOW: labels of L(v) per wave work unit
+    const uint32_t win = env_u32("HSDL_CLEAN_WINDOW", kTileWindow, 1, kMaxWindow);
+    const uint32_t gcap = tile_cap_for(mx[0]);
+    const uint64_t gwords =
+        small_vals ? tile_words<uint16_t>(gcap, K1) : tile_words<uint32_t>(gcap, K1);
+    if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
+    // the heads' lists are streamed from a hop-ordered 32-bit copy of all
+    // labels, or from the index when fields or memory do not allow it
+    const bool copy =
+        use32 && hop_sort && take_scratch(dev, kCsSrt, srt, idx->total * 4) == HSDL_OK;
+    if (copy) {
+      hipLaunchKernelGGL(k_clean_sort<Pair32>, dim3(grid), dim3(256), 0, st,
+                         Pair32{hop_bits, dist_bits}, 0u, n, (uint32_t)idx->K, off, lab,
+                         srt.as<uint32_t>(), hcnt.as<uint32_t>());
       HSDL_HIP(hipGetLastError());
     } else {
       (void)hipGetLastError();
-      use32 = false;
+      width = 8;
     }
-  }
-  const Stream64 s64{idx->lab.as<unsigned long long>()};
-  const Stream32 s32{lab32.as<uint32_t>(), hop_bits, dist_bits,
-                     use32 && hop_sort ? hcnt.as<uint32_t>() : nullptr, (uint32_t)idx->K};
-  auto launch = [&](auto kern, auto str) {
-    hipLaunchKernelGGL(kern, dim3(tgrid), dim3(kTileThreads), lds_bytes, st, n, (uint32_t)idx->K,
-                       idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(), str,
-                       keep.as<uint8_t>(), new_len.as<uint32_t>(), redo.as<uint32_t>(), cnt,
-                       lds_slots, gtile.as<uint32_t>(), gwords, win, indexed);
-  };
-  const uint64_t t_kern = now_ns();  // buffers and the 32-bit copy's set-up end here
-  if (small_vals) {
-    if (use32) launch(k_clean_tile<uint16_t, Stream32>, s32);
-    else launch(k_clean_tile<uint16_t, Stream64>, s64);
-  } else {
-    if (use32) launch(k_clean_tile<uint32_t, Stream32>, s32);
-    else launch(k_clean_tile<uint32_t, Stream64>, s64);
-  }
-  HSDL_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_clean_seq<false>, dim3(grid), dim3(kCleanWaves * kWave), 0, st,
-                     (uint32_t)idx->K, idx->off.as<unsigned long long>(),
-                     idx->lab.as<unsigned long long>(), keep.as<uint8_t>(),
-                     new_len.as<uint32_t>(), redo.as<uint32_t>(), cnt, cnt + 1, nullptr, 0u);
-  HSDL_HIP(hipGetLastError());
-  DevBuf long_bits;
-  if (mx[0] > kSeqBitsPerWave) {
-    // vertices with more labels than an LDS bit set holds: keep bits in a
-    // global slice per wave (few waves: such vertices are rare)
-    const uint32_t lgrid = 64;
-    const uint32_t words = (mx[0] + 31) / 32;
-    if ((rc = long_bits.alloc((uint64_t)lgrid * kCleanWaves * words * 4))) return rc;
-    hipLaunchKernelGGL(k_clean_seq<true>, dim3(lgrid), dim3(kCleanWaves * kWave), 0, st,
-                       (uint32_t)idx->K, idx->off.as<unsigned long long>(),
-                       idx->lab.as<unsigned long long>(), keep.as<uint8_t>(),
-                       new_len.as<uint32_t>(), redo.as<uint32_t>(), cnt, cnt + 1,
-                       long_bits.as<uint32_t>(), words);
+    auto launch = [&](auto kern, auto str) {
+      hipLaunchKernelGGL(kern, dim3(tgrid), dim3(kTileThreads), lds_bytes, st, n,
+                         (uint32_t)idx->K, off, lab, str, redo.as<uint32_t>(), cnt, lds_slots,
+                         gtile.as<uint32_t>(), gwords, win, indexed);
+    };
+    const Stream32 s32{srt.as<uint32_t>(), hop_bits, dist_bits, hcnt.as<uint32_t>(),
+                       (uint32_t)idx->K};
+    const Stream64 s64{lab};
+    if (small_vals) {
+      if (copy) launch(k_clean_tile<uint16_t, Stream32>, s32);
+      else launch(k_clean_tile<uint16_t, Stream64>, s64);
+    } else {
+      if (copy) launch(k_clean_tile<uint32_t, Stream32>, s32);
+      else launch(k_clean_tile<uint32_t, Stream64>, s64);
+    }
     HSDL_HIP(hipGetLastError());
   }
   uint32_t hc[6] = {0, 0, 0, 0, 0, 0};
   HSDL_HIP(hipMemcpyAsync(hc, ctr.p, 24, hipMemcpyDeviceToHost, st));
   HSDL_HIP(hipStreamSynchronize(st));
   const uint64_t t_passes = now_ns();
-  if (hc[1] & 2u) return fail(HSDL_EINVAL, "a vertex holds more than 32 labels of one hub");
-  if (hc[1]) return fail(HSDL_EDEVICE, "clean: keep-bit scratch smaller than a list");
-  if ((rc = scan_counts_u32(new_len.as<uint32_t>(), noff.as<uint64_t>(), n, st))) return rc;
-  uint64_t total = 0;
-  HSDL_HIP(hipMemcpy(&total, noff.as<uint64_t>() + n, 8, hipMemcpyDeviceToHost));
-  if ((rc = take_scratch(dev, kCsLab, nlab, std::max<uint64_t>(total, 1) * 8))) return rc;
-  DevBuf npar;
-  if (idx->has_parents && (rc = npar.alloc(std::max<uint64_t>(total, 1) * 4))) return rc;
-  hipLaunchKernelGGL(k_compact, dim3(grid), dim3(256), 0, st, n, idx->off.as<unsigned long long>(),
-                     idx->lab.as<unsigned long long>(), keep.as<uint8_t>(),
-                     noff.as<unsigned long long>(), nlab.as<unsigned long long>(),
-                     idx->has_parents ? idx->par.as<uint32_t>() : nullptr,
-                     idx->has_parents ? npar.as<uint32_t>() : nullptr);
-  HSDL_HIP(hipGetLastError());
-  HSDL_HIP(hipStreamSynchronize(st));
-  // the replaced arrays are kept for the next clean's new ones
-  std::swap(idx->off, noff);
-  std::swap(idx->lab, nlab);
-  idx->lab32.release();
-  idx->q32.store(0, std::memory_order_release);
-  give_scratch(dev, kCsOff, noff);
-  give_scratch(dev, kCsLab, nlab);
-  if (idx->has_parents) idx->par = std::move(npar);
-  idx->total = total;
+  // nothing falls: the index stays as it is
+  if (hc[0]) {
+    if ((rc = take_scratch(dev, kCsKeep, keep, std::max<uint64_t>(idx->total, 1))) ||
+        (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull)) ||
+        (rc = take_scratch(dev, kCsOff, noff, (n + 1ull) * 8)))
+      return rc;
+    HSDL_HIP(hipMemsetAsync(keep.p, 1, idx->total, st));
+    hipLaunchKernelGGL(k_clean_keep_all, dim3(grid), dim3(256), 0, st, n, off,
+                       new_len.as<uint32_t>());
+    HSDL_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_clean_seq<false>, dim3(grid), dim3(kCleanWaves * kWave), 0, st,
+                       (uint32_t)idx->K, off, lab, keep.as<uint8_t>(), new_len.as<uint32_t>(),
+                       redo.as<uint32_t>(), cnt, cnt + 3, nullptr, 0u);
+    HSDL_HIP(hipGetLastError());
+    DevBuf long_bits;
+    if (mx[0] > kSeqBitsPerWave) {
+      // vertices with more labels than an LDS bit set holds: keep bits in a
+      // global slice per wave (few waves: such vertices are rare)
+      const uint32_t lgrid = 64;
+      const uint32_t words = (mx[0] + 31) / 32;
+      if ((rc = long_bits.alloc((uint64_t)lgrid * kCleanWaves * words * 4))) return rc;
+      hipLaunchKernelGGL(k_clean_seq<true>, dim3(lgrid), dim3(kCleanWaves * kWave), 0, st,
+                         (uint32_t)idx->K, off, lab, keep.as<uint8_t>(), new_len.as<uint32_t>(),
+                         redo.as<uint32_t>(), cnt, cnt + 3, long_bits.as<uint32_t>(), words);
+      HSDL_HIP(hipGetLastError());
+    }
+    uint32_t bad = 0;
+    HSDL_HIP(hipMemcpyAsync(&bad, cnt + 3, 4, hipMemcpyDeviceToHost, st));
+    HSDL_HIP(hipStreamSynchronize(st));
+    if (bad & 2u) return fail(HSDL_EINVAL, "a vertex holds more than 32 labels of one hub");
+    if (bad) return fail(HSDL_EDEVICE, "clean: keep-bit scratch smaller than a list");
+    if ((rc = scan_counts_u32(new_len.as<uint32_t>(), noff.as<uint64_t>(), n, st))) return rc;
+    uint64_t total = 0;
+    HSDL_HIP(hipMemcpy(&total, noff.as<uint64_t>() + n, 8, hipMemcpyDeviceToHost));
+    if ((rc = take_scratch(dev, kCsLab, nlab, std::max<uint64_t>(total, 1) * 8))) return rc;
+    DevBuf npar;
+    if (idx->has_parents && (rc = npar.alloc(std::max<uint64_t>(total, 1) * 4))) return rc;
+    hipLaunchKernelGGL(k_compact, dim3(grid), dim3(256), 0, st, n, off, lab, keep.as<uint8_t>(),
+                       noff.as<unsigned long long>(), nlab.as<unsigned long long>(),
+                       idx->has_parents ? idx->par.as<uint32_t>() : nullptr,
+                       idx->has_parents ? npar.as<uint32_t>() : nullptr);
+    HSDL_HIP(hipGetLastError());
+    HSDL_HIP(hipStreamSynchronize(st));
+    // the replaced arrays are kept for the next clean's new ones
+    std::swap(idx->off, noff);
+    std::swap(idx->lab, nlab);
+    idx->lab32.release();
+    idx->q32.store(0, std::memory_order_release);
+    give_scratch(dev, kCsOff, noff);
+    give_scratch(dev, kCsLab, nlab);
+    if (idx->has_parents) idx->par = std::move(npar);
+    idx->total = total;
+  }
   idx->cleaned = true;
-  idx->stats.labels_cleaned = total;
+  idx->stats.labels_cleaned = idx->total;
   idx->stats.clean_passes = hc[0] ? 2 : 1;
   idx->stats.clean_seq_vertices = hc[0];
   idx->stats.clean_label_reads = (uint64_t)hc[4] | ((uint64_t)hc[5] << 32);
-  idx->stats.clean_label_bytes = use32 ? 4 : 8;
+  idx->stats.clean_label_bytes = (uint32_t)width;
   const uint64_t t_end = now_ns();
   idx->stats.t_clean_s = (t_end - t0) * 1e-9;
   if (getenv("HSDL_VERBOSE"))
-    fprintf(stderr, "[hsdl] clean: %.3f s set-up, %.3f s passes, %.3f s compaction\n",
+    fprintf(stderr, "[hsdl] clean: %.3f s set-up, %.3f s pass 1, %.3f s pass 2 and compaction\n",
             (t_kern - t0) * 1e-9, (t_passes - t_kern) * 1e-9, (t_end - t_passes) * 1e-9);
   return HSDL_OK;
 }

@@ -193,8 +193,8 @@ int hsdl_graph_groups(const hsdl_graph *g, uint32_t method, uint32_t max_size, u
 int hsdl_clean(hsdl_index *idx);
 
 /* Frees the working buffers hsdl_clean keeps on a device (-1: every device)
- * for the next clean: its flags, counts, 32-bit label copy and tile arena,
- * and the index arrays a clean replaced; and the staging buffers (pinned and
+ * for the next clean: its flags, counts, hop-ordered label copy and tile
+ * arena, and the index arrays a clean replaced; and the staging buffers (pinned and
  * device memory, at most 4 x 16 MB) that hsdl_query and hsdl_extract_paths
  * keep for the next call.  No counterpart in the reference
  * (memory management of this library); the graph's build buffers go with
@@ -219,16 +219,18 @@ typedef struct hsdl_stats {
   uint64_t prune_label_reads;       /* labels of L(y) streamed by the prune */
   uint64_t prune_tile_reads;        /* labels of L(s) staged into tiles     */
   uint64_t clean_seq_vertices;      /* vertices the clean walked in order   */
-  uint64_t clean_label_reads;       /* labels of the heads' lists L(u) read
-                                       by the clean's first pass            */
+  uint64_t clean_label_reads;       /* labels read by the clean's first pass:
+                                       of the heads' lists L(u), or of L(v)
+                                       walked (64 pairs each) where it tests
+                                       L(v)'s pairs (short lists)           */
   double t_parents_s;               /* parent derivation (opts.parents),
                                        included in t_generate_s            */
   uint32_t prune_label_bytes;       /* bytes per label of L(y) the prune
                                        streamed: 4 when hub, hop and dist
                                        fit one word (a 32-bit copy of the
                                        label pool), else 8                  */
-  uint32_t clean_label_bytes;       /* same for the heads' lists the clean's
-                                       first pass streamed (0: no clean)   */
+  uint32_t clean_label_bytes;       /* same for the lists the clean's first
+                                       pass walked (0: no clean)           */
   uint64_t prune_row_slots;         /* dense (hub, vertex) slots the prune's
                                        row items scanned for candidates     */
 } hsdl_stats;

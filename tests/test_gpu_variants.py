@@ -194,3 +194,58 @@ def test_host_calls_in_parts():
             jobs += [pool.submit(paths, 90001, 11 * i) for i in range(6)]
             assert all(j.result() for j in jobs)
         H.release_scratch()
+
+
+@pytest.mark.parametrize("pairs,stream32,piece", [("0", "1", None), ("0", "0", None), ("1", "1", None),
+                                                  ("2", "1", None), ("2", "0", None),
+                                                  ("2", "1", "3000"), ("2", "0", "1")])
+def test_clean_forms(monkeypatch, pairs, stream32, piece):
+    """The clean's first pass over tiles, over label pairs and as the mean list
+    length chooses, from 32-bit and 8-byte lists, whole and in slices down to
+    one list: redundant sets of short and of long lists (past 2,048 labels, a
+    workgroup each), hubs ranked below their vertex, empty lists, K = 1 and
+    15, and sets that lose nothing: the oracle's clean."""
+    monkeypatch.setenv("HSDL_CLEAN_PAIRS", pairs)
+    monkeypatch.setenv("HSDL_STREAM32", stream32)
+    if piece:
+        monkeypatch.setenv("HSDL_CLEAN_SLICE", piece)
+    rng = np.random.default_rng(29)
+
+    def check(name, K, off, hub, hop, dist):
+        print(f"[clean] {name} pairs={pairs} stream32={stream32} slice={piece}", flush=True)
+        off = np.asarray(off, np.uint64)
+        n = len(off) - 1
+        want = O.clean(O.labels_from_arrays(n, off.astype(np.int64), hub, hop, dist))
+        idx = H.Index.from_labels(n, K, off, hub, hop, dist)
+        idx.clean()
+        same_labels(idx, want.arrays())
+        return want.total()
+
+    for n, K, wmax, group in ((900, 4, 50, 32), (500, 15, 3, 64), (300, 2, 30000, 9), (65, 1, 5, 7),
+                              (3500, 3, 1000, 3000)):
+        off, hub, hop, dist = O.kround_grouped(csr_of(ragged(n, n + K, wmax)), K, group).arrays()
+        check(f"groups n={n} K={K}", K, off, hub, hop, dist)
+    # some labels (u, h, d) of v also at u as (v, h, d); every third list empty
+    off, hub, hop, dist = O.kround(csr_of(ragged(1200, 8, 40)), 4).arrays()
+    v = np.repeat(np.arange(1200), np.diff(np.asarray(off).astype(np.int64)))
+    rows = np.stack([v, hub, hop, dist], 1).astype(np.int64)
+    pick = (rng.random(len(v)) < 0.3) & (rows[:, 2] > 0)
+    rows = np.concatenate([rows, rows[pick][:, [1, 0, 2, 3]]])
+    rows = rows[rows[:, 0] % 3 > 0]
+    rows = rows[np.lexsort((rows[:, 2], rows[:, 1], rows[:, 0]))]
+    off = np.concatenate([[0], np.cumsum(np.bincount(rows[:, 0], minlength=1200))])
+    check("hubs below", 4, off, rows[:, 1].astype(np.uint32), rows[:, 2].astype(np.uint8),
+          rows[:, 3].astype(np.int32))
+    # lists of 2,047, 2,048, 2,049 and 4,500 labels over hubs that share ten
+    # first hubs; the last ones' hop-2 labels fall through them now and then
+    W, U = 10, 4600
+    lists = [[(x, 0, 0)] for x in range(W)]
+    lists += [[(w, 1, int(rng.integers(1, 50))) for w in range(W)] + [(u, 0, 0)]
+              for u in range(W, W + U)]
+    for i, (size, top) in enumerate(((2047, 3), (2048, 120), (2049, 3), (4500, 3), (4500, 120))):
+        a = [(w, 1, int(rng.integers(top, 50 + top))) for w in range(W)]
+        a += [(u, 2, int(rng.integers(1, top))) for u in range(W, size - 1)]
+        lists.append(a + [(W + U + i, 0, 0)])
+    off = np.concatenate([[0], np.cumsum([len(x) for x in lists])])
+    hub, hop, dist = np.array([e for x in lists for e in x]).T
+    check("long", 3, off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32))
