@@ -111,6 +111,7 @@ struct Ctrl {
   uint32_t heavy_ctr;   // next heavy piece (k_expand_heavy)
   uint32_t row_mode;    // this round's prune takes row items (k_prune_rows)
   uint32_t row_ctr[8];  // next row item of each XCD's queue
+  uint32_t wave_items;  // hub slots the list prune takes a wave each
   // the running batch attempt (k_set_batch): the kernels take these instead
   // of their arguments' s0 / B / tag, so one captured batch replays for any
   uint32_t bs0, bB, btag;
@@ -141,6 +142,9 @@ struct GenArgs {
   uint32_t row_run;      // y-blocks per row item (one tile build per item)
   uint32_t row_block;    // vertices per y-block (a multiple of 1024)
   uint32_t claim_max;    // candidates a prune wave claims at once, at most
+  uint32_t wave_min;     // least hub slots for wave items (kInf32: none)
+  uint32_t wave_cands;   // most candidates of a wave item
+  uint32_t wave_slots;   // its tile's slots (a power of two)
   uint32_t idx_tiles;    // LDS tiles of more labels than this are indexed (kInf32: none)
   uint32_t direct_tiles; // LDS tiles addressed by hub id, where they fit
   uint32_t group_min;    // least frontier groups per chunk of the light expansion
@@ -188,6 +192,7 @@ struct GenArgs {
   uint32_t *hub_off;
   uint32_t *hub_cur;
   uint32_t *chunk_off;
+  uint32_t *wave_hubs;  // hub slots of the round's wave items
   Item *F0;
   Item *F1;
   uint32_t *frank;  // per item of the next frontier: its rank among its vertex's new labels
@@ -370,10 +375,15 @@ __global__ void k_batch_begin(GenArgs a) {
   }
 }
 
+// hub_ccnt: a hub slot's candidates of the round, with this bit where the hub's
+// tile of the round fits a prune wave's slice of LDS
+constexpr uint32_t kSmallTile = 1u << 31;
+
 __global__ void k_round_prep(GenArgs a) {
   with_batch(a);
   for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < a.B; b += gridDim.x * blockDim.x) {
-    a.hub_ccnt[b] = 0;
+    a.hub_ccnt[b] = a.B >= a.wave_min && tile_view(a, hub_of(a, b)).len <= a.wave_slots / 2
+                        ? kSmallTile : 0u;
     a.hub_cur[b] = 0;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -916,47 +926,91 @@ __global__ void __launch_bounds__(kGroupThreads) k_count(GenArgs a) {
 }
 
 // One workgroup: hub_off = exclusive scan of hub_ccnt; chunk_off[b] =
-// sum_{b'<b} ceil(hub_ccnt[b'] / tile).  An overflowed batch gets no work.
-// Each wave scans a contiguous range 64 entries per step (coalesced loads,
-// a wave scan per step, the carry in a register) after the waves' totals
-// give it its start.
+// sum_{b'<b} ceil(hub_ccnt[b'] / tile), over the hubs that are not wave items;
+// wave_hubs: those that are.  An overflowed batch gets no work.  Each wave
+// scans a contiguous range 64 entries per step (coalesced loads, a wave scan
+// per step, the carry in a register) after the waves' totals give it its
+// start.  The loads of kScanSteps steps are issued together, and kept for the
+// second pass where they are all of the batch: the round trips are what it costs.
+constexpr uint32_t kScanSteps = 16;
 __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
   with_batch(a);
-  __shared__ uint32_t wsum[1024 / kWave], wcsum[1024 / kWave];
+  __shared__ uint32_t wsum[1024 / kWave], wcsum[1024 / kWave], wbig[1024 / kWave],
+      wsmall[1024 / kWave];
   const uint32_t t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
   const uint32_t nw = blockDim.x / kWave;
   const uint32_t B = a.B, tile = a.tile;
   const uint32_t per_w = ((B + nw - 1) / nw + kWave - 1) & ~(kWave - 1);
   const uint32_t lo = min(B, w * per_w), hi = min(B, lo + per_w);
-  uint32_t s = 0, cs = 0;
-  for (uint32_t b = lo + lane; b < hi; b += kWave) {
-    const uint32_t c = a.hub_ccnt[b];
-    s += (c + tile - 1) / tile;
-    cs += c;
+  uint32_t v[kScanSteps];
+  auto load = [&](uint32_t b0) {
+#pragma unroll
+    for (uint32_t r = 0; r < kScanSteps; ++r) {
+      const uint32_t b = b0 + r * kWave + lane;
+      v[r] = b < hi ? a.hub_ccnt[b] : 0u;
+    }
+  };
+  // hub slot's candidates, and whether it may be a wave item
+  auto count = [](uint32_t x) { return x & ~kSmallTile; };
+  auto is_small = [&](uint32_t x) {
+    return x > kSmallTile && x - kSmallTile <= a.wave_cands;
+  };
+  // work items of c candidates (the division only where a hub of the step has
+  // more than one)
+  auto chunks = [&](uint32_t c) {
+    return __ballot(c > tile) ? (c + tile - 1) / tile : (c ? 1u : 0u);
+  };
+  uint32_t s = 0, cs = 0, big = 0, small = 0;
+  for (uint32_t b0 = lo; b0 < hi; b0 += kScanSteps * kWave) {
+    load(b0);
+#pragma unroll
+    for (uint32_t r = 0; r < kScanSteps; ++r) {
+      const uint32_t k = chunks(count(v[r]));
+      s += k;
+      big += is_small(v[r]) ? 0u : k;
+      small += is_small(v[r]) ? 1u : 0u;
+      cs += count(v[r]);
+    }
   }
   s = wave_sum_u32(s);
   cs = wave_sum_u32(cs);
+  big = wave_sum_u32(big);
+  small = wave_sum_u32(small);
   if (lane == 0) {
     wsum[w] = s;
     wcsum[w] = cs;
+    wbig[w] = big;
+    wsmall[w] = small;
   }
   __syncthreads();
-  uint32_t run = 0, runc = 0;
+  uint32_t nsmall = 0;
+  for (uint32_t x = 0; x < nw; ++x) nsmall += wsmall[x];
+  const bool waves = nsmall >= a.wave_min;
+  uint32_t run = 0, runc = 0, runs = 0;
   for (uint32_t x = 0; x < w; ++x) {
-    run += wsum[x];
+    run += waves ? wbig[x] : wsum[x];
     runc += wcsum[x];
+    runs += wsmall[x];
   }
-  for (uint32_t b0 = lo; b0 < hi; b0 += kWave) {
-    const uint32_t b = b0 + lane;
-    const uint32_t c = b < hi ? a.hub_ccnt[b] : 0u;
-    const uint32_t k = (c + tile - 1) / tile;
-    const uint32_t ik = wave_incl_scan_u32(k), ic = wave_incl_scan_u32(c);
-    if (b < hi) {
-      a.chunk_off[b] = run + ik - k;
-      a.hub_off[b] = runc + ic - c;
+  for (uint32_t b0 = lo; b0 < hi; b0 += kScanSteps * kWave) {
+    if (hi - lo > kScanSteps * kWave) load(b0);
+#pragma unroll
+    for (uint32_t r = 0; r < kScanSteps; ++r) {
+      if (b0 + r * kWave >= hi) break;
+      const uint32_t b = b0 + r * kWave + lane, c = count(v[r]);
+      const bool sm = waves && is_small(v[r]);
+      const uint32_t all = chunks(c), k = sm ? 0u : all;
+      const uint32_t ik = wave_incl_scan_u32(k), ic = wave_incl_scan_u32(c);
+      if (b < hi) {
+        a.chunk_off[b] = run + ik - k;
+        a.hub_off[b] = runc + ic - c;
+      }
+      const unsigned long long m = __ballot(sm);
+      if (sm) a.wave_hubs[runs + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = b;
+      runs += (uint32_t)__popcll(m);
+      run += (uint32_t)__shfl((int)ik, kWave - 1, kWave);
+      runc += (uint32_t)__shfl((int)ic, kWave - 1, kWave);
     }
-    run += (uint32_t)__shfl((int)ik, kWave - 1, kWave);
-    runc += (uint32_t)__shfl((int)ic, kWave - 1, kWave);
   }
   if (t < 8) a.ctrl->row_ctr[t] = 0;
   if (t == blockDim.x - 1) {
@@ -968,6 +1022,7 @@ __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
     a.hub_off[B] = runc;
     a.ctrl->row_mode = rows ? 1u : 0u;
     a.ctrl->total_chunks = (dead || rows) ? 0u : run;
+    a.ctrl->wave_items = (dead || rows || !waves) ? 0u : nsmall;
     a.ctrl->work_ctr = 0;
     a.ctrl->cand_total += a.ctrl->cand_round;
     a.ctrl->item_total += min(a.ctrl->fcnt[a.cur], a.fcap);
@@ -1085,6 +1140,19 @@ template <class V> __device__ inline uint32_t hop_off(const GenArgs &, unsigned 
   return label_hop(l) << vs;
 }
 
+// (hub, hop hb, distance db) into a record tile
+template <class V>
+__device__ inline void tile_insert(const GenArgs &a, uint32_t *rec, uint32_t cap, uint32_t stride,
+                                   uint32_t hub, uint32_t hb, uint32_t db) {
+  uint32_t slot = hash_slot(hub, cap);
+  for (;;) {
+    const uint32_t prev = atomicCAS(&rec[slot * stride], kInf32, hub);
+    if (prev == kInf32 || prev == hub) break;
+    slot = (slot + 1) & (cap - 1);
+  }
+  V *vals = reinterpret_cast<V *>(rec + slot * stride + 1);
+  for (uint32_t ha = 0; ha + hb <= a.h; ++ha) atomic_min_v(&vals[ha], db);
+}
 template <class V>
 __device__ void build_tile(const GenArgs &a, uint32_t s, const ListView &view, uint32_t *rec,
                            uint32_t cap) {
@@ -1109,14 +1177,7 @@ __device__ void build_tile(const GenArgs &a, uint32_t s, const ListView &view, u
   for (uint32_t i = threadIdx.x; i < view.len; i += blockDim.x) {
     uint32_t hub, hb, db;
     pool_label(a, st + view.at(i), hub, hb, db);
-    uint32_t slot = hash_slot(hub, cap);
-    for (;;) {
-      const uint32_t prev = atomicCAS(&rec[slot * stride], kInf32, hub);
-      if (prev == kInf32 || prev == hub) break;
-      slot = (slot + 1) & (cap - 1);
-    }
-    V *vals = reinterpret_cast<V *>(rec + slot * stride + 1);
-    for (uint32_t ha = 0; ha + hb <= a.h; ++ha) atomic_min_v(&vals[ha], db);
+    tile_insert<V>(a, rec, cap, stride, hub, hb, db);
   }
   __syncthreads();
 }
@@ -1633,21 +1694,157 @@ __device__ __attribute__((always_inline)) inline void tile_prune(
     run((glb_ptr<const uint32_t>)gkeys);
 }
 
+// Wave items: hub slots with few candidates and a short list L(s), a wave each,
+// the tile in the wave's slice of the workgroup's LDS.  Such an item is a chain of
+// round trips (the hub's extents, its list and the candidates' vertices, their
+// slots and list extents, their lists) with a step or two of work at its end, so
+// what counts is how many run at once: 8,192 waves instead of 512 workgroups,
+// whose sixteen waves shared some eight candidates.  A batch of the 1024 x 1024
+// grid at K = 8 (10,240 hubs, 84,000 candidates per round): 43 us per round
+// instead of 135, the build 272 -> 170 ms.  At most 16 candidates per wave item
+// 180 ms, 32 or 64 170 ms.  Rounds with few such hubs keep a workgroup per item:
+// its waves take a hub's candidates at the same time (from 256, 1,024 or 4,096
+// hubs on measures the same: batches grow past that line in one step).
+template <class V, class LT>
+__device__ __attribute__((always_inline)) inline void prune_wave_items(
+    const GenArgs &a, Item *Fn, uint32_t items, uint32_t *lds, Item *sh_acc, uint32_t *sh_acc_n,
+    unsigned long long &wave_reads, unsigned long long &wave_tile) {
+  constexpr uint32_t kAhead = 4;  // candidates whose lists' first steps are in flight
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t K1 = a.K + 1;
+  const uint32_t stride = rec_words<V>(K1), sh = rec_shift<V>(K1);
+  uint32_t *rec = lds + wib * (a.wave_slots << sh);
+  const LT *pool = stream_pool<LT>(a);
+  // consecutive items (whose cost falls slowly along the batch) go to
+  // different workgroups
+  for (uint32_t i = blockIdx.x + wib * gridDim.x; i < items;
+       i += gridDim.x * (kPruneThreads / kWave)) {
+    const uint32_t b = __builtin_amdgcn_readfirstlane(a.wave_hubs[i]);
+    const uint32_t s = __builtin_amdgcn_readfirstlane(hub_of(a, b));
+    const uint32_t *run = a.cgroup + a.hub_off[b];
+    const uint32_t n = __builtin_amdgcn_readfirstlane(a.hub_ccnt[b] & ~kSmallTile);
+    uint32_t y = 0, dy = 0;
+    if (lane < n) y = run[lane];
+    const ListView sv = tile_view(a, s);
+    const LT *Ls = pool + a.seg_start[s];
+    ListView vw{0, 0, 0, 0};
+    unsigned long long st = 0;
+    if (lane < n) {
+      dy = slot_dist(a, a.cand_d[slot_at(a, b, y)]);
+      st = a.seg_start[y];
+      const uint32_t len = a.seg_len[y];
+      uint32_t sorted = 0, pre = 1;
+      if (a.hcnt && a.h > 1) {
+        sorted = a.sorted_len[y];
+        pre = hop_prefix(a, y, a.h - 1);
+      }
+      vw = cand_view(a, len, sorted, pre);
+    }
+    const uint32_t svn = __builtin_amdgcn_readfirstlane(sv.len);
+    LT t0 = 0;
+    if (svn) t0 = Ls[sv.at(min(lane, svn - 1))];
+    auto rl = [](uint32_t v, uint32_t j) { return (uint32_t)__builtin_amdgcn_readlane(v, j); };
+    auto list_of = [&](uint32_t j) {
+      return pool + (((unsigned long long)rl((uint32_t)(st >> 32), j) << 32) | rl((uint32_t)st, j));
+    };
+    auto view_of = [&](uint32_t j) {
+      return ListView{rl(vw.a0, j), rl(vw.na, j), rl(vw.b0, j), rl(vw.len, j)};
+    };
+    LT f[kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j)
+      f[j] = first_step(list_of(min(j, n - 1)), view_of(min(j, n - 1)));
+    // the tile, at a load factor of 1/8 to 1/2
+    const uint32_t cap = min(a.wave_slots, pow2_at_least(4ull * svn + 4));
+    uint4 *fill = reinterpret_cast<uint4 *>(rec);
+    const uint4 ones = make_uint4(kInf32, kInf32, kInf32, kInf32);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t j = lane; j < (cap << sh) / 4; j += kWave) fill[j] = ones;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t j = lane; j < svn; j += kWave) {
+      if (j >= kWave) t0 = Ls[sv.at(j)];
+      uint32_t hub, hb, db;
+      unpack(a, t0, hub, hb, db);
+      tile_insert<V>(a, rec, cap, stride, hub, hb, db);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    wave_tile += svn;
+    unsigned long long kept = 0;
+    for (uint32_t j0 = 0; j0 < n; j0 += kAhead) {
+#pragma unroll
+      for (uint32_t j = 0; j < kAhead; ++j) {
+        const uint32_t c = j0 + j;
+        if (c >= n) break;
+        uint32_t reads = 0;
+        const bool pruned =
+            witness_search<V>(a, list_of(c), view_of(c), f[j], rl(dy, c),
+                              (lds_ptr<const uint32_t>)rec, cap, sh, reads);
+        const uint32_t nx = min(c + kAhead, n - 1);
+        f[j] = first_step(list_of(nx), view_of(nx));
+        wave_reads += reads;
+        if (!pruned) kept |= 1ull << c;
+      }
+    }
+    const uint32_t nk = (uint32_t)__popcll(kept);
+    if (!nk) continue;
+    // accepted labels: staged for the workgroup while its slots last, else
+    // published by the wave
+    const bool mine = (kept >> lane) & 1ull;
+    const uint32_t rank = (uint32_t)__popcll(kept & lt_mask);
+    uint32_t at = kInf32;
+    if (lane == 0) {
+      uint32_t seen = *sh_acc_n;
+      while (seen + nk <= kAccSlots) {
+        const uint32_t got = atomicCAS(sh_acc_n, seen, seen + nk);
+        if (got == seen) {
+          at = seen;
+          break;
+        }
+        seen = got;
+      }
+    }
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (at != kInf32) {
+      if (mine) sh_acc[at + rank] = Item{b, y, dy};
+      continue;
+    }
+    uint32_t r = 1;
+    if (mine) r = atomicAdd(&a.add_cnt[y], 1u);
+    const unsigned long long tm = __ballot(mine && r == 0);
+    uint32_t fb = 0, tb = 0;
+    if (lane == 0) {
+      fb = atomicAdd(&a.ctrl->fcnt[a.cur ^ 1], nk);
+      if (fb + nk > a.fcap) atomicOr(&a.ctrl->overflow, kOvfFront);
+      if (tm) tb = atomicAdd(&a.ctrl->touched_cnt, (uint32_t)__popcll(tm));
+    }
+    fb = __builtin_amdgcn_readfirstlane(fb);
+    tb = __builtin_amdgcn_readfirstlane(tb);
+    if (mine && fb + rank < a.fcap) {
+      Fn[fb + rank] = Item{b, y, dy};
+      a.frank[fb + rank] = r;
+    }
+    if (mine && r == 0) a.touched[tb + (uint32_t)__popcll(tm & lt_mask)] = y;
+  }
+}
+
 // LT: label type of the stream (uint32_t: the pool's 32-bit copy).
 template <class V, class LT>
 __global__ void __launch_bounds__(kPruneThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_prune(GenArgs a) {
   with_batch(a);
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ uint32_t sh_w, sh_acc_n, sh_acc_base, sh_next, sh_touch_n, sh_touch_base;
   __shared__ uint32_t sh_item, sh_item_end, sh_rows;
   __shared__ Item sh_acc[kAccSlots];
   __shared__ uint32_t sh_rank[kAccSlots];
   __shared__ uint32_t sh_touch[kAccSlots];
+  __shared__ unsigned long long sh_reads[2];
   const int lane = lane_id();
   Item *Fn = frontier(a, a.cur ^ 1);
   uint32_t tile_b = kInf32;  // hub slot whose tile is in LDS
-  unsigned long long wave_reads = 0, tile_reads = 0;
+  unsigned long long wave_reads = 0, wave_tile = 0;
   const uint64_t gwords = a.gtile_cap / gridDim.x;
   uint32_t *gkeys = a.gtile + (uint64_t)blockIdx.x * gwords;
   const uint32_t total = a.ctrl->total_chunks;
@@ -1659,13 +1856,20 @@ k_prune(GenArgs a) {
   const uint64_t cands = a.hub_off[a.B];
   const uint32_t claim =
       cands ? (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, (64ull * total) / cands)) : 1u;
+  const uint32_t items = a.ctrl->wave_items;
+  if (blockIdx.x >= items && (uint64_t)blockIdx.x * claim >= total) return;
   if (threadIdx.x == 0) {
+    sh_reads[0] = sh_reads[1] = 0;
     sh_item = blockIdx.x * claim;
     sh_item_end = sh_item + claim;
     sh_acc_n = 0;
     sh_touch_n = 0;
   }
   __syncthreads();
+  if (items) {
+    prune_wave_items<V, LT>(a, Fn, items, lds, sh_acc, &sh_acc_n, wave_reads, wave_tile);
+    __syncthreads();
+  }
   for (;;) {
     if (threadIdx.x == 0) {
       if (sh_item == sh_item_end) {
@@ -1694,7 +1898,7 @@ k_prune(GenArgs a) {
     const uint32_t b = lo;
     const uint32_t s = hub_of(a, b);
     const uint32_t c_beg = (w - a.chunk_off[b]) * a.tile;
-    const uint32_t c_end = min(a.hub_ccnt[b], c_beg + a.tile);
+    const uint32_t c_end = min(a.hub_ccnt[b] & ~kSmallTile, c_beg + a.tile);
     // the staged labels of earlier items are published once this item's
     // could overflow the staging slots (c_end - c_beg <= tile <= kAccSlots)
     if (sh_acc_n + (c_end - c_beg) > kAccSlots)
@@ -1716,7 +1920,7 @@ k_prune(GenArgs a) {
     if (tile_b != b) {
       tile_build<V>(a, s, sv, plan, lds, gkeys, sh_rows);
       tile_b = plan.kind == kTileArena ? kInf32 : b;
-      tile_reads += sv.len;
+      if (threadIdx.x == 0) wave_tile += sv.len;
     }
     auto accept = [&](uint32_t, uint32_t y, uint32_t d) {
       sh_acc[atomicAdd(&sh_acc_n, 1u)] = Item{b, y, d};
@@ -1725,8 +1929,13 @@ k_prune(GenArgs a) {
     __syncthreads();
   }
   publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
-  if (lane == 0 && wave_reads) atomicAdd(&a.ctrl->label_reads, wave_reads);
-  if (threadIdx.x == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
+  if (lane == 0) {
+    if (wave_reads) atomicAdd(&sh_reads[0], wave_reads);
+    if (wave_tile) atomicAdd(&sh_reads[1], wave_tile);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2 && sh_reads[threadIdx.x])
+    atomicAdd(threadIdx.x ? &a.ctrl->tile_reads : &a.ctrl->label_reads, sh_reads[threadIdx.x]);
 }
 
 // --------------------------------------------------------- prune, by rows
@@ -2813,7 +3022,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
       (rc = g.take(kScTouched, n * 4ull)) || (rc = g.take(kScFgrp, n * 16ull)) ||
       (group && (rc = g.take(kScHubSlot, n * 4ull))) ||
       (rc = g.take(kScHubCcnt, (Bmax + 1ull) * 4)) || (rc = g.take(kScHubOff, (Bmax + 1ull) * 4)) ||
-      (rc = g.take(kScHubCur, (Bmax + 1ull) * 4)) || (rc = g.take(kScChunkOff, (Bmax + 1ull) * 4)) ||
+      (rc = g.take(kScHubCur, (Bmax + 1ull) * 4)) || (rc = g.take(kScChunkOff, (2ull * Bmax + 1) * 4)) ||
       (rc = g.take(kScGtile, gtile0 * 4)) || (rc = g.take(kScCtrl, sizeof(Ctrl))) ||
       (rc = g.take(kScHeavy, (uint64_t)heavy_cap * sizeof(HeavyItem))) ||
       (use32 && !g.pool32.p && (rc = g.pool32.alloc(pool0 * 4))))
@@ -2894,6 +3103,13 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   }
   a.piece_pairs = env_u32("HSDL_PIECE_PAIRS", 16384, 1, 1u << 16);
   a.lds_slots = lds_slots;
+  // wave items (tuning knobs HSDL_WAVE_ITEMS, the least hub slots of a round
+  // that take them, 0 for never; HSDL_WAVE_CANDS, the most candidates of one)
+  a.wave_slots = lds_slots / (kPruneThreads / kWave);
+  a.wave_slots = a.wave_slots ? pow2_at_most(a.wave_slots) : 0u;
+  a.wave_cands = env_u32("HSDL_WAVE_CANDS", 32, 1, kWave);
+  a.wave_min = env_u32("HSDL_WAVE_ITEMS", 1024, 0, kInf32 - 1);
+  if (!a.wave_min || a.wave_slots < 4 || plain) a.wave_min = kInf32;
   DevBuf hubs_buf, in_group;
   if (group) {
     std::vector<uint8_t> mark(n, 0);
@@ -2937,6 +3153,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   a.hub_off = g.hub_off.as<uint32_t>();
   a.hub_cur = g.hub_cur.as<uint32_t>();
   a.chunk_off = g.chunk_off.as<uint32_t>();
+  a.wave_hubs = a.chunk_off + Bmax + 1;
   a.gtile = g.gtile.as<uint32_t>();
   a.gtile_cap = gtile0;
   a.ctrl = g.ctrl.as<Ctrl>();

@@ -91,6 +91,50 @@ def test_expansion_shapes(monkeypatch, heavy, piece):
     same_labels(H.hop_constrained_two_hop_labels_generation(g, 6), O.kround(csr_of(g), 6).arrays())
 
 
+@pytest.mark.parametrize("items,cands", [("1", "64"), ("1", "3"), ("300", "64"), ("0", "32")])
+@pytest.mark.parametrize("stream32", ["1", "0"])
+def test_prune_wave_items(monkeypatch, items, cands, stream32):
+    """Hubs with few candidates and a short list take a wave each (from the
+    first such hub, from the 300th, never), beside hubs that do not; batches
+    whose workgroups accept more labels than their staging holds, 16- and
+    32-bit tile values, tiles of few slots, lists read whole, and a group's
+    hubs: the oracle's labels."""
+    monkeypatch.setenv("HSDL_WAVE_ITEMS", items)
+    monkeypatch.setenv("HSDL_WAVE_CANDS", cands)
+    monkeypatch.setenv("HSDL_STREAM32", stream32)
+    monkeypatch.setenv("HSDL_PRUNE_ROWS", "0")
+    monkeypatch.setenv("HSDL_LANDMARKS", "0")
+
+    def check(g, K, **kw):
+        c = csr_of(g)
+        print(f"[wave items] n={c.n} K={K} {kw} items={items} cands={cands} s32={stream32}",
+              flush=True)
+        same_labels(H.hop_constrained_two_hop_labels_generation(g, K, **kw),
+                    O.kround(c, K).arrays())
+
+    for n, K, wmax, ef in ((2500, 4, 100, 8), (2500, 3, 30000, 4), (700, 7, 3, 4), (300, 15, 20, 2)):
+        g = ragged(n, n + K, wmax, ef)
+        check(g, K)
+        check(g, K, hub_batch=n)
+        check(g, K, hub_batch=n, lds_tile_slots=64)
+    g = H.Graph.grid(61, 67, 3, 1, 300)
+    check(g, 8, hub_batch=2000)
+    check(H.Graph.grid(31, 67, 3, 1, 300), 15, hub_batch=2000)
+    monkeypatch.setenv("HSDL_HOP_ZONES", "0")
+    check(g, 5, hub_batch=2000)
+    monkeypatch.delenv("HSDL_HOP_ZONES")
+    n, K = 2400, 4
+    g = ragged(n, 5, 50)
+    hubs = np.arange(1, n, 3, dtype=np.uint32)
+    gid = np.ones(n, np.uint32)
+    gid[hubs] = 0
+    got = H.hop_constrained_two_hop_labels_generation(g, K, hubs=hubs, hub_batch=800)
+    ref = O.kround_gid(csr_of(g), K, gid).arrays()
+    keep = np.isin(ref[1], hubs)
+    for x, y in zip(got.labels()[1:], ref[1:]):
+        assert np.array_equal(x, np.asarray(y)[keep])
+
+
 @pytest.mark.parametrize("q32,slots", [("1", "1024"), ("1", "64"), ("0", "1024")])
 def test_query_forms(monkeypatch, q32, slots):
     """Queries from the hop-ordered 32-bit copy (parts that fit the table, and
