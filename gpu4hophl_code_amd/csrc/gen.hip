@@ -106,7 +106,6 @@ struct Ctrl {
   uint32_t maxlen;
   uint32_t expand_ctr;  // next chunk of 64 frontier groups (k_expand)
   uint32_t gcnt;        // frontier groups of the running round
-  uint32_t cand_round;  // candidates the running round's expansion opened
   uint32_t heavy_cnt;   // pieces pushed to the heavy list this round
   uint32_t heavy_ctr;   // next heavy piece (k_expand_heavy)
   uint32_t row_mode;    // this round's prune takes row items (k_prune_rows)
@@ -118,6 +117,12 @@ struct Ctrl {
   uint32_t lm_on;                // the landmark test runs in this batch
   unsigned long long lm_tested;  // (label, edge) pairs the landmark test looked at
   unsigned long long lm_caught;  // of these, rejected
+  // what the running round's expansion adds up, a line per XCD (k_chunk_scan
+  // takes it into the totals above and clears it)
+  struct alignas(128) Tally {
+    unsigned long long edges, caught;
+    uint32_t cands;
+  } tally[8];
 };
 
 // A piece of a large frontier group: its cnt labels (at pool offset off)
@@ -148,6 +153,7 @@ struct GenArgs {
   uint32_t idx_tiles;    // LDS tiles of more labels than this are indexed (kInf32: none)
   uint32_t direct_tiles; // LDS tiles addressed by hub id, where they fit
   uint32_t group_min;    // least frontier groups per chunk of the light expansion
+  uint32_t expand_waves; // waves of the light expansion
   uint32_t heavy_pairs;  // frontier groups with more pairs go to heavy pieces
   uint32_t piece_pairs;  // pairs per heavy piece (whole edges)
   uint32_t lds_slots;  // LDS tile capacity (slots)
@@ -375,6 +381,24 @@ __global__ void k_batch_begin(GenArgs a) {
   }
 }
 
+// Frontier groups per chunk of the light expansion: 64 once that leaves every
+// wave a chunk; smaller rounds spread over the waves, since a chunk's steps are a
+// chain of memory round trips (64 groups of up to heavy_pairs pairs took a wave
+// 60 us, which was the whole round on graphs of a few thousand vertices and on
+// grids) -- but no chunk below about 64 edges, or the waves' claims on the flat
+// list cost more than the chains (builds at 1,024 / 4,096 vertices and the
+// 1024 x 1024 grid: one group and up 2.55 / 5.1 / 426 ms, 32 edges 2.57 / 4.84 /
+// 367, 64 2.60 / 4.79 / 343, 128 2.77 / 5.0 / 344, 256 2.83 / 5.4 / 363, always
+// 64 groups 2.93 / 6.15 / 363)
+__device__ inline uint32_t light_groups(const GenArgs &a, uint32_t gcnt) {
+  return min((uint32_t)kWave, max(a.group_min, (gcnt + a.expand_waves - 1) / a.expand_waves));
+}
+__device__ inline uint32_t light_chunks(const GenArgs &a, uint32_t gcnt) {
+  const uint32_t gw = light_groups(a, gcnt);
+  return (gcnt + gw - 1) / gw;
+}
+constexpr uint32_t kFirstBlock = 64;  // flat-list entries each wave of a chunk starts with
+
 // hub_ccnt: a hub slot's candidates of the round, with this bit where the hub's
 // tile of the round fits a prune wave's slice of LDS
 constexpr uint32_t kSmallTile = 1u << 31;
@@ -388,13 +412,12 @@ __global__ void k_round_prep(GenArgs a) {
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.ctrl->fcnt[a.cur ^ 1] = 0;
-    a.ctrl->ccnt = 0;
+    a.ctrl->ccnt = min(a.expand_waves, (light_chunks(a, a.ctrl->gcnt) + 3u) & ~3u) * kFirstBlock;
     a.ctrl->touched_cnt = 0;
     a.ctrl->work_ctr = 0;
     a.ctrl->expand_ctr = 0;
     a.ctrl->heavy_cnt = 0;
     a.ctrl->heavy_ctr = 0;
-    a.ctrl->cand_round = 0;
   }
 }
 
@@ -493,35 +516,48 @@ __global__ void __launch_bounds__(256) k_lm_build(GenArgs a, uint32_t *lm, uint3
 
 // Flat-list space is reserved per wave in blocks of kListBlock entries (one
 // atomic on the list counter per block instead of one per step); unused
-// tails are filled with empty entries that the counting and grouping skip.
+// tails are filled with empty entries that the counting and grouping skip.  A
+// wave's first block in the light expansion is shorter and needs no atomic: in
+// the rounds of a 1024 x 1024 grid a wave opens some twenty candidates, and
+// 4,096 first blocks of 512 were 96 % padding.
 constexpr uint32_t kListBlock = 512;
 constexpr unsigned long long kEmptyEntry = ~0ull;
 
 struct ListRes {
-  uint32_t base = 0, used = kListBlock;  // starts exhausted
-  uint32_t cands = 0;                    // candidates opened, not yet added to cand_round
-  uint32_t caught = 0;                   // pairs a landmark rejected (per lane)
+  uint32_t base = 0, used = kListBlock, size = kListBlock;  // starts exhausted
+  uint32_t cands = 0;   // candidates opened
+  uint32_t caught = 0;  // pairs a landmark rejected (per lane)
 };
 
-// Writes empty entries over [base+used, base+kListBlock) (whole wave).
+// Writes empty entries over [base+used, base+size) (whole wave).
 __device__ inline void list_pad(const GenArgs &a, const ListRes &r) {
-  for (uint32_t i = r.used + (uint32_t)lane_id(); i < kListBlock; i += kWave)
+  for (uint32_t i = r.used + (uint32_t)lane_id(); i < r.size; i += kWave)
     if (r.base + i < a.ccap) a.cflat[r.base + i] = kEmptyEntry;
 }
 
-// End of a kernel: pad the open block and add the wave's counts (edges: pairs
-// this lane relaxed).
+// End of an expansion kernel (whole workgroup): pads the waves' open blocks and
+// adds their counts (edges: pairs this lane relaxed) to the round's tally, one
+// atomic per workgroup and count on one of eight lines: on one line, an atomic
+// per wave and count, the counts alone took tens of microseconds per round.
 __device__ inline void list_close(const GenArgs &a, const ListRes &r, uint64_t edges) {
+  __shared__ unsigned long long sum[3];
+  if (threadIdx.x < 3) sum[threadIdx.x] = 0;
   list_pad(a, r);
   edges = wave_sum_u64(edges);
   const uint64_t caught = a.lm && a.h > 1 ? wave_sum_u64(r.caught) : 0;
-  if (lane_id() != 0) return;
-  if (r.cands) atomicAdd(&a.ctrl->cand_round, r.cands);
-  if (!edges) return;
-  atomicAdd(&a.ctrl->edge_total, (unsigned long long)edges);
-  if (a.lm && a.h > 1) {
-    atomicAdd(&a.ctrl->lm_tested, (unsigned long long)edges);
-    if (caught) atomicAdd(&a.ctrl->lm_caught, (unsigned long long)caught);
+  __syncthreads();
+  if (lane_id() == 0 && edges) {
+    atomicAdd(&sum[0], (unsigned long long)edges);
+    if (caught) atomicAdd(&sum[1], (unsigned long long)caught);
+    if (r.cands) atomicAdd(&sum[2], (unsigned long long)r.cands);
+  }
+  __syncthreads();
+  if (threadIdx.x < 3 && sum[threadIdx.x]) {
+    Ctrl::Tally *t = &a.ctrl->tally[blockIdx.x % 8];
+    if (threadIdx.x == 2)
+      atomicAdd(&t->cands, (uint32_t)sum[2]);
+    else
+      atomicAdd(threadIdx.x ? &t->caught : &t->edges, sum[threadIdx.x]);
   }
 }
 
@@ -552,12 +588,13 @@ __device__ inline void list_open(const GenArgs &a, bool first, uint32_t kb, uint
   const unsigned long long firsts = __ballot(first);
   if (firsts) {
     const uint32_t cnt = (uint32_t)__popcll(firsts);
-    if (res.used + cnt > kListBlock) {
+    if (res.used + cnt > res.size) {
       list_pad(a, res);
       uint32_t nb = 0;
       if (lane == 0) nb = atomicAdd(&a.ctrl->ccnt, kListBlock);
       res.base = __shfl(nb, 0, kWave);
       res.used = 0;
+      res.size = kListBlock;
     }
     if (first) {
       const uint32_t pos = res.base + res.used + (uint32_t)__popcll(firsts & lt_mask);
@@ -621,19 +658,16 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   const int lane = lane_id();
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   uint64_t edges_seen = 0;
-  ListRes res;
   const uint32_t wave_id = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
-  // groups per chunk: 64 once that leaves every wave a chunk; smaller rounds
-  // spread over the waves, since a chunk's steps are a chain of memory round
-  // trips (64 groups of up to heavy_pairs pairs took a wave 60 us, which was
-  // the whole round on graphs of a few thousand vertices and on grids)
-  // -- but no chunk below about 64 edges, or the waves' claims on the flat list
-  // cost more than the chains (builds at 1,024 / 4,096 vertices and the
-  // 1024 x 1024 grid: one group and up 2.55 / 5.1 / 426 ms, 32 edges 2.57 /
-  // 4.84 / 367, 64 2.60 / 4.79 / 343, 128 2.77 / 5.0 / 344, 256 2.83 / 5.4 /
-  // 363, always 64 groups 2.93 / 6.15 / 363)
-  const uint32_t gw = min((uint32_t)kWave, max(a.group_min, (gcnt + nwaves - 1) / nwaves));
+  const uint32_t gw = light_groups(a, gcnt);
+  // the first list block of each wave is its own (k_round_prep), as far as the
+  // workgroups that hold a chunk go
+  if ((uint64_t)blockIdx.x * 4 * gw >= gcnt) return;
+  ListRes res;
+  res.base = wave_id * kFirstBlock;
+  res.used = 0;
+  res.size = kFirstBlock;
   for (bool first = true;; first = false) {
     // chunks of gw groups: a wave's first chunk is its own id and later ones
     // come from a counter (waves with nothing to do never touch it; dealing
@@ -642,6 +676,7 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
     // 0.258 s that way against 0.042 s)
     uint32_t chunk = wave_id;
     if (!first) {
+      if ((uint64_t)nwaves * gw >= gcnt) break;  // every chunk was a first one
       if (lane == 0) chunk = nwaves + atomicAdd(&a.ctrl->expand_ctr, 1u);
       chunk = __shfl(chunk, 0, kWave);
     }
@@ -868,8 +903,14 @@ __global__ void __launch_bounds__(256) k_expand_heavy(GenArgs a) {
 // batch's slot rows (or always / never by the policy), and only while an XCD
 // queue's item count fits its 32-bit counter.  A batch of one hub has no list
 // reads to share: the plain form never takes row items unless forced.
+__device__ inline uint32_t round_cands(const GenArgs &a) {
+  uint32_t c = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) c += a.ctrl->tally[x].cands;
+  return c;
+}
 __device__ inline bool rows_chosen(const GenArgs &a) {
-  const uint32_t cands = a.ctrl->cand_round;
+  const uint32_t cands = round_cands(a);
   const uint64_t queue_items =
       (uint64_t)a.B * (((uint64_t)a.n + (uint64_t)a.row_block * kXcds - 1) /
                        ((uint64_t)a.row_block * kXcds));
@@ -1024,7 +1065,20 @@ __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
     a.ctrl->total_chunks = (dead || rows) ? 0u : run;
     a.ctrl->wave_items = (dead || rows || !waves) ? 0u : nsmall;
     a.ctrl->work_ctr = 0;
-    a.ctrl->cand_total += a.ctrl->cand_round;
+    a.ctrl->cand_total += round_cands(a);
+    unsigned long long edges = 0, caught = 0;
+    for (int x = 0; x < 8; ++x) {
+      Ctrl::Tally *y = &a.ctrl->tally[x];
+      edges += y->edges;
+      caught += y->caught;
+      y->edges = y->caught = 0;
+      y->cands = 0;
+    }
+    a.ctrl->edge_total += edges;
+    if (a.lm && a.h > 1) {
+      a.ctrl->lm_tested += edges;
+      a.ctrl->lm_caught += caught;
+    }
     a.ctrl->item_total += min(a.ctrl->fcnt[a.cur], a.fcap);
   }
 }
@@ -1970,6 +2024,7 @@ k_prune_rows(GenArgs a) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t sh_b, sh_k, sh_kn, sh_q, sh_next, sh_rows;
   __shared__ uint32_t sh_nf, sh_acc, sh_touch, sh_acc_base, sh_touch_base;
+  __shared__ unsigned long long sh_reads;
   __shared__ uint32_t sh_step[kRowSteps];  // candidates of each step
   __shared__ uint32_t sh_y0[kRowSteps];    // first vertex of each step
   // candidates: offset in the steps (13 bits), with 16-bit distances the
@@ -1982,6 +2037,7 @@ k_prune_rows(GenArgs a) {
   Item *Fn = frontier(a, a.cur ^ 1);
   uint32_t tile_b = kInf32;  // hub slot whose tile is in LDS
   unsigned long long wave_reads = 0, tile_reads = 0, row_slots = 0;
+  if (tid == 0) sh_reads = 0;
   const uint64_t gwords = a.gtile_cap / gridDim.x;
   uint32_t *gkeys = a.gtile + (uint64_t)blockIdx.x * gwords;
   const uint32_t nblk = (uint32_t)(((uint64_t)a.n + a.row_block - 1) / a.row_block);
@@ -2154,7 +2210,9 @@ k_prune_rows(GenArgs a) {
       __syncthreads();
     }
   }
-  if (lane == 0 && wave_reads) atomicAdd(&a.ctrl->label_reads, wave_reads);
+  if (lane == 0 && wave_reads) atomicAdd(&sh_reads, wave_reads);
+  __syncthreads();
+  if (tid == 0 && sh_reads) atomicAdd(&a.ctrl->label_reads, sh_reads);
   if (tid == 0 && tile_reads) atomicAdd(&a.ctrl->tile_reads, tile_reads);
   if (tid == 0 && row_slots) atomicAdd(&a.ctrl->row_slots, row_slots);
 }
@@ -2249,7 +2307,10 @@ __global__ void __launch_bounds__(256) k_finalize(GenArgs a) {
     }
     a.add_cnt[y] = 0;
   }
-  if (mx) atomicMax(&a.ctrl->maxlen, mx);
+  mx = wave_max_u32(mx);
+  if (lane_id() == 0 &&
+      mx > __hip_atomic_load(&a.ctrl->maxlen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(&a.ctrl->maxlen, mx);
   if (blockIdx.x == 0 && threadIdx.x == 0) a.ctrl->gcnt = keep ? min(cnt, a.n) : 0u;
 }
 
@@ -3101,6 +3162,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     // (either setting of the knob also keeps hash tiles only)
     a.direct_tiles = getenv("HSDL_PRUNE_INDEXED") ? 0u : 1u;
   }
+  a.expand_waves = (uint32_t)g.grid * 4;
   a.piece_pairs = env_u32("HSDL_PIECE_PAIRS", 16384, 1, 1u << 16);
   a.lds_slots = lds_slots;
   // wave items (tuning knobs HSDL_WAVE_ITEMS, the least hub slots of a round
