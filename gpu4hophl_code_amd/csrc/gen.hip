@@ -2438,6 +2438,74 @@ __device__ inline void hop_scatter(const GenArgs &a, unsigned long long st, uint
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// Lists of up to sort_held labels: a wave holds the list in registers, so each
+// label is read and written once and nothing but registers limits the waves in
+// flight (the sort of a short list is three round trips: its extents, its labels,
+// the stores).  A wave looks at 64 vertices, or fewer where that gives every
+// wave some.
+template <class LT> constexpr uint32_t sort_held = 4096 / sizeof(LT);
+template <class LT>
+__global__ void __launch_bounds__(256) k_hop_sort_short(GenArgs a, LT *pool, uint32_t alpha_div) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const unsigned long long lt_mask = (1ull << lane) - 1ull;
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
+  const uint32_t per = min((uint32_t)kWave, (a.n + nwaves - 1) / nwaves);
+  const uint32_t K1 = a.K + 1;
+  constexpr uint32_t kRegs = sort_held<LT> / kWave;
+  for (uint64_t base = (uint64_t)wave * per; base < a.n; base += (uint64_t)nwaves * per) {
+    const uint32_t v = (uint32_t)base + lane;
+    bool need = false;
+    uint32_t vlen = 0;
+    unsigned long long vst = 0;
+    if (lane < per && v < a.n) {
+      vlen = a.seg_len[v];
+      vst = a.seg_start[v];
+      const uint32_t sorted = a.sorted_len[v];
+      need = vlen > sorted && vlen <= sort_held<LT> && (uint64_t)(vlen - sorted) * alpha_div > sorted;
+    }
+    for (unsigned long long todo = __ballot(need); todo; todo &= todo - 1) {
+      const uint32_t i = (uint32_t)(__ffsll((long long)todo) - 1);
+      const uint32_t y = (uint32_t)base + i;
+      const uint32_t len = __builtin_amdgcn_readlane(vlen, i);
+      LT *L = pool + (((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(vst >> 32), i)
+                       << 32) |
+                      (uint32_t)__builtin_amdgcn_readlane((uint32_t)vst, i));
+      LT l[kRegs];
+      uint32_t dst[kRegs];
+#pragma unroll
+      for (uint32_t r = 0; r < kRegs; ++r) {
+        l[r] = 0;
+        if (r * kWave < len) l[r] = L[min(r * kWave + lane, len - 1)];
+      }
+      auto hop = [&](uint32_t r) {
+        uint32_t hub, x, d;
+        unpack(a, l[r], hub, x, d);
+        return r * kWave + lane < len ? x : kInf32;
+      };
+#pragma unroll
+      for (uint32_t r = 0; r < kRegs; ++r) dst[r] = 0;
+      uint32_t run = 0, pre = 0;  // pre: lane x - 1, labels of hop <= x
+      for (uint32_t x = 0; x < K1; ++x) {
+#pragma unroll
+        for (uint32_t r = 0; r < kRegs; ++r) {
+          if (r * kWave >= len) break;
+          const bool here = hop(r) == x;
+          const unsigned long long m = __ballot(here);
+          if (here) dst[r] = run + (uint32_t)__popcll(m & lt_mask);
+          run += (uint32_t)__popcll(m);
+        }
+        if (lane + 1 == x) pre = run;
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < kRegs; ++r)
+        if (r * kWave + lane < len) L[dst[r]] = l[r];
+      if (lane < a.hcnt_stride) a.hcnt[(uint64_t)y * a.hcnt_stride + lane] = pre;
+      if (lane == 0) a.sorted_len[y] = len;
+    }
+  }
+}
+
 // Lists of up to lds_labels labels are scattered in the wave's LDS slice
 // (one read and one write of each label in HBM), longer ones in its slice of
 // `tmp` in HBM (two of each).
@@ -2450,6 +2518,7 @@ __global__ void __launch_bounds__(256) k_hop_sort(GenArgs a, unsigned long long 
   const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
   const uint32_t wib = threadIdx.x / kWave;  // wave in block
   const bool p32 = tmp32 != nullptr;
+  const uint32_t held = p32 ? sort_held<uint32_t> : sort_held<unsigned long long>;
   unsigned long long *t64 = tmp + (uint64_t)wave * per_wave;
   uint32_t *t32 = p32 ? tmp32 + (uint64_t)wave * per_wave : nullptr;
   // LDS: 4 slices of lds_labels u64, then 4 of lds_labels u32; a build
@@ -2465,7 +2534,7 @@ __global__ void __launch_bounds__(256) k_hop_sort(GenArgs a, unsigned long long 
     bool need = false;
     if (v < a.n) {
       const uint32_t len = a.seg_len[v], sorted = a.sorted_len[v];
-      need = len > sorted && (uint64_t)(len - sorted) * alpha_div > sorted &&
+      need = len > sorted && len > held && (uint64_t)(len - sorted) * alpha_div > sorted &&
              (len <= per_wave || len <= lds_labels);
     }
     unsigned long long todo = __ballot(need);
@@ -2873,6 +2942,14 @@ static int enqueue_batch(Gen &g, uint32_t s0, uint32_t B, uint32_t K, uint32_t n
 // list so far (grown here); a list that outgrows them before the next growth
 // is left unsorted, which only costs reads.
 static int sort_zones(Gen &g, uint32_t maxlen, uint32_t resort_div) {
+  if (g.a.pool32)
+    hipLaunchKernelGGL(k_hop_sort_short<uint32_t>, dim3(g.grid * 2), dim3(256), 0, g.st, g.a,
+                       g.a.pool32, resort_div);
+  else
+    hipLaunchKernelGGL(k_hop_sort_short<unsigned long long>, dim3(g.grid * 2), dim3(256), 0, g.st,
+                       g.a, g.a.pool, resort_div);
+  HSDL_HIP(hipGetLastError());
+  if (maxlen <= (g.a.pool32 ? sort_held<uint32_t> : sort_held<unsigned long long>)) return HSDL_OK;
   if (!g.sort_grid) g.sort_grid = std::max(1, g.grid / 4);  // 256 threads: 4 waves each
   const uint64_t waves = (uint64_t)g.sort_grid * 4;
   // tuning knob HSDL_SORT_SLICE caps the slice (longer lists stay unsorted)
