@@ -179,7 +179,8 @@ struct GenArgs {
   uint32_t *sorted_len;
   uint32_t *hcnt;
   uint32_t hcnt_stride;  // K - 1
-  uint32_t *add_cnt;
+  uint32_t *add_cnt;   // labels a vertex gains in the round, counted by the prune
+  uint32_t *base_len;  // its list's length before them (k_reserve, for k_append)
   uint32_t *touched;
   FGroup *fgrp;               // frontier groups (n entries)
   uint32_t *hub_slot;         // group builds: hub slot of each hub of the batch
@@ -368,19 +369,6 @@ __global__ void k_fill_u32(uint32_t *p, uint64_t n, uint32_t val) {
 
 // The first frontier: every hub of the batch with its self label (position
 // 0 of its list), one group each.
-__global__ void k_batch_begin(GenArgs a) {
-  with_batch(a);
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < a.B; b += gridDim.x * blockDim.x) {
-    const uint32_t s = hub_of(a, b);
-    a.fgrp[b] = FGroup{s, 1u, a.seg_start[s]};
-    if (a.hubs) a.hub_slot[s] = b;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    a.ctrl->fcnt[a.cur] = a.B;
-    a.ctrl->gcnt = a.B;
-  }
-}
-
 // Frontier groups per chunk of the light expansion: 64 once that leaves every
 // wave a chunk; smaller rounds spread over the waves, since a chunk's steps are a
 // chain of memory round trips (64 groups of up to heavy_pairs pairs took a wave
@@ -403,8 +391,9 @@ constexpr uint32_t kFirstBlock = 64;  // flat-list entries each wave of a chunk 
 // tile of the round fits a prune wave's slice of LDS
 constexpr uint32_t kSmallTile = 1u << 31;
 
-__global__ void k_round_prep(GenArgs a) {
-  with_batch(a);
+// Sets up round a.h, whose frontier has gcnt groups (all threads of the kernel
+// before the round: the batch's first or the last round's k_append).
+__device__ inline void round_prep(const GenArgs &a, uint32_t gcnt) {
   for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < a.B; b += gridDim.x * blockDim.x) {
     a.hub_ccnt[b] = a.B >= a.wave_min && tile_view(a, hub_of(a, b)).len <= a.wave_slots / 2
                         ? kSmallTile : 0u;
@@ -412,13 +401,27 @@ __global__ void k_round_prep(GenArgs a) {
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.ctrl->fcnt[a.cur ^ 1] = 0;
-    a.ctrl->ccnt = min(a.expand_waves, (light_chunks(a, a.ctrl->gcnt) + 3u) & ~3u) * kFirstBlock;
+    a.ctrl->ccnt = min(a.expand_waves, (light_chunks(a, gcnt) + 3u) & ~3u) * kFirstBlock;
     a.ctrl->touched_cnt = 0;
     a.ctrl->work_ctr = 0;
     a.ctrl->expand_ctr = 0;
     a.ctrl->heavy_cnt = 0;
     a.ctrl->heavy_ctr = 0;
   }
+}
+
+__global__ void k_batch_begin(GenArgs a) {
+  with_batch(a);
+  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < a.B; b += gridDim.x * blockDim.x) {
+    const uint32_t s = hub_of(a, b);
+    a.fgrp[b] = FGroup{s, 1u, a.seg_start[s]};
+    if (a.hubs) a.hub_slot[s] = b;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    a.ctrl->fcnt[a.cur] = a.B;
+    a.ctrl->gcnt = a.B;
+  }
+  round_prep(a, a.B);
 }
 
 // ---------------------------------------------------------------- expand
@@ -661,7 +664,7 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   const uint32_t wave_id = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
   const uint32_t gw = light_groups(a, gcnt);
-  // the first list block of each wave is its own (k_round_prep), as far as the
+  // the first list block of each wave is its own (round_prep), as far as the
   // workgroups that hold a chunk go
   if ((uint64_t)blockIdx.x * 4 * gw >= gcnt) return;
   ListRes res;
@@ -920,21 +923,55 @@ __device__ inline bool rows_chosen(const GenArgs &a) {
 }
 
 // Per-hub candidate counts of a round that takes list items: a workgroup
-// takes 2048 consecutive entries of the flat list, counts their hubs in an
-// LDS hash and adds each hub's count with one global atomic.
+// takes consecutive entries of the flat list, counts their hubs in an LDS hash
+// and adds each hub's count with one global atomic.  2,048 entries, or 512 in
+// rounds whose list is then still a workgroup's work or less for each (a grid's
+// rounds: 262,144 entries, which 128 workgroups had to themselves).
 constexpr uint32_t kGroupThreads = 256;
 constexpr uint32_t kGroupPer = 8;                                 // entries per thread
-constexpr uint32_t kGroupChunk = kGroupThreads * kGroupPer;       // 2048
-constexpr uint32_t kGroupSlots = 2 * kGroupChunk;                 // load factor <= 1/2
-static_assert(kGroupSlots == 4096, "hubs hash to 12 bits");
+constexpr uint32_t kGroupFew = 2;                                 // the same, short lists
+constexpr uint32_t kGroupSlots = 2 * kGroupPer * kGroupThreads;   // load factor <= 1/2
+__device__ inline bool group_few(uint32_t cnt) {
+  return cnt <= gridDim.x * (kGroupFew * kGroupThreads);
+}
 
-// LDS hash slot of hub slot b (inserted when absent)
+// LDS hash slot of hub slot b among 2 * kPer * kGroupThreads (inserted when
+// absent)
+template <uint32_t kPer>
 __device__ inline uint32_t group_slot(uint32_t *hkey, uint32_t b) {
-  uint32_t sl = (b * 0x9E3779B1u) >> 20;  // 12 bits: kGroupSlots = 4096
+  constexpr uint32_t slots = 2 * kPer * kGroupThreads;
+  static_assert((slots & (slots - 1)) == 0, "a power of two");
+  uint32_t sl = (b * 0x9E3779B1u) >> (__builtin_clz(slots) + 1);
   for (;;) {
     const uint32_t prev = atomicCAS(&hkey[sl], kInf32, b);
     if (prev == kInf32 || prev == b) return sl;
-    sl = (sl + 1) & (kGroupSlots - 1);
+    sl = (sl + 1) & (slots - 1);
+  }
+}
+
+template <uint32_t kPer>
+__device__ inline void count_hubs(const GenArgs &a, uint32_t cnt, uint32_t *hkey, uint32_t *hcnt) {
+  constexpr uint32_t chunk = kPer * kGroupThreads, slots = 2 * chunk;
+  const uint32_t tid = threadIdx.x;
+  for (uint64_t c0 = (uint64_t)blockIdx.x * chunk; c0 < cnt; c0 += (uint64_t)gridDim.x * chunk) {
+    unsigned long long e[kPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r) {
+      const uint64_t i = c0 + r * kGroupThreads + tid;
+      e[r] = i < cnt ? a.cflat[i] : kEmptyEntry;
+    }
+    for (uint32_t i = tid; i < slots; i += kGroupThreads) {
+      hkey[i] = kInf32;
+      hcnt[i] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r)
+      if (e[r] != kEmptyEntry) atomicAdd(&hcnt[group_slot<kPer>(hkey, (uint32_t)(e[r] >> 32))], 1u);
+    __syncthreads();
+    for (uint32_t i = tid; i < slots; i += kGroupThreads)
+      if (hcnt[i]) atomicAdd(&a.hub_ccnt[hkey[i]], hcnt[i]);
+    __syncthreads();
   }
 }
 
@@ -945,25 +982,10 @@ __global__ void __launch_bounds__(kGroupThreads) k_count(GenArgs a) {
   if (a.ctrl->overflow || rows_chosen(a)) return;
   // reserved blocks may reach past the list's end; only empty entries lie there
   const uint32_t cnt = min(a.ctrl->ccnt, a.ccap);
-  const uint32_t tid = threadIdx.x;
-  for (uint64_t c0 = (uint64_t)blockIdx.x * kGroupChunk; c0 < cnt;
-       c0 += (uint64_t)gridDim.x * kGroupChunk) {
-    for (uint32_t i = tid; i < kGroupSlots; i += kGroupThreads) {
-      hkey[i] = kInf32;
-      hcnt[i] = 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < kGroupPer; ++r) {
-      const uint64_t i = c0 + r * kGroupThreads + tid;
-      const unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
-      if (e != kEmptyEntry) atomicAdd(&hcnt[group_slot(hkey, (uint32_t)(e >> 32))], 1u);
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < kGroupSlots; i += kGroupThreads)
-      if (hcnt[i]) atomicAdd(&a.hub_ccnt[hkey[i]], hcnt[i]);
-    __syncthreads();
-  }
+  if (group_few(cnt))
+    count_hubs<kGroupFew>(a, cnt, hkey, hcnt);
+  else
+    count_hubs<kGroupPer>(a, cnt, hkey, hcnt);
 }
 
 // One workgroup: hub_off = exclusive scan of hub_ccnt; chunk_off[b] =
@@ -1083,11 +1105,53 @@ __global__ void __launch_bounds__(1024) k_chunk_scan(GenArgs a) {
   }
 }
 
-// Scatter of the flat candidates into per-hub runs.  A workgroup takes 2048
-// consecutive entries, counts their hubs in an LDS hash, reserves each hub's
-// space with one global atomic and writes the entries: one global atomic per
-// (chunk, hub) instead of one per (wave, hub), so hubs with millions of
-// candidates do not serialize the scatter on their counters.
+// Scatter of the flat candidates into per-hub runs.  A workgroup takes the
+// consecutive entries that k_count's would, counts their hubs in an LDS hash,
+// reserves each hub's space with one global atomic and writes the entries: one
+// global atomic per (chunk, hub) instead of one per (wave, hub), so hubs with
+// millions of candidates do not serialize the scatter on their counters.
+template <uint32_t kPer>
+__device__ inline void group_hubs(const GenArgs &a, uint32_t cnt, uint32_t *hkey, uint32_t *hcnt,
+                                  uint32_t *hbase) {
+  constexpr uint32_t chunk = kPer * kGroupThreads, slots = 2 * chunk;
+  const uint32_t tid = threadIdx.x;
+  for (uint64_t c0 = (uint64_t)blockIdx.x * chunk; c0 < cnt; c0 += (uint64_t)gridDim.x * chunk) {
+    unsigned long long e[kPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r) {
+      const uint64_t i = c0 + r * kGroupThreads + tid;
+      e[r] = i < cnt ? a.cflat[i] : kEmptyEntry;
+    }
+    for (uint32_t i = tid; i < slots; i += kGroupThreads) {
+      hkey[i] = kInf32;
+      hcnt[i] = 0;
+    }
+    __syncthreads();
+    uint32_t slot[kPer], rank[kPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r) {
+      slot[r] = kInf32;
+      rank[r] = 0;
+      if (e[r] != kEmptyEntry) {
+        slot[r] = group_slot<kPer>(hkey, (uint32_t)(e[r] >> 32));
+        rank[r] = atomicAdd(&hcnt[slot[r]], 1u);
+      }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < slots; i += kGroupThreads) {
+      const uint32_t c = hcnt[i];
+      if (c) {
+        const uint32_t b = hkey[i];
+        hbase[i] = a.hub_off[b] + atomicAdd(&a.hub_cur[b], c);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r)
+      if (slot[r] != kInf32) a.cgroup[hbase[slot[r]] + rank[r]] = (uint32_t)e[r];
+    __syncthreads();
+  }
+}
 
 __global__ void __launch_bounds__(kGroupThreads) k_group(GenArgs a) {
   with_batch(a);
@@ -1097,46 +1161,10 @@ __global__ void __launch_bounds__(kGroupThreads) k_group(GenArgs a) {
   if (a.ctrl->overflow || a.ctrl->row_mode) return;
   // reserved blocks may reach past the list's end; only empty entries lie there
   const uint32_t cnt = min(a.ctrl->ccnt, a.ccap);
-  const uint32_t tid = threadIdx.x;
-  for (uint64_t c0 = (uint64_t)blockIdx.x * kGroupChunk; c0 < cnt;
-       c0 += (uint64_t)gridDim.x * kGroupChunk) {
-    for (uint32_t i = tid; i < kGroupSlots; i += kGroupThreads) {
-      hkey[i] = kInf32;
-      hcnt[i] = 0;
-    }
-    __syncthreads();
-    uint32_t slot[kGroupPer], yv[kGroupPer];
-#pragma unroll
-    for (uint32_t r = 0; r < kGroupPer; ++r) {
-      const uint64_t i = c0 + r * kGroupThreads + tid;
-      slot[r] = kInf32;
-      yv[r] = 0;
-      const unsigned long long e = i < cnt ? a.cflat[i] : kEmptyEntry;
-      if (e != kEmptyEntry) {
-        yv[r] = (uint32_t)e;
-        const uint32_t sl = group_slot(hkey, (uint32_t)(e >> 32));
-        slot[r] = sl;
-        atomicAdd(&hcnt[sl], 1u);
-      }
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < kGroupSlots; i += kGroupThreads) {
-      const uint32_t c = hcnt[i];
-      if (c) {
-        const uint32_t b = hkey[i];
-        hbase[i] = a.hub_off[b] + atomicAdd(&a.hub_cur[b], c);
-        hcnt[i] = 0;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < kGroupPer; ++r) {
-      if (slot[r] == kInf32) continue;
-      const uint32_t rank = atomicAdd(&hcnt[slot[r]], 1u);
-      a.cgroup[hbase[slot[r]] + rank] = yv[r];
-    }
-    __syncthreads();
-  }
+  if (group_few(cnt))
+    group_hubs<kGroupFew>(a, cnt, hkey, hcnt, hbase);
+  else
+    group_hubs<kGroupPer>(a, cnt, hkey, hcnt, hbase);
 }
 
 // ----------------------------------------------------------------- prune
@@ -2218,64 +2246,122 @@ k_prune_rows(GenArgs a) {
 }
 
 // -------------------------------------------------------- reserve / append
+// The lists [st, st + len) of the lanes with `grow` move to ns (whole wave).
+// Lists of up to kMoveShort labels are taken together, 64 labels per load
+// whatever lists they lie in; longer ones one at a time.
+constexpr uint32_t kMoveShort = 256;
+template <class LT>
+__device__ inline void move_lists(LT *pool, bool grow, unsigned long long st,
+                                  unsigned long long ns, uint32_t len) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t part = grow && len <= kMoveShort ? len : 0u;
+  const uint32_t incl = wave_incl_scan_u32(part), excl = incl - part;
+  const uint32_t total = __shfl(incl, kWave - 1, kWave);
+  const unsigned long long from = st - excl, to = ns - excl;
+  constexpr int kStep = 4;  // loads in flight together
+  for (uint32_t j0 = 0; j0 < total; j0 += kStep * kWave) {
+    LT l[kStep];
+    unsigned long long d[kStep];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const uint32_t j = min(j0 + u * kWave + lane, total - 1);
+      int k = 0;  // largest k with excl_k <= j: empty lists are skipped over
+#pragma unroll
+      for (int step = 32; step > 0; step >>= 1) {
+        const uint32_t e = __shfl(excl, k + step, kWave);
+        if (e <= j) k += step;
+      }
+      d[u] = __shfl(to, k, kWave) + j;
+      l[u] = pool[__shfl(from, k, kWave) + j];
+    }
+#pragma unroll
+    for (int u = 0; u < kStep; ++u)
+      if (j0 + u * kWave + lane < total) pool[d[u]] = l[u];
+  }
+  for (unsigned long long m = __ballot(grow && len > kMoveShort); m; m &= m - 1) {
+    const int i = __ffsll((long long)m) - 1;
+    const uint32_t n = __shfl(len, i, kWave);
+    const LT *src = pool + __shfl(st, i, kWave);
+    LT *dst = pool + __shfl(ns, i, kWave);
+    for (uint32_t q = lane; q < n; q += kWave) dst[q] = src[q];
+  }
+}
+
 __global__ void __launch_bounds__(256) k_reserve(GenArgs a) {
   with_batch(a);
   const int lane = lane_id();
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
   const uint32_t cnt = a.ctrl->touched_cnt;
+  // a lost frontier item leaves a counted label unwritten: publish nothing
+  // (the host rolls the batch back)
+  const bool keep = !(a.ctrl->overflow & kOvfFront);
+  uint32_t mx = 0;
   // 64 touched vertices per wave step (lane i: the step's vertex i), with one
   // pool reservation for all of them that outgrow their segments: in a
   // batch's first rounds most vertices grow, and one reservation per vertex
   // on the single pool counter serialised them
   for (uint32_t t0 = wave * kWave; t0 < cnt; t0 += nwaves * kWave) {
     const uint32_t t = t0 + (uint32_t)lane;
-    uint32_t y = 0, len = 0, ncap = 0;
+    uint32_t y = 0, len = 0, add = 0, cap = 0, ncap = 0;
+    unsigned long long st = 0;
     if (t < cnt) {
       y = a.touched[t];
       len = a.seg_len[y];
-      const uint32_t cap = a.seg_cap[y];
-      const uint32_t need = len + a.add_cnt[y];
-      if (need > cap) ncap = (max(need, cap * 2u) + 7u) & ~7u;
+      cap = a.seg_cap[y];
+      st = a.seg_start[y];
+      add = a.add_cnt[y];
+      if (len + add > cap) ncap = (max(len + add, cap * 2u) + 7u) & ~7u;
     }
-    const unsigned long long grow = __ballot(ncap != 0);
-    if (!grow) continue;
-    const unsigned long long incl = wave_incl_scan_u64(ncap);
-    const unsigned long long total = __shfl(incl, kWave - 1, kWave);
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(&a.ctrl->pool_top, total);
-    base = __shfl(base, 0, kWave);
-    if (base + total > a.pool_cap) {
-      if (lane == 0) atomicOr(&a.ctrl->overflow, kOvfPool);
-      continue;
-    }
-    const unsigned long long ns = base + incl - ncap;
-    // each growing vertex's labels move to its new segment, the whole wave
-    // copying one vertex at a time
-    for (unsigned long long m = grow; m; m &= m - 1) {
-      const int j = __ffsll((long long)m) - 1;
-      const uint32_t yj = __shfl(y, j, kWave), lj = __shfl(len, j, kWave);
-      const unsigned long long nsj = __shfl(ns, j, kWave);
-      const unsigned long long os = a.seg_start[yj];
+    if (__ballot(ncap != 0)) {
+      const unsigned long long incl = wave_incl_scan_u64(ncap);
+      const unsigned long long total = __shfl(incl, kWave - 1, kWave);
+      unsigned long long base = 0;
+      if (lane == 0) base = atomicAdd(&a.ctrl->pool_top, total);
+      base = __shfl(base, 0, kWave);
+      if (base + total > a.pool_cap) {
+        if (lane == 0) atomicOr(&a.ctrl->overflow, kOvfPool);
+        ncap = 0;
+      }
+      const unsigned long long ns = base + incl - ncap;
       if (a.pool)
-        for (uint32_t i = lane; i < lj; i += kWave) a.pool[nsj + i] = a.pool[os + i];
-      if (a.pool32)
-        for (uint32_t i = lane; i < lj; i += kWave) a.pool32[nsj + i] = a.pool32[os + i];
+        move_lists(a.pool, ncap != 0, st, ns, len);
+      else
+        move_lists(a.pool32, ncap != 0, st, ns, len);
+      if (ncap) {
+        a.seg_start[y] = st = ns;
+        a.seg_cap[y] = cap = ncap;
+      }
     }
-    if (ncap) {
-      a.seg_start[y] = ns;
-      a.seg_cap[y] = ncap;
+    if (t < cnt) {
+      a.base_len[y] = len;
+      a.add_cnt[y] = 0;
+      if (keep) {
+        // capped: when the pool ran out some appends are dropped
+        const uint32_t nl = min(len + add, cap);
+        a.seg_len[y] = nl;
+        mx = max(mx, nl);
+        // the next round's frontier group of y: the labels it gains
+        a.fgrp[t] = FGroup{y, nl - len, st + len};
+      }
     }
   }
+  mx = wave_max_u32(mx);
+  if (lane == 0 &&
+      mx > __hip_atomic_load(&a.ctrl->maxlen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(&a.ctrl->maxlen, mx);
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctrl->gcnt = keep ? min(cnt, a.n) : 0u;
 }
 
+// Writes the accepted labels behind their vertices' lists and sets up the next
+// round.
 __global__ void __launch_bounds__(256) k_append(GenArgs a) {
   with_batch(a);
   const Item *Fn = frontier(a, a.cur ^ 1);
   const uint32_t cnt = min(a.ctrl->fcnt[a.cur ^ 1], a.fcap);
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
     const Item it = Fn[i];
-    const uint32_t p = a.seg_len[it.y] + a.frank[i];
+    const uint32_t p = a.base_len[it.y] + a.frank[i];
     if (p < a.seg_cap[it.y]) {
       const unsigned long long at = a.seg_start[it.y] + p;
       const uint32_t hub = hub_of(a, it.b);
@@ -2285,33 +2371,11 @@ __global__ void __launch_bounds__(256) k_append(GenArgs a) {
       atomicOr(&a.ctrl->overflow, kOvfPool);
     }
   }
-}
-
-__global__ void __launch_bounds__(256) k_finalize(GenArgs a) {
-  with_batch(a);
-  const uint32_t cnt = a.ctrl->touched_cnt;
-  // a lost frontier item leaves a counted label unwritten: publish nothing
-  // (the host rolls the batch back)
-  const bool keep = !(a.ctrl->overflow & kOvfFront);
-  uint32_t mx = 0;
-  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < cnt; t += gridDim.x * blockDim.x) {
-    const uint32_t y = a.touched[t];
-    if (keep) {
-      // capped: when the pool ran out some appends were dropped
-      const uint32_t len = a.seg_len[y];
-      const uint32_t nl = min(len + a.add_cnt[y], a.seg_cap[y]);
-      a.seg_len[y] = nl;
-      mx = max(mx, nl);
-      // the next round's frontier group of y: the labels it just gained
-      a.fgrp[t] = FGroup{y, nl - len, a.seg_start[y] + len};
-    }
-    a.add_cnt[y] = 0;
-  }
-  mx = wave_max_u32(mx);
-  if (lane_id() == 0 &&
-      mx > __hip_atomic_load(&a.ctrl->maxlen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-    atomicMax(&a.ctrl->maxlen, mx);
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctrl->gcnt = keep ? min(cnt, a.n) : 0u;
+  if (a.h == a.K) return;
+  const uint32_t gcnt = a.ctrl->gcnt;
+  a.h += 1;
+  a.cur ^= 1;
+  round_prep(a, gcnt);
 }
 
 // Removes the labels of the batch's hubs (the batch being rolled back): they
@@ -2442,7 +2506,9 @@ __device__ inline void hop_scatter(const GenArgs &a, unsigned long long st, uint
 // label is read and written once and nothing but registers limits the waves in
 // flight (the sort of a short list is three round trips: its extents, its labels,
 // the stores).  A wave looks at 64 vertices, or fewer where that gives every
-// wave some.
+// wave some.  Against LDS slices of 64 KB per workgroup (eight waves per CU) for
+// all lists: 0.40 -> 0.03 ms of a 4,096-vertex build, 13.3 -> 6.6 ms at R-MAT
+// 262,144 (K = 5), 19.2 -> 13.4 ms on the 1024 x 1024 grid (K = 8).
 template <class LT> constexpr uint32_t sort_held = 4096 / sizeof(LT);
 template <class LT>
 __global__ void __launch_bounds__(256) k_hop_sort_short(GenArgs a, LT *pool, uint32_t alpha_div) {
@@ -2839,12 +2905,12 @@ static int alloc_lists(Gen &g, uint32_t ccap, uint32_t fcap) {
 // sequence depends only on the buffers, K and whether row items may run.
 static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows) {
   a.cur = 0;
+  a.h = 1;
   // grid-stride loops over the batch's hubs: sized for the largest batch
   const int small_grid = (int)std::min<uint32_t>((g.bmax + 255) / 256, 1024);
   hipLaunchKernelGGL(k_batch_begin, dim3(small_grid), dim3(256), 0, g.st, a);
   for (uint32_t h = 1; h <= K; ++h) {
     a.h = h;
-    hipLaunchKernelGGL(k_round_prep, dim3(small_grid), dim3(256), 0, g.st, a);
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 0], g.st);
     hipLaunchKernelGGL(k_expand, dim3(g.grid), dim3(256), 0, g.st, a);
     hipLaunchKernelGGL(k_expand_heavy, dim3(g.grid), dim3(256), 0, g.st, a);
@@ -2874,7 +2940,6 @@ static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows) {
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 3], g.st);
     hipLaunchKernelGGL(k_reserve, dim3(g.grid), dim3(256), 0, g.st, a);
     hipLaunchKernelGGL(k_append, dim3(g.grid), dim3(256), 0, g.st, a);
-    hipLaunchKernelGGL(k_finalize, dim3(g.grid), dim3(256), 0, g.st, a);
     a.cur ^= 1;
   }
 }
@@ -2926,7 +2991,7 @@ static int enqueue_batch(Gen &g, uint32_t s0, uint32_t B, uint32_t K, uint32_t n
   hipLaunchKernelGGL(k_set_batch, dim3(1), dim3(1), 0, g.st, g.a.ctrl, s0, B, g.a.tag,
                      g.lm_on ? 1u : 0u);
   const bool rows = B > 1 || g.a.row_policy == 2;
-  // one graph launch per batch instead of 1 + 11 K launches (the plain form
+  // one graph launch per batch instead of 1 + 9 K launches (the plain form
   // is bound by the host's launch rate); not with per-launch timing events
   if (g.use_graph && !g.timing && batch_graph(g, K, rows)) {
     HSDL_HIP(hipGraphLaunch(g.gexec[rows ? 1 : 0], g.st));
@@ -3071,9 +3136,9 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
       "HSDL_LIST_INIT",
       (uint32_t)std::min<uint64_t>(std::max<uint64_t>((uint64_t)n * 8, 8u << 20), 1u << 30), 64,
       1u << 30);
-  // per vertex: segment start, length, capacity, add counter, touched
+  // per vertex: segment start, length, capacity, add counter, base, touched
   // entry, frontier group (16 B), hub slot, hop zone counts
-  const uint64_t vert_bytes = (uint64_t)n * (8 + 4 * 4 + 16 + 4 + 4 * (uint64_t)K);
+  const uint64_t vert_bytes = (uint64_t)n * (8 + 5 * 4 + 16 + 4 + 4 * (uint64_t)K);
   // dense dedupe slots: at most 1/slot_div of the budget (tuning knob
   // HSDL_SLOT_DIV), <= 65536 hubs
   const bool plain = opts->mode == HSDL_MODE_PLAIN;
@@ -3156,7 +3221,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   if ((!use32 && !g.pool.p && (rc = g.pool.alloc(pool0 * 8))) ||
       (rc = g.take(kScSegStart, n * 8ull)) ||
       (rc = g.take(kScSegLen, n * 4ull)) || (rc = g.take(kScSegCap, n * 4ull)) ||
-      (rc = g.take(kScAddCnt, n * 4ull)) ||
+      (rc = g.take(kScAddCnt, n * 8ull)) ||
       (rc = g.take(kScTouched, n * 4ull)) || (rc = g.take(kScFgrp, n * 16ull)) ||
       (group && (rc = g.take(kScHubSlot, n * 4ull))) ||
       (rc = g.take(kScHubCcnt, (Bmax + 1ull) * 4)) || (rc = g.take(kScHubOff, (Bmax + 1ull) * 4)) ||
@@ -3273,6 +3338,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   a.hcnt = zones ? g.hcnt.as<uint32_t>() : nullptr;
   a.hcnt_stride = K - 1;
   a.add_cnt = g.add_cnt.as<uint32_t>();
+  a.base_len = a.add_cnt + n;
   a.touched = g.touched.as<uint32_t>();
   a.fgrp = g.fgrp.as<FGroup>();
   a.hub_slot = group ? g.hub_slot.as<uint32_t>() : nullptr;
