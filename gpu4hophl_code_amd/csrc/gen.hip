@@ -3059,12 +3059,23 @@ static int sort_zones(Gen &g, uint32_t maxlen, uint32_t resort_div) {
 // an eighth of the scanned edges, both fixed by the graph and the schedule,
 // so the schedule repeats from run to run -- or, with HSDL_TUNER=time, its
 // wall-clock duration.
+// Batches double, or grow eightfold while the last one was below 1/16 of the
+// target (what follows is then below half of it: the work per hub falls along
+// the ranking): a small batch costs its rounds' launches whatever is in them.
+// The first batch has 64 hubs, or as many as 2^23 slots hold up to 512: its
+// candidates of a round then fit the smallest flat list (2^23 entries).  From 64
+// and doubling always, on the same kernels: 1,024 / 4,096 / 40,001 vertices 2.25 /
+// 3.9 / 36.1 -> 1.48 / 2.33 / 31.5 ms, a group of 65,536 15.1 -> 12.8 ms, R-MAT
+// 262,144 202 -> 201 ms; fourfold 1.45 / 2.45 / 31.9 / 13.2 / 201; a first batch of
+// 1,024 1.45 / 2.5 / 31.9 / 13.1 / 201.
+constexpr double kTuneFar = 16, kTuneGrow = 8;
 struct BatchTuner {
+  static uint32_t first(uint32_t n) { return std::min(512u, std::max(64u, (1u << 23) / n)); }
   uint32_t B, Bmax;
   double target;
   uint32_t next(double last) {
     double f = last > 0 ? target / last : 2.0;
-    f = std::min(2.0, std::max(0.5, f));
+    f = std::min(f > kTuneFar ? kTuneGrow : 2.0, std::max(0.5, f));
     uint64_t nb = (uint64_t)std::llround(B * f);
     nb = std::max<uint64_t>(1, std::min<uint64_t>(nb, Bmax));
     B = (uint32_t)nb;
@@ -3144,7 +3155,8 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   const bool plain = opts->mode == HSDL_MODE_PLAIN;
   const uint32_t slot_div = env_u32("HSDL_SLOT_DIV", 4, 2, 64);
   uint32_t Bmax =
-      (uint32_t)std::min<uint64_t>({g.budget / slot_div / (4ull * n), (uint64_t)n, 1ull << 16});
+      (uint32_t)std::min<uint64_t>({g.budget / slot_div / (4ull * n), (uint64_t)n,
+                                    (nhubs + 15ull) & ~15ull, 1ull << 16});
   if (plain) Bmax = 1;
   if (opts->hub_batch) Bmax = std::min<uint32_t>(opts->hub_batch, Bmax);
   if (Bmax == 0) return fail(HSDL_ENOMEM, "HBM budget below one hub's dedupe slots");
@@ -3425,7 +3437,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   const double tune_target =
       tune_time ? env_u32("HSDL_BATCH_TARGET_US", 50000, 100, 10000000) * 1e-6
                 : (double)env_u32("HSDL_BATCH_TARGET_WORK", 1600000000u, 1000, 4000000000u);
-  BatchTuner tuner{plain ? 1u : std::min<uint32_t>(tune_cap, 64u), tune_cap, tune_target};
+  BatchTuner tuner{plain ? 1u : std::min(tune_cap, BatchTuner::first(n)), tune_cap, tune_target};
   if (opts->hub_batch) tuner.B = std::min(opts->hub_batch, Bmax);
   uint64_t batches = 0, redos = 0;
   const uint64_t t_loop = now_ns();  // set-up (buffers, lists) ends here
