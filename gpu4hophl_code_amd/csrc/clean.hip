@@ -14,10 +14,10 @@
 //     never larger: when it removes nothing from L(v), the sequential walk
 //     keeps every label of v as well.  Pass 1 has no order dependence: it
 //     tests the pairs of L(v)'s labels densely against a distance bound and
-//     looks L(u) up for the few that pass it; long lists take k_clean_tile.
-//  2. k_clean_seq: vertices where pass 1 would remove something are walked
-//     group by group in order with keep bits in LDS, exactly as the
-//     reference does.
+//     looks L(u) up for the few that pass it; long lists, and few of them, take
+//     k_clean_tile.
+//  2. k_clean_seq: of vertices where pass 1 would remove something, the labels
+//     are decided in rounds that reach exactly what the sequential walk does.
 // A K-round, rank-ordered generation already satisfies the predicate (its
 // acceptance test is the all-earlier test over the same final lists), so on
 // this engine's own output pass 1 removes nothing and pass 2 never runs; the
@@ -36,9 +36,10 @@
 
 namespace hsdl {
 
-constexpr uint32_t kCleanWaves = 4;            // waves per workgroup (pass 2)
-constexpr uint32_t kSeqBitsPerWave = 65536;    // max labels per vertex (pass 2)
-constexpr uint32_t kSeqWordsPerWave = kSeqBitsPerWave / 32;
+constexpr uint32_t kSeqThreads = 512;          // pass 2: eight waves per vertex
+constexpr uint32_t kSeqBits = 65536;           // labels whose bits its LDS holds
+constexpr uint32_t kSeqWords = kSeqBits / 32;
+constexpr uint32_t kSeqStage = 4096;           // labels it stages in LDS
 constexpr uint32_t kTileThreads = 1024;        // pass 1: sixteen waves per vertex
 constexpr uint32_t kTileWindow = 4;            // labels of L(v) per work unit (default)
 constexpr uint32_t kMaxWindow = 64;            // largest window
@@ -59,12 +60,6 @@ constexpr uint32_t kTileLdsBytes = 78 * 1024 + 16;
 constexpr uint32_t kIdxBits = 12;
 constexpr uint32_t kIdxRows = (1u << kIdxBits) - 1;
 constexpr uint32_t kGroupFast = 4;             // group sizes with the unrolled check
-
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // lower bound of hub w in lab[lo, hi)
 __device__ inline uint32_t lb_hub(const unsigned long long *lab, uint32_t lo, uint32_t hi,
@@ -120,8 +115,10 @@ struct Pair64 {
 };
 
 // m[u * K + x - 1], x = 1..K: least distance of L(u)'s labels of hop <= x and
-// hub < u (m may be null); maxima[0], [1]: the longest list and the largest
-// distance.  A wave per vertex.
+// hub < u (m may be null).  maxima: the longest list and the largest distance, in
+// kMaxLines copies 64 bytes apart (an atomic per wave and value on one line took
+// 80 us of a 4,096-vertex clean).  A wave per vertex.
+constexpr uint32_t kMaxLines = 32, kMaxStride = 16;
 __global__ void __launch_bounds__(256) k_clean_min(uint32_t n, uint32_t K,
                                                    const unsigned long long *off,
                                                    const unsigned long long *lab, uint32_t *m,
@@ -157,13 +154,16 @@ __global__ void __launch_bounds__(256) k_clean_min(uint32_t n, uint32_t K,
     if (lane < K) m[(uint64_t)u * K + lane] = mine;
   }
   md = wave_max_u32(md);
-  // (one atomic per wave that could raise the maxima)
+  __shared__ uint32_t top[2];
+  if (threadIdx.x < 2) top[threadIdx.x] = 0;
+  __syncthreads();
   if (lane == 0) {
-    if (ml > __hip_atomic_load(&maxima[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      atomicMax(&maxima[0], ml);
-    if (md > __hip_atomic_load(&maxima[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      atomicMax(&maxima[1], md);
+    atomicMax(&top[0], ml);
+    atomicMax(&top[1], md);
   }
+  __syncthreads();
+  if (threadIdx.x < 2 && top[threadIdx.x])
+    atomicMax(&maxima[(blockIdx.x % kMaxLines) * kMaxStride + threadIdx.x], top[threadIdx.x]);
 }
 
 // The labels of vertices [v0, v1) in hop order (index order within a hop), from
@@ -418,8 +418,8 @@ k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long lon
     atomicAdd(reinterpret_cast<unsigned long long *>(ctr) + 2, (unsigned long long)streamed);
 }
 
-// ------------------------------------------------- pass 1, long lists
-// Long lists (a mean above kPairMean labels): k_clean_tile, a workgroup of
+// ------------------------------------------- pass 1, long lists or few
+// Long lists (a mean above kPairMean labels) and few: k_clean_tile, a workgroup of
 // sixteen waves per vertex.  It builds a hash tile of L(v) (hub -> per-hop
 // prefix minimum distance; in LDS, or in the workgroup's slice of a global arena
 // for long lists), then the waves take windows of L(v) in turn, find the windows'
@@ -431,7 +431,11 @@ k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long lon
 // (672 labels per list) takes 164 ms that way (1.1 TB past L2) against 64 ms with
 // tiles, 40,001 vertices (531) 7.4 against 6.3 ms, a group of 65,536 (190) 2.5
 // against 3.8 ms, and the 1024 x 1024 grid (66; 8-byte lists) 10.0 against 24.5 ms.
+// Few lists keep the tiles as well: a wave per list leaves most of the chip idle
+// below some 8,192 lists (1,024 lists of 37 labels 175 us against 110, 4,096 of 69
+// 275 against 211 us).
 constexpr uint64_t kPairMean = 256;
+constexpr uint32_t kPairLists = 8192;
 // The heads' lists L(u) are streamed from the index's 8-byte labels, or from
 // a 32-bit copy of them (hub | hop | dist fields) when the fields fit one
 // word: the first pass reads far more list labels than anything else and
@@ -794,149 +798,221 @@ __global__ void k_clean_keep_all(uint32_t n, const unsigned long long *off, uint
 }
 
 // ---------------------------------------------------------------- pass 2
-// The reference's sequential walk for the vertices in `list`.  For a group of
-// hub u the 64 lanes stream L(u); each lane binary-searches its label's hub
-// w < u in the decided prefix of L(v) and folds the kept matches into per-hop
-// minima m[x] (x = h1 + h2).  A wave min-reduction and a prefix-min over x
-// give the best pair for every hop budget; the group's labels are then
-// decided in hop order, adding the pairs through hub u itself.
-// kLong = false: lists of up to kSeqBitsPerWave labels, keep bits in LDS;
-// longer lists are left to the kLong = true launch, whose keep bits live in
-// the wave's slice of `gbits` (gwords words): read and written with
-// agent-scope atomics, so every lane sees lane 0's updates without relying
-// on the vector L1.  A hub group of more than 32 labels (impossible with one
-// label per (hub, hop) and K <= 15, which import and generation guarantee)
-// sets bad bit 2 instead of overflowing the group's bit mask.
+// The reference's sequential walk for the vertices in `list`, decided in rounds
+// instead of in order.  A label is kept when no pair with earlier labels that may
+// still be kept removes it, and falls when a pair with one that is known to be
+// kept does; either is what the walk decides, whose kept set lies between the
+// two.  The first label left open by a round has only decided ones before it, so
+// a round decides at least that one; nearly all are decided by the first two.
+// A workgroup of eight waves per vertex: the waves take windows of L(v) in
+// turn, and for a group of hub u (with an open label) the 64 lanes stream L(u);
+// each lane searches its label's hub w < u in L(v) and folds the pairs into
+// per-hop minima m[x] (x = h1 + h2), one set over the labels that may be kept and
+// one over those that are.  A wave min-reduction and a prefix-min over x give the
+// best pair for every hop budget; the group's labels are then decided in hop
+// order, adding the pairs through hub u itself.
+// What binds is the searches' latency: eight waves with a list in 48 KB of LDS, three
+// workgroups per CU.  Walking a list in order, a wave per list, took its groups'
+// chains of round trips one after the other: 3,001 vertices with redundant labels
+// 2.03 ms, most of it the longest lists', against 0.74 ms (sixteen waves, one
+// workgroup per CU: 1.14; lists dealt out instead of claimed: 0.90).
+// kLong = false: lists of up to kSeqBits labels, their kept and fallen bits in
+// LDS (and the list itself up to kSeqStage labels); longer lists are left to the
+// kLong = true launch, whose bits live in the workgroup's slice of `gbits` (2 *
+// gwords words): read and written with agent-scope atomics, so every wave sees the
+// others' updates without relying on the vector L1.  A hub group of more than 32
+// labels (impossible with one label per (hub, hop) and K <= 15, which import and
+// generation guarantee) sets bad bit 2 instead of overflowing the group's mask.
 template <bool kLong>
-__global__ void __launch_bounds__(256) k_clean_seq(uint32_t K, const unsigned long long *off,
-                                                   const unsigned long long *lab, uint8_t *keep,
-                                                   uint32_t *new_len, const uint32_t *list,
-                                                   const uint32_t *list_cnt, uint32_t *bad,
-                                                   uint32_t *gbits, uint32_t gwords) {
-  __shared__ uint32_t bits_all[kLong ? 1 : kCleanWaves * kSeqWordsPerWave];
-  const int lane = lane_id();
-  const uint32_t wv = threadIdx.x / kWave;
-  const uint32_t K1 = K + 1;
-  const uint32_t wave = blockIdx.x * kCleanWaves + wv;
-  const uint32_t nwaves = gridDim.x * kCleanWaves;
-  uint32_t *const gb_slice = kLong ? gbits + (uint64_t)wave * gwords : nullptr;
-  auto bit_word = [&](uint32_t i) -> uint32_t {
+__global__ void __launch_bounds__(kSeqThreads) k_clean_seq(
+    uint32_t K, const unsigned long long *off, const unsigned long long *lab, uint8_t *keep,
+    uint32_t *new_len, const uint32_t *list, const uint32_t *list_cnt, uint32_t *next_list,
+    uint32_t *bad, uint32_t *gbits, uint32_t gwords) {
+  __shared__ unsigned long long stage[kLong ? 1 : kSeqStage];
+  __shared__ uint32_t bits[kLong ? 1 : 2 * kSeqWords];  // kept, then fallen
+  __shared__ uint32_t sh_next, sh_open, sh_bad, sh_kept, sh_list;
+  const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id();
+  const uint32_t words_max = kLong ? gwords : kSeqWords;
+  uint32_t *const slice = kLong ? gbits + (uint64_t)blockIdx.x * 2 * gwords : bits;
+  // 32 bits of a set from position i on (fallen: set 1)
+  auto word = [&](uint32_t set, uint32_t i) -> uint32_t {
+    uint32_t *w = slice + set * words_max + i;
     if constexpr (kLong)
-      return __hip_atomic_load(gb_slice + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else
-      return bits_all[wv * kSeqWordsPerWave + i];
+      return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
-  auto bits_sync = [&]() {
-    if constexpr (kLong) {
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
-      __builtin_amdgcn_wave_barrier();
-    } else {
-      wave_lds_sync();
-    }
+  auto bit = [&](uint32_t set, uint32_t i) { return (word(set, i >> 5) >> (i & 31)) & 1u; };
+  auto put = [&](uint32_t set, uint32_t i) {
+    atomicOr(slice + set * words_max + (i >> 5), 1u << (i & 31));
   };
   const uint32_t cnt = *list_cnt;
-  for (uint32_t li = wave; li < cnt; li += nwaves) {
+  // a workgroup's first list is its own id, later ones come from a counter
+  auto claim = [&]() {
+    __syncthreads();  // the shared state is the next list's
+    if (tid == 0) sh_list = gridDim.x + atomicAdd(next_list, 1u);
+    __syncthreads();
+    return sh_list;
+  };
+  for (uint32_t li = blockIdx.x; li < cnt; li = claim()) {
     const uint32_t v = list[li];
     const unsigned long long vb = off[v];
     const uint32_t len = (uint32_t)(off[v + 1] - vb);
     const unsigned long long *Lv = lab + vb;
-    if (kLong ? (len <= kSeqBitsPerWave) : (len > kSeqBitsPerWave)) continue;  // the other launch's
-    if (kLong && (len + 31) / 32 > gwords) {
-      if (lane == 0) atomicOr(bad, 1u);
+    if (kLong ? (len <= kSeqBits) : (len > kSeqBits)) continue;  // the other launch's
+    const uint32_t words = (len + 31) / 32;
+    if (kLong && words > gwords) {
+      if (tid == 0) atomicOr(bad, 1u);
       continue;
     }
-    for (uint32_t i = lane; i < (len + 31) / 32; i += kWave) {
+    for (uint32_t i = tid; i < 2 * words; i += kSeqThreads) {
+      uint32_t *w = slice + (i < words ? i : words_max + i - words);
       if constexpr (kLong)
-        __hip_atomic_store(gb_slice + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       else
-        bits_all[wv * kSeqWordsPerWave + i] = 0;
+        *w = 0;
     }
-    bits_sync();
-    uint32_t kept_total = 0;
-    uint32_t gb = 0;
-    while (gb < len) {
-      const uint32_t u = label_hub(Lv[gb]);
-      uint32_t ge = gb + 1;
-      while (ge < len && label_hub(Lv[ge]) == u) ++ge;  // <= K+1 labels
-      if (ge - gb > 32) {  // see above: cannot happen on valid input
-        if (lane == 0) atomicOr(bad, 2u);
-        break;
-      }
-      uint32_t m[kMaxK + 1];
+    const bool staged = !kLong && len <= kSeqStage;
+    if (staged)
+      for (uint32_t i = tid; i < len; i += kSeqThreads) stage[i] = Lv[i];
+    const lds_ptr<const unsigned long long> Sv = (lds_ptr<const unsigned long long>)stage;
+    auto at = [&](uint32_t i) -> unsigned long long {
+      if (staged) return Sv[i];
+      return Lv[i];
+    };
+    if (tid == 0) sh_next = sh_open = sh_bad = sh_kept = 0;
+    __syncthreads();
+    for (;;) {
+      for (;;) {
+        uint32_t p0 = 0;
+        if (lane == 0) p0 = atomicAdd(&sh_next, kTileWindow);
+        p0 = __builtin_amdgcn_readfirstlane(p0);
+        if (p0 >= len) break;
+        for (uint32_t gb = p0; gb < min(len, p0 + kTileWindow); ++gb) {
+          const uint32_t u = __builtin_amdgcn_readfirstlane(label_hub(at(gb)));
+          if (gb > 0 && label_hub(at(gb - 1)) == u) continue;  // not a group's head
+          // the group [gb, ge) of at most K + 1 labels, the most its labels allow,
+          // and what is decided of it
+          uint32_t ge = gb, maxd = 0, maxh = 0, kept = 0, fell = 0;
+          while (ge < len && ge - gb <= 32 && label_hub(at(ge)) == u) {
+            if (ge - gb < 32) {
+              kept |= bit(0, ge) << (ge - gb);
+              fell |= bit(1, ge) << (ge - gb);
+            }
+            maxd = max(maxd, label_dist(at(ge)));
+            maxh = max(maxh, label_hop(at(ge)));
+            ++ge;
+          }
+          const uint32_t size = ge - gb;
+          if (size > 32) {  // see above: cannot happen on valid input
+            if (lane == 0) atomicOr(&sh_bad, 2u);
+            continue;
+          }
+          const uint32_t all = size == 32 ? ~0u : (1u << size) - 1u;
+          if ((kept | fell) == all) continue;
+          uint32_t ma[kMaxK + 1], mk[kMaxK + 1];
 #pragma unroll
-      for (uint32_t x = 0; x <= kMaxK; ++x) m[x] = kInf32;
-      const unsigned long long ub = off[u];
-      const uint32_t ulen = (uint32_t)(off[u + 1] - ub);
-      const unsigned long long *Lu = lab + ub;
-      if (gb > 0) {
-        for (uint32_t j = lane; j < ulen; j += kWave) {
-          const unsigned long long l = Lu[j];
-          const uint32_t w = label_hub(l);
-          if (w >= u) continue;
-          const uint32_t h1 = label_hop(l), d1 = label_dist(l);
-          for (uint32_t p = lb_hub(Lv, 0, gb, w); p < gb; ++p) {
-            const unsigned long long q = Lv[p];
-            if (label_hub(q) != w) break;
-            if (!((bit_word(p >> 5) >> (p & 31)) & 1u)) continue;
-            const uint32_t x = h1 + label_hop(q);
-            if (x <= K) {
-              const uint32_t s = d1 + label_dist(q);
+          for (uint32_t x = 0; x <= kMaxK; ++x) ma[x] = mk[x] = kInf32;
+          const unsigned long long ub = off[u];
+          const uint32_t ulen = (uint32_t)(off[u + 1] - ub);
+          const unsigned long long *Lu = lab + ub;
+          for (uint32_t j = lane; gb > 0 && j < ulen; j += kWave) {
+            const unsigned long long l = Lu[j];
+            const uint32_t w = label_hub(l), h1 = label_hop(l), d1 = label_dist(l);
+            if (w >= u || h1 > maxh || d1 > maxd) continue;
+            uint32_t p = 0, hi = gb;
+            while (p < hi) {
+              const uint32_t mid = (p + hi) >> 1;
+              if (label_hub(at(mid)) < w) p = mid + 1; else hi = mid;
+            }
+            for (; p < gb; ++p) {
+              const unsigned long long q = at(p);
+              if (label_hub(q) != w) break;
+              const uint32_t x = h1 + label_hop(q), sum = d1 + label_dist(q);
+              if (x > maxh || sum > maxd || bit(1, p)) continue;
+              const bool sure = bit(0, p);
 #pragma unroll
-              for (uint32_t xx = 0; xx <= kMaxK; ++xx)
-                if (xx == x) m[xx] = min(m[xx], s);
+              for (uint32_t y = 0; y <= kMaxK; ++y)
+                if (y == x) {
+                  ma[y] = min(ma[y], sum);
+                  if (sure) mk[y] = min(mk[y], sum);
+                }
             }
           }
+          // L(u)'s own labels (hub u): found by search, since a list may also
+          // hold hubs ranked below its vertex (imported label sets)
+          const uint32_t ub0 = lb_hub(Lu, 0, ulen, u);
+          uint32_t ra = kInf32, rk = kInf32;
+#pragma unroll
+          for (uint32_t x = 0; x <= kMaxK; ++x) {
+            if (x <= K) {
+              ra = min(ra, wave_min_u32(ma[x]));
+              rk = min(rk, wave_min_u32(mk[x]));
+            }
+            ma[x] = ra;
+            mk[x] = rk;
+          }
+          // decide the group's open labels in order (all lanes compute the same)
+          uint32_t nk = 0, nf = 0;
+          for (uint32_t i = 0; i < size; ++i) {
+            if (((kept | fell) >> i) & 1u) continue;
+            const unsigned long long l = at(gb + i);
+            const uint32_t h = label_hop(l), d = label_dist(l);
+            uint32_t best_any = kInf32, best_kept = kInf32;
+#pragma unroll
+            for (uint32_t x = 0; x <= kMaxK; ++x)
+              if (x == h) {
+                best_any = ma[x];
+                best_kept = mk[x];
+              }
+            // pairs through hub u: L(u)'s hub-u labels x earlier labels of this group
+            for (uint32_t k2 = 0; k2 < i; ++k2) {
+              if (((fell | nf) >> k2) & 1u) continue;
+              const bool sure = ((kept | nk) >> k2) & 1u;
+              const unsigned long long q = at(gb + k2);
+              for (uint32_t t = ub0; t < ulen; ++t) {
+                const unsigned long long r = Lu[t];
+                if (label_hub(r) != u) break;
+                if (label_hop(r) + label_hop(q) > h) continue;
+                const uint32_t sum = label_dist(r) + label_dist(q);
+                best_any = min(best_any, sum);
+                if (sure) best_kept = min(best_kept, sum);
+              }
+            }
+            if (best_any > d)
+              nk |= 1u << i;
+            else if (best_kept <= d)
+              nf |= 1u << i;
+          }
+          if (lane < size && ((nk >> lane) & 1u)) put(0, gb + lane);
+          if (lane < size && ((nf >> lane) & 1u)) put(1, gb + lane);
+          if (lane == 0 && (kept | fell | nk | nf) != all) atomicOr(&sh_open, 1u);
         }
       }
-      // L(u)'s own labels (hub u): found by search, since a list may also
-      // hold hubs ranked below its vertex (imported label sets)
-      const uint32_t ub0 = lb_hub(Lu, 0, ulen, u);
-      uint32_t M[kMaxK + 1];
-      uint32_t run = kInf32;
-#pragma unroll
-      for (uint32_t x = 0; x <= kMaxK; ++x) {
-        const uint32_t r = (x < K1) ? wave_min_u32(m[x]) : kInf32;
-        run = min(run, r);
-        M[x] = run;
-      }
-      // decide the group's labels in order (all lanes compute the same)
-      uint32_t newbits = 0;  // relative to gb; groups hold <= 16 labels
-      for (uint32_t i = gb; i < ge; ++i) {
-        const unsigned long long l = Lv[i];
-        const uint32_t h = label_hop(l), d = label_dist(l);
-        uint32_t best = kInf32;
-#pragma unroll
-        for (uint32_t x = 0; x <= kMaxK; ++x)
-          if (x == h) best = M[x];
-        // pairs through hub u: L(u)'s hub-u labels x kept labels of this group
-        for (uint32_t k2 = gb; k2 < i; ++k2) {
-          if (!((newbits >> (k2 - gb)) & 1u)) continue;
-          const unsigned long long q = Lv[k2];
-          const uint32_t h2 = label_hop(q), d2 = label_dist(q);
-          for (uint32_t t = ub0; t < ulen; ++t) {
-            const unsigned long long r = Lu[t];
-            if (label_hub(r) != u) break;
-            if (label_hop(r) + h2 <= h) best = min(best, label_dist(r) + d2);
-          }
-        }
-        if (best > d) newbits |= 1u << (i - gb);
-      }
-      if (lane == 0) {
-        for (uint32_t i = gb; i < ge; ++i)
-          if ((newbits >> (i - gb)) & 1u) {
-            if constexpr (kLong)
-              atomicOr(gb_slice + (i >> 5), 1u << (i & 31));
-            else
-              atomicOr(&bits_all[wv * kSeqWordsPerWave + (i >> 5)], 1u << (i & 31));
-          }
-      }
-      kept_total += __popc(newbits);
-      bits_sync();
-      gb = ge;
+      __syncthreads();
+      const bool again = sh_open && !sh_bad;
+      __syncthreads();
+      if (!again) break;
+      // (reset behind the loop's test and ahead of a barrier: at the head of the
+      // loop this condition met the one before it, and the compiler sent the other
+      // lanes of the wave through the barrier without lane 0)
+      if (tid == 0) sh_next = sh_open = 0;
+      __syncthreads();
     }
-    for (uint32_t i = lane; i < len; i += kWave) keep[vb + i] = (bit_word(i >> 5) >> (i & 31)) & 1u;
-    if (lane == 0) new_len[v] = kept_total;
-    bits_sync();
+    if (sh_bad) {
+      if (tid == 0) atomicOr(bad, sh_bad);
+    } else {
+      uint32_t k = 0;
+      for (uint32_t i = tid; i < len; i += kSeqThreads) {
+        const uint32_t one = bit(0, i);
+        keep[vb + i] = (uint8_t)one;
+        k += one;
+      }
+      k = wave_sum_u32(k);
+      if (lane == 0 && k) atomicAdd(&sh_kept, k);
+      __syncthreads();
+      if (tid == 0) new_len[v] = sh_kept;
+    }
   }
 }
 
@@ -1042,10 +1118,11 @@ int clean_index(hsdl_index *idx) {
          {kCsKeep, kCsNewLen, kCsRedo, kCsSrt, kCsHcnt, kCsMins, kCsLongs, kCsCtr, kCsGtile}};
   if ((rc = take_scratch(dev, kCsRedo, redo, n * 4ull + 4)) ||
       (rc = take_scratch(dev, kCsHcnt, hcnt, (uint64_t)n * idx->K * 4)) ||
-      (rc = take_scratch(dev, kCsCtr, ctr, 64)))
+      (rc = take_scratch(dev, kCsCtr, ctr, (1 + kMaxLines) * kMaxStride * 4)))
     return rc;
-  uint32_t *cnt = ctr.as<uint32_t>();  // see k_clean_pairs; [3]: pass 2's error bits; [8], [9]: maxima
-  HSDL_HIP(hipMemsetAsync(cnt, 0, 64, st));
+  // counters (k_clean_pairs; [3]: pass 2's error bits, [6], [7]: its lists), then the maxima's lines
+  uint32_t *cnt = ctr.as<uint32_t>();
+  HSDL_HIP(hipMemsetAsync(cnt, 0, (1 + kMaxLines) * kMaxStride * 4, st));
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, idx->device);
   const int grid = std::max(1, cus * 8);
@@ -1056,16 +1133,18 @@ int clean_index(hsdl_index *idx) {
   // order, no hop-ordered copy)
   const bool hop_sort = env_u32("HSDL_CLEAN_HOP_SORT", 1, 0, 1);
   const uint32_t form = hop_sort ? env_u32("HSDL_CLEAN_PAIRS", 1, 0, 2) : 0u;
-  const bool pairs = form == 2 || (form == 1 && idx->total <= kPairMean * n);
+  const bool pairs = form == 2 || (form == 1 && n >= kPairLists && idx->total <= kPairMean * n);
   if (pairs && ((rc = take_scratch(dev, kCsLongs, longs, n * 4ull + 4)) ||
                 (rc = take_scratch(dev, kCsMins, mins, (uint64_t)n * idx->K * 4))))
     return rc;
   hipLaunchKernelGGL(k_clean_min, dim3(grid), dim3(256), 0, st, n, (uint32_t)idx->K, off, lab,
-                     pairs ? mins.as<uint32_t>() : nullptr, cnt + 8);
+                     pairs ? mins.as<uint32_t>() : nullptr, cnt + kMaxStride);
   HSDL_HIP(hipGetLastError());
-  uint32_t mx[2] = {0, 0};
-  HSDL_HIP(hipMemcpyAsync(mx, cnt + 8, 8, hipMemcpyDeviceToHost, st));
+  uint32_t lines[kMaxLines * kMaxStride], mx[2] = {0, 0};
+  HSDL_HIP(hipMemcpyAsync(lines, cnt + kMaxStride, sizeof(lines), hipMemcpyDeviceToHost, st));
   HSDL_HIP(hipStreamSynchronize(st));
+  for (uint32_t x = 0; x < kMaxLines; ++x)
+    for (int y = 0; y < 2; ++y) mx[y] = std::max(mx[y], lines[x * kMaxStride + y]);
   // 32-bit copies of the labels when hub, hop and distance fit one word
   // (tuning knob HSDL_STREAM32=0: 8-byte ones)
   uint32_t hub_bits = 1, hop_bits = 1, dist_bits = 1;
@@ -1189,20 +1268,21 @@ int clean_index(hsdl_index *idx) {
     hipLaunchKernelGGL(k_clean_keep_all, dim3(grid), dim3(256), 0, st, n, off,
                        new_len.as<uint32_t>());
     HSDL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_clean_seq<false>, dim3(grid), dim3(kCleanWaves * kWave), 0, st,
+    hipLaunchKernelGGL(k_clean_seq<false>, dim3(cus * 3), dim3(kSeqThreads), 0, st,
                        (uint32_t)idx->K, off, lab, keep.as<uint8_t>(), new_len.as<uint32_t>(),
-                       redo.as<uint32_t>(), cnt, cnt + 3, nullptr, 0u);
+                       redo.as<uint32_t>(), cnt, cnt + 6, cnt + 3, nullptr, 0u);
     HSDL_HIP(hipGetLastError());
     DevBuf long_bits;
-    if (mx[0] > kSeqBitsPerWave) {
-      // vertices with more labels than an LDS bit set holds: keep bits in a
-      // global slice per wave (few waves: such vertices are rare)
+    if (mx[0] > kSeqBits) {
+      // vertices with more labels than an LDS bit set holds: bits in a global
+      // slice per workgroup (few workgroups: such vertices are rare)
       const uint32_t lgrid = 64;
       const uint32_t words = (mx[0] + 31) / 32;
-      if ((rc = long_bits.alloc((uint64_t)lgrid * kCleanWaves * words * 4))) return rc;
-      hipLaunchKernelGGL(k_clean_seq<true>, dim3(lgrid), dim3(kCleanWaves * kWave), 0, st,
+      if ((rc = long_bits.alloc((uint64_t)lgrid * 2 * words * 4))) return rc;
+      hipLaunchKernelGGL(k_clean_seq<true>, dim3(lgrid), dim3(kSeqThreads), 0, st,
                          (uint32_t)idx->K, off, lab, keep.as<uint8_t>(), new_len.as<uint32_t>(),
-                         redo.as<uint32_t>(), cnt, cnt + 3, long_bits.as<uint32_t>(), words);
+                         redo.as<uint32_t>(), cnt, cnt + 7, cnt + 3, long_bits.as<uint32_t>(),
+                         words);
       HSDL_HIP(hipGetLastError());
     }
     uint32_t bad = 0;

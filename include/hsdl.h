@@ -218,7 +218,7 @@ typedef struct hsdl_stats {
   uint64_t prune_launches;
   uint64_t prune_label_reads;       /* labels of L(y) streamed by the prune */
   uint64_t prune_tile_reads;        /* labels of L(s) staged into tiles     */
-  uint64_t clean_seq_vertices;      /* vertices the clean walked in order   */
+  uint64_t clean_seq_vertices;      /* vertices with labels that may fall   */
   uint64_t clean_label_reads;       /* labels read by the clean's first pass:
                                        of the heads' lists L(u), or of L(v)
                                        walked (64 pairs each) where it tests

@@ -293,3 +293,29 @@ def test_clean_forms(monkeypatch, pairs, stream32, piece):
     off = np.concatenate([[0], np.cumsum([len(x) for x in lists])])
     hub, hop, dist = np.array([e for x in lists for e in x]).T
     check("long", 3, off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32))
+
+
+@pytest.mark.parametrize("n,K,top", [(40, 2, 3), (130, 3, 4), (130, 3, 12), (90, 15, 6)])
+def test_clean_decides_chains_in_rounds(n, K, top):
+    """Lists over all hubs with random hops and small distances: most labels
+    fall, many through labels that fall themselves, so a round of the clean's
+    second pass leaves labels open for the next: the oracle's clean, and a clean
+    of the result changes nothing that the oracle's does not."""
+    rng = np.random.default_rng(n + K + top)
+    offs, rows = [0], []
+    for v in range(n):
+        for u in range(v):
+            for h in sorted(set(rng.integers(1, K + 1, 2).tolist())):
+                rows.append((u, h, int(rng.integers(1, top)) + (K - h) * (top > 8)))
+        rows.append((v, 0, 0))
+        offs.append(len(rows))
+    hub, hop, dist = np.array(rows).T
+    off = np.array(offs, np.uint64)
+    arrays = (off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32))
+    for turn in range(2):
+        print(f"[rounds] n={n} K={K} top={top} turn={turn} labels={len(arrays[1])}", flush=True)
+        want = O.clean(O.labels_from_arrays(n, np.asarray(arrays[0]).astype(np.int64), *arrays[1:]))
+        idx = H.Index.from_labels(n, K, *arrays)
+        idx.clean()
+        same_labels(idx, want.arrays())
+        arrays = idx.labels()
