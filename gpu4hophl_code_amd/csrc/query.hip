@@ -430,93 +430,6 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
   return HSDL_OK;
 }
 
-// ------------------------------------------------------------- staging
-static std::mutex g_stage_mu;
-// (never destroyed: no device call may run while the process ends)
-static std::vector<Stage *> &stage_pool() {
-  static std::vector<Stage *> *pool = new std::vector<Stage *>();
-  return *pool;
-}
-
-Stage::~Stage() {
-  for (int i = 0; i < 2; ++i) {
-    if (st[i]) (void)hipStreamDestroy(st[i]);
-    if (h[i]) (void)hipHostFree(h[i]);
-  }
-}
-
-int StageLease::take(int dev, size_t bytes, int slots, bool device) {
-  {
-    std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    for (size_t i = 0; i < pool.size(); ++i)
-      if (pool[i]->dev == dev) {
-        s_ = pool[i];
-        pool.erase(pool.begin() + i);
-        break;
-      }
-  }
-  if (!s_) {
-    s_ = new Stage();
-    s_->dev = dev;
-  }
-  size_t want = 64u << 10;
-  while (want < bytes) want *= 2;
-  for (int i = 0; i < slots; ++i) {
-    if (!s_->st[i]) HSDL_HIP(hipStreamCreateWithFlags(&s_->st[i], hipStreamNonBlocking));
-    if (s_->hbytes[i] < bytes) {
-      if (s_->h[i]) (void)hipHostFree(s_->h[i]);
-      s_->h[i] = nullptr;
-      s_->hbytes[i] = 0;
-      HSDL_HIP(hipHostMalloc((void **)&s_->h[i], want, hipHostMallocMapped | hipHostMallocCoherent));
-      s_->hbytes[i] = want;
-    }
-    if (device && s_->d[i].bytes < bytes) {
-      const int rc = s_->d[i].alloc(want);
-      if (rc) return rc;
-    }
-  }
-  return HSDL_OK;
-}
-
-StageLease::~StageLease() {
-  if (!s_) return;
-  bool keep = true;
-  for (int i = 0; i < 2; ++i) {
-    // (a call that failed half-way may have work in flight)
-    if (s_->st[i]) (void)hipStreamSynchronize(s_->st[i]);
-    keep = keep && s_->hbytes[i] <= kStageBytes && s_->d[i].bytes <= kStageBytes;
-  }
-  if (keep) {
-    std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    int kept = 0;
-    for (Stage *x : pool) kept += x->dev == s_->dev;
-    if (kept < kStagesKept) {
-      pool.push_back(s_);
-      return;
-    }
-  }
-  delete s_;
-}
-
-void release_stages(int dev) {
-  std::vector<Stage *> gone;
-  {
-    std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    for (size_t i = pool.size(); i-- > 0;)
-      if (dev < 0 || pool[i]->dev == dev) {
-        gone.push_back(pool[i]);
-        pool.erase(pool.begin() + i);
-      }
-  }
-  for (Stage *x : gone) {
-    (void)hipSetDevice(x->dev);
-    delete x;
-  }
-}
-
 }  // namespace hsdl
 
 using namespace hsdl;
