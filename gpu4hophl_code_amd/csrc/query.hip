@@ -74,8 +74,101 @@ struct QChunk {
       : per((uint32_t)min<uint64_t>(kWave, (nq + waves - 1) / waves)) {}
 };
 
-// hcnt[v * K + x], x < K: labels of v of hop <= x.  below: the index holds
-// hubs ranked below their vertex.  slots: table slots per wave, a power of two.
+// The least distance of (s, t, k), k > 0, s != t, over this lane's pairs
+// (kInf32: none).  kTeam: a workgroup's work, its threads in step, else a wave's.
+// hcnt[v * K + x], x < K: labels of v of hop <= x.  below: the index holds hubs
+// ranked below their vertex.  T: a table of `slots`, a power of two.
+template <bool kTeam>
+__device__ inline uint32_t join32(const Lab32 &fmt, uint32_t K,
+                                  const unsigned long long *__restrict__ off,
+                                  const uint32_t *__restrict__ lab,
+                                  const uint32_t *__restrict__ hcnt, uint32_t below, uint32_t s,
+                                  uint32_t t, int k, lds_ptr<uint32_t> T, uint32_t slots) {
+  constexpr uint32_t kN = kTeam ? kQThreads : kWave;
+  const uint32_t id = kTeam ? threadIdx.x : (uint32_t)lane_id();
+  auto sync = [] {
+    if constexpr (kTeam)
+      __syncthreads();
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  uint32_t a = s, b = t;
+  unsigned long long abeg = off[s], bbeg = off[t];
+  uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
+  if (alen > blen) {
+    const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
+    const uint32_t l = alen; alen = blen; blen = l;
+    a = t;
+    b = s;
+  }
+  const uint32_t *A = lab + abeg, *B = lab + bbeg;
+  const uint32_t kk = (uint32_t)k, c = kk >> 1;
+  // labels of v of hop <= x
+  auto upto = [&](uint32_t v, uint32_t len, uint32_t x) {
+    return x < K ? hcnt[(uint64_t)v * K + x] : len;
+  };
+  const uint32_t a0 = upto(a, alen, 0), b0 = upto(b, blen, 0);  // self labels
+  const uint32_t ac = upto(a, alen, c), bc = upto(b, blen, kk - 1 - c);
+  const uint32_t a1 = upto(a, alen, kk - 1), b1 = upto(b, blen, kk - 1);
+  const uint32_t ak = upto(a, alen, kk), bk = upto(b, blen, kk);
+  uint32_t best = kInf32;       // pairs of hops >= 1
+  uint32_t at_a = kInf32, at_b = kInf32;  // labels of hub a in L(b), of b in L(a)
+
+  // Labels [beg, end) of L, four steps' loads at a time; use(l, own) sees every
+  // label (a lane past the end a copy of the last one, own = false).
+  auto walk = [&](const uint32_t *L, uint32_t beg, uint32_t end, auto &&use) {
+    for (uint32_t j = beg; j < end; j += 4 * kN) {
+      uint32_t l[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) l[u] = L[min(j + u * kN + id, end - 1)];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (j + u * kN < end) use(l[u], j + u * kN + id < end);
+    }
+  };
+  auto endpoint = [&](uint32_t l, uint32_t other, uint32_t &at) {
+    if (fmt.hub(l) == other) at = min(at, fmt.dist(l));
+  };
+  // hashes X[xb, xe), probes with Y[yb, ye)
+  auto join = [&](const uint32_t *X, uint32_t xb, uint32_t xe, const uint32_t *Y, uint32_t yb,
+                  uint32_t ye) {
+    while (xb < xe && yb < ye) {
+      // at most half the table; a quarter where it has room
+      const uint32_t part = min(xe - xb, slots / 2);
+      const uint32_t cap =
+          min(slots, 1u << (32 - __builtin_clz(max(64u, 4u * part) - 1)));
+      for (uint32_t i = id; i < cap * 4 / 16; i += kN) ((lds_ptr<u32x4>)T)[i] = u32x4{0, 0, 0, 0};
+      sync();
+      walk(X, xb, xb + part, [&](uint32_t l, bool own) {
+        if (!own) return;
+        uint32_t slot = hash_slot(fmt.hub(l), cap);
+        while (atomicCAS((uint32_t *)&T[slot], 0u, l) != 0u) slot = (slot + 1) & (cap - 1);
+      });
+      sync();
+      walk(Y, yb, ye, [&](uint32_t l, bool) {
+        const uint32_t w = fmt.hub(l), h = fmt.hop(l), d = fmt.dist(l);
+        uint32_t slot = hash_slot(w, cap);
+        uint32_t x = T[slot];
+        while (x != 0) {
+          if (fmt.hub(x) == w && fmt.hop(x) + h <= kk) best = min(best, d + fmt.dist(x));
+          slot = (slot + 1) & (cap - 1);
+          x = T[slot];
+        }
+      });
+      sync();
+      xb += part;
+    }
+  };
+  if (below || b > a) walk(B, b0, bk, [&](uint32_t l, bool) { endpoint(l, a, at_a); });
+  if (below || a > b) walk(A, a0, ak, [&](uint32_t l, bool) { endpoint(l, b, at_b); });
+  join(A, a0, ac, B, b0, b1);
+  join(B, b0, bc, A, ac, a1);
+  if (a0) best = min(best, at_a);
+  if (b0) best = min(best, at_b);
+  return best;
+}
+
+// A wave per query.  slots: table slots per wave.
 __global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
           const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt, uint32_t below,
@@ -99,96 +192,124 @@ k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restric
     for (unsigned long long todo = __ballot(vk > 0 && vs < n && vt < n && vs != vt); todo;
          todo &= todo - 1) {
       const int qi = __ffsll((long long)todo) - 1;
-      const uint32_t s = __builtin_amdgcn_readlane(vs, qi), t = __builtin_amdgcn_readlane(vt, qi);
-      const int k = __builtin_amdgcn_readlane(vk, qi);
-      uint32_t a = s, b = t;
-      unsigned long long abeg = off[s], bbeg = off[t];
-      uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
-      if (alen > blen) {
-        const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
-        const uint32_t l = alen; alen = blen; blen = l;
-        a = t;
-        b = s;
-      }
-      const uint32_t *A = lab + abeg, *B = lab + bbeg;
-      const uint32_t kk = (uint32_t)k, c = kk >> 1;
-      // labels of v of hop <= x
-      auto upto = [&](uint32_t v, uint32_t len, uint32_t x) {
-        return x < K ? hcnt[(uint64_t)v * K + x] : len;
-      };
-      const uint32_t a0 = upto(a, alen, 0), b0 = upto(b, blen, 0);  // self labels
-      const uint32_t ac = upto(a, alen, c), bc = upto(b, blen, kk - 1 - c);
-      const uint32_t a1 = upto(a, alen, kk - 1), b1 = upto(b, blen, kk - 1);
-      const uint32_t ak = upto(a, alen, kk), bk = upto(b, blen, kk);
-      uint32_t best = kInf32;       // pairs of hops >= 1
-      uint32_t at_a = kInf32, at_b = kInf32;  // labels of hub a in L(b), of b in L(a)
-
-      // Labels [beg, end) of L, four steps' loads at a time; use(l) sees every
-      // label (a lane past the end a copy of the last one).
-      auto walk = [&](const uint32_t *L, uint32_t beg, uint32_t end, auto &&use) {
-        for (uint32_t j = beg; j < end; j += 4 * kWave) {
-          uint32_t l[4];
-#pragma unroll
-          for (uint32_t u = 0; u < 4; ++u) l[u] = L[min(j + u * kWave + lane, end - 1)];
-#pragma unroll
-          for (uint32_t u = 0; u < 4; ++u)
-            if (j + u * kWave < end) use(l[u]);
-        }
-      };
-      auto endpoint = [&](uint32_t l, uint32_t other, uint32_t &at) {
-        if (fmt.hub(l) == other) at = min(at, fmt.dist(l));
-      };
-      // hashes X[xb, xe), probes with Y[yb, ye)
-      auto join = [&](const uint32_t *X, uint32_t xb, uint32_t xe, const uint32_t *Y, uint32_t yb,
-                      uint32_t ye) {
-        while (xb < xe && yb < ye) {
-          // at most half the table; a quarter where it has room
-          const uint32_t part = min(xe - xb, slots / 2);
-          const uint32_t cap =
-              min(slots, 1u << (32 - __builtin_clz(max(64u, 4u * part) - 1)));
-          for (uint32_t i = lane; i < cap * 4 / 16; i += kWave)
-            ((lds_ptr<u32x4>)T)[i] = u32x4{0, 0, 0, 0};
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          for (uint32_t j = xb; j < xb + part; j += kWave) {
-            const uint32_t l = X[min(j + lane, xb + part - 1)];
-            if (j + lane < xb + part) {
-              uint32_t slot = hash_slot(fmt.hub(l), cap);
-              while (atomicCAS((uint32_t *)&T[slot], 0u, l) != 0u) slot = (slot + 1) & (cap - 1);
-            }
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          walk(Y, yb, ye, [&](uint32_t l) {
-            const uint32_t w = fmt.hub(l), h = fmt.hop(l), d = fmt.dist(l);
-            uint32_t slot = hash_slot(w, cap);
-            uint32_t x = T[slot];
-            while (x != 0) {
-              if (fmt.hub(x) == w && fmt.hop(x) + h <= kk) best = min(best, d + fmt.dist(x));
-              slot = (slot + 1) & (cap - 1);
-              x = T[slot];
-            }
-          });
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          xb += part;
-        }
-      };
-      if (below || b > a) walk(B, b0, bk, [&](uint32_t l) { endpoint(l, a, at_a); });
-      if (below || a > b) walk(A, a0, ak, [&](uint32_t l) { endpoint(l, b, at_b); });
-      join(A, a0, ac, B, b0, b1);
-      join(B, b0, bc, A, ac, a1);
-      if (a0) best = min(best, at_a);
-      if (b0) best = min(best, at_b);
-      best = wave_min_u32(best);
+      const uint32_t best = wave_min_u32(
+          join32<false>(fmt, K, off, lab, hcnt, below, __builtin_amdgcn_readlane(vs, qi),
+                        __builtin_amdgcn_readlane(vt, qi), __builtin_amdgcn_readlane(vk, qi), T,
+                        slots));
       if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
     }
     if (mine) out[q0 + lane] = ans;
   }
 }
 
+// A workgroup per query, for calls of few queries (use_team): the longest lists'
+// queries decide when such a call ends, and its waves would idle beside them.
+// join(s, t, k) is called by all threads of the workgroup.
+template <class J>
+__device__ inline void team_queries(uint32_t n, uint64_t nq, const uint32_t *__restrict__ qs,
+                                    const uint32_t *__restrict__ qt,
+                                    const int8_t *__restrict__ qk, int32_t *out, J &&join) {
+  __shared__ uint32_t least[kQWaves];
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  for (uint64_t q = blockIdx.x; q < nq; q += gridDim.x) {
+    const uint32_t s = __builtin_amdgcn_readfirstlane(qs[q]);
+    const uint32_t t = __builtin_amdgcn_readfirstlane(qt[q]);
+    const int k = __builtin_amdgcn_readfirstlane((int)qk[q]);
+    uint32_t best = kInf32;
+    if (k > 0 && s < n && t < n && s != t)  // the same for every thread
+      best = wave_min_u32(join(s, t, k));
+    if (lane_id() == 0) least[wib] = best;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w < kQWaves; ++w) best = min(best, least[w]);
+    if (threadIdx.x == 0)
+      out[q] = k >= 0 && s == t && s < n ? 0 : best == kInf32 ? INT32_MAX : (int32_t)best;
+    __syncthreads();  // `least` and the join's LDS are the next query's
+  }
+}
+
+// slots: table slots of the workgroup.
+__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_query32_team(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
+               const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt,
+               uint32_t below, uint64_t nq, const uint32_t *__restrict__ qs,
+               const uint32_t *__restrict__ qt, const int8_t *__restrict__ qk, int32_t *out,
+               uint32_t slots) {
+  extern __shared__ uint4 qlds[];
+  team_queries(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
+    return join32<true>(fmt, K, off, lab, hcnt, below, s, t, k,
+                        (lds_ptr<uint32_t>)reinterpret_cast<uint32_t *>(qlds), slots);
+  });
+}
+
 // 8-byte labels: pieces of the longer list B in LDS, searched by the shorter
 // list A's labels.  Both are hub-sorted, so a chunk of A whose hubs lie below
 // the piece is never read again; a run of B cut by a piece's end is found in
 // both pieces.
+// kTeam: a workgroup's work (pieces of four times the size, the waves taking
+// chunks of A in turn), else a wave's.  Returns the least distance of (s, t, k),
+// k > 0, s != t, over this lane's pairs.
 constexpr uint32_t kQPiece = 512;  // labels, 4 KB per wave
+template <bool kTeam>
+__device__ inline uint32_t join64(const unsigned long long *__restrict__ off,
+                                  const unsigned long long *__restrict__ lab, uint32_t s,
+                                  uint32_t t, uint32_t kk, lds_ptr<unsigned long long> P) {
+  constexpr uint32_t kN = kTeam ? kQThreads : kWave, kPiece = kTeam ? kQWaves * kQPiece : kQPiece;
+  const uint32_t lane = (uint32_t)lane_id(), id = kTeam ? threadIdx.x : lane;
+  auto sync = [] {
+    if constexpr (kTeam)
+      __syncthreads();
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  unsigned long long abeg = off[s], bbeg = off[t];
+  uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
+  if (alen > blen) {
+    const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
+    const uint32_t l = alen; alen = blen; blen = l;
+  }
+  const unsigned long long *A = lab + abeg, *B = lab + bbeg;
+  uint32_t best = kInf32;
+  // this wave's chunks of A below j0 are done
+  uint32_t j0 = kTeam ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * kWave : 0u;
+  for (uint32_t p0 = 0; p0 < blen && (kTeam || j0 < alen); p0 += kPiece) {
+    const uint32_t m = min(kPiece, blen - p0);
+    for (uint32_t i = id; i < m; i += 4 * kN) {
+      unsigned long long l[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) l[u] = B[p0 + min(i + u * kN, m - 1)];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (i + u * kN < m) P[i + u * kN] = l[u];
+    }
+    sync();
+    const uint32_t lo_hub = label_hub(P[0]), hi_hub = label_hub(P[m - 1]);
+    for (uint32_t j = j0; j < alen; j += kN) {
+      const unsigned long long a = A[min(j + lane, alen - 1)];
+      const uint32_t w = label_hub(a), h1 = label_hop(a);
+      if (__builtin_amdgcn_readlane(w, 0) > hi_hub) break;
+      if (__builtin_amdgcn_readlane(w, kWave - 1) < lo_hub) {
+        j0 = j + kN;
+        continue;
+      }
+      if (w < lo_hub || w > hi_hub || h1 > kk) continue;
+      // first label of the piece with hub >= w (there is one)
+      uint32_t lo = 0, hi = m - 1;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
+      }
+      for (uint32_t x = lo; x < m; ++x) {  // <= K + 1 labels, hops ascending
+        const unsigned long long l = P[x];
+        if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
+        best = min(best, label_dist(a) + label_dist(l));
+      }
+    }
+    sync();
+  }
+  return best;
+}
+
 __global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_query64(uint32_t n, const unsigned long long *__restrict__ off,
           const unsigned long long *__restrict__ lab, uint64_t nq,
@@ -197,7 +318,6 @@ k_query64(uint32_t n, const unsigned long long *__restrict__ off,
   __shared__ unsigned long long stage[kQWaves][kQPiece];
   const uint32_t lane = (uint32_t)lane_id();
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  lds_ptr<unsigned long long> P = (lds_ptr<unsigned long long>)stage[wib];
   const uint64_t waves = (uint64_t)gridDim.x * kQWaves;
   const QChunk ch(nq, waves);
   for (uint64_t q0 = ((uint64_t)blockIdx.x * kQWaves + wib) * ch.per; q0 < nq;
@@ -212,58 +332,24 @@ k_query64(uint32_t n, const unsigned long long *__restrict__ off,
     for (unsigned long long todo = __ballot(vk > 0 && vs < n && vt < n && vs != vt); todo;
          todo &= todo - 1) {
       const int qi = __ffsll((long long)todo) - 1;
-      const uint32_t s = __builtin_amdgcn_readlane(vs, qi), t = __builtin_amdgcn_readlane(vt, qi);
-      const int k = __builtin_amdgcn_readlane(vk, qi);
-      const uint32_t kk = (uint32_t)k;
-      unsigned long long abeg = off[s], bbeg = off[t];
-      uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
-      if (alen > blen) {
-        const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
-        const uint32_t l = alen; alen = blen; blen = l;
-      }
-      const unsigned long long *A = lab + abeg, *B = lab + bbeg;
-      uint32_t best = kInf32;
-      uint32_t j0 = 0;  // chunks of A below this one are done
-      for (uint32_t p0 = 0; p0 < blen && j0 < alen; p0 += kQPiece) {
-        const uint32_t m = min(kQPiece, blen - p0);
-        for (uint32_t i = lane; i < m; i += 4 * kWave) {
-          unsigned long long l[4];
-#pragma unroll
-          for (uint32_t u = 0; u < 4; ++u) l[u] = B[p0 + min(i + u * kWave, m - 1)];
-#pragma unroll
-          for (uint32_t u = 0; u < 4; ++u)
-            if (i + u * kWave < m) P[i + u * kWave] = l[u];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const uint32_t lo_hub = label_hub(P[0]), hi_hub = label_hub(P[m - 1]);
-        for (uint32_t j = j0; j < alen; j += kWave) {
-          const unsigned long long a = A[min(j + lane, alen - 1)];
-          const uint32_t w = label_hub(a), h1 = label_hop(a);
-          if (__builtin_amdgcn_readlane(w, 0) > hi_hub) break;
-          if (__builtin_amdgcn_readlane(w, kWave - 1) < lo_hub) {
-            j0 = j + kWave;
-            continue;
-          }
-          if (w < lo_hub || w > hi_hub || h1 > kk) continue;
-          // first label of the piece with hub >= w (there is one)
-          uint32_t lo = 0, hi = m - 1;
-          while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
-          }
-          for (uint32_t x = lo; x < m; ++x) {  // <= K + 1 labels, hops ascending
-            const unsigned long long l = P[x];
-            if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
-            best = min(best, label_dist(a) + label_dist(l));
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      }
-      best = wave_min_u32(best);
+      const uint32_t best = wave_min_u32(join64<false>(
+          off, lab, __builtin_amdgcn_readlane(vs, qi), __builtin_amdgcn_readlane(vt, qi),
+          (uint32_t)__builtin_amdgcn_readlane(vk, qi), (lds_ptr<unsigned long long>)stage[wib]));
       if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
     }
     if (mine) out[q0 + lane] = ans;
   }
+}
+
+__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_query64_team(uint32_t n, const unsigned long long *__restrict__ off,
+               const unsigned long long *__restrict__ lab, uint64_t nq,
+               const uint32_t *__restrict__ qs, const uint32_t *__restrict__ qt,
+               const int8_t *__restrict__ qk, int32_t *out) {
+  __shared__ unsigned long long stage[kQWaves * kQPiece];
+  team_queries(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
+    return join64<true>(off, lab, s, t, (uint32_t)k, (lds_ptr<unsigned long long>)stage);
+  });
 }
 
 // Workgroups resident at once on a device (the persistent grid), cached per
@@ -395,6 +481,26 @@ static uint32_t query_slots(const hsdl_index *idx) {
   return pow2_at_most(env_u32("HSDL_QUERY_SLOTS", mean <= 1024 ? 1024 : 2048, 64, 4096));
 }
 
+// Whether a call's queries get a workgroup each: up to the square of the mean list
+// length, within [2,048, 32,768].  A call ends with its longest list's query, and a
+// call of few queries leaves waves idle beside it; many queries fill the chip
+// anyway, and a wave per query does the less work.  Team / wave, us:
+//   672 labels per list (R-MAT 262,144, K = 5): 1,024 queries 38 / 108, 8,192 61 /
+//   139, 65,536 196 / 260, 131,072 362 / 391, 262,144 686 / 622, 2^22 9.7 / 5.6 ms
+//   (8-byte labels, 1,024: 27 / 58, 65,536: 268 / 348, 262,144: 887 / 936)
+//   190 (65,536, K = 4): 1,024 24 / 34, 32,768 105 / 110, 65,536 171 / 127
+//   63 (grid, K = 8, 8-byte): 1,024 16 / 16, 8,192 22 / 18, 65,536 87 / 35
+// Alone, a team would serve up to some 200,000 queries of long lists; but calls in
+// flight together, as a server's batches are, share the chip: 2^20 requests in
+// batches of up to 65,536 take 6.9 ms with teams up to 2,048 queries, 7.2 up to
+// 32,768, 9.0 up to 65,536.
+// Tuning knob HSDL_QUERY_TEAM: the most queries of such a call.
+static bool use_team(const hsdl_index *idx, uint64_t nq) {
+  const uint64_t mean = idx->n ? std::min<uint64_t>(idx->total / idx->n, 1024) : 0;
+  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>(mean * mean, 2048), 1u << 15);
+  return nq <= env_u32("HSDL_QUERY_TEAM", (uint32_t)most, 0, 0xFFFFFFFFu);
+}
+
 int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const uint32_t *d_t,
                  const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc) {
   if (nq == 0) return HSDL_OK;
@@ -411,18 +517,19 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
   const bool copy = want32 && idx->q32.load(std::memory_order_acquire) == 1;
   const uint32_t slots = copy ? query_slots(idx) : 0;
   const size_t lds = (size_t)slots * 4 * kQWaves;
-  const uint32_t grid = (uint32_t)std::min<uint64_t>((nq + kQWaves - 1) / kQWaves,
+  const bool team = use_team(idx, nq);
+  const uint32_t grid = (uint32_t)std::min<uint64_t>(team ? nq : (nq + kQWaves - 1) / kQWaves,
                                                      query_grid(idx->device, copy, lds));
   if (copy) {
     const uint32_t db = idx->q32_dist_bits, pb = idx->q32_hop_bits;
-    hipLaunchKernelGGL(k_query32, dim3(grid), dim3(kQThreads), lds, st,
+    hipLaunchKernelGGL(team ? k_query32_team : k_query32, dim3(grid), dim3(kQThreads), lds, st,
                        Lab32{db, pb + db, (1u << pb) - 1u, (1u << db) - 1u}, idx->n,
                        (uint32_t)idx->K, idx->off.as<unsigned long long>(),
                        idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total,
-                       idx->hubs_below ? 1u : 0u,
-                       (uint64_t)nq, d_s, d_t, d_k, d_out, slots);
+                       idx->hubs_below ? 1u : 0u, (uint64_t)nq, d_s, d_t, d_k, d_out,
+                       team ? slots * kQWaves : slots);
   } else {
-    hipLaunchKernelGGL(k_query64, dim3(grid), dim3(kQThreads), 0, st, idx->n,
+    hipLaunchKernelGGL(team ? k_query64_team : k_query64, dim3(grid), dim3(kQThreads), 0, st, idx->n,
                        idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
                        (uint64_t)nq, d_s, d_t, d_k, d_out);
   }

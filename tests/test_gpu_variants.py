@@ -135,20 +135,23 @@ def test_prune_wave_items(monkeypatch, items, cands, stream32):
         assert np.array_equal(x, np.asarray(y)[keep])
 
 
+@pytest.mark.parametrize("team", ["0", "6000"])
 @pytest.mark.parametrize("q32,slots", [("1", "1024"), ("1", "64"), ("0", "1024")])
-def test_query_forms(monkeypatch, q32, slots):
+def test_query_forms(monkeypatch, q32, slots, team):
     """Queries from the hop-ordered 32-bit copy (parts that fit the table, and
     with 64 slots parts hashed in many pieces) and from the 8-byte labels (lists
-    of one piece of 512 labels and of several): every k from 0 past K, on a
+    of one piece of 512 labels and of several), a wave or a workgroup per query
+    (a call's 6,000 are the most that take one): every k from 0 past K, on a
     graph of long lists, short lists at K = 15, a group's index (vertices
     without their self label) and an imported set with hubs ranked below their
     vertex: the oracle's answers."""
     monkeypatch.setenv("HSDL_QUERY32", q32)
     monkeypatch.setenv("HSDL_QUERY_SLOTS", slots)
+    monkeypatch.setenv("HSDL_QUERY_TEAM", team)
     rng = np.random.default_rng(17)
 
     def check(name, idx, want, n, K):
-        print(f"[query] {name} q32={q32} slots={slots}", flush=True)
+        print(f"[query] {name} q32={q32} slots={slots} team={team}", flush=True)
         s, t = rng.integers(0, n, (2, 6000)).astype(np.uint32)
         t[:50] = s[:50]
         k = rng.integers(-1, K + 3, 6000).astype(np.int8)
