@@ -255,9 +255,11 @@ int derive_parents(hsdl_index *idx, const hsdl_graph *g, hipStream_t st);
 // Query launch used by hsdl_query_device and the server.
 // may_alloc: the call may make the index's 32-bit query copy (device memory
 // of 4 B per label, kept with the index); without it the query reads the
-// copy only when an earlier call made it.
+// copy only when an earlier call made it.  shared: other calls are in flight on the
+// device at the same time.
 int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const uint32_t *d_t,
-                 const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc = true);
+                 const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc = true,
+                 bool shared = false);
 // Makes the index's 32-bit query copy now, when it fits (synchronous).
 int prepare_query(const hsdl_index *idx);
 

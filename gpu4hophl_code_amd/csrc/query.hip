@@ -75,16 +75,16 @@ struct QChunk {
 };
 
 // The least distance of (s, t, k), k > 0, s != t, over this lane's pairs
-// (kInf32: none).  kTeam: a workgroup's work, its threads in step, else a wave's.
+// (kInf32: none).  kN threads' work: a wave's, or a workgroup's in step.
 // hcnt[v * K + x], x < K: labels of v of hop <= x.  below: the index holds hubs
 // ranked below their vertex.  T: a table of `slots`, a power of two.
-template <bool kTeam>
+template <uint32_t kN>
 __device__ inline uint32_t join32(const Lab32 &fmt, uint32_t K,
                                   const unsigned long long *__restrict__ off,
                                   const uint32_t *__restrict__ lab,
                                   const uint32_t *__restrict__ hcnt, uint32_t below, uint32_t s,
                                   uint32_t t, int k, lds_ptr<uint32_t> T, uint32_t slots) {
-  constexpr uint32_t kN = kTeam ? kQThreads : kWave;
+  constexpr bool kTeam = kN > kWave;
   const uint32_t id = kTeam ? threadIdx.x : (uint32_t)lane_id();
   auto sync = [] {
     if constexpr (kTeam)
@@ -193,7 +193,7 @@ k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restric
          todo &= todo - 1) {
       const int qi = __ffsll((long long)todo) - 1;
       const uint32_t best = wave_min_u32(
-          join32<false>(fmt, K, off, lab, hcnt, below, __builtin_amdgcn_readlane(vs, qi),
+          join32<kWave>(fmt, K, off, lab, hcnt, below, __builtin_amdgcn_readlane(vs, qi),
                         __builtin_amdgcn_readlane(vt, qi), __builtin_amdgcn_readlane(vk, qi), T,
                         slots));
       if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
@@ -205,11 +205,11 @@ k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restric
 // A workgroup per query, for calls of few queries (use_team): the longest lists'
 // queries decide when such a call ends, and its waves would idle beside them.
 // join(s, t, k) is called by all threads of the workgroup.
-template <class J>
+template <uint32_t kN, class J>
 __device__ inline void team_queries(uint32_t n, uint64_t nq, const uint32_t *__restrict__ qs,
                                     const uint32_t *__restrict__ qt,
                                     const int8_t *__restrict__ qk, int32_t *out, J &&join) {
-  __shared__ uint32_t least[kQWaves];
+  __shared__ uint32_t least[kN / kWave];
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   for (uint64_t q = blockIdx.x; q < nq; q += gridDim.x) {
     const uint32_t s = __builtin_amdgcn_readfirstlane(qs[q]);
@@ -221,7 +221,7 @@ __device__ inline void team_queries(uint32_t n, uint64_t nq, const uint32_t *__r
     if (lane_id() == 0) least[wib] = best;
     __syncthreads();
 #pragma unroll
-    for (uint32_t w = 0; w < kQWaves; ++w) best = min(best, least[w]);
+    for (uint32_t w = 0; w < kN / kWave; ++w) best = min(best, least[w]);
     if (threadIdx.x == 0)
       out[q] = k >= 0 && s == t && s < n ? 0 : best == kInf32 ? INT32_MAX : (int32_t)best;
     __syncthreads();  // `least` and the join's LDS are the next query's
@@ -229,16 +229,17 @@ __device__ inline void team_queries(uint32_t n, uint64_t nq, const uint32_t *__r
 }
 
 // slots: table slots of the workgroup.
-__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+template <uint32_t kN>
+__global__ void __launch_bounds__(kN) __attribute__((amdgpu_waves_per_eu(8)))
 k_query32_team(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
                const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt,
                uint32_t below, uint64_t nq, const uint32_t *__restrict__ qs,
                const uint32_t *__restrict__ qt, const int8_t *__restrict__ qk, int32_t *out,
                uint32_t slots) {
   extern __shared__ uint4 qlds[];
-  team_queries(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
-    return join32<true>(fmt, K, off, lab, hcnt, below, s, t, k,
-                        (lds_ptr<uint32_t>)reinterpret_cast<uint32_t *>(qlds), slots);
+  team_queries<kN>(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
+    return join32<kN>(fmt, K, off, lab, hcnt, below, s, t, k,
+                      (lds_ptr<uint32_t>)reinterpret_cast<uint32_t *>(qlds), slots);
   });
 }
 
@@ -246,15 +247,16 @@ k_query32_team(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__re
 // list A's labels.  Both are hub-sorted, so a chunk of A whose hubs lie below
 // the piece is never read again; a run of B cut by a piece's end is found in
 // both pieces.
-// kTeam: a workgroup's work (pieces of four times the size, the waves taking
-// chunks of A in turn), else a wave's.  Returns the least distance of (s, t, k),
+// kN threads' work: a wave's, or a workgroup's (a piece of 512 labels per wave,
+// the waves taking chunks of A in turn).  Returns the least distance of (s, t, k),
 // k > 0, s != t, over this lane's pairs.
 constexpr uint32_t kQPiece = 512;  // labels, 4 KB per wave
-template <bool kTeam>
+template <uint32_t kN>
 __device__ inline uint32_t join64(const unsigned long long *__restrict__ off,
                                   const unsigned long long *__restrict__ lab, uint32_t s,
                                   uint32_t t, uint32_t kk, lds_ptr<unsigned long long> P) {
-  constexpr uint32_t kN = kTeam ? kQThreads : kWave, kPiece = kTeam ? kQWaves * kQPiece : kQPiece;
+  constexpr bool kTeam = kN > kWave;
+  constexpr uint32_t kPiece = kN / kWave * kQPiece;
   const uint32_t lane = (uint32_t)lane_id(), id = kTeam ? threadIdx.x : lane;
   auto sync = [] {
     if constexpr (kTeam)
@@ -332,7 +334,7 @@ k_query64(uint32_t n, const unsigned long long *__restrict__ off,
     for (unsigned long long todo = __ballot(vk > 0 && vs < n && vt < n && vs != vt); todo;
          todo &= todo - 1) {
       const int qi = __ffsll((long long)todo) - 1;
-      const uint32_t best = wave_min_u32(join64<false>(
+      const uint32_t best = wave_min_u32(join64<kWave>(
           off, lab, __builtin_amdgcn_readlane(vs, qi), __builtin_amdgcn_readlane(vt, qi),
           (uint32_t)__builtin_amdgcn_readlane(vk, qi), (lds_ptr<unsigned long long>)stage[wib]));
       if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
@@ -341,14 +343,15 @@ k_query64(uint32_t n, const unsigned long long *__restrict__ off,
   }
 }
 
-__global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
+template <uint32_t kN>
+__global__ void __launch_bounds__(kN) __attribute__((amdgpu_waves_per_eu(8)))
 k_query64_team(uint32_t n, const unsigned long long *__restrict__ off,
                const unsigned long long *__restrict__ lab, uint64_t nq,
                const uint32_t *__restrict__ qs, const uint32_t *__restrict__ qt,
                const int8_t *__restrict__ qk, int32_t *out) {
-  __shared__ unsigned long long stage[kQWaves * kQPiece];
-  team_queries(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
-    return join64<true>(off, lab, s, t, (uint32_t)k, (lds_ptr<unsigned long long>)stage);
+  __shared__ unsigned long long stage[kN / kWave * kQPiece];
+  team_queries<kN>(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
+    return join64<kN>(off, lab, s, t, (uint32_t)k, (lds_ptr<unsigned long long>)stage);
   });
 }
 
@@ -482,7 +485,7 @@ static uint32_t query_slots(const hsdl_index *idx) {
 }
 
 // Whether a call's queries get a workgroup each: up to the square of the mean list
-// length, within [2,048, 32,768].  A call ends with its longest list's query, and a
+// length, within [2,048, 131,072].  A call ends with its longest list's query, and a
 // call of few queries leaves waves idle beside it; many queries fill the chip
 // anyway, and a wave per query does the less work.  Team / wave, us:
 //   672 labels per list (R-MAT 262,144, K = 5): 1,024 queries 38 / 108, 8,192 61 /
@@ -490,19 +493,22 @@ static uint32_t query_slots(const hsdl_index *idx) {
 //   (8-byte labels, 1,024: 27 / 58, 65,536: 268 / 348, 262,144: 887 / 936)
 //   190 (65,536, K = 4): 1,024 24 / 34, 32,768 105 / 110, 65,536 171 / 127
 //   63 (grid, K = 8, 8-byte): 1,024 16 / 16, 8,192 22 / 18, 65,536 87 / 35
-// Alone, a team would serve up to some 200,000 queries of long lists; but calls in
-// flight together, as a server's batches are, share the chip: 2^20 requests in
-// batches of up to 65,536 take 6.9 ms with teams up to 2,048 queries, 7.2 up to
-// 32,768, 9.0 up to 65,536.
+// Calls in flight together (shared: a server's batches) have the chip filled by each
+// other: there up to 32,768 at most (2^20 requests in batches of up to 65,536: 6.9 ms
+// with teams up to 2,048 queries, 7.2 up to 32,768, 9.0 up to 65,536).
+// Up to kWideQueries, which that many workgroups of eight waves take at once, a
+// team has eight waves.
 // Tuning knob HSDL_QUERY_TEAM: the most queries of such a call.
-static bool use_team(const hsdl_index *idx, uint64_t nq) {
+constexpr uint64_t kWideQueries = 1024;
+static bool use_team(const hsdl_index *idx, uint64_t nq, bool shared) {
   const uint64_t mean = idx->n ? std::min<uint64_t>(idx->total / idx->n, 1024) : 0;
-  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>(mean * mean, 2048), 1u << 15);
+  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>(mean * mean, 2048), shared ? 1u << 15 : 1u << 17);
   return nq <= env_u32("HSDL_QUERY_TEAM", (uint32_t)most, 0, 0xFFFFFFFFu);
 }
 
 int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const uint32_t *d_t,
-                 const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc) {
+                 const int8_t *d_k, int32_t *d_out, hipStream_t st, bool may_alloc,
+                 bool shared) {
   if (nq == 0) return HSDL_OK;
   const bool want32 = env_u32("HSDL_QUERY32", 1, 0, 1) != 0;
   if (want32 && may_alloc && !idx->q32.load(std::memory_order_acquire)) {
@@ -517,19 +523,26 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
   const bool copy = want32 && idx->q32.load(std::memory_order_acquire) == 1;
   const uint32_t slots = copy ? query_slots(idx) : 0;
   const size_t lds = (size_t)slots * 4 * kQWaves;
-  const bool team = use_team(idx, nq);
-  const uint32_t grid = (uint32_t)std::min<uint64_t>(team ? nq : (nq + kQWaves - 1) / kQWaves,
-                                                     query_grid(idx->device, copy, lds));
+  const bool team = use_team(idx, nq, shared);
+  const bool wide = team && nq <= kWideQueries && lds <= 32 * 1024;  // 64 KB at most
+  const uint32_t threads = wide ? 2 * kQThreads : kQThreads;
+  const uint32_t fill = query_grid(idx->device, copy, lds) / (threads / kQThreads);
+  const uint32_t grid =
+      (uint32_t)std::min<uint64_t>(team ? nq : (nq + kQWaves - 1) / kQWaves, std::max(1u, fill));
   if (copy) {
     const uint32_t db = idx->q32_dist_bits, pb = idx->q32_hop_bits;
-    hipLaunchKernelGGL(team ? k_query32_team : k_query32, dim3(grid), dim3(kQThreads), lds, st,
+    hipLaunchKernelGGL(wide ? k_query32_team<2 * kQThreads>
+                            : team ? k_query32_team<kQThreads> : k_query32,
+                       dim3(grid), dim3(threads), lds * (threads / kQThreads), st,
                        Lab32{db, pb + db, (1u << pb) - 1u, (1u << db) - 1u}, idx->n,
                        (uint32_t)idx->K, idx->off.as<unsigned long long>(),
                        idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total,
                        idx->hubs_below ? 1u : 0u, (uint64_t)nq, d_s, d_t, d_k, d_out,
-                       team ? slots * kQWaves : slots);
+                       team ? slots * (threads / kWave) : slots);
   } else {
-    hipLaunchKernelGGL(team ? k_query64_team : k_query64, dim3(grid), dim3(kQThreads), 0, st, idx->n,
+    hipLaunchKernelGGL(wide ? k_query64_team<2 * kQThreads>
+                            : team ? k_query64_team<kQThreads> : k_query64,
+                       dim3(grid), dim3(threads), 0, st, idx->n,
                        idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
                        (uint64_t)nq, d_s, d_t, d_k, d_out);
   }

@@ -124,7 +124,7 @@ static void launch_slot(hsdl_server *srv, Slot &sl) {
   const uint8_t *d = copy ? sl.d_req.as<uint8_t>() : sl.h_req;
   int32_t *out = copy ? sl.d_out.as<int32_t>() : sl.h_out;
   if (launch_query(srv->idx, n, (const uint32_t *)d, (const uint32_t *)(d + 4 * n),
-                   (const int8_t *)(d + 8 * n), out, sl.st) != HSDL_OK)
+                   (const int8_t *)(d + 8 * n), out, sl.st, true, true) != HSDL_OK)
     srv->error = HSDL_EDEVICE;
   sl.t_kernel = srv->tracing ? now_ns() : 0;
   if (copy) {

@@ -140,8 +140,8 @@ def test_prune_wave_items(monkeypatch, items, cands, stream32):
 def test_query_forms(monkeypatch, q32, slots, team):
     """Queries from the hop-ordered 32-bit copy (parts that fit the table, and
     with 64 slots parts hashed in many pieces) and from the 8-byte labels (lists
-    of one piece of 512 labels and of several), a wave or a workgroup per query
-    (a call's 6,000 are the most that take one): every k from 0 past K, on a
+    of one piece of 512 labels and of several), a wave or a workgroup of
+    four (6,000 queries) or eight waves (1,000 and one) per query: every k from 0 past K, on a
     graph of long lists, short lists at K = 15, a group's index (vertices
     without their self label) and an imported set with hubs ranked below their
     vertex: the oracle's answers."""
@@ -155,7 +155,9 @@ def test_query_forms(monkeypatch, q32, slots, team):
         s, t = rng.integers(0, n, (2, 6000)).astype(np.uint32)
         t[:50] = s[:50]
         k = rng.integers(-1, K + 3, 6000).astype(np.int8)
-        assert np.array_equal(idx.query(s, t, k), O.query(want, s, t, k))
+        ans = O.query(want, s, t, k)
+        for m in (6000, 1000, 1):
+            assert np.array_equal(idx.query(s[:m], t[:m], k[:m]), ans[:m])
 
     def imported(off, hub, hop, dist, K):
         o = O.labels_from_arrays(len(off) - 1, off, hub, hop, dist)
