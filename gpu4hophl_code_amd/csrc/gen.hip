@@ -645,6 +645,16 @@ __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uin
   return relaxed;
 }
 
+// Whether an earlier kernel stopped the batch, or another workgroup of this one
+// did: read once for the workgroup, whose waves meet at barriers further on.
+__device__ inline bool batch_stopped(const GenArgs &a) {
+  __shared__ uint32_t stopped;
+  if (threadIdx.x == 0)
+    stopped = __hip_atomic_load(&a.ctrl->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(stopped) != 0;
+}
+
 // Round h's expansion.  A wave takes 64 frontier groups (vertex x and the
 // labels x gained in round h-1, of many hubs) and walks the pairs (edge of x
 // above the batch's first hub, label of the group) edge-major: consecutive
@@ -654,7 +664,6 @@ __device__ inline bool relax_edge(const GenArgs &a, bool valid, uint32_t kb, uin
 // work (rank pruning).
 __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   with_batch(a);
-  if (a.ctrl->overflow) return;  // the batch is rolled back and run again
   const FGroup *G = a.fgrp;
   const uint32_t gcnt = min(a.ctrl->gcnt, a.n);
   const uint32_t lo_hub = hub_of(a, 0);
@@ -667,6 +676,7 @@ __global__ void __launch_bounds__(256) k_expand(GenArgs a) {
   // the first list block of each wave is its own (round_prep), as far as the
   // workgroups that hold a chunk go
   if ((uint64_t)blockIdx.x * 4 * gw >= gcnt) return;
+  if (batch_stopped(a)) return;  // the batch is rolled back and run again
   ListRes res;
   res.base = wave_id * kFirstBlock;
   res.used = 0;
@@ -785,12 +795,12 @@ constexpr int kHeavySteps = 4;   // edge steps with their loads in flight togeth
 __global__ void __launch_bounds__(256) k_expand_heavy(GenArgs a) {
   with_batch(a);
   __shared__ uint32_t sh_h;
-  if (a.ctrl->overflow) return;
   const uint32_t lane = (uint32_t)lane_id();
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
   const uint32_t wv = threadIdx.x / kWave, nwv = 256 / kWave;
   const uint32_t cnt = min(a.ctrl->heavy_cnt, a.heavy_cap);
   if (blockIdx.x >= cnt) return;  // uniform: most launches find no pieces
+  if (batch_stopped(a)) return;
   ListRes res;
   uint64_t edges_seen = 0;
   const bool lm = a.lm && a.h > 1;
