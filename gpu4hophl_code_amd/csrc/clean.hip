@@ -830,7 +830,11 @@ __global__ void __launch_bounds__(kSeqThreads) k_clean_seq(
     uint32_t *bad, uint32_t *gbits, uint32_t gwords) {
   __shared__ unsigned long long stage[kLong ? 1 : kSeqStage];
   __shared__ uint32_t bits[kLong ? 1 : 2 * kSeqWords];  // kept, then fallen
-  __shared__ uint32_t sh_next, sh_open, sh_bad, sh_kept, sh_list;
+  // a round's next window and whether it leaves labels open: three sets in turn,
+  // the next round's cleared while this one runs, so that nothing is reset where
+  // the rounds' loop turns
+  __shared__ uint32_t sh_next[3], sh_open[3];
+  __shared__ uint32_t sh_bad, sh_kept, sh_list;
   const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id();
   const uint32_t words_max = kLong ? gwords : kSeqWords;
   uint32_t *const slice = kLong ? gbits + (uint64_t)blockIdx.x * 2 * gwords : bits;
@@ -846,18 +850,20 @@ __global__ void __launch_bounds__(kSeqThreads) k_clean_seq(
   auto put = [&](uint32_t set, uint32_t i) {
     atomicOr(slice + set * words_max + (i >> 5), 1u << (i & 31));
   };
-  const uint32_t cnt = *list_cnt;
+  // every value that decides a loop with barriers in it is made scalar: the
+  // compiler then branches for the whole wave, never for some of its lanes
+  const uint32_t cnt = __builtin_amdgcn_readfirstlane(*list_cnt);
   // a workgroup's first list is its own id, later ones come from a counter
   auto claim = [&]() {
     __syncthreads();  // the shared state is the next list's
     if (tid == 0) sh_list = gridDim.x + atomicAdd(next_list, 1u);
     __syncthreads();
-    return sh_list;
+    return (uint32_t)__builtin_amdgcn_readfirstlane(sh_list);
   };
   for (uint32_t li = blockIdx.x; li < cnt; li = claim()) {
-    const uint32_t v = list[li];
+    const uint32_t v = __builtin_amdgcn_readfirstlane(list[li]);
     const unsigned long long vb = off[v];
-    const uint32_t len = (uint32_t)(off[v + 1] - vb);
+    const uint32_t len = __builtin_amdgcn_readfirstlane((uint32_t)(off[v + 1] - vb));
     const unsigned long long *Lv = lab + vb;
     if (kLong ? (len <= kSeqBits) : (len > kSeqBits)) continue;  // the other launch's
     const uint32_t words = (len + 31) / 32;
@@ -880,12 +886,15 @@ __global__ void __launch_bounds__(kSeqThreads) k_clean_seq(
       if (staged) return Sv[i];
       return Lv[i];
     };
-    if (tid == 0) sh_next = sh_open = sh_bad = sh_kept = 0;
+    if (tid < 3) sh_next[tid] = sh_open[tid] = 0;
+    if (tid == 0) sh_bad = sh_kept = 0;
     __syncthreads();
-    for (;;) {
+    for (uint32_t round = 0;; round = round == 2 ? 0 : round + 1) {
+      // (last read before the barrier that ended the round before this one)
+      if (tid == 0) sh_next[round == 2 ? 0 : round + 1] = sh_open[round == 2 ? 0 : round + 1] = 0;
       for (;;) {
         uint32_t p0 = 0;
-        if (lane == 0) p0 = atomicAdd(&sh_next, kTileWindow);
+        if (lane == 0) p0 = atomicAdd(&sh_next[round], kTileWindow);
         p0 = __builtin_amdgcn_readfirstlane(p0);
         if (p0 >= len) break;
         for (uint32_t gb = p0; gb < min(len, p0 + kTileWindow); ++gb) {
@@ -986,20 +995,14 @@ __global__ void __launch_bounds__(kSeqThreads) k_clean_seq(
           }
           if (lane < size && ((nk >> lane) & 1u)) put(0, gb + lane);
           if (lane < size && ((nf >> lane) & 1u)) put(1, gb + lane);
-          if (lane == 0 && (kept | fell | nk | nf) != all) atomicOr(&sh_open, 1u);
+          if (lane == 0 && (kept | fell | nk | nf) != all) atomicOr(&sh_open[round], 1u);
         }
       }
       __syncthreads();
-      const bool again = sh_open && !sh_bad;
-      __syncthreads();
-      if (!again) break;
-      // (reset behind the loop's test and ahead of a barrier: at the head of the
-      // loop this condition met the one before it, and the compiler sent the other
-      // lanes of the wave through the barrier without lane 0)
-      if (tid == 0) sh_next = sh_open = 0;
-      __syncthreads();
+      // (a group too large is met in the first round: no later one sets sh_bad)
+      if (!__builtin_amdgcn_readfirstlane(sh_open[round] && !sh_bad)) break;
     }
-    if (sh_bad) {
+    if (__builtin_amdgcn_readfirstlane(sh_bad)) {
       if (tid == 0) atomicOr(bad, sh_bad);
     } else {
       uint32_t k = 0;

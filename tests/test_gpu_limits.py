@@ -24,3 +24,39 @@ def test_lists_that_run_out_inside_an_expansion(monkeypatch, heavy):
         g = ragged(n, n + K, wmax, 16)
         same_labels(H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=batch),
                     O.kround(csr_of(g), K).arrays())
+
+
+@pytest.mark.parametrize("pad", [0, 5000])
+def test_clean_of_chains_over_many_rounds(pad):
+    """Lists whose labels each fall through the one before, if that one is
+    kept: at K = 15 the decisions run along chains of 15, over windows that
+    different waves take, so a list needs several rounds of the clean's second
+    pass.  Chains of every length side by side in 2,000 lists, with and without
+    hubs between them that push the list out of LDS: the oracle's clean."""
+    K = 15
+    rng = np.random.default_rng(pad + 1)
+    lists = [[(0, 0, 0)]]
+    # hub x: a label through hub x - 1, so that a kept (x - 1, h, d) removes (x, h + 1, d + 1)
+    lists += [[(x - 1, 1, 1), (x, 0, 0)] for x in range(1, 400 + pad)]
+    for v in range(2000 if not pad else 300):
+        x, rows = 0, []
+        while x < 380:
+            for i in range(int(rng.integers(1, K + 1))):
+                # now and then a distance too small to fall
+                rows.append((x, i + 1, 40 + i - 3 * int(rng.random() < 0.05)))
+                x += 1
+            x += int(rng.integers(1, 4))
+        rows = [r for r in rows if r[0] < 400]
+        if v % 3 == 0:
+            rows += [(400 + u, 1 + u % K, 1 + u % 7) for u in range(pad)]
+        lists.append(rows + [(len(lists), 0, 0)])
+    off = np.concatenate([[0], np.cumsum([len(x) for x in lists])])
+    hub, hop, dist = np.array([e for x in lists for e in x]).T
+    hub, hop, dist = hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32)
+    n = len(lists)
+    want = O.clean(O.labels_from_arrays(n, off.astype(np.int64), hub, hop, dist))
+    print(f"[chains] n={n} labels={len(hub)} kept={want.total()}", flush=True)
+    assert want.total() < len(hub) - n
+    idx = H.Index.from_labels(n, K, off.astype(np.uint64), hub, hop, dist)
+    idx.clean()
+    same_labels(idx, want.arrays())
