@@ -2127,7 +2127,7 @@ k_prune_rows(GenArgs a) {
     const uint32_t kSubs = a.row_block / kPruneThreads;
     const uint32_t steps = sh_kn * kSubs;
     for (uint32_t g0 = 0; g0 < steps; g0 += kRowSteps) {
-      uint32_t v[kRowSteps];
+      uint32_t v[kRowSteps], scanned = 0;
       auto load_slots = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (uint32_t u = 0; u < kRowSteps; ++u) {
@@ -2137,10 +2137,11 @@ k_prune_rows(GenArgs a) {
           const uint32_t y_end = i < steps ? min(a.n, (kb + 1) * a.row_block) : 0u;
           if (tid == u) sh_y0[u] = y0;
           v[u] = y0 + tid < y_end ? a.cand_d[slot_at(a, b, y0 + tid)] : kInf32;
-          row_slots += y0 < y_end ? min(kPruneThreads, y_end - y0) : 0u;
+          scanned += y0 < y_end ? min(kPruneThreads, y_end - y0) : 0u;
         }
       };
       load_slots();
+      row_slots += scanned;  // once, however many pieces the candidates take
       if (tid < kRowSteps) sh_step[tid] = 0;
       __syncthreads();
 #pragma unroll

@@ -60,3 +60,20 @@ def test_clean_of_chains_over_many_rounds(pad):
     idx = H.Index.from_labels(n, K, off.astype(np.uint64), hub, hop, dist)
     idx.clean()
     same_labels(idx, want.arrays())
+
+
+@pytest.mark.parametrize("n", [9001, 20000, 70000])
+def test_row_slots_count_each_scan_once(monkeypatch, n):
+    """Stars: the centre has every other vertex as a candidate, so a row item's
+    candidates fill the LDS list several times over and its slots are loaded
+    again for each further piece.  prune_row_slots counts a scan of a slot once:
+    the rows of n slots of the centre's batch, in the one round with candidates."""
+    monkeypatch.setenv("HSDL_PRUNE_ROWS", "2")
+    u = np.zeros(n - 1, np.uint32)
+    v = np.arange(1, n, dtype=np.uint32)
+    g = H.Graph.from_edges(n, u, v, np.full(n - 1, 3, np.int32))
+    for K in (1, 3):
+        print(f"[row slots] n={n} K={K}", flush=True)
+        idx = H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=64)
+        same_labels(idx, O.kround(csr_of(g), K).arrays())
+        assert idx.stats()["prune_row_slots"] == 64 * n
