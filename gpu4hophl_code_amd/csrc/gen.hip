@@ -3527,6 +3527,8 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
       fix.cand_total = c_ok.cand_total;
       fix.item_total = c_ok.item_total;
       fix.edge_total = c_ok.edge_total;
+      fix.lm_tested = c_ok.lm_tested;  // one attempt decides whether the test stays
+      fix.lm_caught = c_ok.lm_caught;
       HSDL_HIP(hipMemcpyAsync(g.ctrl.p, &fix, sizeof(Ctrl), hipMemcpyHostToDevice, g.st));
       HSDL_HIP(hipStreamSynchronize(g.st));
       g.h_grow += (now_ns() - tg) * 1e-9;

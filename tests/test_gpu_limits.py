@@ -77,3 +77,37 @@ def test_row_slots_count_each_scan_once(monkeypatch, n):
         idx = H.hop_constrained_two_hop_labels_generation(g, K, hub_batch=64)
         same_labels(idx, O.kround(csr_of(g), K).arrays())
         assert idx.stats()["prune_row_slots"] == 64 * n
+
+
+def test_a_retried_batch_counts_its_landmark_tests_once(monkeypatch):
+    """A batch whose landmark tests reject nothing ends the test from 4,096
+    tests on.  Hubs 16..31 of this graph make 2,880 of them, in a round whose
+    candidates outgrow 2,048 list entries: run again with larger lists the batch
+    still counts 2,880, so the later hubs, where landmarks reject most pairs,
+    open as many candidates as without the retry."""
+    monkeypatch.setenv("HSDL_HEAVY_PAIRS", "65536")
+    edges, n = [], 32
+    for x in range(16, 32):  # 60 neighbours each, three more behind each of those
+        for _ in range(60):
+            y, n = n, n + 1
+            edges.append((x, y, 5))
+            for _ in range(3):
+                edges.append((y, n, 5))
+                n += 1
+    rng = np.random.default_rng(8)
+    late = np.arange(n, n + 180)  # next to hubs 0..7, and among themselves far apart
+    n += 180
+    edges += [(x, y, 1) for x in range(8) for y in late]
+    edges += [(x, y, 50) for x, y in rng.choice(late, (800, 2)) if x != y]
+    u, v, w = np.array(edges).T
+    g = H.Graph.from_edges(n, u.astype(np.uint32), v.astype(np.uint32), w.astype(np.int32))
+    want = O.kround(csr_of(g), 2).arrays()
+    cands = []
+    for lists in (None, "2048"):
+        if lists:
+            monkeypatch.setenv("HSDL_LIST_INIT", lists)
+        print(f"[retried batch] n={n} lists={lists}", flush=True)
+        idx = H.hop_constrained_two_hop_labels_generation(g, 2, hub_batch=16)
+        same_labels(idx, want)
+        cands.append(idx.stats()["candidates"])
+    assert cands[0] == cands[1]
