@@ -2765,10 +2765,12 @@ struct Gen {
   double t_expand = 0, t_prune = 0;
   uint64_t n_prune = 0;
   double h_grow = 0, h_enqueue = 0, h_wait = 0;  // host-side phase timers (verbose)
+  uint64_t list_bytes() const {
+    return cflat.bytes + cgroup.bytes + F0.bytes + F1.bytes + frank.bytes;
+  }
   uint64_t held() const {
-    return fixed + pool.bytes + pool32.bytes + cflat.bytes + cgroup.bytes + F0.bytes + F1.bytes +
-           frank.bytes +
-           gtile.bytes + sort_tmp.bytes + sort_tmp32.bytes;
+    return fixed + pool.bytes + pool32.bytes + list_bytes() + gtile.bytes + sort_tmp.bytes +
+           sort_tmp32.bytes;
   }
   // Whether the build may hold `want` bytes beside the landmark chunks; the
   // rows only save time, so they go when the build needs their room.
@@ -3079,14 +3081,21 @@ static int sort_zones(Gen &g, uint32_t maxlen, uint32_t resort_div) {
 // 3.9 / 36.1 -> 1.48 / 2.33 / 31.5 ms, a group of 65,536 15.1 -> 12.8 ms, R-MAT
 // 262,144 202 -> 201 ms; fourfold 1.45 / 2.45 / 31.9 / 13.2 / 201; a first batch of
 // 1,024 1.45 / 2.5 / 31.9 / 13.1 / 201.
+// The eightfold step and the larger first batch are for builds with room: a batch
+// that outgrows its lists where larger ones would take the build past half its
+// budget runs again at the size that doubling from 64 had reached, on the lists it
+// has, and the batches double from there on (grown lists stay, and what they hold
+// the label pool may need later).
 constexpr double kTuneFar = 16, kTuneGrow = 8;
+constexpr uint32_t kTuneFirst = 64;
 struct BatchTuner {
-  static uint32_t first(uint32_t n) { return std::min(512u, std::max(64u, (1u << 23) / n)); }
+  static uint32_t first(uint32_t n) { return std::min(512u, std::max(kTuneFirst, (1u << 23) / n)); }
   uint32_t B, Bmax;
   double target;
+  bool far = true;  // batches may grow more than twofold
   uint32_t next(double last) {
     double f = last > 0 ? target / last : 2.0;
-    f = std::min(f > kTuneFar ? kTuneGrow : 2.0, std::max(0.5, f));
+    f = std::min(far && f > kTuneFar ? kTuneGrow : 2.0, std::max(0.5, f));
     uint64_t nb = (uint64_t)std::llround(B * f);
     nb = std::max<uint64_t>(1, std::min<uint64_t>(nb, Bmax));
     B = (uint32_t)nb;
@@ -3451,6 +3460,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   BatchTuner tuner{plain ? 1u : std::min(tune_cap, BatchTuner::first(n)), tune_cap, tune_target};
   if (opts->hub_batch) tuner.B = std::min(opts->hub_batch, Bmax);
   uint64_t batches = 0, redos = 0;
+  uint32_t done_B = 0;  // hubs of the last batch that completed
   const uint64_t t_loop = now_ns();  // set-up (buffers, lists) ends here
   uint32_t s0 = 0;
   Ctrl c{}, c_ok{};  // c_ok: counters after the last batch that completed
@@ -3497,15 +3507,23 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
       HSDL_HIP(hipGetLastError());
       HSDL_HIP(hipStreamSynchronize(g.st));
       const uint64_t used = std::min<uint64_t>(c.pool_top, g.a.pool_cap);
+      bool overshot = false;  // larger than doubling had made it, on lists that may not grow
       if ((c.overflow & kOvfPool) && (rc = grow_pool(g, used, used * 2))) return rc;
       if ((c.overflow & kOvfArena) && (rc = grow_gtile(g))) return rc;
       if (c.overflow & (kOvfCand | kOvfFront)) {
         const uint64_t nc = std::max<uint64_t>((uint64_t)g.a.ccap * 2, (uint64_t)c.ccnt * 5 / 4);
         const uint64_t nf = std::max<uint64_t>((uint64_t)g.a.fcap * 2, nc);
         const uint32_t occ = g.a.ccap, ofc = g.a.fcap;
-        const bool grown = nc <= 0xFFFFFFF0ull && nf <= 0xFFFFFFF0ull &&
+        const uint32_t doubled = done_B ? 2 * done_B : kTuneFirst;
+        const bool roomy = g.held() - g.list_bytes() + nc * 12 + nf * (2 * sizeof(Item) + 4) <=
+                           g.budget / 2;
+        overshot = !opts->hub_batch && B > doubled && !roomy;
+        const bool grown = !overshot && nc <= 0xFFFFFFF0ull && nf <= 0xFFFFFFF0ull &&
                            alloc_lists(g, (uint32_t)nc, (uint32_t)nf) == HSDL_OK;
-        if (!grown) {
+        if (overshot) {
+          tuner.far = false;
+          tuner.B = doubled;
+        } else if (!grown) {
           // lists of twice the size do not fit: the batch runs again at half
           // its hubs with lists of the old sizes, which fitted (a chosen
           // hub_batch or a one-hub batch cannot shrink)
@@ -3516,6 +3534,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
           g.a.ccap = g.a.fcap = 0;  // the old buffers may be gone
           if ((rc = alloc_lists(g, occ, ofc))) return rc;
           tuner.B = std::max(1u, B / 2);
+          tuner.far = false;
         }
       }
       // the counters restart from the last completed batch (the attempt's
@@ -3536,7 +3555,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
         fprintf(stderr, "[hsdl] batch s0=%u B=%u overflow=%u: pool %llu, arena %llu, lists %u/%u; redo\n",
                 s0, B, c.overflow, (unsigned long long)g.a.pool_cap,
                 (unsigned long long)g.a.gtile_cap, g.a.ccap, g.a.fcap);
-      if (++redos > 64) return fail(HSDL_ENOMEM, "buffers kept overflowing");
+      if (!overshot && ++redos > 64) return fail(HSDL_ENOMEM, "buffers kept overflowing");
       continue;
     }
     // keep headroom: grow the pool between batches when it is half full
@@ -3563,6 +3582,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
     if (zones && B > 1 && s0 + B < nhubs && (rc = sort_zones(g, c.maxlen, resort_div)))
       return rc;
     s0 += B;
+    done_B = B;
     ++batches;
     const double dt = (now_ns() - tb) * 1e-9;
     if (g.verbose)

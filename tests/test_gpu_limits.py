@@ -111,3 +111,19 @@ def test_a_retried_batch_counts_its_landmark_tests_once(monkeypatch):
         same_labels(idx, want)
         cands.append(idx.stats()["candidates"])
     assert cands[0] == cands[1]
+
+
+@pytest.mark.parametrize("mb", [1400, 1520, 1700])
+def test_growing_batches_leave_the_budget_to_the_pool(mb):
+    """Builds within budgets that hold the labels as long as the candidate lists
+    stay small: batches that grow eightfold outgrow the lists, and lists
+    grown for them would leave the label pool no room to grow in.  The labels of
+    a build without such a limit."""
+    K = 5
+    g = H.Graph.rmat(15, 16, 7, 1, 40000)
+    want = H.hop_constrained_two_hop_labels_generation(g, K, hbm_budget=60 << 30).labels()
+    g = H.Graph.rmat(15, 16, 7, 1, 40000)  # another handle: nothing kept from the first build
+    print(f"[tight budget] {mb} MB", flush=True)
+    idx = H.hop_constrained_two_hop_labels_generation(g, K, hbm_budget=mb << 20,
+                                                      pool_init_labels=4 * len(want[1]))
+    same_labels(idx, want)
