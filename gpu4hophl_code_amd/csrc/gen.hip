@@ -179,8 +179,7 @@ struct GenArgs {
   uint32_t *sorted_len;
   uint32_t *hcnt;
   uint32_t hcnt_stride;  // K - 1
-  uint32_t *add_cnt;   // labels a vertex gains in the round, counted by the prune
-  uint32_t *base_len;  // its list's length before them (k_reserve, for k_append)
+  uint32_t *fill;  // a vertex's list length with the labels the round's prune accepted so far
   uint32_t *touched;
   FGroup *fgrp;               // frontier groups (n entries)
   uint32_t *hub_slot;         // group builds: hub slot of each hub of the batch
@@ -202,7 +201,7 @@ struct GenArgs {
   uint32_t *wave_hubs;  // hub slots of the round's wave items
   Item *F0;
   Item *F1;
-  uint32_t *frank;  // per item of the next frontier: its rank among its vertex's new labels
+  uint32_t *fpos;  // per item of the next frontier: its label's place in its vertex's list
   HeavyItem *heavy;
   uint32_t heavy_cap;
   uint32_t *gtile;
@@ -351,7 +350,7 @@ __global__ void k_init_labels(GenArgs a, uint32_t c0) {
     a.seg_start[v] = v * c0;
     a.seg_len[v] = 1;
     a.seg_cap[v] = c0;
-    a.add_cnt[v] = 0;
+    a.fill[v] = 1;
     if (a.pool) a.pool[v * c0] = pack_label((uint32_t)v, 0, 0);
     if (a.pool32) a.pool32[v * c0] = pack32(a, (uint32_t)v, 0, 0);
     if (a.hcnt) {
@@ -1591,21 +1590,21 @@ __device__ bool witness_search(const GenArgs &a, const LT *L, const ListView &vi
 constexpr uint32_t kAccSlots = 256;
 
 // Publishes the staged accepted labels (whole workgroup; the caller has
-// synchronised after staging): per-vertex add counts, the vertices touched
+// synchronised after staging): their vertices' lengths, the vertices touched
 // for the first time this round gathered in LDS, one reservation each on the
 // frontier and the touched list, then the writes.  Empties the staging.
 __device__ inline void publish_accepted(const GenArgs &a, Item *Fn, Item *sh_acc,
-                                        uint32_t *sh_rank, uint32_t *sh_touch, uint32_t &sh_acc_n,
+                                        uint32_t *sh_pos, uint32_t *sh_touch, uint32_t &sh_acc_n,
                                         uint32_t &sh_acc_base, uint32_t &sh_touch_n,
                                         uint32_t &sh_touch_base) {
   const uint32_t nacc = sh_acc_n;
   for (uint32_t i = threadIdx.x; i < nacc; i += blockDim.x) {
     const uint32_t y = sh_acc[i].y;
-    // the count before this label is its rank among y's new labels (the
-    // append's slot past y's list)
-    const uint32_t r = atomicAdd(&a.add_cnt[y], 1u);
-    if (r == 0) sh_touch[atomicAdd(&sh_touch_n, 1u)] = y;
-    sh_rank[i] = r;
+    // the length before this label is its place in y's list
+    const uint32_t len = a.seg_len[y];
+    const uint32_t at = atomicAdd(&a.fill[y], 1u);
+    if (at == len) sh_touch[atomicAdd(&sh_touch_n, 1u)] = y;
+    sh_pos[i] = at;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1619,7 +1618,7 @@ __device__ inline void publish_accepted(const GenArgs &a, Item *Fn, Item *sh_acc
   for (uint32_t i = threadIdx.x; i < nacc; i += blockDim.x)
     if (sh_acc_base + i < a.fcap) {
       Fn[sh_acc_base + i] = sh_acc[i];
-      a.frank[sh_acc_base + i] = sh_rank[i];
+      a.fpos[sh_acc_base + i] = sh_pos[i];
     }
   const uint32_t ntouch = sh_touch_n;
   for (uint32_t i = threadIdx.x; i < ntouch; i += blockDim.x)
@@ -1902,9 +1901,12 @@ __device__ __attribute__((always_inline)) inline void prune_wave_items(
       if (mine) sh_acc[at + rank] = Item{b, y, dy};
       continue;
     }
-    uint32_t r = 1;
-    if (mine) r = atomicAdd(&a.add_cnt[y], 1u);
-    const unsigned long long tm = __ballot(mine && r == 0);
+    uint32_t len = 0, pos = 1;
+    if (mine) {
+      len = a.seg_len[y];
+      pos = atomicAdd(&a.fill[y], 1u);
+    }
+    const unsigned long long tm = __ballot(mine && pos == len);
     uint32_t fb = 0, tb = 0;
     if (lane == 0) {
       fb = atomicAdd(&a.ctrl->fcnt[a.cur ^ 1], nk);
@@ -1915,9 +1917,9 @@ __device__ __attribute__((always_inline)) inline void prune_wave_items(
     tb = __builtin_amdgcn_readfirstlane(tb);
     if (mine && fb + rank < a.fcap) {
       Fn[fb + rank] = Item{b, y, dy};
-      a.frank[fb + rank] = r;
+      a.fpos[fb + rank] = pos;
     }
-    if (mine && r == 0) a.touched[tb + (uint32_t)__popcll(tm & lt_mask)] = y;
+    if (mine && pos == len) a.touched[tb + (uint32_t)__popcll(tm & lt_mask)] = y;
   }
 }
 
@@ -1930,7 +1932,7 @@ k_prune(GenArgs a) {
   __shared__ uint32_t sh_w, sh_acc_n, sh_acc_base, sh_next, sh_touch_n, sh_touch_base;
   __shared__ uint32_t sh_item, sh_item_end, sh_rows;
   __shared__ Item sh_acc[kAccSlots];
-  __shared__ uint32_t sh_rank[kAccSlots];
+  __shared__ uint32_t sh_pos[kAccSlots];
   __shared__ uint32_t sh_touch[kAccSlots];
   __shared__ unsigned long long sh_reads[2];
   const int lane = lane_id();
@@ -1994,7 +1996,7 @@ k_prune(GenArgs a) {
     // the staged labels of earlier items are published once this item's
     // could overflow the staging slots (c_end - c_beg <= tile <= kAccSlots)
     if (sh_acc_n + (c_end - c_beg) > kAccSlots)
-      publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
+      publish_accepted(a, Fn, sh_acc, sh_pos, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
     const uint32_t *run = a.cgroup + a.hub_off[b];
     auto cands = [&](uint32_t i, uint32_t &y, uint32_t &dy) {
       y = run[i];
@@ -2020,7 +2022,7 @@ k_prune(GenArgs a) {
     tile_prune<V, LT>(a, b, c_beg, c_end, cands, accept, plan, lds, gkeys, sh_next, wave_reads);
     __syncthreads();
   }
-  publish_accepted(a, Fn, sh_acc, sh_rank, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
+  publish_accepted(a, Fn, sh_acc, sh_pos, sh_touch, sh_acc_n, sh_acc_base, sh_touch_n, sh_touch_base);
   if (lane == 0) {
     if (wave_reads) atomicAdd(&sh_reads[0], wave_reads);
     if (wave_tile) atomicAdd(&sh_reads[1], wave_tile);
@@ -2196,26 +2198,29 @@ k_prune_rows(GenArgs a) {
             [&](uint32_t i, uint32_t, uint32_t) { list[i] |= 1u << 31; }, plan, lds, gkeys,
             sh_next, wave_reads);
         __syncthreads();
-        // the accepted labels: per-vertex add counts (the count before a label
-        // is its rank among the vertex's new labels, the append's slot past its
-        // list), one reservation each on the frontier and the touched list
-        uint32_t ry[2], rr[2], rd[2], at[2], tat[2];
-        bool acc[2];
+        // the accepted labels: their vertices' lengths (the length before a label
+        // is its place in the list), one reservation each on the frontier and the
+        // touched list
+        uint32_t ry[2], rp[2], rd[2], at[2], tat[2];
+        bool acc[2], fst[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const uint32_t i = u * kPruneThreads + tid;
           const uint32_t e = i < cnt ? list[i] : 0u;
           acc[u] = e >> 31;
-          ry[u] = rr[u] = rd[u] = at[u] = tat[u] = 0;
+          ry[u] = rp[u] = rd[u] = at[u] = tat[u] = 0;
+          fst[u] = false;
           if (acc[u]) {
             ry[u] = vertex(e);
             rd[u] = dist_of(e, ry[u]);
-            rr[u] = atomicAdd(&a.add_cnt[ry[u]], 1u);
+            const uint32_t len = a.seg_len[ry[u]];
+            rp[u] = atomicAdd(&a.fill[ry[u]], 1u);
+            fst[u] = rp[u] == len;
           }
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const uint64_t m = __ballot(acc[u]), mt = __ballot(acc[u] && rr[u] == 0);
+          const uint64_t m = __ballot(acc[u]), mt = __ballot(fst[u]);
           if (!m) continue;
           if (lane == 0) {
             at[u] = atomicAdd(&sh_acc, (uint32_t)__popcll(m));
@@ -2239,9 +2244,9 @@ k_prune_rows(GenArgs a) {
             const uint32_t p = sh_acc_base + at[u];
             if (p < a.fcap) {
               Fn[p] = Item{b, ry[u], rd[u]};
-              a.frank[p] = rr[u];
+              a.fpos[p] = rp[u];
             }
-            if (rr[u] == 0) a.touched[sh_touch_base + tat[u]] = ry[u];
+            if (fst[u]) a.touched[sh_touch_base + tat[u]] = ry[u];
           }
         }
         __syncthreads();
@@ -2321,7 +2326,7 @@ __global__ void __launch_bounds__(256) k_reserve(GenArgs a) {
       len = a.seg_len[y];
       cap = a.seg_cap[y];
       st = a.seg_start[y];
-      add = a.add_cnt[y];
+      add = a.fill[y] - len;
       if (len + add > cap) ncap = (max(len + add, cap * 2u) + 7u) & ~7u;
     }
     if (__ballot(ncap != 0)) {
@@ -2344,17 +2349,12 @@ __global__ void __launch_bounds__(256) k_reserve(GenArgs a) {
         a.seg_cap[y] = cap = ncap;
       }
     }
-    if (t < cnt) {
-      a.base_len[y] = len;
-      a.add_cnt[y] = 0;
-      if (keep) {
-        // capped: when the pool ran out some appends are dropped
-        const uint32_t nl = min(len + add, cap);
-        a.seg_len[y] = nl;
-        mx = max(mx, nl);
-        // the next round's frontier group of y: the labels it gains
-        a.fgrp[t] = FGroup{y, nl - len, st + len};
-      }
+    // (where the pool ran out y gains nothing)
+    if (t < cnt && keep && len + add <= cap) {
+      a.seg_len[y] = len + add;
+      mx = max(mx, len + add);
+      // the next round's frontier group of y: the labels it gains
+      a.fgrp[t] = FGroup{y, add, st + len};
     }
   }
   mx = wave_max_u32(mx);
@@ -2364,23 +2364,21 @@ __global__ void __launch_bounds__(256) k_reserve(GenArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) a.ctrl->gcnt = keep ? min(cnt, a.n) : 0u;
 }
 
-// Writes the accepted labels behind their vertices' lists and sets up the next
-// round.
+// Writes the accepted labels into their vertices' lists, which k_reserve has
+// lengthened, and sets up the next round.
 __global__ void __launch_bounds__(256) k_append(GenArgs a) {
   with_batch(a);
   const Item *Fn = frontier(a, a.cur ^ 1);
   const uint32_t cnt = min(a.ctrl->fcnt[a.cur ^ 1], a.fcap);
+  const bool stopped = a.ctrl->overflow != 0;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
     const Item it = Fn[i];
-    const uint32_t p = a.base_len[it.y] + a.frank[i];
-    if (p < a.seg_cap[it.y]) {
-      const unsigned long long at = a.seg_start[it.y] + p;
-      const uint32_t hub = hub_of(a, it.b);
-      if (a.pool) a.pool[at] = pack_label(hub, a.h, it.d);
-      if (a.pool32) a.pool32[at] = pack32(a, hub, a.h, it.d);
-    } else {
-      atomicOr(&a.ctrl->overflow, kOvfPool);
-    }
+    const uint32_t p = a.fpos[i];
+    if (stopped && p >= a.seg_len[it.y]) continue;  // not lengthened
+    const unsigned long long at = a.seg_start[it.y] + p;
+    const uint32_t hub = hub_of(a, it.b);
+    if (a.pool) a.pool[at] = pack_label(hub, a.h, it.d);
+    if (a.pool32) a.pool32[at] = pack32(a, hub, a.h, it.d);
   }
   if (a.h == a.K) return;
   const uint32_t gcnt = a.ctrl->gcnt;
@@ -2407,7 +2405,7 @@ __global__ void __launch_bounds__(256) k_rollback(GenArgs a) {
       --len;
     }
     a.seg_len[v] = len;
-    a.add_cnt[v] = 0;
+    a.fill[v] = len;
   }
 }
 
@@ -2725,23 +2723,23 @@ static int upload_graph(hsdl_graph *g, int dev) {
 
 // Slots of hsdl_graph::scratch for Gen's buffers.
 enum ScratchId : int {
-  kScSegStart, kScSegLen, kScSegCap, kScAddCnt, kScTouched, kScFgrp, kScHubSlot,
+  kScSegStart, kScSegLen, kScSegCap, kScFill, kScTouched, kScFgrp, kScHubSlot,
   kScSortedLen, kScHcnt, kScSortTmp, kScSortTmp32, kScCflat, kScCgroup, kScHubCcnt, kScHubOff,
   kScHubCur, kScChunkOff, kScF0, kScF1, kScGtile, kScCtrl, kScHeavy, kScExpKeys, kScExpSorted,
-  kScExpTmp, kScFrank, kScLm, kScCount
+  kScExpTmp, kScFpos, kScLm, kScCount
 };
 static_assert(kScCount <= hsdl_graph::kScratch, "scratch slots");
 
 struct Gen {
   GenArgs a{};
   hsdl_graph *mg = nullptr;  // the graph whose scratch the buffers come from and go back to
-  DevBuf pool, pool32, seg_start, seg_len, seg_cap, add_cnt, touched, fgrp, hub_slot;
+  DevBuf pool, pool32, seg_start, seg_len, seg_cap, fill, touched, fgrp, hub_slot;
   DevBuf sorted_len, hcnt, sort_tmp, sort_tmp32;  // hop zones
   uint32_t sort_per_wave = 0;                     // labels per wave slice of sort_tmp
   int sort_grid = 0;
   DevBuf cflat, cgroup, hub_ccnt, hub_off, hub_cur, chunk_off, F0, F1, gtile, ctrl, heavy;
   DevBuf exp_keys, exp_sorted, exp_tmp;  // export: 32-bit keys, sorted keys, sort space
-  DevBuf frank;                          // ranks of the next frontier's items
+  DevBuf fpos;                           // list places of the next frontier's items
   DevBuf lm;                             // landmark chunks (k_lm_build)
   bool lm_on = false;
   uint64_t budget = 0;  // device bytes the build may hold
@@ -2766,7 +2764,7 @@ struct Gen {
   uint64_t n_prune = 0;
   double h_grow = 0, h_enqueue = 0, h_wait = 0;  // host-side phase timers (verbose)
   uint64_t list_bytes() const {
-    return cflat.bytes + cgroup.bytes + F0.bytes + F1.bytes + frank.bytes;
+    return cflat.bytes + cgroup.bytes + F0.bytes + F1.bytes + fpos.bytes;
   }
   uint64_t held() const {
     return fixed + pool.bytes + pool32.bytes + list_bytes() + gtile.bytes + sort_tmp.bytes +
@@ -2785,10 +2783,10 @@ struct Gen {
     return true;
   }
   DevBuf *by_id(int id) {
-    DevBuf *t[kScCount] = {&seg_start, &seg_len, &seg_cap, &add_cnt, &touched, &fgrp,
+    DevBuf *t[kScCount] = {&seg_start, &seg_len, &seg_cap, &fill, &touched, &fgrp,
                            &hub_slot, &sorted_len, &hcnt, &sort_tmp, &sort_tmp32, &cflat, &cgroup,
                            &hub_ccnt, &hub_off, &hub_cur, &chunk_off, &F0, &F1, &gtile, &ctrl,
-                           &heavy, &exp_keys, &exp_sorted, &exp_tmp, &frank, &lm};
+                           &heavy, &exp_keys, &exp_sorted, &exp_tmp, &fpos, &lm};
     return t[id];
   }
   // Buffer `id` of at least n bytes: the graph's kept one when it is large
@@ -2897,16 +2895,16 @@ static int alloc_lists(Gen &g, uint32_t ccap, uint32_t fcap) {
   if (fcap != g.a.fcap) {
     g.F0.release();
     g.F1.release();
-    g.frank.release();
+    g.fpos.release();
     if (!g.fits(g.held() + (uint64_t)fcap * (2 * sizeof(Item) + 4)))
       return fail(HSDL_ENOMEM, "frontier lists exceed the HBM budget");
     if ((rc = g.take(kScF0, (uint64_t)fcap * sizeof(Item))) ||
         (rc = g.take(kScF1, (uint64_t)fcap * sizeof(Item))) ||
-        (rc = g.take(kScFrank, (uint64_t)fcap * 4)))
+        (rc = g.take(kScFpos, (uint64_t)fcap * 4)))
       return rc;
     g.a.F0 = g.F0.as<Item>();
     g.a.F1 = g.F1.as<Item>();
-    g.a.frank = g.frank.as<uint32_t>();
+    g.a.fpos = g.fpos.as<uint32_t>();
     g.a.fcap = fcap;
   }
   return HSDL_OK;
@@ -2962,7 +2960,7 @@ static bool same_buffers(const GenArgs &x, const GenArgs &y) {
   return x.pool == y.pool && x.pool_cap == y.pool_cap && x.pool32 == y.pool32 &&
          x.gtile == y.gtile && x.gtile_cap == y.gtile_cap && x.cflat == y.cflat &&
          x.cgroup == y.cgroup && x.ccap == y.ccap && x.F0 == y.F0 && x.F1 == y.F1 &&
-         x.frank == y.frank && x.fcap == y.fcap && x.lm == y.lm;
+         x.fpos == y.fpos && x.fcap == y.fcap && x.lm == y.lm;
 }
 
 // Captures the batch sequence (with or without the row-item prune) into a
@@ -3167,9 +3165,9 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
       "HSDL_LIST_INIT",
       (uint32_t)std::min<uint64_t>(std::max<uint64_t>((uint64_t)n * 8, 8u << 20), 1u << 30), 64,
       1u << 30);
-  // per vertex: segment start, length, capacity, add counter, base, touched
+  // per vertex: segment start, length, capacity, fill, touched
   // entry, frontier group (16 B), hub slot, hop zone counts
-  const uint64_t vert_bytes = (uint64_t)n * (8 + 5 * 4 + 16 + 4 + 4 * (uint64_t)K);
+  const uint64_t vert_bytes = (uint64_t)n * (8 + 4 * 4 + 16 + 4 + 4 * (uint64_t)K);
   // dense dedupe slots: at most 1/slot_div of the budget (tuning knob
   // HSDL_SLOT_DIV), <= 65536 hubs
   const bool plain = opts->mode == HSDL_MODE_PLAIN;
@@ -3253,7 +3251,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   if ((!use32 && !g.pool.p && (rc = g.pool.alloc(pool0 * 8))) ||
       (rc = g.take(kScSegStart, n * 8ull)) ||
       (rc = g.take(kScSegLen, n * 4ull)) || (rc = g.take(kScSegCap, n * 4ull)) ||
-      (rc = g.take(kScAddCnt, n * 8ull)) ||
+      (rc = g.take(kScFill, n * 4ull)) ||
       (rc = g.take(kScTouched, n * 4ull)) || (rc = g.take(kScFgrp, n * 16ull)) ||
       (group && (rc = g.take(kScHubSlot, n * 4ull))) ||
       (rc = g.take(kScHubCcnt, (Bmax + 1ull) * 4)) || (rc = g.take(kScHubOff, (Bmax + 1ull) * 4)) ||
@@ -3369,8 +3367,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   a.sorted_len = zones ? g.sorted_len.as<uint32_t>() : nullptr;
   a.hcnt = zones ? g.hcnt.as<uint32_t>() : nullptr;
   a.hcnt_stride = K - 1;
-  a.add_cnt = g.add_cnt.as<uint32_t>();
-  a.base_len = a.add_cnt + n;
+  a.fill = g.fill.as<uint32_t>();
   a.touched = g.touched.as<uint32_t>();
   a.fgrp = g.fgrp.as<FGroup>();
   a.hub_slot = group ? g.hub_slot.as<uint32_t>() : nullptr;

@@ -127,3 +127,34 @@ def test_growing_batches_leave_the_budget_to_the_pool(mb):
     idx = H.hop_constrained_two_hop_labels_generation(g, K, hbm_budget=mb << 20,
                                                       pool_init_labels=4 * len(want[1]))
     same_labels(idx, want)
+
+
+@pytest.mark.parametrize("scale,K,batch,group,budget", [
+    (14, 5, 64, True, 260762640), (14, 2, 1, False, 176436256), (13, 1, 16, False, 163329296)])
+def test_least_budgets(monkeypatch, scale, K, batch, group, budget):
+    """The least budgets of builds whose buffers never grow, as the per-vertex
+    state, slots, lists, pool and tile arena of a 256-CU device add up to: any
+    further array per vertex would refuse them."""
+    monkeypatch.setenv("HSDL_LIST_INIT", "2000000")
+    monkeypatch.setenv("HSDL_HEAVY_CAP", "4096")
+    g = H.Graph.rmat(scale, 8, 7, 1, 100)
+    hubs = np.arange(0, g.n, 3, dtype=np.uint32) if group else None
+    print(f"[least budget] scale={scale} K={K} batch={batch} group={group}", flush=True)
+    idx = H.hop_constrained_two_hop_labels_generation(g, K, hbm_budget=budget, hubs=hubs,
+                                                      pool_init_labels=400 * g.n, hub_batch=batch)
+    if not group:
+        same_labels(idx, O.kround(csr_of(g), K).arrays())
+
+
+@pytest.mark.parametrize("stream32", ["1", "0"])
+def test_pool_that_runs_out_between_vertices(monkeypatch, stream32):
+    """A pool that takes some vertices' longer segments and not others', so that
+    part of a round's labels is written before the batch is rolled back and run
+    again: the oracle's labels."""
+    monkeypatch.setenv("HSDL_STREAM32", stream32)
+    for n, K, batch, extra in ((3000, 4, 64, 40), (3000, 4, 700, 3000), (1300, 5, 0, 9)):
+        print(f"[pool] n={n} K={K} batch={batch} extra={extra} stream32={stream32}", flush=True)
+        g = ragged(n, n + K, 60, 16)
+        same_labels(H.hop_constrained_two_hop_labels_generation(
+            g, K, hub_batch=batch, pool_init_labels=16 * n + extra),
+            O.kround(csr_of(g), K).arrays())
