@@ -239,16 +239,30 @@ __device__ inline bool has_partner(const unsigned long long *__restrict__ lab,
   return false;
 }
 
+// The walk of a list is quadratic in its length, and so are its lookups where the
+// bound rejects little (a long list whose heads have short ones).  A list goes on
+// to the tiles, which take |L(u)| probes per label, once 64 of its labels walk past
+// kPairWalk others, or a wave's lookups of 64 pairs pass kPairLooks per 64 labels
+// (no list of R-MAT and grid builds of 26 to 311 labels per list does).
+// Lists of 16,000 labels over heads of 20, whose pairs all pass the bound and find
+// nothing: 64 of them 128 -> 4.7 ms (tiles alone 4.8), 4 of 60,000 1,640 -> 14 (14);
+// whose pairs all fail it: 10 -> 4.7 (5.2) and 114 -> 11 (10).
+constexpr int32_t kPairWalk = 2048;
+constexpr int32_t kPairLooks = 16;
+enum : uint32_t { kPairsKeep, kPairsRemove, kPairsLeave };
+
 // Whether some pair of v's labels removes one of the 64 labels from position i0
 // of the hop-ordered list L (whole wave).  hc: v's prefix counts; q: the wave's
-// queue of 128 entries (position of j << 6 | lane of i).
+// queue of 128 entries (position of j << 6 | lane of i); look: lookups the wave has
+// left for this list.
 template <class F>
-__device__ bool chunk_removes(const F &f, uint32_t v, uint32_t K,
+__device__ uint32_t chunk_removes(const F &f, uint32_t v, uint32_t K,
                               const unsigned long long *__restrict__ off,
                               const unsigned long long *__restrict__ lab,
                               const typename F::T *__restrict__ L,
                               const uint32_t *__restrict__ hc, const uint32_t *__restrict__ m,
-                              uint32_t len, uint32_t i0, lds_ptr<uint32_t> q, uint64_t &streamed) {
+                              uint32_t len, uint32_t i0, lds_ptr<uint32_t> q, int32_t &look,
+                              uint64_t &streamed) {
   using T = typename F::T;
   const uint32_t lane = (uint32_t)lane_id();
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
@@ -260,7 +274,10 @@ __device__ bool chunk_removes(const F &f, uint32_t v, uint32_t K,
   const uint32_t hmax = __builtin_amdgcn_readfirstlane(wave_max_u32(act ? h : 0u));
   uint32_t qn = 0;
   bool hit = false;
+  int32_t walk = kPairWalk;
+  look += (int32_t)kPairLooks;
   auto look_up = [&](uint32_t cnt) {
+    --look;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t e = q[lane];
     const int il = (int)(e & 63u);
@@ -286,6 +303,8 @@ __device__ bool chunk_removes(const F &f, uint32_t v, uint32_t K,
       const T *Z = L + j;
       if (Z[0] >= umax) break;
       streamed += 32;
+      walk -= 32;
+      if ((walk | look) < 0) return kPairsLeave;
       uint32_t mask = 0;
 #pragma unroll
       for (uint32_t t = 0; t < 32; ++t) {
@@ -308,13 +327,13 @@ __device__ bool chunk_removes(const F &f, uint32_t v, uint32_t K,
           const uint32_t rest = q[kWave + lane];
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           if (lane < qn) q[lane] = rest;
-          if (__ballot(hit)) return true;
+          if (__ballot(hit)) return kPairsRemove;
         }
       }
     }
   }
   if (qn) look_up(qn);
-  return __ballot(hit) != 0;
+  return __ballot(hit) ? kPairsRemove : kPairsKeep;
 }
 
 // Whether two labels of one hub group of v's list [vb, vb + len) remove the
@@ -342,18 +361,21 @@ __device__ inline bool group_removes(uint32_t v, const unsigned long long *__res
 }
 
 // ctr[0]: redo count, ctr[1]: long lists of the slice, ctr[2]: next vertex of
-// the slice (kLong: next entry of `longs`), ctr[4..5]: labels read (u64).
+// the slice (kLong: next entry of `longs`), ctr[4..5]: labels read (u64), ctr[8]:
+// lists left to the tiles.
 // kLong = false: a wave per vertex, lists of more than kCleanLong labels are
 // left in `longs`.  kLong = true: a workgroup per list of `longs`, its waves
 // taking the chunks in turn.
-constexpr uint32_t kCleanLong = 2048;
+// (64 lists of 2,000 labels: a wave each 3.3 ms, a workgroup each 1.0; from 512
+// labels on a group build's clean takes 6 % longer.)
+constexpr uint32_t kCleanLong = 1024;
 constexpr uint32_t kCleanClaim = 4;  // vertices a wave claims at once
 template <class F, bool kLong>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
 k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long long *__restrict__ off,
               const unsigned long long *__restrict__ lab, const typename F::T *__restrict__ srt,
               const uint32_t *__restrict__ hcnt, const uint32_t *__restrict__ m, uint32_t *redo,
-              uint32_t *longs, uint32_t *ctr) {
+              uint32_t *longs, uint32_t *left, uint32_t *ctr) {
   __shared__ uint32_t queue[256 / kWave][2 * kWave];
   __shared__ uint32_t sh_l, sh_c, sh_hit;
   const uint32_t lane = (uint32_t)lane_id();
@@ -374,12 +396,15 @@ k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long lon
           if (lane == 0) longs[atomicAdd(&ctr[1], 1u)] = v;
           continue;
         }
-        bool gone = false;
-        for (uint32_t i0 = 0; i0 < len && !gone; i0 += kWave)
-          gone = group_removes(v, off, lab, vb, len, i0) ||
-                 chunk_removes(f, v, K, off, lab, srt + (vb - base), hcnt + (uint64_t)(v - v0) * K,
-                               m, len, i0, q, streamed);
-        if (gone && lane == 0) redo[atomicAdd(&ctr[0], 1u)] = v;
+        uint32_t end = kPairsKeep;
+        int32_t look = 0;
+        for (uint32_t i0 = 0; i0 < len && end == kPairsKeep; i0 += kWave)
+          end = group_removes(v, off, lab, vb, len, i0)
+                    ? kPairsRemove
+                    : chunk_removes(f, v, K, off, lab, srt + (vb - base),
+                                    hcnt + (uint64_t)(v - v0) * K, m, len, i0, q, look, streamed);
+        if (end == kPairsRemove && lane == 0) redo[atomicAdd(&ctr[0], 1u)] = v;
+        if (end == kPairsLeave && lane == 0) left[atomicAdd(&ctr[8], 1u)] = v;
       }
     }
   } else {
@@ -396,6 +421,7 @@ k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long lon
       const uint32_t v = longs[li];
       const unsigned long long vb = off[v];
       const uint32_t len = (uint32_t)(off[v + 1] - vb);
+      int32_t look = 0;
       for (;;) {
         uint32_t c = 0;
         if (lane == 0) c = atomicAdd(&sh_c, 1u);
@@ -403,14 +429,20 @@ k_clean_pairs(F f, uint32_t v0, uint32_t v1, uint32_t K, const unsigned long lon
         const uint32_t seen = __hip_atomic_load(&sh_hit, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
         if ((uint64_t)c * kWave >= len || __builtin_amdgcn_readfirstlane(seen)) break;
-        if (group_removes(v, off, lab, vb, len, c * kWave) ||
-            chunk_removes(f, v, K, off, lab, srt + (vb - base), hcnt + (uint64_t)(v - v0) * K, m,
-                          len, c * kWave, q, streamed))
-          if (lane == 0)
-            __hip_atomic_store(&sh_hit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t end =
+            group_removes(v, off, lab, vb, len, c * kWave)
+                ? kPairsRemove
+                : chunk_removes(f, v, K, off, lab, srt + (vb - base), hcnt + (uint64_t)(v - v0) * K,
+                                m, len, c * kWave, q, look, streamed);
+        if (end != kPairsKeep && lane == 0) atomicOr(&sh_hit, end);
       }
       __syncthreads();
-      if (threadIdx.x == 0 && sh_hit) redo[atomicAdd(&ctr[0], 1u)] = v;
+      if (threadIdx.x == 0 && sh_hit) {
+        if (sh_hit & kPairsRemove)
+          redo[atomicAdd(&ctr[0], 1u)] = v;
+        else
+          left[atomicAdd(&ctr[8], 1u)] = v;
+      }
       __syncthreads();
     }
   }
@@ -718,11 +750,11 @@ __device__ __attribute__((always_inline)) inline bool clean_vertex(
   return sh_removed != 0;
 }
 
-// ctr[0]: redo count, ctr[2]: next vertex, ctr[4..5]: labels of L(u) read (u64).  gtile: per-workgroup arena slices
+// The n vertices from 0, or those of `list`.  ctr[0]: redo count, ctr[2]: next vertex, ctr[4..5]: labels of L(u) read (u64).  gtile: per-workgroup arena slices
 // of gwords words for tiles above lds_slots slots.
 template <class V, class S>
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)))
-k_clean_tile(uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
+k_clean_tile(uint32_t n, const uint32_t *list, uint32_t K, const unsigned long long *__restrict__ off,
              const unsigned long long *__restrict__ lab, S str,
              uint32_t *redo, uint32_t *ctr, uint32_t lds_slots, uint32_t *gtile,
              uint64_t gwords, uint32_t win, uint32_t indexed) {
@@ -744,8 +776,9 @@ k_clean_tile(uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
     __syncthreads();
     // wave-uniform values are made explicit, so the list offsets and hubs are
     // scalar loads and the loops over them carry no per-lane masks
-    const uint32_t v = __builtin_amdgcn_readfirstlane(sh_v);
-    if (v >= n) break;
+    const uint32_t next = __builtin_amdgcn_readfirstlane(sh_v);
+    if (next >= n) break;
+    const uint32_t v = list ? list[next] : next;
     const unsigned long long vb = off[v];
     const uint32_t len = (uint32_t)(off[v + 1] - vb);
     const unsigned long long *Lv = lab + vb;
@@ -1137,7 +1170,9 @@ int clean_index(hsdl_index *idx) {
   const bool hop_sort = env_u32("HSDL_CLEAN_HOP_SORT", 1, 0, 1);
   const uint32_t form = hop_sort ? env_u32("HSDL_CLEAN_PAIRS", 1, 0, 2) : 0u;
   const bool pairs = form == 2 || (form == 1 && n >= kPairLists && idx->total <= kPairMean * n);
+  // (the lists that the pairs leave to the tiles stand where the lengths will)
   if (pairs && ((rc = take_scratch(dev, kCsLongs, longs, n * 4ull + 4)) ||
+                (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull)) ||
                 (rc = take_scratch(dev, kCsMins, mins, (uint64_t)n * idx->K * 4))))
     return rc;
   hipLaunchKernelGGL(k_clean_min, dim3(grid), dim3(256), 0, st, n, (uint32_t)idx->K, off, lab,
@@ -1158,6 +1193,52 @@ int clean_index(hsdl_index *idx) {
       env_u32("HSDL_STREAM32", 1, 0, 1) && hub_bits + hop_bits + dist_bits <= 32;
   uint64_t width = use32 ? 4 : 8;
   const uint64_t t_kern = now_ns();
+  // k_clean_tile over `cnt` vertices (those of `list`, if any), streaming the hop-
+  // ordered 32-bit copy of all labels, or the index
+  auto tiles = [&](uint32_t count, const uint32_t *list, bool copy) -> int {
+    const uint32_t K1 = (uint32_t)idx->K + 1;
+    const bool small_vals = mx[1] < 0xFFFFu;
+    // indexed LDS tiles need hub << kIdxBits to fit a word (tuning knob
+    // HSDL_CLEAN_INDEXED=0: per-slot values only)
+    const uint32_t indexed =
+        (uint64_t)n <= (1ull << (32 - kIdxBits)) ? env_u32("HSDL_CLEAN_INDEXED", 1, 0, 1) : 0u;
+    const uint32_t slot_bytes = 4 + K1 * (small_vals ? 2 : 4);
+    // tuning knob HSDL_CLEAN_LDS_SLOTS caps the LDS tile (small values send
+    // every vertex to the global arena)
+    uint32_t lds_slots = (kTileLdsBytes - 16) / slot_bytes;
+    lds_slots = env_u32("HSDL_CLEAN_LDS_SLOTS", lds_slots, 1, lds_slots);
+    const size_t lds_bytes = (size_t)lds_slots * slot_bytes + 16;
+    const int tgrid = std::max(1, cus * 2);
+    // tuning knob HSDL_CLEAN_WINDOW: labels of L(v) per wave work unit
+    const uint32_t win = env_u32("HSDL_CLEAN_WINDOW", kTileWindow, 1, kMaxWindow);
+    const uint32_t gcap = tile_cap_for(mx[0]);
+    const uint64_t gwords =
+        small_vals ? tile_words<uint16_t>(gcap, K1) : tile_words<uint32_t>(gcap, K1);
+    if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
+    auto launch = [&](auto kern, auto str) {
+      hipLaunchKernelGGL(kern, dim3(tgrid), dim3(kTileThreads), lds_bytes, st, count, list,
+                         (uint32_t)idx->K, off, lab, str, redo.as<uint32_t>(), cnt, lds_slots,
+                         gtile.as<uint32_t>(), gwords, win, indexed);
+    };
+    const Stream32 s32{srt.as<uint32_t>(), hop_bits, dist_bits, hcnt.as<uint32_t>(),
+                       (uint32_t)idx->K};
+    const Stream64 s64{lab};
+    if (small_vals) {
+      if (copy) launch(k_clean_tile<uint16_t, Stream32>, s32);
+      else launch(k_clean_tile<uint16_t, Stream64>, s64);
+    } else {
+      if (copy) launch(k_clean_tile<uint32_t, Stream32>, s32);
+      else launch(k_clean_tile<uint32_t, Stream64>, s64);
+    }
+    HSDL_HIP(hipGetLastError());
+    return HSDL_OK;
+  };
+  uint32_t hc[9] = {};  // the counters (k_clean_pairs)
+  auto counters = [&]() -> int {
+    HSDL_HIP(hipMemcpyAsync(hc, ctr.p, sizeof(hc), hipMemcpyDeviceToHost, st));
+    HSDL_HIP(hipStreamSynchronize(st));
+    return HSDL_OK;
+  };
   if (pairs) {
     // The hop-ordered copy holds a slice of the vertices: all of them up to
     // kSliceBytes (tuning knob HSDL_CLEAN_SLICE: labels), fewer when there is no
@@ -1192,13 +1273,15 @@ int clean_index(hsdl_index *idx) {
         HSDL_HIP(hipMemsetAsync(cnt + 1, 0, 8, st));
         hipLaunchKernelGGL((k_clean_pairs<F, false>), dim3(grid), dim3(256), 0, st, f, v0, v1,
                            (uint32_t)idx->K, off, lab, srt.as<T>(), hcnt.as<uint32_t>(),
-                           mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(), cnt);
+                           mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(),
+                           new_len.as<uint32_t>(), cnt);
         HSDL_HIP(hipGetLastError());
         if (mx[0] > kCleanLong) {
           HSDL_HIP(hipMemsetAsync(cnt + 2, 0, 4, st));
           hipLaunchKernelGGL((k_clean_pairs<F, true>), dim3(grid), dim3(256), 0, st, f, v0, v1,
                              (uint32_t)idx->K, off, lab, srt.as<T>(), hcnt.as<uint32_t>(),
-                             mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(), cnt);
+                             mins.as<uint32_t>(), redo.as<uint32_t>(), longs.as<uint32_t>(),
+                             new_len.as<uint32_t>(), cnt);
           HSDL_HIP(hipGetLastError());
         }
         v0 = v1;
@@ -1207,26 +1290,13 @@ int clean_index(hsdl_index *idx) {
     };
     if (idx->total && (rc = use32 ? pass1(Pair32{hop_bits, dist_bits}) : pass1(Pair64{})))
       return rc;
+    if ((rc = counters())) return rc;
+    if (hc[8]) {
+      HSDL_HIP(hipMemsetAsync(cnt + 2, 0, 4, st));
+      if ((rc = tiles(hc[8], new_len.as<uint32_t>(), use32 && hoff.empty())) || (rc = counters()))
+        return rc;
+    }
   } else {
-    const uint32_t K1 = (uint32_t)idx->K + 1;
-    const bool small_vals = mx[1] < 0xFFFFu;
-    // indexed LDS tiles need hub << kIdxBits to fit a word (tuning knob
-    // HSDL_CLEAN_INDEXED=0: per-slot values only)
-    const uint32_t indexed =
-        (uint64_t)n <= (1ull << (32 - kIdxBits)) ? env_u32("HSDL_CLEAN_INDEXED", 1, 0, 1) : 0u;
-    const uint32_t slot_bytes = 4 + K1 * (small_vals ? 2 : 4);
-    // tuning knob HSDL_CLEAN_LDS_SLOTS caps the LDS tile (small values send
-    // every vertex to the global arena)
-    uint32_t lds_slots = (kTileLdsBytes - 16) / slot_bytes;
-    lds_slots = env_u32("HSDL_CLEAN_LDS_SLOTS", lds_slots, 1, lds_slots);
-    const size_t lds_bytes = (size_t)lds_slots * slot_bytes + 16;
-    const int tgrid = std::max(1, cus * 2);
-    // tuning knob HSDL_CLEAN_WINDOW: labels of L(v) per wave work unit
-    const uint32_t win = env_u32("HSDL_CLEAN_WINDOW", kTileWindow, 1, kMaxWindow);
-    const uint32_t gcap = tile_cap_for(mx[0]);
-    const uint64_t gwords =
-        small_vals ? tile_words<uint16_t>(gcap, K1) : tile_words<uint32_t>(gcap, K1);
-    if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
     // the heads' lists are streamed from a hop-ordered 32-bit copy of all
     // labels, or from the index when fields or memory do not allow it
     const bool copy =
@@ -1240,31 +1310,13 @@ int clean_index(hsdl_index *idx) {
       (void)hipGetLastError();
       width = 8;
     }
-    auto launch = [&](auto kern, auto str) {
-      hipLaunchKernelGGL(kern, dim3(tgrid), dim3(kTileThreads), lds_bytes, st, n,
-                         (uint32_t)idx->K, off, lab, str, redo.as<uint32_t>(), cnt, lds_slots,
-                         gtile.as<uint32_t>(), gwords, win, indexed);
-    };
-    const Stream32 s32{srt.as<uint32_t>(), hop_bits, dist_bits, hcnt.as<uint32_t>(),
-                       (uint32_t)idx->K};
-    const Stream64 s64{lab};
-    if (small_vals) {
-      if (copy) launch(k_clean_tile<uint16_t, Stream32>, s32);
-      else launch(k_clean_tile<uint16_t, Stream64>, s64);
-    } else {
-      if (copy) launch(k_clean_tile<uint32_t, Stream32>, s32);
-      else launch(k_clean_tile<uint32_t, Stream64>, s64);
-    }
-    HSDL_HIP(hipGetLastError());
+    if ((rc = tiles(n, nullptr, copy)) || (rc = counters())) return rc;
   }
-  uint32_t hc[6] = {0, 0, 0, 0, 0, 0};
-  HSDL_HIP(hipMemcpyAsync(hc, ctr.p, 24, hipMemcpyDeviceToHost, st));
-  HSDL_HIP(hipStreamSynchronize(st));
   const uint64_t t_passes = now_ns();
   // nothing falls: the index stays as it is
   if (hc[0]) {
     if ((rc = take_scratch(dev, kCsKeep, keep, std::max<uint64_t>(idx->total, 1))) ||
-        (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull)) ||
+        (!new_len.p && (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull))) ||
         (rc = take_scratch(dev, kCsOff, noff, (n + 1ull) * 8)))
       return rc;
     HSDL_HIP(hipMemsetAsync(keep.p, 1, idx->total, st));
@@ -1324,8 +1376,9 @@ int clean_index(hsdl_index *idx) {
   const uint64_t t_end = now_ns();
   idx->stats.t_clean_s = (t_end - t0) * 1e-9;
   if (getenv("HSDL_VERBOSE"))
-    fprintf(stderr, "[hsdl] clean: %.3f s set-up, %.3f s pass 1, %.3f s pass 2 and compaction\n",
-            (t_kern - t0) * 1e-9, (t_passes - t_kern) * 1e-9, (t_end - t_passes) * 1e-9);
+    fprintf(stderr, "[hsdl] clean: %.3f s set-up, %.3f s pass 1 (%u lists left to tiles), "
+            "%.3f s pass 2 and compaction\n",
+            (t_kern - t0) * 1e-9, (t_passes - t_kern) * 1e-9, hc[8], (t_end - t_passes) * 1e-9);
   return HSDL_OK;
 }
 

@@ -158,3 +158,62 @@ def test_pool_that_runs_out_between_vertices(monkeypatch, stream32):
         same_labels(H.hop_constrained_two_hop_labels_generation(
             g, K, hub_batch=batch, pool_init_labels=16 * n + extra),
             O.kround(csr_of(g), K).arrays())
+
+
+def skewed(rng, n, short, longs, size, K, far):
+    """n - longs lists of up to `short` even hubs, then `longs` lists of `size`
+    odd ones: pairs of a long list's labels find no partner in its heads' lists,
+    but for its few even hubs.  far: distances fall with the hop, so that no pair
+    passes the clean's distance bound; else nearly all do."""
+    lists, base = [], n - longs
+    for v in range(n):
+        if v < base:
+            u = np.sort(rng.choice((v + 1) // 2, min(v // 2, short), replace=False)) * 2
+            u = u[u < v]
+            hop, dist = rng.integers(1, K + 1, len(u)), rng.integers(1, 10, len(u))
+        else:
+            odd = rng.choice(base // 2, size, replace=False) * 2 + 1
+            u = np.unique(np.concatenate([odd, rng.choice(base // 2, 5) * 2]))
+            hop = rng.integers(1, K + 1, len(u))
+            dist = 1000 * (K - hop) + 500 + rng.integers(0, 400, len(u)) if far else \
+                rng.integers(5, 60, len(u))
+        lists.append((np.append(u, v), np.append(hop, 0), np.append(dist, 0)))
+    off = np.concatenate([[0], np.cumsum([len(x[0]) for x in lists])]).astype(np.uint64)
+    hub, hop, dist = (np.concatenate([x[i] for x in lists]) for i in range(3))
+    return off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32)
+
+
+@pytest.mark.parametrize("stream32,piece", [("1", None), ("0", None), ("1", "9000")])
+@pytest.mark.parametrize("far", [False, True])
+def test_clean_leaves_costly_lists_to_the_tiles(monkeypatch, stream32, piece, far):
+    """Lists whose pairs are too many for the clean's pair form go on to the
+    tiles: from a wave's lists and from a workgroup's (past 1,024 labels), from
+    32-bit and 8-byte copies, whole and sliced, beside lists that stay: the
+    oracle's clean."""
+    monkeypatch.setenv("HSDL_CLEAN_PAIRS", "2")
+    monkeypatch.setenv("HSDL_STREAM32", stream32)
+    if piece:
+        monkeypatch.setenv("HSDL_CLEAN_SLICE", piece)
+    rng = np.random.default_rng(12)
+    for n, short, longs, size, K in ((5000, 20, 12, 1900, 5), (5000, 20, 40, 1000, 5), (17000, 10, 3, 8300, 4),
+                                     (2000, 9, 200, 300, 15)):
+        a = skewed(rng, n, short, longs, size, K, far)
+        want = O.clean(O.labels_from_arrays(n, a[0].astype(np.int64), *a[1:]))
+        print(f"[skewed clean] n={n} size={size} far={far} kept={want.total()} of {len(a[1])}",
+              flush=True)
+        idx = H.Index.from_labels(n, K, *a)
+        idx.clean()
+        same_labels(idx, want.arrays())
+
+
+def test_clean_of_a_few_long_lists_is_not_quadratic():
+    """Four lists of 60,000 labels whose heads have twenty each: 0.34 s by pairs
+    alone, a twentieth of that where they go on to the tiles."""
+    a = skewed(np.random.default_rng(3), 140000, 20, 4, 60000, 5, False)
+    sec = []
+    for _ in range(3):
+        idx = H.Index.from_labels(140000, 5, *a)
+        idx.clean()
+        sec.append(idx.stats()["t_clean_s"])
+    print(f"[long lists] {sec}", flush=True)
+    assert min(sec) < 0.1
