@@ -27,13 +27,14 @@
 // lists and hashes a smaller one.  Labels of hop k matter only for hub a or b,
 // which ranks above the list's vertex: only the lower-ranked endpoint's list is
 // read that far, unless the index holds hubs ranked below their vertex
-// (imported label sets may).  A part of more labels than half the table is
-// hashed and probed in pieces.  What binds is instructions (a probe about 15
+// (imported label sets may).  A query with a part of more labels than half the
+// table reads the 8-byte labels as k_query64 does; hashing it in pieces streamed
+// the other list once per piece (20,000 queries between lists of 5,000 labels 1.37
+// ms, now 0.52).  What binds is instructions (a probe about 15
 // for 64 labels, a turn of its chain 10): 2^22 queries of an R-MAT 262,144
-// index at K = 5 (672 labels per list, k uniform in 1..5) take 5.98 ms, 701 M
+// index at K = 5 (672 labels per list, k uniform in 1..5) take 5.24 ms, 800 M
 // q/s; a workgroup of four waves per query, with both whole lists in registers
-// and LDS, took 19.2 ms.  512 or 2,048 table slots per wave: 13.4 and 10.2 ms
-// (chunked parts; fewer waves resident).
+// and LDS, took 19.2 ms.
 //
 // k_query64 reads the index's 8-byte labels, in (hub, hop, dist) order, where
 // there is no copy (fields wider than 32 bits, no memory, none made yet).  The
@@ -74,16 +75,120 @@ struct QChunk {
       : per((uint32_t)min<uint64_t>(kWave, (nq + waves - 1) / waves)) {}
 };
 
+// 8-byte labels: pieces of the longer list B in LDS, searched by the shorter
+// list A's labels.  Both are hub-sorted, so a chunk of A whose hubs lie below
+// the piece is never read again; a run of B cut by a piece's end is found in
+// both pieces.
+// kN threads' work: a wave's, or a workgroup's (a piece of 512 labels per wave,
+// the waves taking chunks of A in turn).  Returns the least distance of (s, t, k),
+// k > 0, s != t, over this lane's pairs.
+constexpr uint32_t kQPiece = 512;  // labels, 4 KB per wave
+// Where B is far the longer, A's labels search it in memory: 100,000 queries of a
+// list of 20 labels and one of 16,000 (60,000) 0.87 -> 0.11 ms (2.6 -> 0.12).  The
+// search is a chain of a dozen loads: between lists of up to 8,192 labels that lie
+// in HBM (R-MAT 2^20 vertices, K = 5) it loses to the pieces, 9.2 against 8.4 ms.
+constexpr uint32_t kQSearchLen = 8192;
+constexpr uint32_t kQSearchRatio = 64;
+__device__ inline bool searched(uint32_t alen, uint32_t blen) {
+  return blen > kQSearchLen && (uint64_t)alen * kQSearchRatio <= blen;
+}
+template <uint32_t kN>
+__device__ inline uint32_t join64(const unsigned long long *__restrict__ off,
+                                  const unsigned long long *__restrict__ lab, uint32_t s,
+                                  uint32_t t, uint32_t kk, lds_ptr<unsigned long long> P) {
+  constexpr bool kTeam = kN > kWave;
+  constexpr uint32_t kPiece = kN / kWave * kQPiece;
+  const uint32_t lane = (uint32_t)lane_id(), id = kTeam ? threadIdx.x : lane;
+  auto sync = [] {
+    if constexpr (kTeam)
+      __syncthreads();
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  unsigned long long abeg = off[s], bbeg = off[t];
+  uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
+  if (alen > blen) {
+    const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
+    const uint32_t l = alen; alen = blen; blen = l;
+  }
+  const unsigned long long *A = lab + abeg, *B = lab + bbeg;
+  uint32_t best = kInf32;
+  // this wave's chunks of A below j0 are done
+  uint32_t j0 = kTeam ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * kWave : 0u;
+  if (searched(alen, blen)) {
+    for (; j0 < alen; j0 += kN) {
+      const unsigned long long a = A[min(j0 + lane, alen - 1)];
+      const uint32_t w = label_hub(a), h1 = label_hop(a);
+      if (h1 > kk) continue;
+      uint32_t lo = 0, hi = blen;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (label_hub(B[mid]) < w) lo = mid + 1; else hi = mid;
+      }
+      for (; lo < blen; ++lo) {  // <= K + 1 labels, hops ascending
+        const unsigned long long l = B[lo];
+        if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
+        best = min(best, label_dist(a) + label_dist(l));
+      }
+    }
+    return best;
+  }
+  for (uint32_t p0 = 0; p0 < blen && (kTeam || j0 < alen); p0 += kPiece) {
+    const uint32_t m = min(kPiece, blen - p0);
+    for (uint32_t i = id; i < m; i += 4 * kN) {
+      unsigned long long l[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) l[u] = B[p0 + min(i + u * kN, m - 1)];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (i + u * kN < m) P[i + u * kN] = l[u];
+    }
+    sync();
+    const uint32_t lo_hub = label_hub(P[0]), hi_hub = label_hub(P[m - 1]);
+    for (uint32_t j = j0; j < alen; j += kN) {
+      const unsigned long long a = A[min(j + lane, alen - 1)];
+      const uint32_t w = label_hub(a), h1 = label_hop(a);
+      if (__builtin_amdgcn_readlane(w, 0) > hi_hub) break;
+      if (__builtin_amdgcn_readlane(w, kWave - 1) < lo_hub) {
+        j0 = j + kN;
+        continue;
+      }
+      if (w < lo_hub || w > hi_hub || h1 > kk) continue;
+      // first label of the piece with hub >= w (there is one)
+      uint32_t lo = 0, hi = m - 1;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
+      }
+      for (uint32_t x = lo; x < m; ++x) {  // <= K + 1 labels, hops ascending
+        const unsigned long long l = P[x];
+        if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
+        best = min(best, label_dist(a) + label_dist(l));
+      }
+    }
+    sync();
+  }
+  return best;
+}
+
+// LDS words of a wave of the query copy's kernels: its table, or a piece of 8-byte
+// labels.
+__host__ __device__ inline uint32_t slice_words(uint32_t slots) {
+  return slots > 2 * kQPiece ? slots : 2 * kQPiece;
+}
+
 // The least distance of (s, t, k), k > 0, s != t, over this lane's pairs
 // (kInf32: none).  kN threads' work: a wave's, or a workgroup's in step.
 // hcnt[v * K + x], x < K: labels of v of hop <= x.  below: the index holds hubs
-// ranked below their vertex.  T: a table of `slots`, a power of two.
+// ranked below their vertex.  T: slice_words per wave, a table of `slots`, a power
+// of two.  lab64: the 8-byte labels.
 template <uint32_t kN>
 __device__ inline uint32_t join32(const Lab32 &fmt, uint32_t K,
                                   const unsigned long long *__restrict__ off,
                                   const uint32_t *__restrict__ lab,
                                   const uint32_t *__restrict__ hcnt, uint32_t below, uint32_t s,
-                                  uint32_t t, int k, lds_ptr<uint32_t> T, uint32_t slots) {
+                                  uint32_t t, int k, lds_ptr<uint32_t> T, uint32_t slots,
+                                  const unsigned long long *__restrict__ lab64) {
   constexpr bool kTeam = kN > kWave;
   const uint32_t id = kTeam ? threadIdx.x : (uint32_t)lane_id();
   auto sync = [] {
@@ -111,6 +216,9 @@ __device__ inline uint32_t join32(const Lab32 &fmt, uint32_t K,
   const uint32_t ac = upto(a, alen, c), bc = upto(b, blen, kk - 1 - c);
   const uint32_t a1 = upto(a, alen, kk - 1), b1 = upto(b, blen, kk - 1);
   const uint32_t ak = upto(a, alen, kk), bk = upto(b, blen, kk);
+  // a part that outgrows the table, or a list that is searched
+  if (__builtin_expect(max(ac - a0, bc - b0) > slots / 2 || searched(alen, blen), 0))
+    return join64<kN>(off, lab64, s, t, kk, (lds_ptr<unsigned long long>)T);
   uint32_t best = kInf32;       // pairs of hops >= 1
   uint32_t at_a = kInf32, at_b = kInf32;  // labels of hub a in L(b), of b in L(a)
 
@@ -132,32 +240,28 @@ __device__ inline uint32_t join32(const Lab32 &fmt, uint32_t K,
   // hashes X[xb, xe), probes with Y[yb, ye)
   auto join = [&](const uint32_t *X, uint32_t xb, uint32_t xe, const uint32_t *Y, uint32_t yb,
                   uint32_t ye) {
-    while (xb < xe && yb < ye) {
-      // at most half the table; a quarter where it has room
-      const uint32_t part = min(xe - xb, slots / 2);
-      const uint32_t cap =
-          min(slots, 1u << (32 - __builtin_clz(max(64u, 4u * part) - 1)));
-      for (uint32_t i = id; i < cap * 4 / 16; i += kN) ((lds_ptr<u32x4>)T)[i] = u32x4{0, 0, 0, 0};
-      sync();
-      walk(X, xb, xb + part, [&](uint32_t l, bool own) {
-        if (!own) return;
-        uint32_t slot = hash_slot(fmt.hub(l), cap);
-        while (atomicCAS((uint32_t *)&T[slot], 0u, l) != 0u) slot = (slot + 1) & (cap - 1);
-      });
-      sync();
-      walk(Y, yb, ye, [&](uint32_t l, bool) {
-        const uint32_t w = fmt.hub(l), h = fmt.hop(l), d = fmt.dist(l);
-        uint32_t slot = hash_slot(w, cap);
-        uint32_t x = T[slot];
-        while (x != 0) {
-          if (fmt.hub(x) == w && fmt.hop(x) + h <= kk) best = min(best, d + fmt.dist(x));
-          slot = (slot + 1) & (cap - 1);
-          x = T[slot];
-        }
-      });
-      sync();
-      xb += part;
-    }
+    if (xb >= xe || yb >= ye) return;
+    // at most half the table; a quarter where it has room
+    const uint32_t cap = min(slots, 1u << (32 - __builtin_clz(max(64u, 4u * (xe - xb)) - 1)));
+    for (uint32_t i = id; i < cap * 4 / 16; i += kN) ((lds_ptr<u32x4>)T)[i] = u32x4{0, 0, 0, 0};
+    sync();
+    walk(X, xb, xe, [&](uint32_t l, bool own) {
+      if (!own) return;
+      uint32_t slot = hash_slot(fmt.hub(l), cap);
+      while (atomicCAS((uint32_t *)&T[slot], 0u, l) != 0u) slot = (slot + 1) & (cap - 1);
+    });
+    sync();
+    walk(Y, yb, ye, [&](uint32_t l, bool) {
+      const uint32_t w = fmt.hub(l), h = fmt.hop(l), d = fmt.dist(l);
+      uint32_t slot = hash_slot(w, cap);
+      uint32_t x = T[slot];
+      while (x != 0) {
+        if (fmt.hub(x) == w && fmt.hop(x) + h <= kk) best = min(best, d + fmt.dist(x));
+        slot = (slot + 1) & (cap - 1);
+        x = T[slot];
+      }
+    });
+    sync();
   };
   if (below || b > a) walk(B, b0, bk, [&](uint32_t l, bool) { endpoint(l, a, at_a); });
   if (below || a > b) walk(A, a0, ak, [&](uint32_t l, bool) { endpoint(l, b, at_b); });
@@ -173,11 +277,13 @@ __global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(
 k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restrict__ off,
           const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt, uint32_t below,
           uint64_t nq, const uint32_t *__restrict__ qs, const uint32_t *__restrict__ qt,
-          const int8_t *__restrict__ qk, int32_t *out, uint32_t slots) {
+          const int8_t *__restrict__ qk, int32_t *out, uint32_t slots,
+          const unsigned long long *__restrict__ lab64) {
   extern __shared__ uint4 qlds[];  // 16-byte stores clear the tables
   const uint32_t lane = (uint32_t)lane_id();
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  lds_ptr<uint32_t> T = (lds_ptr<uint32_t>)(reinterpret_cast<uint32_t *>(qlds) + wib * slots);
+  lds_ptr<uint32_t> T =
+      (lds_ptr<uint32_t>)(reinterpret_cast<uint32_t *>(qlds) + wib * slice_words(slots));
   const uint64_t waves = (uint64_t)gridDim.x * kQWaves;
   const QChunk ch(nq, waves);
   for (uint64_t q0 = ((uint64_t)blockIdx.x * kQWaves + wib) * ch.per; q0 < nq;
@@ -195,7 +301,7 @@ k_query32(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__restric
       const uint32_t best = wave_min_u32(
           join32<kWave>(fmt, K, off, lab, hcnt, below, __builtin_amdgcn_readlane(vs, qi),
                         __builtin_amdgcn_readlane(vt, qi), __builtin_amdgcn_readlane(vk, qi), T,
-                        slots));
+                        slots, lab64));
       if ((int)lane == qi) ans = best == kInf32 ? INT32_MAX : (int32_t)best;
     }
     if (mine) out[q0 + lane] = ans;
@@ -235,81 +341,12 @@ k_query32_team(Lab32 fmt, uint32_t n, uint32_t K, const unsigned long long *__re
                const uint32_t *__restrict__ lab, const uint32_t *__restrict__ hcnt,
                uint32_t below, uint64_t nq, const uint32_t *__restrict__ qs,
                const uint32_t *__restrict__ qt, const int8_t *__restrict__ qk, int32_t *out,
-               uint32_t slots) {
+               uint32_t slots, const unsigned long long *__restrict__ lab64) {
   extern __shared__ uint4 qlds[];
   team_queries<kN>(n, nq, qs, qt, qk, out, [&](uint32_t s, uint32_t t, int k) {
     return join32<kN>(fmt, K, off, lab, hcnt, below, s, t, k,
-                      (lds_ptr<uint32_t>)reinterpret_cast<uint32_t *>(qlds), slots);
+                      (lds_ptr<uint32_t>)reinterpret_cast<uint32_t *>(qlds), slots, lab64);
   });
-}
-
-// 8-byte labels: pieces of the longer list B in LDS, searched by the shorter
-// list A's labels.  Both are hub-sorted, so a chunk of A whose hubs lie below
-// the piece is never read again; a run of B cut by a piece's end is found in
-// both pieces.
-// kN threads' work: a wave's, or a workgroup's (a piece of 512 labels per wave,
-// the waves taking chunks of A in turn).  Returns the least distance of (s, t, k),
-// k > 0, s != t, over this lane's pairs.
-constexpr uint32_t kQPiece = 512;  // labels, 4 KB per wave
-template <uint32_t kN>
-__device__ inline uint32_t join64(const unsigned long long *__restrict__ off,
-                                  const unsigned long long *__restrict__ lab, uint32_t s,
-                                  uint32_t t, uint32_t kk, lds_ptr<unsigned long long> P) {
-  constexpr bool kTeam = kN > kWave;
-  constexpr uint32_t kPiece = kN / kWave * kQPiece;
-  const uint32_t lane = (uint32_t)lane_id(), id = kTeam ? threadIdx.x : lane;
-  auto sync = [] {
-    if constexpr (kTeam)
-      __syncthreads();
-    else
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  };
-  unsigned long long abeg = off[s], bbeg = off[t];
-  uint32_t alen = (uint32_t)(off[s + 1] - abeg), blen = (uint32_t)(off[t + 1] - bbeg);
-  if (alen > blen) {
-    const unsigned long long x = abeg; abeg = bbeg; bbeg = x;
-    const uint32_t l = alen; alen = blen; blen = l;
-  }
-  const unsigned long long *A = lab + abeg, *B = lab + bbeg;
-  uint32_t best = kInf32;
-  // this wave's chunks of A below j0 are done
-  uint32_t j0 = kTeam ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * kWave : 0u;
-  for (uint32_t p0 = 0; p0 < blen && (kTeam || j0 < alen); p0 += kPiece) {
-    const uint32_t m = min(kPiece, blen - p0);
-    for (uint32_t i = id; i < m; i += 4 * kN) {
-      unsigned long long l[4];
-#pragma unroll
-      for (uint32_t u = 0; u < 4; ++u) l[u] = B[p0 + min(i + u * kN, m - 1)];
-#pragma unroll
-      for (uint32_t u = 0; u < 4; ++u)
-        if (i + u * kN < m) P[i + u * kN] = l[u];
-    }
-    sync();
-    const uint32_t lo_hub = label_hub(P[0]), hi_hub = label_hub(P[m - 1]);
-    for (uint32_t j = j0; j < alen; j += kN) {
-      const unsigned long long a = A[min(j + lane, alen - 1)];
-      const uint32_t w = label_hub(a), h1 = label_hop(a);
-      if (__builtin_amdgcn_readlane(w, 0) > hi_hub) break;
-      if (__builtin_amdgcn_readlane(w, kWave - 1) < lo_hub) {
-        j0 = j + kN;
-        continue;
-      }
-      if (w < lo_hub || w > hi_hub || h1 > kk) continue;
-      // first label of the piece with hub >= w (there is one)
-      uint32_t lo = 0, hi = m - 1;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
-      }
-      for (uint32_t x = lo; x < m; ++x) {  // <= K + 1 labels, hops ascending
-        const unsigned long long l = P[x];
-        if (label_hub(l) != w || h1 + label_hop(l) > kk) break;
-        best = min(best, label_dist(a) + label_dist(l));
-      }
-    }
-    sync();
-  }
-  return best;
 }
 
 __global__ void __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(8)))
@@ -522,7 +559,7 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
   }
   const bool copy = want32 && idx->q32.load(std::memory_order_acquire) == 1;
   const uint32_t slots = copy ? query_slots(idx) : 0;
-  const size_t lds = (size_t)slots * 4 * kQWaves;
+  const size_t lds = copy ? (size_t)slice_words(slots) * 4 * kQWaves : 0;
   const bool team = use_team(idx, nq, shared);
   const bool wide = team && nq <= kWideQueries && lds <= 32 * 1024;  // 64 KB at most
   const uint32_t threads = wide ? 2 * kQThreads : kQThreads;
@@ -538,7 +575,7 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
                        (uint32_t)idx->K, idx->off.as<unsigned long long>(),
                        idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total,
                        idx->hubs_below ? 1u : 0u, (uint64_t)nq, d_s, d_t, d_k, d_out,
-                       team ? slots * (threads / kWave) : slots);
+                       team ? slots * (threads / kWave) : slots, idx->lab.as<unsigned long long>());
   } else {
     hipLaunchKernelGGL(wide ? k_query64_team<2 * kQThreads>
                             : team ? k_query64_team<kQThreads> : k_query64,

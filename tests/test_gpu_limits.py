@@ -1,5 +1,7 @@
 """Builds, cleans and host calls at the limits of their buffers, lists and
 counters.  Labels, answers and counts are integers: every comparison is exact."""
+import time
+
 import numpy as np
 import pytest
 
@@ -217,3 +219,64 @@ def test_clean_of_a_few_long_lists_is_not_quadratic():
         sec.append(idx.stats()["t_clean_s"])
     print(f"[long lists] {sec}", flush=True)
     assert min(sec) < 0.1
+
+
+def mixed_lists(rng, n, sizes, K, top):
+    """n - len(sizes) lists of up to 20 hubs, then one of each of `sizes`."""
+    base, rows = n - len(sizes), []
+    for v in range(n):
+        m = min(v, int(rng.integers(0, 21))) if v < base else sizes[v - base]
+        u = np.sort(rng.choice(min(v, base), m, replace=False)) if m else np.zeros(0, int)
+        rows.append((np.append(u, v), np.append(rng.integers(1, K + 1, m), 0),
+                     np.append(rng.integers(1, top, m), 0)))
+    off = np.concatenate([[0], np.cumsum([len(x[0]) for x in rows])]).astype(np.uint64)
+    hub, hop, dist = (np.concatenate([x[i] for x in rows]) for i in range(3))
+    return off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32)
+
+
+@pytest.mark.parametrize("team", ["0", "6000"])
+@pytest.mark.parametrize("q32,slots", [("1", "1024"), ("1", "2048"), ("0", "1024")])
+def test_query_of_lists_far_above_the_mean(monkeypatch, q32, slots, team):
+    """A few long lists among many short ones: parts that fill the table to the
+    last slot and outgrow it (answered from the 8-byte labels, in pieces), and
+    lists past 8,192 labels that a short one searches, beside every other pair
+    of lengths, a wave, four and eight waves per query: the oracle's answers."""
+    monkeypatch.setenv("HSDL_QUERY32", q32)
+    monkeypatch.setenv("HSDL_QUERY_SLOTS", slots)
+    monkeypatch.setenv("HSDL_QUERY_TEAM", team)
+    rng = np.random.default_rng(41)
+    n, K = 20000, 5
+    sizes = [128, 129, 510, 514, 1023, 1030, 2600, 5200, 8191, 8193, 8200, 12000, 12000]
+    a = mixed_lists(rng, n, sizes, K, 2000)
+    want = O.labels_from_arrays(n, a[0].astype(np.int64), *a[1:])
+    idx = H.Index.from_labels(n, K, *a)
+    s, t = rng.integers(0, n, (2, 6000))
+    s[:4000] = n - len(sizes) + rng.integers(0, len(sizes), 4000)
+    t[2000:4000] = n - len(sizes) + rng.integers(0, len(sizes), 2000)
+    s, t = s.astype(np.uint32), t.astype(np.uint32)
+    swap = rng.random(6000) < 0.5
+    s, t = np.where(swap, t, s), np.where(swap, s, t)
+    k = rng.integers(-1, K + 3, 6000).astype(np.int8)
+    ans = O.query(want, s, t, k)
+    for m in (6000, 1000, 1):
+        print(f"[long lists] q32={q32} slots={slots} team={team} queries={m}", flush=True)
+        o = 1500
+        sl = slice(0, m) if m > 1000 else slice(o, o + m)
+        assert np.array_equal(idx.query(s[sl], t[sl], k[sl]), ans[sl])
+
+
+def test_queries_of_a_short_and_a_long_list_are_quick():
+    """100,000 queries of a list of at most 20 labels and one of 60,000: 0.2 ms
+    with their copies, and 5 ms where all of the long list is read."""
+    rng = np.random.default_rng(6)
+    n, nq = 70000, 100000
+    idx = H.Index.from_labels(n, 5, *mixed_lists(rng, n, [60000] * 16, 5, 2000))
+    s, t = rng.integers(100, 60000, nq).astype(np.uint32), rng.integers(n - 16, n, nq).astype(np.uint32)
+    k = rng.integers(2, 6, nq).astype(np.int8)
+    sec = []
+    for _ in range(6):
+        t0 = time.perf_counter()
+        idx.query(s, t, k)
+        sec.append(time.perf_counter() - t0)
+    print(f"[short and long] {sec}", flush=True)
+    assert min(sec) < 2e-3
