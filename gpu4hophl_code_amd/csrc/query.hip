@@ -514,33 +514,51 @@ int prepare_query(const hsdl_index *idx) {
 
 // Table slots per wave: a list part is a few hundred labels, hashed at a load
 // of a quarter where the table has room; 1,024 slots are 16 KB per workgroup
-// and keep a CU's 32 waves resident, and indexes of longer lists take twice
-// that for 20 waves.  Tuning knob HSDL_QUERY_SLOTS (a power of two from 64).
-static uint32_t query_slots(const hsdl_index *idx) {
-  const uint64_t mean = idx->n ? idx->total / idx->n : 0;
-  return pow2_at_most(env_u32("HSDL_QUERY_SLOTS", mean <= 1024 ? 1024 : 2048, 64, 4096));
+// and keep a CU's 32 waves resident.  2^21 queries of R-MAT 2^20 vertices (1,218
+// labels per list) with 512 / 1,024 / 2,048 / 4,096 slots: 5.05 / 4.70 / 8.4 / 8.7 ms;
+// of 262,144 (672): 3.20 / 2.80 / 4.5 / 5.5.  Tuning knob HSDL_QUERY_SLOTS (a power of
+// two from 64).
+static uint32_t query_slots() { return pow2_at_most(env_u32("HSDL_QUERY_SLOTS", 1024, 64, 4096)); }
+
+static uint64_t mean_labels(const hsdl_index *idx) { return idx->n ? idx->total / idx->n : 0; }
+
+// Whether a call's queries get a workgroup each: up to a quarter of the square of
+// the mean list length, within [2,048, 131,072].  A call ends with its longest list's
+// query, and a call of few queries leaves waves idle beside it; many queries fill
+// the chip anyway, and a wave per query does the less work.  Team / wave, us:
+//   672 labels per list (R-MAT 262,144, K = 5): 8,192 queries 61 / 94, 65,536 211 / 230,
+//   131,072 385 / 337
+//   349 (65,536, K = 4): 32,768 120 / 105, 65,536 181 / 113; 8-byte labels 16,384 67 / 80
+//   123 (16,384, K = 4), 8-byte: 2,048 20 / 22, 4,096 24 / 23, 16,384 48 / 37
+// Calls in flight together (shared: a server's batches) have the chip filled by each
+// other: there up to 32,768 at most.
+// Up to 1,024 queries, or 2,048 of long lists, a team has eight waves: 672 labels,
+// four / eight: 512 27 / 22, 2,048 37 / 35; 1,209: 2,048 60 / 50; 349: 2,048 25 / 27.
+// Tuning knob HSDL_QUERY_TEAM: the most queries of a team call.
+static bool use_team(const hsdl_index *idx, uint64_t nq, bool shared) {
+  const uint64_t mean = std::min<uint64_t>(mean_labels(idx), 1024);
+  const uint64_t most =
+      std::min<uint64_t>(std::max<uint64_t>(mean * mean / 4, 2048), shared ? 1u << 15 : 1u << 17);
+  return nq <= env_u32("HSDL_QUERY_TEAM", (uint32_t)most, 0, 0xFFFFFFFFu);
+}
+static bool use_wide(const hsdl_index *idx, uint64_t nq) {
+  return nq <= (mean_labels(idx) > 512 ? 2048 : 1024);
 }
 
-// Whether a call's queries get a workgroup each: up to the square of the mean list
-// length, within [2,048, 131,072].  A call ends with its longest list's query, and a
-// call of few queries leaves waves idle beside it; many queries fill the chip
-// anyway, and a wave per query does the less work.  Team / wave, us:
-//   672 labels per list (R-MAT 262,144, K = 5): 1,024 queries 38 / 108, 8,192 61 /
-//   139, 65,536 196 / 260, 131,072 362 / 391, 262,144 686 / 622, 2^22 9.7 / 5.6 ms
-//   (8-byte labels, 1,024: 27 / 58, 65,536: 268 / 348, 262,144: 887 / 936)
-//   190 (65,536, K = 4): 1,024 24 / 34, 32,768 105 / 110, 65,536 171 / 127
-//   63 (grid, K = 8, 8-byte): 1,024 16 / 16, 8,192 22 / 18, 65,536 87 / 35
-// Calls in flight together (shared: a server's batches) have the chip filled by each
-// other: there up to 32,768 at most (2^20 requests in batches of up to 65,536: 6.9 ms
-// with teams up to 2,048 queries, 7.2 up to 32,768, 9.0 up to 65,536).
-// Up to kWideQueries, which that many workgroups of eight waves take at once, a
-// team has eight waves.
-// Tuning knob HSDL_QUERY_TEAM: the most queries of such a call.
-constexpr uint64_t kWideQueries = 1024;
-static bool use_team(const hsdl_index *idx, uint64_t nq, bool shared) {
-  const uint64_t mean = idx->n ? std::min<uint64_t>(idx->total / idx->n, 1024) : 0;
-  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>(mean * mean, 2048), shared ? 1u << 15 : 1u << 17);
-  return nq <= env_u32("HSDL_QUERY_TEAM", (uint32_t)most, 0, 0xFFFFFFFFu);
+// Whether a call reads the query copy, where there is one.  A query over it goes
+// through more round trips (prefix counts, table) for fewer labels, so small calls
+// and short lists read the 8-byte labels: up to 3 * 2^30 of queries times the
+// square of the mean list length.  8-byte / copy, us:
+//   123 labels per list: 16,384 queries 37 / 61, 131,072 119 / 132
+//   349: 1,024 20 / 27, 16,384 67 / 70, 32,768 109 / 105
+//   672: 1,024 27 / 30, 4,096 49 / 47, 8,192 71 / 61
+//   1,209: 1,024 36 / 40, 4,096 70 / 69, 8,192 109 / 93
+// (a workgroup of four waves per query over both lists, hub-ordered: 21, 24, 29
+// and 45 at 1,024).  HSDL_QUERY32=1 always reads the copy.
+static bool use_copy(const hsdl_index *idx, uint64_t nq) {
+  if (getenv("HSDL_QUERY32")) return true;
+  const double mean = (double)mean_labels(idx);
+  return (double)nq * mean * mean > 3.0 * 0x1p30;
 }
 
 int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const uint32_t *d_t,
@@ -557,11 +575,12 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
       if (rc) return rc;
     }
   }
-  const bool copy = want32 && idx->q32.load(std::memory_order_acquire) == 1;
-  const uint32_t slots = copy ? query_slots(idx) : 0;
+  const bool copy =
+      want32 && idx->q32.load(std::memory_order_acquire) == 1 && use_copy(idx, nq);
+  const uint32_t slots = copy ? query_slots() : 0;
   const size_t lds = copy ? (size_t)slice_words(slots) * 4 * kQWaves : 0;
   const bool team = use_team(idx, nq, shared);
-  const bool wide = team && nq <= kWideQueries && lds <= 32 * 1024;  // 64 KB at most
+  const bool wide = team && use_wide(idx, nq) && lds <= 32 * 1024;  // 64 KB at most
   const uint32_t threads = wide ? 2 * kQThreads : kQThreads;
   const uint32_t fill = query_grid(idx->device, copy, lds) / (threads / kQThreads);
   const uint32_t grid =

@@ -280,3 +280,26 @@ def test_queries_of_a_short_and_a_long_list_are_quick():
         sec.append(time.perf_counter() - t0)
     print(f"[short and long] {sec}", flush=True)
     assert min(sec) < 2e-3
+
+
+@pytest.mark.parametrize("n,K,ef", [(6000, 4, 16), (3000, 5, 4), (300, 15, 3)])
+def test_query_forms_by_call_size(n, K, ef):
+    """Calls on both sides of every line of the choice between the query copy
+    and the 8-byte labels, and between a wave, four and eight waves per query:
+    the oracle's answers, in one call and over the same requests in another."""
+    g = ragged(n, n, 1000, ef)
+    want = O.kround(csr_of(g), K)
+    idx = H.hop_constrained_two_hop_labels_generation(g, K)
+    mean = idx.label_count() // n
+    line = int(3 * 2 ** 30 / mean ** 2)
+    rng = np.random.default_rng(n)
+    sizes = {1, 2, 63, 64, 65, 1023, 1024, 1025, 2047, 2048, 2049, mean ** 2 // 4, mean ** 2 // 4 + 1,
+             line, line + 1, 150001}
+    most = 150001
+    s, t = rng.integers(0, n, (2, most)).astype(np.uint32)
+    t[:50] = s[:50]
+    k = rng.integers(-1, K + 3, most).astype(np.int8)
+    ans = O.query(want, s, t, k)
+    for m in sorted(x for x in sizes if 0 < x <= most):
+        print(f"[form] n={n} mean={mean} queries={m}", flush=True)
+        assert np.array_equal(idx.query(s[:m], t[:m], k[:m]), ans[:m])
