@@ -303,3 +303,31 @@ def test_query_forms_by_call_size(n, K, ef):
     for m in sorted(x for x in sizes if 0 < x <= most):
         print(f"[form] n={n} mean={mean} queries={m}", flush=True)
         assert np.array_equal(idx.query(s[:m], t[:m], k[:m]), ans[:m])
+
+
+@pytest.mark.parametrize("q32", ["0", "1"])
+@pytest.mark.parametrize("n", [900, 6000])
+def test_team_requests_in_chunks(monkeypatch, q32, n):
+    """A workgroup takes consecutive queries: one, several, 64 and more than 64
+    each, with a remainder at the call's end, queries without a join among
+    them: the oracle's answers, through host arrays, without allocation and
+    served."""
+    monkeypatch.setenv("HSDL_QUERY32", q32)
+    monkeypatch.setenv("HSDL_QUERY_TEAM", "10000000")
+    g = ragged(n, n, 100, 8)
+    want = O.kround(csr_of(g), 3)
+    idx = H.hop_constrained_two_hop_labels_generation(g, 3)
+    rng = np.random.default_rng(n)
+    most = 250007
+    s, t = rng.integers(0, n, (2, most)).astype(np.uint32)
+    t[::7] = s[::7]
+    k = rng.integers(-1, 5, most).astype(np.int8)
+    ans = O.query(want, s, t, k)
+    for m in (1, 1023, 1025, 2047, 2049, 4097, 10001, 131071, 131073, most):
+        print(f"[team chunks] n={n} q32={q32} queries={m}", flush=True)
+        assert np.array_equal(idx.query(s[:m], t[:m], k[:m]), ans[:m])
+        assert np.array_equal(idx.query_noalloc(s[:m], t[:m], k[:m]), ans[:m])
+    srv = H.Server(idx, max_batch=5003, max_wait_us=50, inflight=3)
+    got, _ = srv.replay(s, t, k, np.arange(most, dtype=np.uint64) * 5)
+    srv.close()
+    assert np.array_equal(got, ans)
