@@ -117,6 +117,11 @@ __device__ inline void wave_argmin2(unsigned long long &k1, unsigned long long &
 // a load from L2, 2^17 queries on R-MAT 65,536, K = 5, took 0.88 ms, with the
 // searched list in LDS 0.45 ms (host arrays and copies included 1.49 -> 1.01).
 constexpr uint32_t kPathPiece = 512;  // labels, 4 KB per wave
+// A list of more than kPathSearchLen labels and kPathSearchRatio times the other is
+// searched in memory: 50,000 paths between lists of 9 and 60,000 labels 1.32 -> 0.27
+// ms with their copies, of 5 and 4,000 0.29 -> 0.25.
+constexpr uint32_t kPathSearchLen = 2048;
+constexpr uint32_t kPathSearchRatio = 64;
 __global__ void __launch_bounds__(256) k_paths(size_t nq, const unsigned long long *__restrict__ off,
                                                const unsigned long long *__restrict__ lab,
                                                const uint32_t *__restrict__ par,
@@ -148,6 +153,39 @@ __global__ void __launch_bounds__(256) k_paths(size_t nq, const unsigned long lo
       const unsigned long long *A = lab + (a_is_s ? sb : tb), *B = lab + (a_is_s ? tb : sb);
       const uint32_t alen = a_is_s ? slen : tlen, blen = a_is_s ? tlen : slen;
       uint32_t j0 = 0;
+      // the pairs of A's label `ja` and those from position x of B[p0, p0 + m), held
+      // in P, of its hub
+      auto pairs = [&](auto P, uint32_t p0, uint32_t m, uint32_t x, uint32_t ja,
+                       unsigned long long la) {
+        const uint32_t w = label_hub(la), h1 = label_hop(la);
+        for (; x < m; ++x) {
+          const unsigned long long lb = P[x];
+          if (label_hub(lb) != w || (int32_t)(h1 + label_hop(lb)) > k) break;
+          const unsigned long long c1 =
+              ((unsigned long long)(label_dist(la) + label_dist(lb)) << 32) | w;
+          const uint32_t jb = p0 + x;
+          const unsigned long long c2 =
+              ((unsigned long long)(a_is_s ? ja : jb) << 32) | (a_is_s ? jb : ja);
+          if (c1 < k1 || (c1 == k1 && c2 < k2)) {
+            k1 = c1;
+            k2 = c2;
+          }
+        }
+      };
+      if (blen > kPathSearchLen && (uint64_t)alen * kPathSearchRatio <= blen) {
+        for (; j0 < alen; j0 += kWave) {
+          const uint32_t ja = min(j0 + (uint32_t)lane, alen - 1);
+          const unsigned long long la = A[ja];
+          const uint32_t w = label_hub(la);
+          if ((int32_t)label_hop(la) > k) continue;
+          uint32_t lo = 0, hi = blen;
+          while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (label_hub(B[mid]) < w) lo = mid + 1; else hi = mid;
+          }
+          pairs(B, 0, blen, lo, ja, la);
+        }
+      }
       for (uint32_t p0 = 0; p0 < blen && j0 < alen; p0 += kPathPiece) {
         const uint32_t m = min(kPathPiece, blen - p0);
         for (uint32_t i = lane; i < m; i += 4 * kWave) {
@@ -175,19 +213,7 @@ __global__ void __launch_bounds__(256) k_paths(size_t nq, const unsigned long lo
             const uint32_t mid = (lo + hi) >> 1;
             if (label_hub(P[mid]) < w) lo = mid + 1; else hi = mid;
           }
-          for (uint32_t x = lo; x < m; ++x) {
-            const unsigned long long lb = P[x];
-            if (label_hub(lb) != w || (int32_t)(h1 + label_hop(lb)) > k) break;
-            const unsigned long long c1 =
-                ((unsigned long long)(label_dist(la) + label_dist(lb)) << 32) | w;
-            const uint32_t jb = p0 + x;
-            const unsigned long long c2 =
-                ((unsigned long long)(a_is_s ? ja : jb) << 32) | (a_is_s ? jb : ja);
-            if (c1 < k1 || (c1 == k1 && c2 < k2)) {
-              k1 = c1;
-              k2 = c2;
-            }
-          }
+          pairs(P, p0, m, lo, ja, la);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }

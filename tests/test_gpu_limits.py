@@ -331,3 +331,39 @@ def test_team_requests_in_chunks(monkeypatch, q32, n):
     got, _ = srv.replay(s, t, k, np.arange(most, dtype=np.uint64) * 5)
     srv.close()
     assert np.array_equal(got, ans)
+
+
+@pytest.mark.parametrize("deg", [1000, 2600, 9000])
+def test_paths_between_short_and_long_lists(deg):
+    """A few vertices of the lowest ranks next to very many others: their lists
+    span several staged pieces of 512 labels, or are searched by the other's
+    where that is far shorter (past 2,048 labels); weights 1..2, so that equal
+    sums meet on both sides of a piece's end: the oracle's edges."""
+    n, last = 12000, 6
+    rng = np.random.default_rng(deg)
+    base = n - last
+    u = [np.full(deg, x) for x in range(base, n)]
+    v = [rng.choice(base, deg, replace=False) for _ in range(last)]
+    y = rng.integers(0, base, (2, 3 * n))
+    y = y[:, y[0] != y[1]]
+    u, v = np.concatenate(u + [y[0]]), np.concatenate(v + [y[1]])
+    g = H.Graph.from_edges(n, u.astype(np.uint32), v.astype(np.uint32),
+                           rng.integers(1, 3, len(u)).astype(np.int32))
+    idx = H.hop_constrained_two_hop_labels_generation(g, 2, parents=True)
+    want = O.kround(csr_of(g), 2)
+    lens = np.diff(np.asarray(want.arrays()[0]).astype(np.int64))
+    print(f"[paths] deg={deg} longest={lens.max()} mean={lens.mean():.0f}", flush=True)
+    assert lens.max() > 1024 and lens[-last:].min() > deg
+    short = np.argsort(lens)[:80]
+    assert deg < 2000 or lens[-last:].min() > 64 * lens[short].max()
+    s, t = rng.integers(0, n, (2, 3000)).astype(np.uint32)
+    s[:1800] = base + rng.integers(0, last, 1800)
+    t[:900] = rng.choice(short, 900)
+    t[900:1800] = base + rng.integers(0, last, 900)
+    swap = rng.random(3000) < 0.5
+    s, t = np.where(swap, t, s), np.where(swap, s, t)
+    k = rng.integers(0, 4, 3000).astype(np.int8)
+    edges, counts = idx.paths(s, t, k, cap=3)
+    wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), 3)
+    assert np.array_equal(counts.astype(np.int32), wcounts)
+    assert np.array_equal(edges.astype(np.int32), wedges)
