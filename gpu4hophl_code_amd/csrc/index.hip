@@ -91,12 +91,12 @@ int segmented_sort_labels(uint64_t *d_lab, uint64_t total, const uint64_t *d_off
 }
 
 // ------------------------------------------------------------- staging
+// The pool: plain pointers, so that giving a stage back allocates nothing (it
+// happens in a destructor, where a failed allocation would end the process) and
+// no device call runs while the process ends.
 static std::mutex g_stage_mu;
-// (never destroyed: no device call may run while the process ends)
-static std::vector<Stage *> &stage_pool() {
-  static std::vector<Stage *> *pool = new std::vector<Stage *>();
-  return *pool;
-}
+constexpr int kStageDevices = 64;
+static Stage *g_stages[kStageDevices][kStagesKept];
 
 Stage::~Stage() {
   for (int i = 0; i < 2; ++i) {
@@ -106,13 +106,12 @@ Stage::~Stage() {
 }
 
 int StageLease::take(int dev, size_t bytes, int slots, bool device) {
-  {
+  if (dev >= 0 && dev < kStageDevices) {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    for (size_t i = 0; i < pool.size(); ++i)
-      if (pool[i]->dev == dev) {
-        s_ = pool[i];
-        pool.erase(pool.begin() + i);
+    for (Stage *&x : g_stages[dev])
+      if (x) {
+        s_ = x;
+        x = nullptr;
         break;
       }
   }
@@ -147,33 +146,33 @@ StageLease::~StageLease() {
     if (s_->st[i]) (void)hipStreamSynchronize(s_->st[i]);
     keep = keep && s_->hbytes[i] <= kStageBytes && s_->d[i].bytes <= kStageBytes;
   }
-  if (keep) {
+  if (keep && s_->dev >= 0 && s_->dev < kStageDevices) {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    int kept = 0;
-    for (Stage *x : pool) kept += x->dev == s_->dev;
-    if (kept < kStagesKept) {
-      pool.push_back(s_);
-      return;
-    }
+    for (Stage *&x : g_stages[s_->dev])
+      if (!x) {
+        x = s_;
+        return;
+      }
   }
   delete s_;
 }
 
 void release_stages(int dev) {
-  std::vector<Stage *> gone;
-  {
-    std::lock_guard<std::mutex> g(g_stage_mu);
-    std::vector<Stage *> &pool = stage_pool();
-    for (size_t i = pool.size(); i-- > 0;)
-      if (dev < 0 || pool[i]->dev == dev) {
-        gone.push_back(pool[i]);
-        pool.erase(pool.begin() + i);
+  for (int d = 0; d < kStageDevices; ++d) {
+    if (dev >= 0 && d != dev) continue;
+    Stage *gone[kStagesKept];
+    {
+      std::lock_guard<std::mutex> g(g_stage_mu);
+      for (int i = 0; i < kStagesKept; ++i) {
+        gone[i] = g_stages[d][i];
+        g_stages[d][i] = nullptr;
       }
-  }
-  for (Stage *x : gone) {
-    (void)hipSetDevice(x->dev);
-    delete x;
+    }
+    for (Stage *x : gone) {
+      if (!x) continue;
+      (void)hipSetDevice(d);
+      delete x;
+    }
   }
 }
 
