@@ -263,27 +263,32 @@ int launch_query(const hsdl_index *idx, size_t nq, const uint32_t *d_s, const ui
 // Makes the index's 32-bit query copy now, when it fits (synchronous).
 int prepare_query(const hsdl_index *idx);
 
-// Staging of a host-array call: one or two slots, each a stream, pinned host
-// memory that kernels read and write in place, and device memory (when asked
-// for), of the bytes the call needs up to kStageBytes.  Calls take one from a
-// per-device pool of at most kStagesKept and give it back; a call that finds
-// none makes its own, so calls on several threads never share one.
-// hsdl_release_scratch frees the pool.
+// Staging of a host-array call: a stream and one or two slots of pinned host memory,
+// which kernels read and write in place, of the bytes the call needs up to
+// kStageBytes.  Calls take one from a per-device pool of at most kStagesKept and give
+// it back; a call that finds none makes its own, so calls on several threads never
+// share one.  hsdl_release_scratch frees the pool.
+// A process's first large call pays for what it makes: a stream takes 0.4 to 3 ms, the
+// first asynchronous copy from device memory 6.5 ms.  So the slots share one stream,
+// and kernels store answers where the host reads them.
 constexpr size_t kStageBytes = 4u << 20;  // per slot that is kept
 constexpr int kStagesKept = 4;
 struct Stage {
   int dev = 0;
-  hipStream_t st[2] = {nullptr, nullptr};
+  hipStream_t st = nullptr;
   uint8_t *h[2] = {nullptr, nullptr};
   size_t hbytes[2] = {0, 0};
-  DevBuf d[2];
+  hipEvent_t done[2] = {nullptr, nullptr};  // where a call has two slots
+  int slots = 1;                            // of the running call
+  // after slot x's kernel is launched, and before the host reads its answers
+  int sent(int x);
+  int wait(int x);
   ~Stage();
 };
 class StageLease {
  public:
-  // `slots` slots of at least `bytes` each on the current device `dev`; device:
-  // with device memory of the same size
-  int take(int dev, size_t bytes, int slots, bool device);
+  // `slots` slots of at least `bytes` each on the current device `dev`
+  int take(int dev, size_t bytes, int slots);
   Stage *operator->() const { return s_; }
   ~StageLease();
 
@@ -291,6 +296,10 @@ class StageLease {
   Stage *s_ = nullptr;
 };
 void release_stages(int dev);  // -1: every device
+
+// Brings the pages of an array that is about to be written into memory while a kernel
+// runs: fresh ones cost a fault each otherwise (10 MB of edges 3.4 ms).
+void fault_in(void *p, size_t bytes);
 
 // Whether every entry of a and b lies below n (no early exit: it vectorizes).
 inline bool all_below(const uint32_t *a, const uint32_t *b, size_t cnt, uint32_t n) {

@@ -3,6 +3,7 @@
 #include <cstring>  // rocPRIM's texture iterator uses memset on the host
 
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_segmented_radix_sort.hpp>
 
@@ -99,13 +100,27 @@ constexpr int kStageDevices = 64;
 static Stage *g_stages[kStageDevices][kStagesKept];
 
 Stage::~Stage() {
+  if (st) (void)hipStreamDestroy(st);
   for (int i = 0; i < 2; ++i) {
-    if (st[i]) (void)hipStreamDestroy(st[i]);
+    if (done[i]) (void)hipEventDestroy(done[i]);
     if (h[i]) (void)hipHostFree(h[i]);
   }
 }
 
-int StageLease::take(int dev, size_t bytes, int slots, bool device) {
+int Stage::sent(int x) {
+  if (slots > 1) HSDL_HIP(hipEventRecord(done[x], st));
+  return HSDL_OK;
+}
+
+int Stage::wait(int x) {
+  if (slots > 1)
+    HSDL_HIP(hipEventSynchronize(done[x]));
+  else
+    HSDL_HIP(hipStreamSynchronize(st));
+  return HSDL_OK;
+}
+
+int StageLease::take(int dev, size_t bytes, int slots) {
   if (dev >= 0 && dev < kStageDevices) {
     std::lock_guard<std::mutex> g(g_stage_mu);
     for (Stage *&x : g_stages[dev])
@@ -119,10 +134,15 @@ int StageLease::take(int dev, size_t bytes, int slots, bool device) {
     s_ = new Stage();
     s_->dev = dev;
   }
+  s_->slots = slots;
+  if (!s_->st) HSDL_HIP(hipStreamCreateWithFlags(&s_->st, hipStreamNonBlocking));
+  // a slot that is not kept afterwards has what the call needs and no more
   size_t want = 64u << 10;
-  while (want < bytes) want *= 2;
+  while (want < bytes && want < kStageBytes) want *= 2;
+  want = std::max(want, bytes);
   for (int i = 0; i < slots; ++i) {
-    if (!s_->st[i]) HSDL_HIP(hipStreamCreateWithFlags(&s_->st[i], hipStreamNonBlocking));
+    if (slots > 1 && !s_->done[i])
+      HSDL_HIP(hipEventCreateWithFlags(&s_->done[i], hipEventDisableTiming));
     if (s_->hbytes[i] < bytes) {
       if (s_->h[i]) (void)hipHostFree(s_->h[i]);
       s_->h[i] = nullptr;
@@ -130,22 +150,15 @@ int StageLease::take(int dev, size_t bytes, int slots, bool device) {
       HSDL_HIP(hipHostMalloc((void **)&s_->h[i], want, hipHostMallocMapped | hipHostMallocCoherent));
       s_->hbytes[i] = want;
     }
-    if (device && s_->d[i].bytes < bytes) {
-      const int rc = s_->d[i].alloc(want);
-      if (rc) return rc;
-    }
   }
   return HSDL_OK;
 }
 
 StageLease::~StageLease() {
   if (!s_) return;
-  bool keep = true;
-  for (int i = 0; i < 2; ++i) {
-    // (a call that failed half-way may have work in flight)
-    if (s_->st[i]) (void)hipStreamSynchronize(s_->st[i]);
-    keep = keep && s_->hbytes[i] <= kStageBytes && s_->d[i].bytes <= kStageBytes;
-  }
+  // (a call that failed half-way may have work in flight)
+  if (s_->st) (void)hipStreamSynchronize(s_->st);
+  const bool keep = s_->hbytes[0] <= kStageBytes && s_->hbytes[1] <= kStageBytes;
   if (keep && s_->dev >= 0 && s_->dev < kStageDevices) {
     std::lock_guard<std::mutex> g(g_stage_mu);
     for (Stage *&x : g_stages[s_->dev])
@@ -174,6 +187,18 @@ void release_stages(int dev) {
       delete x;
     }
   }
+}
+
+void fault_in(void *p, size_t bytes) {
+#ifdef MADV_POPULATE_WRITE
+  const uintptr_t page = 4096, b = ((uintptr_t)p + page - 1) & ~(page - 1),
+                  e = ((uintptr_t)p + bytes) & ~(page - 1);
+  // (where the kernel does not know the call, the pages fault as they are written)
+  if (e > b) (void)madvise(reinterpret_cast<void *>(b), e - b, MADV_POPULATE_WRITE);
+#else
+  (void)p;
+  (void)bytes;
+#endif
 }
 
 }  // namespace hsdl

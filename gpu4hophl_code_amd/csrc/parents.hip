@@ -141,6 +141,21 @@ __global__ void __launch_bounds__(256) k_paths(size_t nq, const unsigned long lo
     int32_t k = qk[q];
     uint32_t cnt = 0;
     uint32_t *out = edges + 2 * (size_t)cap * q;
+    // the row's first 64 words are a lane's each and stored together: `edges` is host
+    // memory, where a store is a packet
+    uint32_t row = 0;
+    auto emit = [&](uint32_t v, uint32_t parent) {
+      const uint32_t at = 2 * cnt;
+      if (cnt < cap) {
+        if ((uint32_t)lane == at) row = v;
+        if ((uint32_t)lane == at + 1) row = parent;
+        if (at >= kWave && lane == 0) {
+          out[at] = v;
+          out[at + 1] = parent;
+        }
+      }
+      ++cnt;
+    };
     // every step that emits lowers k; a step that cannot emit ends the walk
     for (int32_t step = 0; step <= 256 && s != t; ++step) {
       const unsigned long long sb = off[s], tb = off[t];
@@ -223,26 +238,20 @@ __global__ void __launch_bounds__(256) k_paths(size_t nq, const unsigned long lo
       const uint32_t p2 = __builtin_amdgcn_readfirstlane(par[tb + (k2 & 0xFFFFFFFFull)]);
       if (p1 == s && p2 == t) break;
       if (p1 != s) {
-        if (lane == 0 && cnt < cap) {
-          out[2 * cnt] = s;
-          out[2 * cnt + 1] = p1;
-        }
-        ++cnt;
+        emit(s, p1);
         s = p1;
         --k;
       }
       if (p2 != t) {
-        if (lane == 0 && cnt < cap) {
-          out[2 * cnt] = t;
-          out[2 * cnt + 1] = p2;
-        }
-        ++cnt;
+        emit(t, p2);
         t = p2;
         --k;
       }
     }
     // slots past the path's end read 0
-    for (uint32_t e = 2 * min(cnt, cap) + (uint32_t)lane; e < 2 * cap; e += kWave) out[e] = 0;
+    if ((uint32_t)lane < 2 * cap) out[lane] = row;
+    for (uint32_t e = max(2 * min(cnt, cap), (uint32_t)kWave) + lane; e < 2 * cap; e += kWave)
+      out[e] = 0;
     if (lane == 0) counts[q] = cnt;
   }
 }
@@ -324,28 +333,27 @@ static int extract_paths_body(const hsdl_index *idx, size_t n, const uint32_t *s
   int dev = 0;
   int rc = use_device(idx->device, &dev);
   if (rc) return rc;
-  // a slot: requests (9 B a query) read in place, then counts and edges, written
-  // in device memory and copied back together
+  // a slot: requests (9 B a query), counts and edges, read and written in place; the
+  // host's part of a slot runs beside the other slot's kernel
   const size_t per = 13 + (size_t)8 * cap;
   // (a query whose edges exceed a kept slot gets slots of its own)
   const size_t most = std::max<size_t>(1, (kStageBytes - 64) / per);
   const size_t part = std::min(n, most >= 4 ? most & ~(size_t)3 : most);
   StageLease stage;
-  if ((rc = stage.take(dev, part * per + 64, n > part ? 2 : 1, true))) return rc;
+  if ((rc = stage.take(dev, part * per + 64, n > part ? 2 : 1))) return rc;
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, idx->device);
   size_t sent = 0, first[2] = {0, 0}, cnt[2] = {0, 0};
   for (int x = 0;; x ^= 1) {
-    uint8_t *h = stage->h[x], *d = stage->d[x].as<uint8_t>();
+    uint8_t *h = stage->h[x];
     uint32_t *hs = reinterpret_cast<uint32_t *>(h), *ht = hs + part;
     int8_t *hk = reinterpret_cast<int8_t *>(ht + part);
-    const size_t at = (part * 9 + 15) & ~(size_t)15;  // counts, then edges
+    uint32_t *hc = reinterpret_cast<uint32_t *>(h + ((part * 9 + 15) & ~(size_t)15));
     if (cnt[x]) {
-      HSDL_HIP(hipStreamSynchronize(stage->st[x]));
-      std::memcpy(counts + first[x], h + at, cnt[x] * 4);
+      if ((rc = stage->wait(x))) return rc;
+      std::memcpy(counts + first[x], hc, cnt[x] * 4);
       if (cap)
-        std::memcpy(edges + (size_t)2 * cap * first[x], h + at + cnt[x] * 4,
-                    (size_t)8 * cap * cnt[x]);
+        std::memcpy(edges + (size_t)2 * cap * first[x], hc + part, (size_t)8 * cap * cnt[x]);
       cnt[x] = 0;
     }
     if (sent < n) {
@@ -354,13 +362,12 @@ static int extract_paths_body(const hsdl_index *idx, size_t n, const uint32_t *s
       std::memcpy(ht, t + sent, m * 4);
       std::memcpy(hk, k + sent, m);
       const size_t blocks = std::min<size_t>((m + 3) / 4, (size_t)cus * 16);
-      hipLaunchKernelGGL(k_paths, dim3((uint32_t)blocks), dim3(256), 0, stage->st[x], m,
+      hipLaunchKernelGGL(k_paths, dim3((uint32_t)blocks), dim3(256), 0, stage->st, m,
                          idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                         idx->par.as<uint32_t>(), hs, ht, hk, cap,
-                         reinterpret_cast<uint32_t *>(d + m * 4), reinterpret_cast<uint32_t *>(d));
+                         idx->par.as<uint32_t>(), hs, ht, hk, cap, hc + part, hc);
       HSDL_HIP(hipGetLastError());
-      HSDL_HIP(hipMemcpyAsync(h + at, d, m * 4 + (size_t)8 * cap * m, hipMemcpyDeviceToHost,
-                              stage->st[x]));
+      if ((rc = stage->sent(x))) return rc;
+      fault_in(edges + (size_t)2 * cap * sent, (size_t)8 * cap * m);
       first[x] = sent;
       cnt[x] = m;
       sent += m;

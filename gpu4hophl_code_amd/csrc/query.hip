@@ -647,11 +647,11 @@ static int query_body(const hsdl_index *idx, size_t n, const uint32_t *s, const 
   int rc = use_device(idx->device, &dev);
   if (rc) return rc;
   // the kernel reads the requests from pinned memory and writes the answers
-  // there; a slot's copies overlap the other slot's queries
+  // there; a slot's copies run beside the other slot's queries
   constexpr size_t kPart = (size_t)1 << 18;
   static_assert(kPart * 13 <= kStageBytes, "a part fits a slot");
   StageLease stage;
-  if ((rc = stage.take(dev, std::min(n, kPart) * 13, n > kPart ? 2 : 1, false))) return rc;
+  if ((rc = stage.take(dev, std::min(n, kPart) * 13, n > kPart ? 2 : 1))) return rc;
   const size_t part = std::min(n, kPart);
   size_t sent = 0, first[2] = {0, 0}, cnt[2] = {0, 0};
   for (int x = 0;; x ^= 1) {
@@ -660,7 +660,7 @@ static int query_body(const hsdl_index *idx, size_t n, const uint32_t *s, const 
     int32_t *ho = reinterpret_cast<int32_t *>(ht + part);
     int8_t *hk = reinterpret_cast<int8_t *>(ho + part);
     if (cnt[x]) {
-      HSDL_HIP(hipStreamSynchronize(stage->st[x]));
+      if ((rc = stage->wait(x))) return rc;
       std::memcpy(out + first[x], ho, cnt[x] * 4);
       cnt[x] = 0;
     }
@@ -669,7 +669,7 @@ static int query_body(const hsdl_index *idx, size_t n, const uint32_t *s, const 
       std::memcpy(hs, s + sent, m * 4);
       std::memcpy(ht, t + sent, m * 4);
       std::memcpy(hk, k + sent, m);
-      if ((rc = launch_query(idx, m, hs, ht, hk, ho, stage->st[x]))) return rc;
+      if ((rc = launch_query(idx, m, hs, ht, hk, ho, stage->st)) || (rc = stage->sent(x))) return rc;
       first[x] = sent;
       cnt[x] = m;
       sent += m;

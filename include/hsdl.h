@@ -194,8 +194,8 @@ int hsdl_clean(hsdl_index *idx);
 
 /* Frees the working buffers hsdl_clean keeps on a device (-1: every device)
  * for the next clean: its flags, counts, hop-ordered label copy and tile
- * arena, and the index arrays a clean replaced; and the staging buffers (pinned and
- * device memory, at most 4 x 16 MB) that hsdl_query and hsdl_extract_paths
+ * arena, and the index arrays a clean replaced; and the staging buffers (pinned
+ * host memory, at most 4 x 8 MB) that hsdl_query and hsdl_extract_paths
  * keep for the next call.  No counterpart in the reference
  * (memory management of this library); the graph's build buffers go with
  * hsdl_graph_release_device. */

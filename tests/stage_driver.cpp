@@ -20,7 +20,7 @@ int main() {
   for (int turn = 0; turn < 2 * hsdl::kStagesKept; ++turn) {
     // (no GPU here: taking the stream fails, the stage itself exists)
     hsdl::StageLease a, b;
-    const int ra = a.take(0, 100, 1, false), rb = b.take(0, 100, 2, true);
+    const int ra = a.take(0, 100, 1), rb = b.take(0, 100, 2);
     if (ra == HSDL_OK || rb == HSDL_OK) {
       std::puts("a GPU answered");
       return 1;

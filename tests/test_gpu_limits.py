@@ -1,5 +1,8 @@
 """Builds, cleans and host calls at the limits of their buffers, lists and
 counters.  Labels, answers and counts are integers: every comparison is exact."""
+import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -367,3 +370,54 @@ def test_paths_between_short_and_long_lists(deg):
     wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), 3)
     assert np.array_equal(counts.astype(np.int32), wcounts)
     assert np.array_equal(edges.astype(np.int32), wedges)
+
+
+@pytest.mark.parametrize("cap", [1, 7, 31, 32, 33, 70])
+def test_path_rows_of_every_width(cap):
+    """Paths of up to 30 edges (K = 15 on a path) into rows below, at and past the 64
+    words that a wave stores at once, cut at the row's end: the oracle's rows."""
+    n, K = 61, 15
+    at = np.argsort(np.abs(np.arange(n) - n // 2), kind="stable")  # the middle ranks first
+    ids = np.argsort(at).astype(np.uint32)
+    g = H.Graph.from_edges(n, ids[:-1], ids[1:], np.full(n - 1, 2, np.int32))
+    idx = H.hop_constrained_two_hop_labels_generation(g, K, parents=True)
+    want = O.kround(csr_of(g), K)
+    s, t = (x.ravel().astype(np.uint32) for x in np.meshgrid(np.arange(n), np.arange(n)))
+    k = np.full(n * n, 40, np.int8)
+    edges, counts = idx.paths(s, t, k, cap=cap)
+    wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), cap)
+    print(f"[path rows] cap={cap} longest={wcounts.max()}", flush=True)
+    assert wcounts.max() == 30
+    assert np.array_equal(counts.astype(np.int32), wcounts)
+    assert np.array_equal(edges.astype(np.int32), wedges)
+
+
+FIRST_CALLS = """
+import sys, time
+import numpy as np
+import gpu4hophl_code_amd as H
+g = H.Graph.rmat(12, 8, 1, 1, 100)
+n = g.info()[0]
+idx = H.hop_constrained_two_hop_labels_generation(g, 4, parents=True)
+rng = np.random.default_rng(1)
+s, t = rng.integers(0, n, (2, 1 << 18)).astype(np.uint32)
+k = rng.integers(1, 5, 1 << 18).astype(np.int8)
+t0 = time.perf_counter()
+idx.paths(s[:1024], t[:1024], k[:1024], cap=4)
+idx.paths(s, t, k, cap=4)
+print(1e3 * (time.perf_counter() - t0))
+"""
+
+
+def test_first_host_calls_of_a_process():
+    """A small and a large path call, the first of their process: 5 ms together, and 16
+    with a second stream and the process's first asynchronous copy in them."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    ms = []
+    for _ in range(3):
+        out = subprocess.run([sys.executable, "-c", FIRST_CALLS], cwd=root, timeout=100,
+                             capture_output=True, text=True)
+        assert out.returncode == 0, out.stderr[-2000:]
+        ms.append(float(out.stdout.split()[-1]))
+        print(f"[first calls] {ms[-1]:.2f} ms", flush=True)
+    assert min(ms) < 11
