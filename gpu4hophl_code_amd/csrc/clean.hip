@@ -1142,18 +1142,20 @@ int clean_index(hsdl_index *idx) {
   } guard{st};
   DevBuf keep, new_len, noff, nlab, redo, ctr, srt, hcnt, mins, longs, gtile;
   const int dev = idx->device;
-  // every buffer taken from the kept ones goes back when the clean ends
+  // every buffer taken from the kept ones goes back when the clean ends (a clean
+  // that failed may have kernels in flight on them)
   struct Give {
+    hipStream_t st;
     int dev;
     DevBuf *b[9];
     int id[9];
     ~Give() {
+      (void)hipStreamSynchronize(st);
       for (int i = 0; i < 9; ++i) give_scratch(dev, id[i], *b[i]);
     }
-  } give{dev, {&keep, &new_len, &redo, &srt, &hcnt, &mins, &longs, &ctr, &gtile},
+  } give{st, dev, {&keep, &new_len, &redo, &srt, &hcnt, &mins, &longs, &ctr, &gtile},
          {kCsKeep, kCsNewLen, kCsRedo, kCsSrt, kCsHcnt, kCsMins, kCsLongs, kCsCtr, kCsGtile}};
   if ((rc = take_scratch(dev, kCsRedo, redo, n * 4ull + 4)) ||
-      (rc = take_scratch(dev, kCsHcnt, hcnt, (uint64_t)n * idx->K * 4)) ||
       (rc = take_scratch(dev, kCsCtr, ctr, (1 + kMaxLines) * kMaxStride * 4)))
     return rc;
   // counters (k_clean_pairs; [3]: pass 2's error bits, [6], [7]: its lists), then the maxima's lines
@@ -1169,12 +1171,23 @@ int clean_index(hsdl_index *idx) {
   // order, no hop-ordered copy)
   const bool hop_sort = env_u32("HSDL_CLEAN_HOP_SORT", 1, 0, 1);
   const uint32_t form = hop_sort ? env_u32("HSDL_CLEAN_PAIRS", 1, 0, 2) : 0u;
-  const bool pairs = form == 2 || (form == 1 && n >= kPairLists && idx->total <= kPairMean * n);
+  bool pairs = form == 2 || (form == 1 && n >= kPairLists && idx->total <= kPairMean * n);
+  const uint64_t hop_bytes = (uint64_t)n * idx->K * 4;
+  // The hop-ordered copy and what belongs to it only save time: where the device has
+  // no room for them, or for what comes after them, the clean goes on without.
+  auto drop_copy = [&] {
+    (void)hipStreamSynchronize(st);
+    for (DevBuf *b : {&srt, &hcnt, &mins, &longs}) b->release();
+  };
   // (the lists that the pairs leave to the tiles stand where the lengths will)
-  if (pairs && ((rc = take_scratch(dev, kCsLongs, longs, n * 4ull + 4)) ||
-                (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull)) ||
-                (rc = take_scratch(dev, kCsMins, mins, (uint64_t)n * idx->K * 4))))
-    return rc;
+  if (pairs && (take_scratch(dev, kCsLongs, longs, n * 4ull + 4) ||
+                take_scratch(dev, kCsNewLen, new_len, n * 4ull) ||
+                take_scratch(dev, kCsMins, mins, hop_bytes) ||
+                take_scratch(dev, kCsHcnt, hcnt, hop_bytes))) {
+    drop_copy();
+    new_len.release();
+    pairs = false;
+  }
   hipLaunchKernelGGL(k_clean_min, dim3(grid), dim3(256), 0, st, n, (uint32_t)idx->K, off, lab,
                      pairs ? mins.as<uint32_t>() : nullptr, cnt + kMaxStride);
   HSDL_HIP(hipGetLastError());
@@ -1214,7 +1227,13 @@ int clean_index(hsdl_index *idx) {
     const uint32_t gcap = tile_cap_for(mx[0]);
     const uint64_t gwords =
         small_vals ? tile_words<uint16_t>(gcap, K1) : tile_words<uint32_t>(gcap, K1);
-    if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
+    if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) {
+      if (!srt.p) return rc;
+      drop_copy();
+      copy = false;
+      width = 8;
+      if ((rc = take_scratch(dev, kCsGtile, gtile, (uint64_t)tgrid * gwords * 4))) return rc;
+    }
     auto launch = [&](auto kern, auto str) {
       hipLaunchKernelGGL(kern, dim3(tgrid), dim3(kTileThreads), lds_bytes, st, count, list,
                          (uint32_t)idx->K, off, lab, str, redo.as<uint32_t>(), cnt, lds_slots,
@@ -1239,20 +1258,23 @@ int clean_index(hsdl_index *idx) {
     HSDL_HIP(hipStreamSynchronize(st));
     return HSDL_OK;
   };
-  if (pairs) {
-    // The hop-ordered copy holds a slice of the vertices: all of them up to
-    // kSliceBytes (tuning knob HSDL_CLEAN_SLICE: labels), fewer when there is no
-    // room for it, at least the longest list.
-    constexpr uint64_t kSliceBytes = 2ull << 30;
-    uint64_t cap = std::min<uint64_t>(idx->total, kSliceBytes / width);
-    cap = std::max<uint64_t>({std::min<uint64_t>(cap, env_u32("HSDL_CLEAN_SLICE", 0xFFFFFFFFu, 1,
-                                                             0xFFFFFFFFu)),
-                              mx[0], 1});
-    constexpr uint64_t kPad = 64;  // labels read past a list's end (masked)
-    while ((rc = take_scratch(dev, kCsSrt, srt, (cap + kPad) * width))) {
-      if (rc != HSDL_ENOMEM || cap <= mx[0]) return rc;
-      cap = std::max<uint64_t>(cap / 2, mx[0]);
+  // The hop-ordered copy of the pairs holds a slice of the vertices: all of them up to
+  // kSliceBytes (tuning knob HSDL_CLEAN_SLICE: labels), fewer when there is no room
+  // for it, at least the longest list.
+  constexpr uint64_t kSliceBytes = 2ull << 30;
+  constexpr uint64_t kPad = 64;  // labels read past a list's end (masked)
+  uint64_t cap = std::min<uint64_t>(idx->total, kSliceBytes / width);
+  cap = std::max<uint64_t>({std::min<uint64_t>(cap, env_u32("HSDL_CLEAN_SLICE", 0xFFFFFFFFu, 1,
+                                                           0xFFFFFFFFu)),
+                            mx[0], 1});
+  while (pairs && take_scratch(dev, kCsSrt, srt, (cap + kPad) * width)) {
+    if (cap <= mx[0]) {
+      drop_copy();
+      pairs = false;
     }
+    cap = std::max<uint64_t>(cap / 2, mx[0]);
+  }
+  if (pairs) {
     std::vector<uint64_t> hoff;
     if (idx->total > cap) {
       hoff.resize(n + 1ull);
@@ -1299,15 +1321,15 @@ int clean_index(hsdl_index *idx) {
   } else {
     // the heads' lists are streamed from a hop-ordered 32-bit copy of all
     // labels, or from the index when fields or memory do not allow it
-    const bool copy =
-        use32 && hop_sort && take_scratch(dev, kCsSrt, srt, idx->total * 4) == HSDL_OK;
+    const bool copy = use32 && hop_sort &&
+                      take_scratch(dev, kCsHcnt, hcnt, hop_bytes) == HSDL_OK &&
+                      take_scratch(dev, kCsSrt, srt, idx->total * 4) == HSDL_OK;
     if (copy) {
       hipLaunchKernelGGL(k_clean_sort<Pair32>, dim3(grid), dim3(256), 0, st,
                          Pair32{hop_bits, dist_bits}, 0u, n, (uint32_t)idx->K, off, lab,
                          srt.as<uint32_t>(), hcnt.as<uint32_t>());
       HSDL_HIP(hipGetLastError());
     } else {
-      (void)hipGetLastError();
       width = 8;
     }
     if ((rc = tiles(n, nullptr, copy)) || (rc = counters())) return rc;
@@ -1315,9 +1337,19 @@ int clean_index(hsdl_index *idx) {
   const uint64_t t_passes = now_ns();
   // nothing falls: the index stays as it is
   if (hc[0]) {
-    if ((rc = take_scratch(dev, kCsKeep, keep, std::max<uint64_t>(idx->total, 1))) ||
-        (!new_len.p && (rc = take_scratch(dev, kCsNewLen, new_len, n * 4ull))) ||
-        (rc = take_scratch(dev, kCsOff, noff, (n + 1ull) * 8)))
+    // (the first pass has ended: its buffers make room)
+    auto with_room = [&](auto &&alloc) -> int {
+      if (alloc() == HSDL_OK) return HSDL_OK;
+      drop_copy();
+      gtile.release();
+      return alloc();
+    };
+    auto take = [&](int id, DevBuf &b, uint64_t bytes) {
+      return with_room([&] { return take_scratch(dev, id, b, bytes); });
+    };
+    if ((rc = take(kCsKeep, keep, std::max<uint64_t>(idx->total, 1))) ||
+        (!new_len.p && (rc = take(kCsNewLen, new_len, n * 4ull))) ||
+        (rc = take(kCsOff, noff, (n + 1ull) * 8)))
       return rc;
     HSDL_HIP(hipMemsetAsync(keep.p, 1, idx->total, st));
     hipLaunchKernelGGL(k_clean_keep_all, dim3(grid), dim3(256), 0, st, n, off,
@@ -1333,7 +1365,8 @@ int clean_index(hsdl_index *idx) {
       // slice per workgroup (few workgroups: such vertices are rare)
       const uint32_t lgrid = 64;
       const uint32_t words = (mx[0] + 31) / 32;
-      if ((rc = long_bits.alloc((uint64_t)lgrid * 2 * words * 4))) return rc;
+      if ((rc = with_room([&] { return long_bits.alloc((uint64_t)lgrid * 2 * words * 4); })))
+        return rc;
       hipLaunchKernelGGL(k_clean_seq<true>, dim3(lgrid), dim3(kSeqThreads), 0, st,
                          (uint32_t)idx->K, off, lab, keep.as<uint8_t>(), new_len.as<uint32_t>(),
                          redo.as<uint32_t>(), cnt, cnt + 7, cnt + 3, long_bits.as<uint32_t>(),
@@ -1348,9 +1381,11 @@ int clean_index(hsdl_index *idx) {
     if ((rc = scan_counts_u32(new_len.as<uint32_t>(), noff.as<uint64_t>(), n, st))) return rc;
     uint64_t total = 0;
     HSDL_HIP(hipMemcpy(&total, noff.as<uint64_t>() + n, 8, hipMemcpyDeviceToHost));
-    if ((rc = take_scratch(dev, kCsLab, nlab, std::max<uint64_t>(total, 1) * 8))) return rc;
+    if ((rc = take(kCsLab, nlab, std::max<uint64_t>(total, 1) * 8))) return rc;
     DevBuf npar;
-    if (idx->has_parents && (rc = npar.alloc(std::max<uint64_t>(total, 1) * 4))) return rc;
+    if (idx->has_parents &&
+        (rc = with_room([&] { return npar.alloc(std::max<uint64_t>(total, 1) * 4); })))
+      return rc;
     hipLaunchKernelGGL(k_compact, dim3(grid), dim3(256), 0, st, n, off, lab, keep.as<uint8_t>(),
                        noff.as<unsigned long long>(), nlab.as<unsigned long long>(),
                        idx->has_parents ? idx->par.as<uint32_t>() : nullptr,

@@ -421,3 +421,34 @@ def test_first_host_calls_of_a_process():
         ms.append(float(out.stdout.split()[-1]))
         print(f"[first calls] {ms[-1]:.2f} ms", flush=True)
     assert min(ms) < 11
+
+
+@pytest.fixture(scope="module")
+def room_driver(tmp_path_factory):
+    """tests/clean_room_driver.cpp, and label sets with redundant labels: short lists, and
+    short lists with long ones that leave the pair form (tiles beside its copy)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    tmp = tmp_path_factory.mktemp("room")
+    exe, lib = str(tmp / "driver"), os.path.join(root, "gpu4hophl_code_amd")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(root, "include"),
+                           os.path.join(root, "tests", "clean_room_driver.cpp"), "-o", exe,
+                           "-rdynamic", "-L", lib, "-lhsdl", "-ldl", f"-Wl,-rpath,{lib}"])
+    dumps = []
+    for sizes in ([], [9000, 12000]):
+        a = mixed_lists(np.random.default_rng(8), 30000, sizes, 5, 300)
+        dumps.append(str(tmp / f"labels{len(sizes)}.bin"))
+        H.Index.from_labels(30000, 5, *a).save(dumps[-1])
+    return exe, dumps
+
+
+@pytest.mark.parametrize("what", ["room", "refused"])
+@pytest.mark.parametrize("longer", [0, 1])
+def test_clean_where_memory_is_short(room_driver, what, longer):
+    """A clean takes no more device memory than its least form (tiles over the index's own
+    labels) has to have: with exactly that much it gives the labels that it
+    gives with all there is.  Each allocation of a clean refused in turn: the same labels, or
+    the documented refusal, the index as it was and the next clean right."""
+    exe, dumps = room_driver
+    out = subprocess.run([exe, dumps[longer], "5", what], timeout=110, capture_output=True, text=True)
+    print(out.stdout, flush=True)
+    assert out.returncode == 0 and f"{what} done" in out.stdout, out.stderr[-2000:]
