@@ -3128,7 +3128,12 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   HSDL_HIP(hipStreamCreateWithFlags(&g.st, hipStreamNonBlocking));
   struct StreamGuard {
     hipStream_t s;
-    ~StreamGuard() { if (s) (void)hipStreamDestroy(s); }
+    // (a build that ends early has kernels in flight on buffers that ~Gen gives to
+    // the graph's next build)
+    ~StreamGuard() {
+      (void)hipStreamSynchronize(s);
+      (void)hipStreamDestroy(s);
+    }
   } sg{g.st};
   g.grid = grid_for_device(dev);
   g.prune_grid = g.grid / 2;

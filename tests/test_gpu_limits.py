@@ -452,3 +452,15 @@ def test_clean_where_memory_is_short(room_driver, what, longer):
     out = subprocess.run([exe, dumps[longer], "5", what], timeout=110, capture_output=True, text=True)
     print(out.stdout, flush=True)
     assert out.returncode == 0 and f"{what} done" in out.stdout, out.stderr[-2000:]
+
+
+def test_build_after_one_that_passed_its_deadline():
+    """A build that ends between batches leaves its buffers to the graph's next build,
+    with a batch's re-sort still queued: the next build's labels are another handle's."""
+    g, other = (H.Graph.rmat(15, 16, 5, 1, 100) for _ in range(2))
+    want = H.hop_constrained_two_hop_labels_generation(other, 4).labels()
+    for batch in (3000, 0, 700):
+        with pytest.raises(H.HSDLError) as e:
+            H.hop_constrained_two_hop_labels_generation(g, 4, hub_batch=batch, deadline_s=1e-6)
+        assert e.value.code == -5
+        same_labels(H.hop_constrained_two_hop_labels_generation(g, 4), want)
