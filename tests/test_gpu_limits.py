@@ -464,3 +464,48 @@ def test_build_after_one_that_passed_its_deadline():
             H.hop_constrained_two_hop_labels_generation(g, 4, hub_batch=batch, deadline_s=1e-6)
         assert e.value.code == -5
         same_labels(H.hop_constrained_two_hop_labels_generation(g, 4), want)
+
+
+@pytest.fixture(scope="module")
+def long_lists():
+    """Vertices of the lowest ranks next to 450 to 6,500 others: lists that grow past what
+    the re-sort holds in registers (1,024 labels, 512 of 8 bytes) and its LDS slices."""
+    degs = [450, 540, 900, 1100, 1340, 1420, 3000, 4000, 4300, 6500]
+    n = 8000
+    base = n - len(degs)
+    rng = np.random.default_rng(17)
+    u = [np.full(d, base + i) for i, d in enumerate(degs)]
+    v = [rng.choice(base, d, replace=False) for d in degs]
+    y = rng.integers(0, base, (2, 2 * n))
+    y = y[:, y[0] != y[1]]
+    u, v = np.concatenate(u + [y[0]]), np.concatenate(v + [y[1]])
+    g = H.Graph.from_edges(n, u.astype(np.uint32), v.astype(np.uint32),
+                           rng.integers(1, 30, len(u)).astype(np.int32))
+    return g, O.kround(csr_of(g), 3).arrays()
+
+
+@pytest.mark.parametrize("stream32,held,default", [("1", 1024, 4080), ("0", 512, 1360)])
+@pytest.mark.parametrize("lds,piece", [(None, None), ("0", None), ("700", None), ("0", "2000"),
+                                       ("700", "2000"), ("1300", "64")])
+def test_resort_of_long_lists(monkeypatch, long_lists, stream32, held, default, lds, piece):
+    """Lists around the re-sort's register limit, its LDS slice and its slice in memory:
+    scattered in LDS, in memory, or left unsorted past a capped slice, in 32- and
+    8-byte labels, over batches that add to lists sorted before: the oracle's labels."""
+    monkeypatch.setenv("HSDL_STREAM32", stream32)
+    monkeypatch.setenv("HSDL_RESORT_DIV", "8")
+    if lds:
+        monkeypatch.setenv("HSDL_SORT_LDS", lds)
+    if piece:
+        monkeypatch.setenv("HSDL_SORT_SLICE", piece)
+    g, want = long_lists
+    lens = np.diff(np.asarray(want[0]).astype(np.int64))
+    in_lds = int(lds or default)
+    most = max(in_lds, int(piece or lens.max()))
+    print(f"[re-sort] stream32={stream32} lds={lds} slice={piece} "
+          f"held={(lens <= held).sum()} lds={((lens > held) & (lens <= in_lds)).sum()} "
+          f"memory={((lens > max(held, in_lds)) & (lens <= most)).sum()} "
+          f"unsorted={(lens > max(held, most)).sum()}", flush=True)
+    assert (lens > max(held, most)).any() if piece else (lens > max(held, in_lds)).any()
+    assert in_lds <= held or ((lens > held) & (lens <= in_lds)).any()
+    for batch in (600, 0):
+        same_labels(H.hop_constrained_two_hop_labels_generation(g, 3, hub_batch=batch), want)
