@@ -1149,8 +1149,9 @@ int clean_index(hsdl_index *idx) {
     int dev;
     DevBuf *b[9];
     int id[9];
+    bool idle = false;
     ~Give() {
-      (void)hipStreamSynchronize(st);
+      if (!idle) (void)hipStreamSynchronize(st);
       for (int i = 0; i < 9; ++i) give_scratch(dev, id[i], *b[i]);
     }
   } give{st, dev, {&keep, &new_len, &redo, &srt, &hcnt, &mins, &longs, &ctr, &gtile},
@@ -1402,6 +1403,7 @@ int clean_index(hsdl_index *idx) {
     if (idx->has_parents) idx->par = std::move(npar);
     idx->total = total;
   }
+  give.idle = true;
   idx->cleaned = true;
   idx->stats.labels_cleaned = idx->total;
   idx->stats.clean_passes = hc[0] ? 2 : 1;

@@ -3128,10 +3128,11 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   HSDL_HIP(hipStreamCreateWithFlags(&g.st, hipStreamNonBlocking));
   struct StreamGuard {
     hipStream_t s;
-    // (a build that ends early has kernels in flight on buffers that ~Gen gives to
-    // the graph's next build)
+    // a build that ends early has kernels in flight on buffers that ~Gen gives to the
+    // graph's next build (the others have waited: a further wait costs 10 us)
+    bool idle = false;
     ~StreamGuard() {
-      (void)hipStreamSynchronize(s);
+      if (!idle) (void)hipStreamSynchronize(s);
       (void)hipStreamDestroy(s);
     }
   } sg{g.st};
@@ -3692,6 +3693,7 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   const uint64_t t_sorted = now_ns();
   // parents (optional): derived from the sorted uncleaned labels and the graph
   if (opts->parents && (rc = derive_parents(idx, hg, g.st))) return cleanup(rc);
+  sg.idle = true;
   const uint64_t t_end = now_ns();
   idx->stats.t_parents_s = (t_end - t_sorted) * 1e-9;
   if (g.verbose)
