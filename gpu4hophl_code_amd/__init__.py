@@ -473,7 +473,8 @@ def hop_constrained_two_hop_labels_generation(graph, K, mode=MODE_BATCHED, hub_b
 
 def release_scratch(device=-1):
     """Frees the working buffers the clean keeps on a device for the next
-    clean (-1: every device)."""
+    clean, and the staging that host-array queries and paths keep (-1: every
+    device)."""
     _check(lib().hsdl_release_scratch(device))
 
 

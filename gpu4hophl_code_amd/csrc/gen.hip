@@ -20,36 +20,40 @@
 // guarantees; labels of hubs > s never pair (L(s) holds hubs <= s only).
 // B = 1 is the plain one-hub-per-launch form.
 //
-// Per round, all on one stream, no host synchronisation:
-//   round_prep  -> zero per-hub counters
+// Per round, all on one stream, no host synchronisation (round_prep, the per-hub
+// counters and the flat list's first blocks, is part of the kernel before the round:
+// the batch's first, or the last round's append):
 //   expand      -> the frontier is grouped by vertex (the labels vertex x
-//                  gained in the last round, of many hubs); a wave takes 64
-//                  groups, binary-searches each x's id-sorted adjacency for
+//                  gained in the last round, of many hubs); a wave takes up to
+//                  64 groups, binary-searches each x's id-sorted adjacency for
 //                  the first neighbour above the batch's first hub and walks
 //                  the (edge, label) pairs edge-major, 64 at a time, so the
 //                  lanes of one edge reach the neighbour's slots of nearby
-//                  hub slots (slot windows, slot_at) in a few sectors;
-//                  candidates are deduplicated by atomicMin on a dense
-//                  per-(hub,vertex) slot that keeps the batch's earlier
-//                  rounds' minima (tagged per batch attempt); the first
-//                  toucher that undercuts them appends (hub,vertex) to a flat
-//                  list
+//                  hub slots (slot windows, slot_at) in a few sectors; large
+//                  groups are cut into pieces (expand_heavy); pairs a landmark
+//                  rejects open nothing, other candidates are deduplicated by
+//                  atomicMin on a dense per-(hub,vertex) slot that keeps the
+//                  batch's earlier rounds' minima (tagged per batch attempt);
+//                  the first toucher that undercuts them appends (hub,vertex)
+//                  to a flat list
 //   count       -> per-hub candidate counts of the flat list (LDS hash per
-//                  2048-entry chunk: one global atomic per chunk and hub)
+//                  2048- or 512-entry chunk: one global atomic per chunk and hub)
 //   chunk_scan  -> per-hub offsets and work items of `tile` candidates
 //   group       -> flat candidates scattered into per-hub runs (hubs tallied
-//                  per 2048-entry chunk in an LDS hash: one global
-//                  reservation per chunk and hub)
+//                  per chunk in an LDS hash: one global reservation per chunk
+//                  and hub)
 //   prune       -> persistent: a workgroup of 16 waves takes a work item,
-//                  stages the hub's labels L(s) in an LDS hash tile (hub ->
-//                  prefix-min dist per hop budget), then the waves take its
-//                  candidates one at a time, stream L(y) 128 labels per step
-//                  with the next step in flight and stop at the first witness
+//                  stages the hub's labels L(s) in an LDS tile (hub ->
+//                  smallest dist per hop), then the waves claim up to 8 of its
+//                  candidates at once, stream each L(y) 128 labels per step
+//                  with the next step in flight and stop at the first witness;
+//                  hubs with few candidates take a wave each, and dense rounds
+//                  take row items instead (prune_rows)
 //   reserve     -> grows label segments that the round's accepted labels
-//                  overflow (bump allocation in a device pool; no locks)
-//   append      -> writes accepted labels
-//   finalize    -> publishes segment lengths; each vertex's new labels
-//                  become its frontier group of the next round
+//                  overflow (bump allocation in a device pool; no locks),
+//                  publishes the new lengths and each vertex's frontier group
+//                  of the next round
+//   append      -> writes the accepted labels behind the old lengths
 // Capacities (label pool, tile arena, candidate and frontier lists) start
 // small; a batch that overflows one raises a flag, the later kernels of the
 // batch stand down, and the host rolls the batch back, grows the buffer and
@@ -366,8 +370,6 @@ __global__ void k_fill_u32(uint32_t *p, uint64_t n, uint32_t val) {
     p[i] = val;
 }
 
-// The first frontier: every hub of the batch with its self label (position
-// 0 of its list), one group each.
 // Frontier groups per chunk of the light expansion: 64 once that leaves every
 // wave a chunk; smaller rounds spread over the waves, since a chunk's steps are a
 // chain of memory round trips (64 groups of up to heavy_pairs pairs took a wave
@@ -409,6 +411,8 @@ __device__ inline void round_prep(const GenArgs &a, uint32_t gcnt) {
   }
 }
 
+// The first frontier: every hub of the batch with its self label (position
+// 0 of its list), one group each.
 __global__ void k_batch_begin(GenArgs a) {
   with_batch(a);
   for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < a.B; b += gridDim.x * blockDim.x) {
@@ -3073,10 +3077,11 @@ static int sort_zones(Gen &g, uint32_t maxlen, uint32_t resort_div) {
 // Batches double, or grow eightfold while the last one was below 1/16 of the
 // target (what follows is then below half of it: the work per hub falls along
 // the ranking): a small batch costs its rounds' launches whatever is in them.
-// The first batch has 64 hubs, or as many as 2^23 slots hold up to 512: its
-// candidates of a round then fit the smallest flat list (2^23 entries).  From 64
-// and doubling always, on the same kernels: 1,024 / 4,096 / 40,001 vertices 2.25 /
-// 3.9 / 36.1 -> 1.48 / 2.33 / 31.5 ms, a group of 65,536 15.1 -> 12.8 ms, R-MAT
+// The first batch has 64 hubs, or as many as 2^23 slots hold up to 512: up to 131,072
+// vertices its candidates of a round are then no more than the smallest flat list has
+// entries (2^23, less what its blocks leave empty).  Larger graphs, and a list
+// that runs out all the same, rely on the batch's rollback.  From 64 and doubling
+// always, on the same kernels: 1,024 / 4,096 / 40,001 vertices 2.25 / 3.9 / 36.1 -> 1.48 / 2.33 / 31.5 ms, a group of 65,536 15.1 -> 12.8 ms, R-MAT
 // 262,144 202 -> 201 ms; fourfold 1.45 / 2.45 / 31.9 / 13.2 / 201; a first batch of
 // 1,024 1.45 / 2.5 / 31.9 / 13.1 / 201.
 // The eightfold step and the larger first batch are for builds with room: a batch

@@ -115,7 +115,7 @@ __device__ inline void wave_argmin2(unsigned long long &k1, unsigned long long &
 // hub, position in L(s), position in L(t)), the pair the reference's merge
 // meets first at the minimum.  A step is a chain of searches: with every probe
 // a load from L2, 2^17 queries on R-MAT 65,536, K = 5, took 0.88 ms, with the
-// searched list in LDS 0.45 ms (host arrays and copies included 1.49 -> 1.01).
+// searched list in LDS 0.45 ms (host arrays and copies included 1.49 -> 0.84).
 constexpr uint32_t kPathPiece = 512;  // labels, 4 KB per wave
 // A list of more than kPathSearchLen labels and kPathSearchRatio times the other is
 // searched in memory: 50,000 paths between lists of 9 and 60,000 labels 1.32 -> 0.27
