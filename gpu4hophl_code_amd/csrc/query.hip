@@ -436,50 +436,143 @@ static uint32_t query_grid(int dev, bool copy, size_t lds) {
 }
 
 // The query copy: every list's labels as 32-bit words in hop order (any order
-// within a hop) and the prefix counts.  A wave per vertex counts its labels'
-// hops, then scatters them.
-__global__ void __launch_bounds__(256) k_pack_query32(uint32_t n, uint32_t K,
-                                                      const unsigned long long *off,
-                                                      const unsigned long long *lab, uint32_t *out,
-                                                      uint32_t *hcnt, uint32_t hsh, uint32_t db) {
+// within a hop) and the prefix counts, a wave per list.  An index's first call waits for
+// it.  Lists of up to kPackHeld labels are read once, held in registers while their
+// labels are ranked hop by hop, and stored from LDS in whole lines.  First calls on
+// R-MAT 262,144 (672 labels per list) 1,275 -> 950 us, on 65,536 at K = 3 / 5 118 / 157 ->
+// 98 / 123, against a wave per list that read it twice and stored label by label (a copy
+// in the index's own order: 520, 70 and 120).
+constexpr uint32_t kPackRegs = 16, kPackHeld = kPackRegs * kWave;
+struct PackArgs {
+  uint32_t n, K;
+  const unsigned long long *off, *lab;
+  uint32_t *out, *hcnt;
+  uint32_t hsh, db;
+  __device__ uint32_t word(unsigned long long l) const {
+    return (label_hub(l) << hsh) | (label_hop(l) << db) | label_dist(l);
+  }
+};
+__global__ void __launch_bounds__(kQThreads) k_pack_short(PackArgs a) {
+  __shared__ uint32_t sorted[kQWaves][kPackHeld];
   const uint32_t lane = (uint32_t)lane_id();
-  const unsigned long long lt_mask = (1ull << lane) - 1ull;
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const uint32_t nwaves = (gridDim.x * blockDim.x) / kWave;
-  for (uint32_t v = wave; v < n; v += nwaves) {
-    const unsigned long long b = off[v];
-    const uint32_t len = (uint32_t)(off[v + 1] - b);
-    uint32_t pos[kMaxK + 1];
+  const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  lds_ptr<uint32_t> T = (lds_ptr<uint32_t>)sorted[wib];
+  const uint32_t wave = blockIdx.x * kQWaves + wib, nwaves = gridDim.x * kQWaves;
+  // the extents of up to 64 lists together
+  const uint32_t per = min((uint32_t)kWave, (a.n + nwaves - 1) / nwaves);
+  for (uint64_t v0 = (uint64_t)wave * per; v0 < a.n; v0 += (uint64_t)nwaves * per) {
+    const uint32_t cnt = (uint32_t)min<uint64_t>(per, a.n - v0);
+    const uint64_t vi = v0 + min(lane, cnt - 1);
+    const unsigned long long vb = a.off[vi];
+    const uint32_t vlen = (uint32_t)min<uint64_t>(a.off[vi + 1] - vb, kInf32);
+    for (uint32_t i = 0; i < cnt; ++i) {
+      const uint32_t len = __builtin_amdgcn_readlane(vlen, i);
+      if (len > kPackHeld) continue;  // k_pack_long's
+      const unsigned long long b =
+          ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(vb >> 32), i) << 32) |
+          (uint32_t)__builtin_amdgcn_readlane((uint32_t)vb, i);
+      const unsigned long long *L = a.lab + b;
+      unsigned long long l[kPackRegs];
+      uint32_t p[kPackRegs], dst[kPackRegs];
 #pragma unroll
-    for (uint32_t x = 0; x <= kMaxK; ++x) pos[x] = 0;
-    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
-      const unsigned long long l = lab[b + min(j0 + lane, len - 1)];
-      const uint32_t hop = j0 + lane < len ? label_hop(l) : kInf32;
+      for (uint32_t r = 0; r < kPackRegs; ++r) {
+        l[r] = 0;
+        if (r * kWave < len) l[r] = L[min(r * kWave + lane, len - 1)];
+      }
 #pragma unroll
-      for (uint32_t x = 0; x <= kMaxK; ++x)
-        if (x <= K) pos[x] += (uint32_t)__popcll(__ballot(hop == x));
+      for (uint32_t r = 0; r < kPackRegs; ++r) {
+        p[r] = a.word(l[r]);
+        dst[r] = 0;
+      }
+      uint32_t run = 0, upto = 0;  // upto: lane x, labels of hop <= x
+      for (uint32_t x = 0; x <= a.K; ++x) {
+#pragma unroll
+        for (uint32_t r = 0; r < kPackRegs; ++r) {
+          if (r * kWave >= len) break;
+          const bool here = __builtin_amdgcn_ubfe(p[r], a.db, a.hsh - a.db) == x;
+          unsigned long long m = __ballot(here);
+          if (len - r * kWave < kWave) m &= (1ull << (len - r * kWave)) - 1ull;
+          if (here)
+            dst[r] = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((uint32_t)m, run));
+          run += (uint32_t)__popcll(m);
+        }
+        if (lane == x) upto = run;
+      }
+      if (lane < a.K) a.hcnt[(v0 + i) * a.K + lane] = upto;
+#pragma unroll
+      for (uint32_t r = 0; r < kPackRegs; ++r)
+        if (r * kWave + lane < len) T[dst[r]] = p[r];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (uint32_t r = 0; r < kPackRegs; ++r)
+        if (r * kWave + lane < len) a.out[b + r * kWave + lane] = T[r * kWave + lane];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    uint32_t run = 0;
+  }
+}
+
+// Longer lists: counted, then read again and scattered, kPackStep * 64 labels in
+// flight.  Lane i looks at list wave + i * waves, so that long lists, which lie
+// together, spread over the waves.  (A workgroup per list that held it in registers:
+// 1,150 us for the longer lists of R-MAT 262,144, this form 600.)
+constexpr uint32_t kPackStep = 4;
+__global__ void __launch_bounds__(kQThreads) k_pack_long(PackArgs a) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t wave = blockIdx.x * kQWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t nwaves = gridDim.x * kQWaves;
+  for (uint64_t v0 = wave; v0 < a.n; v0 += nwaves * kWave) {
+    const uint64_t vi = min<uint64_t>(v0 + lane * nwaves, a.n - 1);
+    for (unsigned long long todo =
+             __ballot(v0 + lane * nwaves < a.n &&
+                      a.off[vi + 1] - a.off[vi] > (unsigned long long)kPackHeld);
+         todo; todo &= todo - 1) {
+      const uint64_t v = v0 + (uint32_t)(__ffsll((long long)todo) - 1) * nwaves;
+      const unsigned long long b = a.off[v];
+      const uint32_t len = (uint32_t)(a.off[v + 1] - b);
+      const unsigned long long *L = a.lab + b;
+      // every label with its hop (past the end: no hop)
+      auto each = [&](auto &&use) {
+        for (uint32_t j0 = 0; j0 < len; j0 += kPackStep * kWave) {
+          unsigned long long l[kPackStep];
 #pragma unroll
-    for (uint32_t x = 0; x <= kMaxK; ++x) {
-      const uint32_t c = pos[x];
-      pos[x] = run;
-      run += c;
-      if (x < K && lane == 0) hcnt[(uint64_t)v * K + x] = run;
-    }
-    for (uint32_t j0 = 0; j0 < len; j0 += kWave) {
-      const unsigned long long l = lab[b + min(j0 + lane, len - 1)];
-      const uint32_t hop = j0 + lane < len ? label_hop(l) : kInf32;
-      uint32_t dst = 0;
+          for (uint32_t r = 0; r < kPackStep; ++r)
+            l[r] = L[min(j0 + r * kWave + lane, len - 1)];
+#pragma unroll
+          for (uint32_t r = 0; r < kPackStep; ++r)
+            if (j0 + r * kWave < len)
+              use(l[r], j0 + r * kWave + lane < len ? label_hop(l[r]) : kInf32);
+        }
+      };
+      uint32_t pos[kMaxK + 1];
+#pragma unroll
+      for (uint32_t x = 0; x <= kMaxK; ++x) pos[x] = 0;
+      each([&](unsigned long long, uint32_t hop) {
+#pragma unroll
+        for (uint32_t x = 0; x <= kMaxK; ++x)
+          if (x <= a.K) pos[x] += (uint32_t)__popcll(__ballot(hop == x));
+      });
+      uint32_t run = 0;
 #pragma unroll
       for (uint32_t x = 0; x <= kMaxK; ++x) {
-        if (x > K) continue;
-        const unsigned long long m = __ballot(hop == x);
-        if (hop == x) dst = pos[x] + (uint32_t)__popcll(m & lt_mask);
-        pos[x] += (uint32_t)__popcll(m);
+        const uint32_t c = pos[x];
+        pos[x] = run;
+        run += c;
+        if (x < a.K && lane == 0) a.hcnt[v * a.K + x] = run;
       }
-      if (hop != kInf32)
-        out[b + dst] = (label_hub(l) << hsh) | (hop << db) | label_dist(l);
+      each([&](unsigned long long l, uint32_t hop) {
+        uint32_t dst = 0;
+#pragma unroll
+        for (uint32_t x = 0; x <= kMaxK; ++x) {
+          if (x > a.K) continue;
+          const unsigned long long m = __ballot(hop == x);
+          if (hop == x)
+            dst = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                            __builtin_amdgcn_mbcnt_lo((uint32_t)m, pos[x]));
+          pos[x] += (uint32_t)__popcll(m);
+        }
+        if (hop != kInf32) a.out[b + dst] = a.word(l);
+      });
     }
   }
 }
@@ -511,10 +604,16 @@ static int ensure_query32(const hsdl_index *idx, hipStream_t st) {
     return HSDL_OK;
   }
   const uint32_t grid = (uint32_t)std::min<uint64_t>(4096, idx->n / kQWaves + 1ull);
-  hipLaunchKernelGGL(k_pack_query32, dim3(grid), dim3(256), 0, st, idx->n, (uint32_t)idx->K,
-                     idx->off.as<unsigned long long>(), idx->lab.as<unsigned long long>(),
-                     idx->lab32.as<uint32_t>(), idx->lab32.as<uint32_t>() + idx->total, pb + db,
-                     db);
+  const PackArgs a{idx->n,
+                   (uint32_t)idx->K,
+                   idx->off.as<unsigned long long>(),
+                   idx->lab.as<unsigned long long>(),
+                   idx->lab32.as<uint32_t>(),
+                   idx->lab32.as<uint32_t>() + idx->total,
+                   pb + db,
+                   db};
+  hipLaunchKernelGGL(k_pack_short, dim3(grid), dim3(kQThreads), 0, st, a);
+  hipLaunchKernelGGL(k_pack_long, dim3(grid), dim3(kQThreads), 0, st, a);
   HSDL_HIP(hipGetLastError());
   // queries on other streams may read the copy as soon as it is marked made
   HSDL_HIP(hipStreamSynchronize(st));

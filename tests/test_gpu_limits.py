@@ -509,3 +509,34 @@ def test_resort_of_long_lists(monkeypatch, long_lists, stream32, held, default, 
     assert in_lds <= held or ((lens > held) & (lens <= in_lds)).any()
     for batch in (600, 0):
         same_labels(H.hop_constrained_two_hop_labels_generation(g, 3, hub_batch=batch), want)
+
+
+def test_query_copy_of_lists_of_every_length():
+    """The query copy holds lists of up to 1,024 labels in a wave's registers, 64 at a time,
+    and reads longer ones twice: empty lists, lists around every 64th length up to
+    1,100 and far longer ones, with hops up to 15, queried through the copy: the oracle's
+    answers."""
+    rng = np.random.default_rng(5)
+    lens = sorted({0, 1, 2, 62, 63, 64, 1022, 1023, 1024, 1025, 1100, 3000, 5001} |
+                  {64 * i + d for i in range(1, 17) for d in (-1, 0, 1)})
+    base, K = 6000, 15
+    rows = [(np.zeros(0, int),) * 3 for _ in range(base)]  # no labels, not even their own
+    for m in lens:
+        u = np.sort(rng.choice(base, m, replace=False))
+        rows.append((u, rng.integers(1, K + 1, m), rng.integers(1, 900, m)))
+    n = len(rows)
+    off = np.concatenate([[0], np.cumsum([len(x[0]) for x in rows])]).astype(np.uint64)
+    hub, hop, dist = (np.concatenate([x[i] for x in rows]) for i in range(3))
+    a = (off, hub.astype(np.uint32), hop.astype(np.uint8), dist.astype(np.int32))
+    want = O.labels_from_arrays(n, off.astype(np.int64), *a[1:])
+    idx = H.Index.from_labels(n, K, *a)
+    s, t = (x.ravel().astype(np.uint32) for x in np.meshgrid(np.arange(base, n), np.arange(base, n)))
+    for kk in (1, 2, 7, 16, 30):
+        k = np.full(len(s), kk, np.int8)
+        print(f"[copy] lists={n - base} queries={len(s)} k={kk}", flush=True)
+        os.environ["HSDL_QUERY32"] = "1"
+        try:
+            got = idx.query(s, t, k)
+        finally:
+            del os.environ["HSDL_QUERY32"]
+        assert np.array_equal(got, O.query(want, s, t, k))
