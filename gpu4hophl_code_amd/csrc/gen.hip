@@ -2065,7 +2065,7 @@ template <class V, class LT>
 __global__ void __launch_bounds__(kPruneThreads) __attribute__((amdgpu_waves_per_eu(8)))
 k_prune_rows(GenArgs a) {
   with_batch(a);
-  extern __shared__ uint32_t lds[];
+  extern __shared__ __align__(16) uint32_t lds[];
   __shared__ uint32_t sh_b, sh_k, sh_kn, sh_q, sh_next, sh_rows;
   __shared__ uint32_t sh_nf, sh_acc, sh_touch, sh_acc_base, sh_touch_base;
   __shared__ unsigned long long sh_reads;
