@@ -116,7 +116,7 @@ struct Ctrl {
   uint32_t row_ctr[8];  // next row item of each XCD's queue
   uint32_t wave_items;  // hub slots the list prune takes a wave each
   // the running batch attempt (k_set_batch): the kernels take these instead
-  // of their arguments' s0 / B / tag, so one captured batch replays for any
+  // of their arguments' s0 / B / tag, so one graph of a batch replays for any
   uint32_t bs0, bB, btag;
   uint32_t lm_on;                // the landmark test runs in this batch
   unsigned long long lm_tested;  // (label, edge) pairs the landmark test looked at
@@ -2753,12 +2753,12 @@ struct Gen {
   size_t lds_bytes = 0;
   bool small_vals = false;  // 16-bit tile values
   uint32_t bmax = 1;        // largest batch (slot rows)
-  // captured batch sequences (without / with the row-item prune) and the
-  // buffers each was captured with
+  // graphs of the batch sequence (without / with the row-item prune) and the
+  // buffers each was made with
   bool use_graph = false;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   GenArgs gkey[2]{};
-  uint64_t graph_captures = 0;
+  uint64_t graphs_made = 0;
   hipStream_t st = nullptr;
   bool verbose = false;
   // kernel timing (events around every expand and prune launch of a batch)
@@ -2914,25 +2914,50 @@ static int alloc_lists(Gen &g, uint32_t ccap, uint32_t fcap) {
   return HSDL_OK;
 }
 
-// Enqueues one batch (K rounds) of hubs [s0, s0+B).
-// The launches of one batch attempt (its K rounds) on g.st.  The kernels
-// read the batch's s0 / B / tag from the control block (k_set_batch), so the
-// sequence depends only on the buffers, K and whether row items may run.
-static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows) {
+// Takes a batch's kernels: launches them on a stream, or adds them to a graph, each
+// after the one before.  (Not by capturing the stream: while a stream is captured, HIP
+// refuses other threads' calls on the legacy stream, their builds among them.)
+struct Sequence {
+  hipStream_t st;
+  hipGraph_t graph;  // null: launch
+  hipGraphNode_t last = nullptr;
+  hipError_t err = hipSuccess;
+  void add(void (*kern)(GenArgs), uint32_t blocks, uint32_t threads, size_t lds, GenArgs a) {
+    if (!graph) {
+      hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), lds, st, a);
+      return;
+    }
+    void *args[] = {&a};
+    hipKernelNodeParams p{};
+    p.func = reinterpret_cast<void *>(kern);
+    p.gridDim = dim3(blocks);
+    p.blockDim = dim3(threads);
+    p.sharedMemBytes = (uint32_t)lds;
+    p.kernelParams = args;
+    hipGraphNode_t node = nullptr;
+    if (err == hipSuccess) err = hipGraphAddKernelNode(&node, graph, &last, last ? 1 : 0, &p);
+    last = node;
+  }
+};
+
+// The kernels of one batch attempt (its K rounds).  They read the batch's s0 / B /
+// tag from the control block (k_set_batch), so the sequence depends only on the
+// buffers, K and whether row items may run.
+static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows, Sequence &seq) {
   a.cur = 0;
   a.h = 1;
   // grid-stride loops over the batch's hubs: sized for the largest batch
   const int small_grid = (int)std::min<uint32_t>((g.bmax + 255) / 256, 1024);
-  hipLaunchKernelGGL(k_batch_begin, dim3(small_grid), dim3(256), 0, g.st, a);
+  seq.add(k_batch_begin, small_grid, 256, 0, a);
   for (uint32_t h = 1; h <= K; ++h) {
     a.h = h;
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 0], g.st);
-    hipLaunchKernelGGL(k_expand, dim3(g.grid), dim3(256), 0, g.st, a);
-    hipLaunchKernelGGL(k_expand_heavy, dim3(g.grid), dim3(256), 0, g.st, a);
+    seq.add(k_expand, g.grid, 256, 0, a);
+    seq.add(k_expand_heavy, g.grid, 256, 0, a);
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 1], g.st);
-    hipLaunchKernelGGL(k_count, dim3(g.grid), dim3(kGroupThreads), 0, g.st, a);
-    hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(1024), 0, g.st, a);
-    hipLaunchKernelGGL(k_group, dim3(g.grid), dim3(kGroupThreads), 0, g.st, a);
+    seq.add(k_count, g.grid, kGroupThreads, 0, a);
+    seq.add(k_chunk_scan, 1, 1024, 0, a);
+    seq.add(k_group, g.grid, kGroupThreads, 0, a);
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 2], g.st);
     {
       // 16- or 32-bit tile values; 32- or 64-bit labels streamed
@@ -2940,7 +2965,7 @@ static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows) {
                                          : k_prune<uint16_t, unsigned long long>)
                              : (a.pool32 ? k_prune<uint32_t, uint32_t>
                                          : k_prune<uint32_t, unsigned long long>);
-      hipLaunchKernelGGL(kp, dim3(g.prune_grid), dim3(kPruneThreads), g.lds_bytes, g.st, a);
+      seq.add(kp, g.prune_grid, kPruneThreads, g.lds_bytes, a);
       // row items instead, when k_chunk_scan chose them (one of the two
       // launches returns at once); never for a one-hub batch unless forced,
       // so the plain form pays no second launch per round
@@ -2949,17 +2974,17 @@ static void launch_rounds(Gen &g, GenArgs a, uint32_t K, bool rows) {
                                            : k_prune_rows<uint16_t, unsigned long long>)
                                : (a.pool32 ? k_prune_rows<uint32_t, uint32_t>
                                            : k_prune_rows<uint32_t, unsigned long long>);
-        hipLaunchKernelGGL(kr, dim3(g.prune_grid), dim3(kPruneThreads), g.lds_bytes, g.st, a);
+        seq.add(kr, g.prune_grid, kPruneThreads, g.lds_bytes, a);
       }
     }
     if (g.timing) (void)hipEventRecord(g.ev[4 * (h - 1) + 3], g.st);
-    hipLaunchKernelGGL(k_reserve, dim3(g.grid), dim3(256), 0, g.st, a);
-    hipLaunchKernelGGL(k_append, dim3(g.grid), dim3(256), 0, g.st, a);
+    seq.add(k_reserve, g.grid, 256, 0, a);
+    seq.add(k_append, g.grid, 256, 0, a);
     a.cur ^= 1;
   }
 }
 
-// The buffers a captured batch has baked in (they change when one grows).
+// The buffers a batch's graph has baked in (they change when one grows).
 static bool same_buffers(const GenArgs &x, const GenArgs &y) {
   return x.pool == y.pool && x.pool_cap == y.pool_cap && x.pool32 == y.pool32 &&
          x.gtile == y.gtile && x.gtile_cap == y.gtile_cap && x.cflat == y.cflat &&
@@ -2967,9 +2992,9 @@ static bool same_buffers(const GenArgs &x, const GenArgs &y) {
          x.fpos == y.fpos && x.fcap == y.fcap && x.lm == y.lm;
 }
 
-// Captures the batch sequence (with or without the row-item prune) into a
-// HIP graph, once per buffer state; false when capture is not possible here
-// (the batch then runs as separate launches).
+// Makes a HIP graph of the batch sequence (with or without the row-item prune), once
+// per buffer state; false when that is not possible here (the batch then runs as
+// separate launches).
 static bool batch_graph(Gen &g, uint32_t K, bool rows) {
   const int v = rows ? 1 : 0;
   if (g.gexec[v] && same_buffers(g.gkey[v], g.a)) return true;
@@ -2978,24 +3003,24 @@ static bool batch_graph(Gen &g, uint32_t K, bool rows) {
     g.gexec[v] = nullptr;
   }
   hipGraph_t graph = nullptr;
-  if (hipStreamBeginCapture(g.st, hipStreamCaptureModeRelaxed) != hipSuccess) {
+  if (hipGraphCreate(&graph, 0) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  launch_rounds(g, g.a, K, rows);
-  const hipError_t e = hipStreamEndCapture(g.st, &graph);
+  Sequence seq{g.st, graph};
+  launch_rounds(g, g.a, K, rows, seq);
   hipGraphExec_t ex = nullptr;
-  const bool ok = e == hipSuccess && graph &&
+  const bool ok = seq.err == hipSuccess &&
                   hipGraphInstantiate(&ex, graph, nullptr, nullptr, 0) == hipSuccess;
-  if (graph) (void)hipGraphDestroy(graph);
+  (void)hipGraphDestroy(graph);
   if (!ok) {
     (void)hipGetLastError();
-    if (g.verbose) fprintf(stderr, "[hsdl] batch graph capture failed; separate launches\n");
+    if (g.verbose) fprintf(stderr, "[hsdl] no batch graph; separate launches\n");
     return false;
   }
   g.gexec[v] = ex;
   g.gkey[v] = g.a;
-  ++g.graph_captures;
+  ++g.graphs_made;
   return true;
 }
 
@@ -3011,7 +3036,8 @@ static int enqueue_batch(Gen &g, uint32_t s0, uint32_t B, uint32_t K, uint32_t n
   if (g.use_graph && !g.timing && batch_graph(g, K, rows)) {
     HSDL_HIP(hipGraphLaunch(g.gexec[rows ? 1 : 0], g.st));
   } else {
-    launch_rounds(g, g.a, K, rows);
+    Sequence seq{g.st, nullptr};
+    launch_rounds(g, g.a, K, rows, seq);
   }
   HSDL_HIP(hipGetLastError());
   return HSDL_OK;
@@ -3703,11 +3729,11 @@ int generate(const hsdl_graph *hg, uint8_t K, const hsdl_opts *opts, const uint3
   idx->stats.t_parents_s = (t_end - t_sorted) * 1e-9;
   if (g.verbose)
     fprintf(stderr, "[hsdl] generate: %.3f s set-up, %.3f s batches (%llu, %llu redo; host enqueue "
-            "%.3f s, wait %.3f s, grow %.3f s; %llu graph captures), %.3f s export (%.3f s sort), "
+            "%.3f s, wait %.3f s, grow %.3f s; %llu graphs made), %.3f s export (%.3f s sort), "
             "%llu labels\n",
             (t_loop - t_csr) * 1e-9, (t_gen - t_loop) * 1e-9, (unsigned long long)batches,
             (unsigned long long)redos,
-            g.h_enqueue, g.h_wait, g.h_grow, (unsigned long long)g.graph_captures,
+            g.h_enqueue, g.h_wait, g.h_grow, (unsigned long long)g.graphs_made,
             (t_end - t_gen) * 1e-9, (t_end - t_sort0) * 1e-9, (unsigned long long)total);
   mg->hint_ccap = g.a.ccap;
   mg->hint_fcap = g.a.fcap;

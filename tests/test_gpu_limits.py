@@ -540,3 +540,41 @@ def test_query_copy_of_lists_of_every_length():
         finally:
             del os.environ["HSDL_QUERY32"]
         assert np.array_equal(got, O.query(want, s, t, k))
+
+
+def test_builds_on_several_threads():
+    """Eight threads build, clean, query and extract paths on graphs of their own at the
+    same time, with the kept buffers released in between: no call is refused for what
+    another thread does, and all answers are the oracle's."""
+    from concurrent.futures import ThreadPoolExecutor
+    sets = []
+    for i in range(4):
+        n, K = 700 + 400 * i, 3 + i % 3
+        c = csr_of(ragged(n, 50 + i, 50))
+        red = O.kround_gid(c, K, (np.arange(n) % 3).astype(np.int32))
+        sets.append((n, K, O.kround(c, K), red, O.clean(red)))
+
+    def work(j):
+        n, K, want, red, cleaned = sets[j % 4]
+        rng = np.random.default_rng(j)
+        g = ragged(n, 50 + j % 4, 50)
+        for r in range(6):
+            idx = H.hop_constrained_two_hop_labels_generation(g, K, parents=True)
+            same_labels(idx, want.arrays())
+            s, t = rng.integers(0, n, (2, 3000)).astype(np.uint32)
+            k = rng.integers(0, K + 3, 3000).astype(np.int8)
+            assert np.array_equal(idx.query(s, t, k), O.query(want, s, t, k))
+            edges, counts = idx.paths(s, t, k, cap=K)
+            wedges, wcounts = O.paths(want, s, t, k.astype(np.int32), K)
+            assert np.array_equal(counts.astype(np.int32), wcounts)
+            assert np.array_equal(edges.astype(np.int32), wedges)
+            off, hub, hop, dist = red.arrays()
+            idx = H.Index.from_labels(n, K, off.astype(np.uint64), hub.astype(np.uint32),
+                                      hop.astype(np.uint8), dist.astype(np.int32))
+            same_labels(H.hop_constrained_clean_L(idx), cleaned.arrays())
+            if r == 3:
+                H.release_scratch()
+        return True
+
+    with ThreadPoolExecutor(8) as pool:
+        assert all(pool.map(work, range(16)))
